@@ -221,8 +221,8 @@ struct aq_unet {
                      const float* G, int gs, int go, const __bf16* X, int xs, int xo, float* dX,
                      int dxs, int dxo) {
       const int ci = kConvs[l].cin, co = kConvs[l].cout;
-      relu_bwd(Vn, co, Y, ys, yo, G, gs, go, true, dypre, bpart, kRedBlocks, grads + boff[l], stream);
-      conv3_wgrad(ci, co, v, dypre, X, xs, xo, wpart, kNSplit, grads + woff[l], stream);
+      relu_bwd(Vn, co, Y, ys, yo, G, gs, go, dypre, stream);
+      conv3_wgrad(ci, co, v, dypre, X, xs, xo, wpart, bpart, kNSplit, grads + woff[l], grads + boff[l], stream);
       if (dX) conv3_dgrad(ci, co, v, dypre, Wt[l], dX, dxs, dxo, stream);
     };
     head_bwd(V1, kHeadC, b5, params + head_w, gy, g16a, bpart, kRedBlocks, grads + head_w, stream);

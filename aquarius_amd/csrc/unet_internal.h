@@ -15,9 +15,9 @@ void conv3_forward(int cin, int cout, const Vol& v, const __bf16* X, int xs, int
 void conv3_dgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* Wt, float* dX,
                  int dxs, int dxo, hipStream_t s);
 void conv3_wgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* X, int xs, int xo,
-                 float* part, int nsplit, float* dW, hipStream_t s);
+                 float* part, float* bpart, int nsplit, float* dW, float* db, hipStream_t s);
 void relu_bwd(long long V, int C, const __bf16* Y, int ys, int yo, const float* dY, int dys, int dyo,
-              bool relu, __bf16* dYpre, float* bpart, int nblk, float* dbias, hipStream_t s);
+              __bf16* dYpre, hipStream_t s);
 void avgpool(const Vol& vo, int C, const __bf16* X, int xs, int xo, __bf16* Y, hipStream_t s);
 void avgpool_bwd(const Vol& vo, int C, const float* dY, float* dX, int dxs, int dxo, hipStream_t s);
 void upsample(const Vol& vi, int C, const __bf16* X, __bf16* Y, int ys, int yo, hipStream_t s);

@@ -333,160 +333,277 @@ void conv3_dgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16
 
 // ------------------------------------------------------------------ weight gradient
 // dW[n, tap, c] = sum_v dYpre[v, n] * X[v + off(tap), c]: per tap an MFMA GEMM
-// (COUT x CIN) with K = voxels. A block owns one tap and a range of W-rows; for
-// each row it stages dYpre and the tap-shifted X row into LDS transposed
-// (channel-major, voxel contiguous), so a lane's 8 consecutive k (voxels) are one
-// aligned 16-byte LDS read. Partial sums per block go to `part`
-// [split][tap][COUT][CIN] and are folded in a fixed order by k_fold_wgrad.
-constexpr int kWgRow = 64;  // max W handled by the row staging (rows padded to 64)
+// (COUT x CIN) with K = voxels, one w row of up to RW voxels at a time. The rows are
+// dealt round-robin to `nsplit` splits; a one-wave block owns a split, one (dd, dh)
+// pair of taps and 16*NTB input channels, and keeps the three dw taps' accumulators
+// over all its rows. Both operands have K as their strided dimension (channels-last),
+// so a row is staged in LDS as it lies in memory -- 16-byte pieces, one zero voxel
+// either side -- and read transposed (ds_read_b64_tr_b16: lane i of 16 receives element
+// i of four consecutive voxels); a dw shift is then an address offset, and one staged X
+// row serves three taps. The next row's pieces are loaded into registers while the
+// current one is multiplied. Partial sums go to `part` [split][tap][COUT][CIN] and are
+// folded in split order by k_fold_wgrad.
+// Bound by LDS reads (1 KB per MFMA when COUT = 16). 8 x 64^3 (the training batch),
+// 48 -> 16: 5,880 -> 228 us, 16 -> 16: 1,878 -> 132 us, 96 -> 32 at 32^3: 3,166 -> 113 us
+// against one tap per block with 2-byte transposing LDS stores.
+constexpr int kWgRow = 64;  // longest row the staging holds
 
-template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void k_conv3_wgrad(Vol v, const __bf16* __restrict__ dY,
-                                                     const __bf16* __restrict__ X, int xs, int xo,
-                                                     float* __restrict__ part, int nsplit) {
-  constexpr int CINP = CIN < 16 ? 16 : CIN;  // N tiles of 16 (first layer has 8 channels)
-  constexpr int MT = COUT / 16, NTL = CINP / 16, TILES = MT * NTL;
-  constexpr int TPW = (TILES + 3) / 4;  // tiles per wave
-  __shared__ __align__(16) __bf16 sDY[COUT][kWgRow];
-  __shared__ __align__(16) __bf16 sX[CINP][kWgRow];
-  const int split = blockIdx.x, tap = blockIdx.y;
-  const int dd = tap / 9 - 1, dh = (tap / 3) % 3 - 1, dw = tap % 3 - 1;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r = lane & 15, q = lane >> 4;
-  const long long nrows = (long long)v.B * v.D * v.H;
-  f32x4 acc[TPW];
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// Eight consecutive k (rows of the LDS tile, `stride` bf16 apart) of column lane % 16,
+// for lane group q = lane / 16: the MFMA operand layout. p: the tile's first row and
+// column; lane i of a group addresses row i / 4, columns 4 (i % 4) .. +3.
+__device__ __forceinline__ bf16x8 lds_read_k8(const __bf16* p, int stride, int lane) {
+  const __bf16* a = p + (8 * (lane >> 4) + ((lane & 15) >> 2)) * stride + 4 * (lane & 3);
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)a);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(a + 4 * stride));
+  return __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+// LDS row stride for C channels: 64 channels are padded so that the four voxels a lane
+// group reads at once fall in distinct banks.
+constexpr int wg_stride(int C) { return C == 64 ? 80 : C; }
+
+template <int CIN, int COUT, int NTB, int RW>
+__global__ __launch_bounds__(64) void k_conv3_wgrad(Vol v, const __bf16* __restrict__ dY,
+                                                    const __bf16* __restrict__ X, int xs, int xo,
+                                                    float* __restrict__ part, int nsplit) {
+  constexpr int MT = COUT / 16, KCH = RW / 32;
+  constexpr int XC = 16 * NTB;                          // staged input channels
+  constexpr int XP = (CIN < 16 ? CIN : XC) / 8;         // 16-byte pieces per voxel
+  constexpr int XST = wg_stride(XC), YST = wg_stride(COUT);
+  constexpr int NX = (RW * XP + 63) / 64, NY = RW * (COUT / 8) / 64;  // pieces per lane
+  static_assert(NY * 64 == RW * (COUT / 8), "whole pieces per lane");
+  __shared__ __align__(16) __bf16 sX[(RW + 2) * XST];
+  __shared__ __align__(16) __bf16 sY[RW * YST];
+  const int lane = threadIdx.x, r = lane & 15, q = lane >> 4;
+  const int split = xcd_block();  // neighbouring splits hold neighbouring rows: one XCD
+  const int dd = (int)blockIdx.y / 3 - 1, dh = (int)blockIdx.y % 3 - 1;
+  const int c0 = (int)blockIdx.z * XC;
+  const bf16x8 zero8 = {};
+  for (int e = lane; e < (RW + 2) * XST / 8; e += 64) *(bf16x8*)&sX[e * 8] = zero8;
+  for (int e = lane; e < RW * YST / 8; e += 64) *(bf16x8*)&sY[e * 8] = zero8;
+  f32x4 acc[3][MT][NTB];
 #pragma unroll
-  for (int i = 0; i < TPW; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int kch = (v.W + 31) / 32;
-  for (long long row = split; row < nrows; row += nsplit) {
-    const int h = (int)(row % v.H);
-    const long long t = row / v.H;
-    const int d = (int)(t % v.D), b = (int)(t / v.D);
+  for (int t = 0; t < 3; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int n = 0; n < NTB; ++n) acc[t][m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int nrows = v.B * v.D * v.H;  // rows of at least 4 voxels: fits 32 bits with the tensors in memory
+  bf16x8 rx[NX], ry[NY];
+  auto load = [&](int row) {
+    const int h = row % v.H, t = row / v.H;
+    const int d = t % v.D, b = t / v.D;
     const int sd = d + dd, sh = h + dh;
-    const bool rowok = sd >= 0 && sd < v.D && sh >= 0 && sh < v.H;
-    __syncthreads();
-    for (int e = threadIdx.x; e < COUT * kWgRow; e += 256) {
-      const int w = e / COUT, n = e - w * COUT;
-      __bf16 val = f2bf(0.f);
-      if (w < v.W) val = dY[vox_id(v, b, d, h, w) * COUT + n];
-      sDY[n][w] = val;
+    const bool ok = sd >= 0 && sd < v.D && sh >= 0 && sh < v.H;
+    const __bf16* py = dY + vox_id(v, b, d, h, 0) * COUT;
+    const __bf16* px = X + vox_id(v, b, ok ? sd : d, ok ? sh : h, 0) * xs + xo + c0;
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int e = i * 64 + lane, w = e / XP, j = e - w * XP;
+      rx[i] = ok && w < v.W ? *(const bf16x8*)(px + (long long)w * xs + j * 8) : zero8;
     }
-    for (int e = threadIdx.x; e < CINP * kWgRow; e += 256) {
-      const int w = e / CINP, c = e - w * CINP;
-      __bf16 val = f2bf(0.f);
-      const int sw = w + dw;
-      if (rowok && c < CIN && w < v.W && sw >= 0 && sw < v.W)
-        val = X[vox_id(v, b, sd, sh, sw) * xs + xo + c];
-      sX[c][w] = val;
+#pragma unroll
+    for (int i = 0; i < NY; ++i) {
+      const int e = i * 64 + lane, w = e / (COUT / 8);
+      ry[i] = w < v.W ? *(const bf16x8*)(py + e * 8) : zero8;
     }
+  };
+  load(split);
+  const int kch = (v.W + 31) / 32;
+  for (int row = split; row < nrows; row += nsplit) {
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const int tile = wave + 4 * i;
-      if (tile >= TILES) break;
-      const int mt = tile / NTL, nt = tile - mt * NTL;
-      for (int kc = 0; kc < kch; ++kc) {
-        const bf16x8 a = *(const bf16x8*)&sDY[mt * 16 + r][kc * 32 + q * 8];
-        const bf16x8 bw = *(const bf16x8*)&sX[nt * 16 + r][kc * 32 + q * 8];
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw, acc[i], 0, 0, 0);
-      }
+    for (int i = 0; i < NX; ++i) {
+      const int e = i * 64 + lane, w = e / XP, j = e - w * XP;
+      if (NX * 64 == RW * XP || w < RW) *(bf16x8*)&sX[(w + 1) * XST + j * 8] = rx[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NY; ++i) {
+      const int e = i * 64 + lane, w = e / (COUT / 8), j = e - w * (COUT / 8);
+      *(bf16x8*)&sY[w * YST + j * 8] = ry[i];
+    }
+    __syncthreads();
+    if (row + nsplit < nrows) load(row + nsplit);
+#pragma unroll
+    for (int kc = 0; kc < KCH; ++kc) {
+      if (kc >= kch) break;
+      bf16x8 a[MT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) a[m] = lds_read_k8(&sY[kc * 32 * YST + m * 16], YST, lane);
+#pragma unroll
+      for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int n = 0; n < NTB; ++n) {
+          bf16x8 x = lds_read_k8(&sX[(kc * 32 + t) * XST + n * 16], XST, lane);
+          // voxel W is outside: its dw = -1 source, voxel W - 1, is not (dY is 0 there,
+          // but 0 times an infinity is not)
+          if (t == 0 && v.W - kc * 32 < 32) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+              if (kc * 32 + q * 8 + j == v.W) x[j] = f2bf(0.f);
+          }
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            acc[t][m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], x, acc[t][m][n], 0, 0, 0);
+        }
     }
   }
 #pragma unroll
-  for (int i = 0; i < TPW; ++i) {
-    const int tile = wave + 4 * i;
-    if (tile >= TILES) break;
-    const int mt = tile / NTL, nt = tile - mt * NTL;
-    const int c = nt * 16 + r;
-    if (c >= CIN) continue;
+  for (int t = 0; t < 3; ++t)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = mt * 16 + q * 4 + j;
-      part[(((long long)split * 27 + tap) * COUT + n) * CIN + c] = acc[i][j];
+    for (int n = 0; n < NTB; ++n) {
+      const int c = c0 + n * 16 + r;
+      if (c >= CIN) continue;
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          part[(((long long)split * 27 + blockIdx.y * 3 + t) * COUT + m * 16 + q * 4 + j) * CIN + c] = acc[t][m][n][j];
     }
-  }
 }
 
-// dW[n][tap*CIN + c] = sum over splits (fixed order) of part[split][tap][n][c].
-__global__ void k_fold_wgrad(const float* __restrict__ part, int nsplit, int cin, int cout,
-                             float* __restrict__ dW) {
-  const long long total = 27LL * cout * cin;
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= total) return;
-  const int c = (int)(e % cin);
-  const long long t2 = e / cin;
-  const int n = (int)(t2 % cout);
-  const int tap = (int)(t2 / cout);
-  float s = 0.f;
-  for (int sp = 0; sp < nsplit; ++sp) s += part[(((long long)sp * 27 + tap) * cout + n) * cin + c];
-  dW[(long long)n * 27 * cin + tap * cin + c] = s;
-}
-
-template <int CIN, int COUT>
-static void wgrad_t(const Vol& v, const __bf16* dY, const __bf16* X, int xs, int xo, float* part,
-                    int nsplit, float* dW, hipStream_t s) {
-  hipLaunchKernelGGL((k_conv3_wgrad<CIN, COUT>), dim3(nsplit, 27), dim3(256), 0, s, v, dY, X, xs, xo, part, nsplit);
-  const long long total = 27LL * CIN * COUT;
-  hipLaunchKernelGGL(k_fold_wgrad, dim3((int)((total + 255) / 256)), dim3(256), 0, s, part, nsplit, CIN, COUT, dW);
-}
-
-void conv3_wgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* X, int xs, int xo,
-                 float* part, int nsplit, float* dW, hipStream_t s) {
-#define AQU_WG(CI, CO) \
-  if (cin == CI && cout == CO) return wgrad_t<CI, CO>(v, dY, X, xs, xo, part, nsplit, dW, s);
-  AQU_WG(8, 16) AQU_WG(16, 16) AQU_WG(16, 32) AQU_WG(32, 32) AQU_WG(32, 64) AQU_WG(64, 64)
-  AQU_WG(96, 32) AQU_WG(48, 16)
-#undef AQU_WG
-}
-
-// ------------------------------------------------------------------ ReLU backward + bias gradient
-// dYpre = dY * (Y > 0) as bf16 (dense, C channels), and per-block per-channel sums
-// of dYpre (bias gradient partials, folded by k_fold_rows). Thread t works on
-// channel t % C, so each channel's partial is summed in a fixed order.
-__global__ void k_relu_bwd(long long V, int C, const __bf16* __restrict__ Y, int ysd, int yo,
-                           const float* __restrict__ dY, int dys, int dyo, bool relu,
-                           __bf16* __restrict__ dYpre, float* __restrict__ bpart, int vox_per_block) {
+// Bias gradient partials: per-block sums of dYpre over vox_per_block voxels. A channel's
+// voxels are dealt to 256 / C slots, each summed in voxel order by one thread (two
+// channels per thread, kBiasAhead loads in flight), then the slots in order.
+constexpr int kBiasBlocks = 512, kBiasAhead = 16;
+__global__ __launch_bounds__(128) void k_bias_part(long long V, int C, const __bf16* __restrict__ dYpre,
+                                                   float* __restrict__ bpart, int vox_per_block) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   __shared__ float red[256];
-  const int c = threadIdx.x % C;
-  const int lanesPerC = 256 / C;
-  const int slot = threadIdx.x / C;
-  float acc = 0.f;
+  const int C2 = C / 2, slots = 256 / C;
+  const int slot = (int)threadIdx.x / C2, c = ((int)threadIdx.x - slot * C2) * 2;
   const long long v0 = (long long)blockIdx.x * vox_per_block;
-  if (slot < lanesPerC) {
-    for (int i = slot; i < vox_per_block; i += lanesPerC) {
-      const long long vv = v0 + i;
-      if (vv >= V) break;
-      float g = dY[vv * dys + dyo + c];
-      if (relu && !(bf2f(Y[vv * ysd + yo + c]) > 0.f)) g = 0.f;
-      const __bf16 gb = f2bf(g);
-      dYpre[vv * C + c] = gb;
-      acc += bf2f(gb);
-    }
+  const int nv = (int)std::max<long long>(0, std::min<long long>(vox_per_block, V - v0));
+  const __bf16* p = dYpre + v0 * C + c;
+  float a0 = 0.f, a1 = 0.f;
+  int i = slot;
+  for (; i + (kBiasAhead - 1) * slots < nv; i += kBiasAhead * slots) {
+    bf16x2 t[kBiasAhead];
+#pragma unroll
+    for (int k = 0; k < kBiasAhead; ++k) t[k] = *(const bf16x2*)(p + (long long)(i + k * slots) * C);
+#pragma unroll
+    for (int k = 0; k < kBiasAhead; ++k) a0 += bf2f(t[k][0]), a1 += bf2f(t[k][1]);
   }
-  red[threadIdx.x] = (slot < lanesPerC) ? acc : 0.f;
+  for (; i < nv; i += slots) {
+    const bf16x2 t = *(const bf16x2*)(p + (long long)i * C);
+    a0 += bf2f(t[0]), a1 += bf2f(t[1]);
+  }
+  red[slot * C + c] = a0;
+  red[slot * C + c + 1] = a1;
   __syncthreads();
-  if (threadIdx.x < C) {
+  if ((int)threadIdx.x < C) {
     float s = 0.f;
-    for (int k = 0; k < lanesPerC; ++k) s += red[k * C + threadIdx.x];
+    for (int k = 0; k < slots; ++k) s += red[k * C + threadIdx.x];
     bpart[(long long)blockIdx.x * C + threadIdx.x] = s;
   }
 }
 
-// out[c] = sum over rows (fixed order) of part[row][c].
-__global__ void k_fold_rows(const float* __restrict__ part, int rows, int C, float* __restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= C) return;
+// dW[n][tap*CIN + c] = sum over splits (in order) of part[split][tap][n][c], and the bias
+// gradient db[n] likewise of bpart[block][n]. The loads of kFoldAhead rows are in
+// flight together; the sums stay in row order.
+constexpr int kFoldAhead = 32;
+__global__ __launch_bounds__(64) void k_fold_wgrad(const float* __restrict__ part, const float* __restrict__ bpart,
+                                                   int nsplit, int cin, int cout, float* __restrict__ dW,
+                                                   float* __restrict__ db) {
+  const int total = 27 * cout * cin;
+  const int e = blockIdx.x * 64 + threadIdx.x;
+  if (e >= total + cout) return;
+  const bool isw = e < total;
+  const float* p = isw ? part + e : bpart + (e - total);
+  const long long stride = isw ? total : cout;
+  const int rows = isw ? nsplit : kBiasBlocks;
   float s = 0.f;
-  for (int r = 0; r < rows; ++r) s += part[(long long)r * C + c];
-  out[c] = s;
+  int sp = 0;
+  for (; sp + kFoldAhead <= rows; sp += kFoldAhead) {
+    float t[kFoldAhead];
+#pragma unroll
+    for (int k = 0; k < kFoldAhead; ++k) t[k] = p[(sp + k) * stride];
+#pragma unroll
+    for (int k = 0; k < kFoldAhead; ++k) s += t[k];
+  }
+  for (; sp < rows; ++sp) s += p[sp * stride];
+  if (!isw) {
+    db[e - total] = s;
+    return;
+  }
+  const int c = e % cin, t2 = e / cin;
+  const int n = t2 % cout, tap = t2 / cout;
+  dW[n * 27 * cin + tap * cin + c] = s;
+}
+
+template <int CIN, int COUT, int NTB>
+static void wgrad_t(const Vol& v, const __bf16* dY, const __bf16* X, int xs, int xo, float* part,
+                    float* bpart, int nsplit, float* dW, float* db, hipStream_t s) {
+  // a split without rows would only add zeros
+  nsplit = std::min(nsplit, v.B * v.D * v.H);
+  const dim3 grid(nsplit, 9, (CIN + 16 * NTB - 1) / (16 * NTB));
+  if (v.W > 32)
+    hipLaunchKernelGGL((k_conv3_wgrad<CIN, COUT, NTB, 64>), grid, dim3(64), 0, s, v, dY, X, xs, xo, part, nsplit);
+  else
+    hipLaunchKernelGGL((k_conv3_wgrad<CIN, COUT, NTB, 32>), grid, dim3(64), 0, s, v, dY, X, xs, xo, part, nsplit);
+  const long long V = (long long)v.B * v.D * v.H * v.W;
+  hipLaunchKernelGGL(k_bias_part, dim3(kBiasBlocks), dim3(128), 0, s, V, COUT, dY, bpart,
+                     (int)((V + kBiasBlocks - 1) / kBiasBlocks));
+  const int total = 27 * CIN * COUT + COUT;
+  hipLaunchKernelGGL(k_fold_wgrad, dim3((total + 63) / 64), dim3(64), 0, s, part, bpart, nsplit, CIN, COUT, dW, db);
+}
+
+void conv3_wgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* X, int xs, int xo,
+                 float* part, float* bpart, int nsplit, float* dW, float* db, hipStream_t s) {
+#define AQU_WG(CI, CO, NTB) \
+  if (cin == CI && cout == CO) return wgrad_t<CI, CO, NTB>(v, dY, X, xs, xo, part, bpart, nsplit, dW, db, s);
+  AQU_WG(8, 16, 1) AQU_WG(16, 16, 1) AQU_WG(16, 32, 1) AQU_WG(32, 32, 2) AQU_WG(32, 64, 2) AQU_WG(64, 64, 2)
+  AQU_WG(96, 32, 3) AQU_WG(48, 16, 3)
+#undef AQU_WG
+}
+
+// ------------------------------------------------------------------ ReLU backward
+// dYpre = dY * (Y > 0) as bf16 (dense, C channels), 8 channels per thread.
+__global__ void k_relu_bwd(long long n8, int C8, const __bf16* __restrict__ Y, int ysd, int yo,
+                           const float* __restrict__ dY, int dys, int dyo, __bf16* __restrict__ dYpre) {
+  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n8) return;
+  const long long vv = e / C8;
+  const int c = (int)(e - vv * C8) * 8;
+  const bf16x8 y = *(const bf16x8*)(Y + vv * ysd + yo + c);
+  const f32x4 g0 = *(const f32x4*)(dY + vv * dys + dyo + c), g1 = *(const f32x4*)(dY + vv * dys + dyo + c + 4);
+  bf16x8 o;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float g = k < 4 ? g0[k & 3] : g1[k & 3];
+    o[k] = f2bf(bf2f(y[k]) > 0.f ? g : 0.f);
+  }
+  *(bf16x8*)(dYpre + e * 8) = o;
+}
+
+// out[c] = sum over rows (in order) of part[row][c], C <= 64: the rows are staged in LDS
+// kFoldRows at a time by the whole block, then thread c adds its column.
+constexpr int kFoldRows = 256;
+__global__ __launch_bounds__(256) void k_fold_rows(const float* __restrict__ part, int rows, int C,
+                                                   float* __restrict__ out) {
+  __shared__ float sp[kFoldRows * 64];
+  float s = 0.f;
+  for (int r0 = 0; r0 < rows; r0 += kFoldRows) {
+    const int nr = min(kFoldRows, rows - r0);
+    __syncthreads();
+    for (int e = threadIdx.x; e < nr * C; e += 256) sp[e] = part[(long long)r0 * C + e];
+    __syncthreads();
+    if ((int)threadIdx.x < C)
+#pragma unroll 16
+      for (int r = 0; r < nr; ++r) s += sp[r * C + threadIdx.x];
+  }
+  if ((int)threadIdx.x < C) out[threadIdx.x] = s;
 }
 
 void relu_bwd(long long V, int C, const __bf16* Y, int ys, int yo, const float* dY, int dys, int dyo,
-              bool relu, __bf16* dYpre, float* bpart, int nblk, float* dbias, hipStream_t s) {
-  const int vpb = (int)((V + nblk - 1) / nblk);
-  hipLaunchKernelGGL(k_relu_bwd, dim3(nblk), dim3(256), 0, s, V, C, Y, ys, yo, dY, dys, dyo, relu,
-                     dYpre, bpart, vpb);
-  hipLaunchKernelGGL(k_fold_rows, dim3((C + 63) / 64), dim3(64), 0, s, bpart, nblk, C, dbias);
+              __bf16* dYpre, hipStream_t s) {
+  const long long n8 = V * (C / 8);
+  hipLaunchKernelGGL(k_relu_bwd, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, s, n8, C / 8, Y, ys, yo, dY, dys,
+                     dyo, dYpre);
 }
 
 // ------------------------------------------------------------------ pooling / upsampling
@@ -635,7 +752,7 @@ void head_bwd(long long V, int C, const __bf16* X, const float* w, const float* 
               float* part, int nblk, float* dwb, hipStream_t s) {
   const int vpb = (int)((V + nblk - 1) / nblk);
   hipLaunchKernelGGL(k_head_bwd, dim3(nblk), dim3(256), 0, s, V, C, X, w, dy, dX, part, vpb);
-  hipLaunchKernelGGL(k_fold_rows, dim3(1), dim3(64), 0, s, part, nblk, C + 1, dwb);
+  hipLaunchKernelGGL(k_fold_rows, dim3(1), dim3(256), 0, s, part, nblk, C + 1, dwb);
 }
 
 // ------------------------------------------------------------------ loss

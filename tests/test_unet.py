@@ -188,6 +188,49 @@ def test_gradients_match_oracle():
     assert rel_l2(g[hw:], want[hw:]) < 5e-3
 
 
+def exact_problem(shape, seed):
+    """A network and batch whose every intermediate is exact: one-hot weights, inputs that
+    stay multiples of 1/8 below 24 through both poolings, 2^k masked voxels, integer
+    targets. Whatever bf16 rounds, it rounds from the same integers on both sides."""
+    rng = np.random.default_rng(seed)
+    blocks, hw, hb, total = U.layout()
+    p = np.zeros(total)
+    for (w, b), (ci, co) in zip(blocks, U.CONVS):
+        k = np.zeros((co, 27, ci))
+        real = 2 if ci == 8 else ci
+        for o, c in enumerate(np.concatenate([rng.permutation(real) for _ in range(-(-co // real))])[:co]):
+            k[o, rng.choice([4, 10, 12, 13, 13, 13, 14, 16, 22]), c] = 1
+        p[w:w + k.size] = k.ravel()
+    p[hw:hw + 16] = rng.choice([-2, -1, 1, 2], 16)
+    vox = int(np.prod(shape))
+    m = np.zeros(vox)
+    m[rng.choice(vox, 1 << (vox.bit_length() - 2), replace=False)] = 1
+    m = m.reshape(shape)
+    x = np.stack([8.0 * rng.integers(0, 4, shape) * m, m], -1)
+    return p, x, rng.integers(-8, 9, shape) * m, m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 4, 4, 4), (2, 4, 8, 36), (1, 8, 4, 60), (1, 4, 12, 28), (3, 4, 4, 64)])
+def test_gradients_at_row_lengths(shape):
+    """Weight and bias gradients where the staged w rows are shorter than, as long as, or
+    a remainder of the kernel's row, and where a level has fewer rows than splits. All
+    values are exact (exact_problem) and the sums stay far below 2^24, so only the last
+    division by the mask count and the FP32 export round."""
+    from aquarius_amd.unet import UNet
+    p, x, t, m = exact_problem(shape, seed=8)
+    net = UNet()
+    net.set_params(p)
+    _, g = net.gradients(x, t, m)
+    _, want = U.loss_and_grads(p, x, t, m, bf=True)
+    blocks, hw, hb, total = U.layout()
+    for l, ((w, b), (ci, co)) in enumerate(zip(blocks, U.CONVS)):
+        assert np.any(want[w:b]) and np.any(want[b:b + co]), l
+        assert np.linalg.norm(g[w:b] - want[w:b]) <= 1e-6 * np.linalg.norm(want[w:b]), l
+        assert np.linalg.norm(g[b:b + co] - want[b:b + co]) <= 1e-6 * np.linalg.norm(want[b:b + co]), l
+    assert rel_l2(g[hw:], want[hw:]) <= 1e-6
+
+
 @pytest.mark.gpu
 def test_gradient_descent_on_gpu_gradients_reduces_loss():
     """Plain gradient descent driven by the GPU gradients (host-tensor path) lowers
