@@ -73,10 +73,10 @@ struct aq_unet {
   long long capV = 0;  // voxels at level 1 (B*D*H*W)
   __bf16 *x0 = nullptr, *a1 = nullptr, *cat1 = nullptr, *p1 = nullptr, *a2 = nullptr,
          *cat2 = nullptr, *p2 = nullptr, *a3 = nullptr, *b3 = nullptr, *a4 = nullptr,
-         *b4 = nullptr, *a5 = nullptr, *b5 = nullptr, *dypre = nullptr;
-  float *y = nullptr, *gy = nullptr, *g16a = nullptr, *g16b = nullptr, *gcat1 = nullptr,
-        *g32a = nullptr, *g32b = nullptr, *gcat2 = nullptr, *g64a = nullptr, *g64b = nullptr,
-        *gp1 = nullptr, *gp2 = nullptr, *target = nullptr, *mask = nullptr;
+         *b4 = nullptr, *a5 = nullptr, *b5 = nullptr;
+  __bf16* dy[2] = {};  // dYpre of the layer in hand and of the one below it
+  float *y = nullptr, *gy = nullptr, *gs1 = nullptr, *gs2 = nullptr, *gp1 = nullptr, *gp2 = nullptr,
+        *target = nullptr, *mask = nullptr;
   float *wpart = nullptr, *bpart = nullptr;
   double *lpart = nullptr, *lout = nullptr, *sig = nullptr;
   std::vector<void*> act_allocs;
@@ -162,17 +162,12 @@ struct aq_unet {
     UTRY(alloc(&b4, V2 * 32, L));
     UTRY(alloc(&a5, V * 16, L));
     UTRY(alloc(&b5, V * 16, L));
-    UTRY(alloc(&dypre, V * 64, L));
+    UTRY(alloc(&dy[0], V * 16, L));
+    UTRY(alloc(&dy[1], V * 16, L));
     UTRY(alloc(&y, V, L));
     UTRY(alloc(&gy, V, L));
-    UTRY(alloc(&g16a, V * 16, L));
-    UTRY(alloc(&g16b, V * 16, L));
-    UTRY(alloc(&gcat1, V * 48, L));
-    UTRY(alloc(&g32a, V2 * 32, L));
-    UTRY(alloc(&g32b, V2 * 32, L));
-    UTRY(alloc(&gcat2, V2 * 96, L));
-    UTRY(alloc(&g64a, V3 * 64, L));
-    UTRY(alloc(&g64b, V3 * 64, L));
+    UTRY(alloc(&gs1, V * 16, L));
+    UTRY(alloc(&gs2, V2 * 32, L));
     UTRY(alloc(&gp1, V2 * 16, L));
     UTRY(alloc(&gp2, V3 * 32, L));
     UTRY(alloc(&target, V, L));
@@ -192,7 +187,7 @@ struct aq_unet {
     const Vol v2{v1.B, v1.D / 2, v1.H / 2, v1.W / 2}, v3{v1.B, v1.D / 4, v1.H / 4, v1.W / 4};
     auto conv = [&](int l, const Vol& v, const __bf16* X, int xs, int xo, __bf16* Y, int ys, int yo) {
       conv3_forward(kConvs[l].cin, kConvs[l].cout, v, X, xs, xo, Wk[l], params + boff[l], Y, ys, yo,
-                    true, stream);
+                    stream);
     };
     conv(0, v1, x0, 8, 0, a1, 16, 0);
     conv(1, v1, a1, 16, 0, cat1, 48, 0);
@@ -212,34 +207,41 @@ struct aq_unet {
     head_fwd(V, kHeadC, b5, params + head_w, params + head_b, y, stream);
   }
 
-  // Backward pass from gy (dL/dy) into grads (every parameter overwritten).
+  // Backward pass from gy (dL/dy) into grads (every parameter overwritten). dYpre (the
+  // gradient at a layer's output through its ReLU, bf16) alternates between dy[0] and
+  // dy[1]; every input-gradient convolution writes the next layer's directly.
   void backward(const Vol& v1) {
     const Vol v2{v1.B, v1.D / 2, v1.H / 2, v1.W / 2}, v3{v1.B, v1.D / 4, v1.H / 4, v1.W / 4};
-    const long long V1 = (long long)v1.B * v1.D * v1.H * v1.W, V2 = V1 / 8, V3 = V1 / 64;
-    // layer l: output Y (stride ys, offset yo) with gradient G (stride gs, offset go), input X.
-    auto layer = [&](int l, const Vol& v, long long Vn, const __bf16* Y, int ys, int yo,
-                     const float* G, int gs, int go, const __bf16* X, int xs, int xo, float* dX,
-                     int dxs, int dxo) {
-      const int ci = kConvs[l].cin, co = kConvs[l].cout;
-      relu_bwd(Vn, co, Y, ys, yo, G, gs, go, dypre, stream);
-      conv3_wgrad(ci, co, v, dypre, X, xs, xo, wpart, bpart, kNSplit, grads + woff[l], grads + boff[l], stream);
-      if (dX) conv3_dgrad(ci, co, v, dypre, Wt[l], dX, dxs, dxo, stream);
+    const long long V1 = (long long)v1.B * v1.D * v1.H * v1.W;
+    auto wgrad = [&](int l, const Vol& v, int k, const __bf16* X, int xs) {
+      conv3_wgrad(kConvs[l].cin, kConvs[l].cout, v, dy[k], X, xs, 0, wpart, bpart, kNSplit, grads + woff[l],
+                  grads + boff[l], stream);
     };
-    head_bwd(V1, kHeadC, b5, params + head_w, gy, g16a, bpart, kRedBlocks, grads + head_w, stream);
-    layer(9, v1, V1, b5, 16, 0, g16a, 16, 0, a5, 16, 0, g16b, 16, 0);        // c5b
-    layer(8, v1, V1, a5, 16, 0, g16b, 16, 0, cat1, 48, 0, gcat1, 48, 0);    // c5a
-    upsample_bwd(v2, 32, gcat1, 48, 16, g32a, stream);                       // -> d b4
-    layer(7, v2, V2, b4, 32, 0, g32a, 32, 0, a4, 32, 0, g32b, 32, 0);        // c4b
-    layer(6, v2, V2, a4, 32, 0, g32b, 32, 0, cat2, 96, 0, gcat2, 96, 0);    // c4a
-    upsample_bwd(v3, 64, gcat2, 96, 32, g64a, stream);                       // -> d b3
-    layer(5, v3, V3, b3, 64, 0, g64a, 64, 0, a3, 64, 0, g64b, 64, 0);        // c3b
-    layer(4, v3, V3, a3, 64, 0, g64b, 64, 0, p2, 32, 0, gp2, 32, 0);        // c3a
-    avgpool_bwd(v3, 32, gp2, gcat2, 96, 0, stream);                          // += d s2
-    layer(3, v2, V2, cat2, 96, 0, gcat2, 96, 0, a2, 32, 0, g32a, 32, 0);    // c2b
-    layer(2, v2, V2, a2, 32, 0, g32a, 32, 0, p1, 16, 0, gp1, 16, 0);        // c2a
-    avgpool_bwd(v2, 16, gp1, gcat1, 48, 0, stream);                          // += d s1
-    layer(1, v1, V1, cat1, 48, 0, gcat1, 48, 0, a1, 16, 0, g16a, 16, 0);    // c1b
-    layer(0, v1, V1, a1, 16, 0, g16a, 16, 0, x0, 8, 0, nullptr, 0, 0);      // c1a
+    auto dgrad_relu = [&](int l, const Vol& v, int k, const __bf16* M, int ms) {
+      conv3_dgrad_relu(kConvs[l].cin, v, dy[k], Wt[l], M, ms, 0, dy[k ^ 1], stream);
+    };
+    head_bwd(V1, b5, params + head_w, gy, dy[0], bpart, kRedBlocks, grads + head_w, stream);
+    wgrad(9, v1, 0, a5, 16);                                                   // c5b
+    dgrad_relu(9, v1, 0, a5, 16);
+    wgrad(8, v1, 1, cat1, 48);                                                 // c5a
+    conv3_dgrad_concat(48, 16, v1, dy[1], Wt[8], gs1, b4, dy[0], stream);      // -> skip 1, c4b
+    wgrad(7, v2, 0, a4, 32);                                                   // c4b
+    dgrad_relu(7, v2, 0, a4, 32);
+    wgrad(6, v2, 1, cat2, 96);                                                 // c4a
+    conv3_dgrad_concat(96, 32, v2, dy[1], Wt[6], gs2, b3, dy[0], stream);      // -> skip 2, c3b
+    wgrad(5, v3, 0, a3, 64);                                                   // c3b
+    dgrad_relu(5, v3, 0, a3, 64);
+    wgrad(4, v3, 1, p2, 32);                                                   // c3a
+    conv3_dgrad(32, 64, v3, dy[1], Wt[4], gp2, stream);
+    skip_bwd(v2, 32, cat2, 96, gs2, gp2, dy[0], stream);
+    wgrad(3, v2, 0, a2, 32);                                                   // c2b
+    dgrad_relu(3, v2, 0, a2, 32);
+    wgrad(2, v2, 1, p1, 16);                                                   // c2a
+    conv3_dgrad(16, 32, v2, dy[1], Wt[2], gp1, stream);
+    skip_bwd(v1, 16, cat1, 48, gs1, gp1, dy[0], stream);
+    wgrad(1, v1, 0, a1, 16);                                                   // c1b
+    dgrad_relu(1, v1, 0, a1, 16);
+    wgrad(0, v1, 1, x0, 8);                                                    // c1a
   }
 
   void adam_step() {
@@ -317,8 +319,8 @@ aq_status nn_infer(const aqf::FlipView& fv, aq_unet* net, const float* src, floa
 }
 
 aq_status upload_input(aq_unet* net, const float* x, long long V) {
-  // x (V*2 floats) -> x0 (bf16, 8 channels) through a staging copy in `y`/`gy`
-  float* stage = net->g16b;  // V*16 floats of scratch, enough for V*2
+  // x (V*2 floats) -> x0 (bf16, 8 channels) through a staging copy
+  float* stage = net->gs1;  // V*16 floats of scratch, enough for V*2
   UHIP(hipMemcpyAsync(stage, x, V * 2 * sizeof(float), hipMemcpyHostToDevice, net->stream));
   host_input(V, stage, net->x0, net->stream);
   return AQ_OK;

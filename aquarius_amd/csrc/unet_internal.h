@@ -11,20 +11,21 @@ struct Vol {
 };
 
 void conv3_forward(int cin, int cout, const Vol& v, const __bf16* X, int xs, int xo, const __bf16* Wk,
-                   const float* bias, __bf16* Y, int ys, int yo, bool relu, hipStream_t s);
-void conv3_dgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* Wt, float* dX,
-                 int dxs, int dxo, hipStream_t s);
+                   const float* bias, __bf16* Y, int ys, int yo, hipStream_t s);
+void conv3_dgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* Wt, float* dX, hipStream_t s);
+void conv3_dgrad_relu(int c, const Vol& v, const __bf16* dY, const __bf16* Wt, const __bf16* M, int ms, int mo,
+                      __bf16* dYpre, hipStream_t s);
+void conv3_dgrad_concat(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* Wt, float* skip,
+                        const __bf16* M, __bf16* up, hipStream_t s);
 void conv3_wgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* X, int xs, int xo,
                  float* part, float* bpart, int nsplit, float* dW, float* db, hipStream_t s);
-void relu_bwd(long long V, int C, const __bf16* Y, int ys, int yo, const float* dY, int dys, int dyo,
-              __bf16* dYpre, hipStream_t s);
+void skip_bwd(const Vol& v, int C, const __bf16* Y, int ys, const float* dS, const float* dP, __bf16* dYpre,
+              hipStream_t s);
 void avgpool(const Vol& vo, int C, const __bf16* X, int xs, int xo, __bf16* Y, hipStream_t s);
-void avgpool_bwd(const Vol& vo, int C, const float* dY, float* dX, int dxs, int dxo, hipStream_t s);
 void upsample(const Vol& vi, int C, const __bf16* X, __bf16* Y, int ys, int yo, hipStream_t s);
-void upsample_bwd(const Vol& vi, int C, const float* dY, int dys, int dyo, float* dX, hipStream_t s);
 void head_fwd(long long V, int C, const __bf16* X, const float* w, const float* b, float* y, hipStream_t s);
-void head_bwd(long long V, int C, const __bf16* X, const float* w, const float* dy, float* dX,
-              float* part, int nblk, float* dwb, hipStream_t s);
+void head_bwd(long long V, const __bf16* X, const float* w, const float* dy, __bf16* dYpre, float* part,
+              int nblk, float* dwb, hipStream_t s);
 void masked_mse(long long V, const float* y, const float* t, const float* m, double* part, int nblk,
                 double* out, float* dy, hipStream_t s);
 void adam(long long n, float* w, const float* g, float* m, float* v, float lr_t, float b1, float b2,

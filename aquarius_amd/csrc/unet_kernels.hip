@@ -20,7 +20,9 @@
 namespace aqu {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kXCD = 8;
 
@@ -52,283 +54,375 @@ __device__ __forceinline__ long long vox_id(const Vol& v, int b, int d, int h, i
 }
 
 // ------------------------------------------------------------------ conv 3x3x3, implicit GEMM
-// Y[v, n] = sum_{tap, c} X[v + off(tap), c] * Wk[n, tap*CIN + c] (+ bias, ReLU),
-// zero padding outside the volume. M = voxels, N = COUT, K = 27*CIN in slices of
-// 32. A wave owns kConvMF fragments of 16 consecutive voxels, so every weight
-// fragment it fetches feeds kConvMF MFMAs and the fragments' input gathers are in
-// flight together. When the layer's weights fit (<= 64 KiB) the block stages them
-// in LDS once, rows padded by 16 bytes so the 16 rows a wave reads fall in
-// distinct banks. With flipped, transposed weights the same kernel computes the
-// input gradient. OUT_F32 writes FP32 (optionally accumulating), else bf16.
-// AQUNET_NO_TILE=1 switches the LDS-tiled forward convolution off (measurements and
-// the tiled-against-untiled test); read at every launch.
+// Y[v, n] = sum_{tap, c} X[v + off(tap), c] * Wk[n, tap*CIN + c], zero padding outside
+// the volume. M = voxels, N = COUT, K = 27*CIN in slices of 32.
+//
+// k_conv3 gathers its input per tap from memory, one fragment of 16 voxels and one
+// 16-channel output tile per wave: the reference for k_conv3_tile's forward pass, run
+// only under AQUNET_NO_TILE=1 (read at every launch).
 static bool conv3_tile_enabled() {
   const char* e = std::getenv("AQUNET_NO_TILE");
   return !(e && e[0] == '1');
 }
 
-constexpr int kConvMF = 4;
-constexpr int kConvVox = 4 * kConvMF * 16;  // voxels per 256-thread block
-
-// MF fragments of 16 voxels per wave; the block computes NTW 16-channel output
-// tiles, tile group blockIdx.y (NTW = COUT/16: all of them). Small grids use MF = 1,
-// NTW = 1 so that they still spread over the CUs; each output value is the same
-// MFMA chain either way.
-template <int CIN, int COUT, bool RELU, bool OUT_F32, bool ACCUM, int MF = kConvMF, int NTW = COUT / 16>
+template <int CIN, int COUT>
 __global__ __launch_bounds__(256) void k_conv3(Vol v, const __bf16* __restrict__ X, int xs, int xo,
                                                const __bf16* __restrict__ Wk,
-                                               const float* __restrict__ bias, void* __restrict__ Yv,
-                                               int ys, int yo) {
+                                               const float* __restrict__ bias, __bf16* __restrict__ Y, int ys,
+                                               int yo) {
   constexpr int K = 27 * CIN;
-  constexpr int NT = NTW;
-  constexpr int RS = K + 8;  // LDS row stride in bf16
-  constexpr bool WLDS = NT * 16 * RS * 2 <= 64 * 1024;
-  __shared__ __align__(16) __bf16 sW[WLDS ? NT * 16 * RS : 8];
-  const int n0 = (int)blockIdx.y * NT * 16;  // first output channel of this block
-  Wk += (long long)n0 * K;
-  if (bias) bias += n0;
-  if (WLDS) {
-    for (int e = threadIdx.x; e < NT * 16 * (K / 8); e += 256) {
-      const int n = e / (K / 8), j = e - n * (K / 8);
-      *(bf16x8*)&sW[n * RS + j * 8] = *(const bf16x8*)(Wk + (long long)n * K + j * 8);
-    }
-    __syncthreads();
-  }
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const long long V = (long long)v.B * v.D * v.H * v.W;
-  const long long wbase = ((long long)xcd_block() * 4 + wave) * (MF * 16);
-  if (wbase >= V) return;
   const int r = lane & 15, q = lane >> 4;
-  VoxelPos p[MF];
-  bool vok[MF];
-#pragma unroll
-  for (int f = 0; f < MF; ++f) {
-    const long long vid = wbase + f * 16 + r;
-    vok[f] = vid < V;
-    p[f] = vox_of(v, vok[f] ? vid : 0);
-  }
-  f32x4 acc[MF][NT];
-#pragma unroll
-  for (int f = 0; f < MF; ++f)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[f][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int n = (int)blockIdx.y * 16 + r;
+  const long long V = (long long)v.B * v.D * v.H * v.W;
+  const long long wbase = ((long long)xcd_block() * 4 + wave) * 16;
+  if (wbase >= V) return;
+  const bool vok = wbase + r < V;
+  const VoxelPos p = vox_of(v, vok ? wbase + r : 0);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   const bf16x8 zero8 = {};
   for (int k0 = 0; k0 < K; k0 += 32) {
     const int k = k0 + q * 8;
     const bool kok = k < K;
     const int tap = k / CIN, c = k - tap * CIN;
-    const int dd = tap / 9 - 1, dh = (tap / 3) % 3 - 1, dw = tap % 3 - 1;
-    bf16x8 a[MF];
-#pragma unroll
-    for (int f = 0; f < MF; ++f) {
-      a[f] = zero8;
-      const int zd = p[f].d + dd, zh = p[f].h + dh, zw = p[f].w + dw;
-      if (kok && vok[f] && zd >= 0 && zd < v.D && zh >= 0 && zh < v.H && zw >= 0 && zw < v.W)
-        a[f] = *(const bf16x8*)(X + vox_id(v, p[f].b, zd, zh, zw) * xs + xo + c);
-    }
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      bf16x8 bw = zero8;
-      if (kok) {
-        if (WLDS)
-          bw = *(const bf16x8*)&sW[(t * 16 + r) * RS + k];
-        else
-          bw = *(const bf16x8*)(Wk + (long long)(t * 16 + r) * K + k);
-      }
-#pragma unroll
-      for (int f = 0; f < MF; ++f)
-        acc[f][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[f], bw, acc[f][t], 0, 0, 0);
-    }
+    const int zd = p.d + tap / 9 - 1, zh = p.h + (tap / 3) % 3 - 1, zw = p.w + tap % 3 - 1;
+    bf16x8 a = zero8;
+    if (kok && vok && zd >= 0 && zd < v.D && zh >= 0 && zh < v.H && zw >= 0 && zw < v.W)
+      a = *(const bf16x8*)(X + vox_id(v, p.b, zd, zh, zw) * xs + xo + c);
+    const bf16x8 bw = kok ? *(const bf16x8*)(Wk + (long long)n * K + k) : zero8;
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw, acc, 0, 0, 0);
   }
 #pragma unroll
-  for (int f = 0; f < MF; ++f)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int n = t * 16 + r;  // within this block's tiles
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const long long o = wbase + f * 16 + q * 4 + i;
-        if (o >= V) continue;
-        float val = acc[f][t][i];
-        if (bias) val += bias[n];
-        if (RELU) val = fmaxf(val, 0.f);
-        if (OUT_F32) {
-          float* Y = (float*)Yv + o * ys + yo + n0 + n;
-          *Y = ACCUM ? *Y + val : val;
-        } else {
-          ((__bf16*)Yv)[o * ys + yo + n0 + n] = f2bf(val);
-        }
-      }
-    }
+  for (int i = 0; i < 4; ++i) {
+    const long long o = wbase + q * 4 + i;
+    if (o < V) Y[o * ys + yo + n] = f2bf(fmaxf(acc[i] + bias[n], 0.f));
+  }
 }
 
 // ------------------------------------------------------------------ conv 3x3x3, input tile in LDS
-// The forward convolution of the layers whose extents divide into tiles: a block owns
-// an output tile of TD x 8 x 16 voxels (d, h, w) of one batch item and NTB 16-channel
-// output tiles (channel group blockIdx.y). The input tile with its one-voxel halo,
-// (TD+2) x 10 x 18 voxels, is staged in LDS CH input channels at a time (zero outside
-// the volume), so each input value is read from memory about 2.5 times per layer
-// instead of once per tap; the A fragments of all 27 taps then come from LDS. Each of
-// the four waves owns MF = 2*TD rows of 16 voxels along w. Voxels sit CH + 8 bf16
-// apart in LDS (CH when CH = 8), which puts the 16-byte reads of 8 consecutive lanes in
-// distinct banks. The k order is (chunk, tap, channel within the chunk): for CIN = CH
-// it is the order of k_conv3.
-template <int CIN, int COUT, int CH, int TD, int NTB, bool RELU>
-__global__ __launch_bounds__(256) void k_conv3_tile(Vol v, const __bf16* __restrict__ X, int xs, int xo,
-                                                    const __bf16* __restrict__ Wk,
-                                                    const float* __restrict__ bias, __bf16* __restrict__ Y,
-                                                    int ys, int yo) {
+// The convolutions of the forward pass and, with flipped transposed weights, the input
+// gradients. A block owns output tiles of TD x 8 x 16 voxels (d, h, w) of one batch item
+// and NTB 16-channel output tiles (channel group blockIdx.y). An input tile with its
+// one-voxel halo, (TD+2) x 10 x 18 voxels, is staged in LDS CH input channels at a time
+// (zero outside the volume), so each input value is read from memory about 2.5 times per
+// layer instead of once per tap; the fragments of all 27 taps then come from LDS. A
+// block walks several tiles when there are many: the next tile's (or channel chunk's)
+// pieces are loaded into registers while the current one is multiplied. Wave w owns the
+// rows h = 2w, 2w + 1 of every plane, so it holds whole 2 x 2 x 2 groups when TD = 2.
+// 8 x 64^3, before (16-bit stores, weights refetched, one tile per block; gradients by
+// gathering per tap, FP32, with separate upsampling, pooling and ReLU passes) and now:
+// forward 16 -> 16 104 -> 67 us, 32 -> 32 at 32^3 38 -> 31 us, 96 -> 32 93 -> 84 us, 48 -> 16
+// 232 -> 230 us; gradients 16 -> 16 147 + 77 -> 69 us, 48 -> 16 277 + 90 -> 169 us. The
+// fragments' LDS reads (1 KB per MFMA with one channel tile) bound the 16-channel layers.
+// The weights are the MFMA's first operand (rows = output channels): lane (r, q) then
+// holds channels 4q .. 4q + 3 of voxel r, one 8- or 16-byte store. LDS voxels sit
+// VS bf16 apart so that the 16-byte reads of 8 consecutive lanes fall in distinct banks.
+// The k order is (chunk, tap, channel within the chunk), the order of k_conv3 when
+// CH = CIN. Extents that are no multiples of the tile compute partial tiles.
+enum { kConvFwd, kConvF32, kConvMask, kConvUp };
+struct ConvOut {
+  const float* bias;  // kConvFwd: + bias, ReLU, bf16
+  void* y;            // bf16 (kConvFwd, kConvMask) or FP32 (kConvF32; kConvUp: channels below `split`)
+  int ys, yo;         // its channel stride and offset
+  const __bf16* m;    // kConvMask / kConvUp: the ReLU outputs whose sign gates the gradient
+  int ms, mo;
+  int split;          // kConvUp: first channel of the upsampled part
+  __bf16* up;         // kConvUp: gated gradient of the coarse tensor, dense
+};
+
+// Offset (in LDS bf16) of tap t from tap 0.
+template <int IH, int IW, int VS>
+__device__ constexpr int tap_off(int t) {
+  return (((t / 9) * IH + (t / 3) % 3) * IW + t % 3) * VS;
+}
+
+// Waves per SIMD the registers must allow: what the tile's LDS leaves room for, at most 3
+// (four 16-channel variants spill at 128 registers).
+constexpr int conv_waves(int CH, int TD) {
+  const int n = 160 * 1024 / ((TD + 2) * 180 * (CH <= 16 ? CH : CH + 8) * 2);
+  return CH == 48 ? 1 : CH >= 32 && n > 2 ? 2 : n > 3 ? 3 : n;
+}
+
+template <int CIN, int COUT, int CH, int TD, int NTB, int EPI>
+__global__ __launch_bounds__(256, conv_waves(CH, TD)) void k_conv3_tile(Vol v, int ntiles, const __bf16* __restrict__ X, int xs, int xo,
+                                                    const __bf16* __restrict__ Wk, ConvOut out) {
   constexpr int TH = 8, TW = 16;
   constexpr int ID = TD + 2, IH = TH + 2, IW = TW + 2;
   constexpr int NV = ID * IH * IW;
-  constexpr int VS = CH == 8 ? 8 : CH + 8;  // LDS voxel stride (bf16)
-  constexpr int MF = TD * TH / 4;           // 16-voxel rows per wave
-  constexpr int KC = 27 * CH;               // k per channel chunk
-  constexpr int NSL = (KC + 31) / 32;
+  constexpr int VS = CH <= 16 ? CH : CH + 8;     // LDS voxel stride (bf16)
+  constexpr int MF = 2 * TD;                      // 16-voxel rows per wave
+  constexpr int NSL = (27 * CH + 31) / 32;        // k slices per chunk
+  constexpr int NC = CIN / CH;
   constexpr int K = 27 * CIN;
-  static_assert(CIN % CH == 0 && CH % 8 == 0, "channel chunks of 8, 16 or 32");
+  constexpr int PV = CH / 8;                      // 16-byte pieces per voxel
+  constexpr int NP = (NV * PV + 255) / 256;       // pieces per thread
+  constexpr int TPS = CH >= 32 ? 1 : 32 / CH;     // taps per slice
+  static_assert(CIN % CH == 0 && CH % 8 == 0 && (CH < 32 ? 32 % CH == 0 : CH % 32 == 0 || CH == 48), "channel chunks");
   __shared__ __align__(16) __bf16 sX[NV * VS];
-  const int ntw = v.W / TW, nth = v.H / TH, ntd = v.D / TD;
-  int t = xcd_block();
-  const int tw = t % ntw;
-  t /= ntw;
-  const int th = t % nth;
-  t /= nth;
-  const int td = t % ntd;
-  const int b = t / ntd;
-  const int d0 = td * TD, h0 = th * TH, w0 = tw * TW;
-  const int n0 = (int)blockIdx.y * NTB * 16;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int r = lane & 15, q = lane >> 4;
-  f32x4 acc[MF][NTB];
-#pragma unroll
-  for (int f = 0; f < MF; ++f)
-#pragma unroll
-    for (int nt = 0; nt < NTB; ++nt) acc[f][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int n0 = (int)blockIdx.y * NTB * 16;
+  const int ntw = (v.W + TW - 1) / TW, nth = (v.H + TH - 1) / TH, ntd = (v.D + TD - 1) / TD;
   const bf16x8 zero8 = {};
-  for (int cc = 0; cc < CIN; cc += CH) {
-    if (cc) __syncthreads();  // every wave is done with the previous chunk
-    for (int e = threadIdx.x; e < NV * (CH / 8); e += 256) {
-      const int vx = e / (CH / 8), j = e - vx * (CH / 8);
+  struct Org {
+    int b, d0, h0, w0;
+  };
+  auto org_of = [&](int t) {
+    Org o;
+    o.w0 = (t % ntw) * TW;
+    t /= ntw;
+    o.h0 = (t % nth) * TH;
+    t /= nth;
+    o.d0 = (t % ntd) * TD;
+    o.b = t / ntd;
+    return o;
+  };
+  bf16x8 rp[NP];
+  auto load = [&](const Org& o, int cc) {
+    const __bf16* base = X + vox_id(v, o.b, o.d0 - 1, o.h0 - 1, o.w0 - 1) * xs + xo + cc;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int e = i * 256 + (int)threadIdx.x;
+      const int vx = e / PV, j = e - vx * PV;
       const int iw = vx % IW, ih = (vx / IW) % IH, id = vx / (IW * IH);
-      const int zd = d0 + id - 1, zh = h0 + ih - 1, zw = w0 + iw - 1;
-      bf16x8 val = zero8;
-      if (zd >= 0 && zd < v.D && zh >= 0 && zh < v.H && zw >= 0 && zw < v.W)
-        val = *(const bf16x8*)(X + vox_id(v, b, zd, zh, zw) * xs + xo + cc + j * 8);
-      *(bf16x8*)&sX[vx * VS + j * 8] = val;
+      const bool ok = (NP * 256 == NV * PV || e < NV * PV) && (unsigned)(o.d0 - 1 + id) < (unsigned)v.D &&
+                      (unsigned)(o.h0 - 1 + ih) < (unsigned)v.H && (unsigned)(o.w0 - 1 + iw) < (unsigned)v.W;
+      rp[i] = ok ? *(const bf16x8*)(base + (long long)((id * v.H + ih) * v.W + iw) * xs + j * 8) : zero8;
     }
-    __syncthreads();
+  };
+  // lane bases: the voxel fragment's, and the weight row's
+  const __bf16* lx = &sX[(2 * wave * IW + r) * VS + (CH >= 32 ? q : q & (PV - 1)) * 8];
+  const __bf16* lw = Wk + (long long)(n0 + r) * K +
+                     (CH >= 32 ? q * 8 : (q / PV) * CIN + (q & (PV - 1)) * 8);
+  // Layers whose weight fragments fit beside the rest keep them in registers across the
+  // block's tiles; the others read them again per tile (wofs hides the invariance).
+  constexpr bool kKeepW = NC * NSL * NTB * 4 <= (TD == 1 ? 108 : 56);
+  int wofs = 0;
+  f32x4 acc[MF][NTB];
+  auto slice = [&](int s, int cc) {
+    bf16x8 w[NTB];
+    // the slice's first tap and, for CH > 32, the channel it starts at
+    constexpr int SPT = CH > 32 ? 1 : 0;
+    const int k = s * 32;
+    const int tap = k / CH, ch = SPT ? k - tap * CH : 0;
+    int off;
+    bool ok = true;
+    if (CH == 48) {  // slices straddle taps: the lane's own
+      const int kl = k + q * 8, t = kl / CH, c = kl - t * CH;
+      ok = kl < 27 * CH;
+      off = ok ? tap_off<IH, IW, VS>(t) + c - q * 8 : 0;
+    } else if (CH >= 32) {
+      off = tap_off<IH, IW, VS>(tap) + ch;
+    } else {
+      const int last = min(tap + TPS - 1, 26);
+      off = tap_off<IH, IW, VS>(tap);
+      if (q / PV >= 1) off = tap_off<IH, IW, VS>(min(tap + 1, last));
+      if (TPS == 4) {
+        if (q == 2) off = tap_off<IH, IW, VS>(min(tap + 2, last));
+        if (q == 3) off = tap_off<IH, IW, VS>(min(tap + 3, last));
+      }
+      ok = tap + TPS <= 27 || tap + q / PV < 27;
+    }
+    const int wo = CH >= 32 ? (CH == CIN ? k : tap * CIN + cc + ch) : tap * CIN + cc;
 #pragma unroll
-    for (int s = 0; s < NSL; ++s) {
-      const int kc = s * 32 + q * 8;
-      const bool kok = kc < KC;
-      const int tap = kok ? kc / CH : 0, c = kc - tap * CH;
-      const int dd = tap / 9, dh = (tap / 3) % 3, dw = tap % 3;
-      bf16x8 bw[NTB];
+    for (int n = 0; n < NTB; ++n) {
+      const __bf16* p = lw + wofs + (long long)n * 16 * K + wo;
+      w[n] = ok ? *(const bf16x8*)p : zero8;
+    }
 #pragma unroll
-      for (int nt = 0; nt < NTB; ++nt)
-        bw[nt] = kok ? *(const bf16x8*)(Wk + (long long)(n0 + nt * 16 + r) * K + tap * CIN + cc + c) : zero8;
+    for (int f = 0; f < MF; ++f) {
+      const int fo = ((f >> 1) * IH + (f & 1)) * IW * VS;
+      bf16x8 x = *(const bf16x8*)(lx + off + fo);
+      if (!ok) x = zero8;
+#pragma unroll
+      for (int n = 0; n < NTB; ++n) acc[f][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[n], x, acc[f][n], 0, 0, 0);
+    }
+  };
+  const int nb = gridDim.x;
+  int t = xcd_block();
+  Org o = org_of(t);
+  load(o, 0);
+  for (; t < ntiles; t += nb) {
+    const Org cur = o;
+#pragma unroll
+    for (int f = 0; f < MF; ++f)
+#pragma unroll
+      for (int n = 0; n < NTB; ++n) acc[f][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ci = 0; ci < NC; ++ci) {
+      if (!kKeepW) asm volatile("" : "+s"(wofs));
+      __syncthreads();  // every wave is done with the previous chunk
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const int e = i * 256 + (int)threadIdx.x;
+        const int vx = e / PV, j = e - vx * PV;
+        if (NP * 256 == NV * PV || e < NV * PV) *(bf16x8*)&sX[vx * VS + j * 8] = rp[i];
+      }
+      __syncthreads();
+      if (ci + 1 < NC) {
+        load(cur, (ci + 1) * CH);
+      } else if (t + nb < ntiles) {
+        o = org_of(t + nb);
+        load(o, 0);
+      }
+#pragma unroll
+      for (int s = 0; s < NSL; ++s) slice(s, ci * CH);
+    }
+    const int w = cur.w0 + r;
+    if (EPI != kConvUp) {
 #pragma unroll
       for (int f = 0; f < MF; ++f) {
-        const int row = wave * MF + f;
-        const int rd = row / TH, rh = row - rd * TH;
-        const bf16x8 a =
-            kok ? *(const bf16x8*)&sX[(((rd + dd) * IH + (rh + dh)) * IW + (r + dw)) * VS + c] : zero8;
+        const int d = cur.d0 + (f >> 1), h = cur.h0 + 2 * wave + (f & 1);
+        if (d >= v.D || h >= v.H || w >= v.W) continue;
+        const long long vi = vox_id(v, cur.b, d, h, w);
 #pragma unroll
-        for (int nt = 0; nt < NTB; ++nt)
-          acc[f][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw[nt], acc[f][nt], 0, 0, 0);
+        for (int n = 0; n < NTB; ++n) {
+          const int c = n0 + n * 16 + q * 4;
+          f32x4 a = acc[f][n];
+          if (EPI == kConvF32) {
+            *(f32x4*)((float*)out.y + vi * out.ys + out.yo + c) = a;
+            continue;
+          }
+          bf16x4 y;
+          if (EPI == kConvFwd) {
+            const f32x4 bs = *(const f32x4u*)(out.bias + c);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[j] = f2bf(fmaxf(a[j] + bs[j], 0.f));
+          } else {
+            const bf16x4 m = *(const bf16x4*)(out.m + vi * out.ms + out.mo + c);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) y[j] = f2bf(bf2f(m[j]) > 0.f ? a[j] : 0.f);
+          }
+          *(bf16x4*)((__bf16*)out.y + vi * out.ys + out.yo + c) = y;
+        }
       }
-    }
-  }
+    } else {
+      // Concatenated input: the skip part is stored as it is; the upsampled part's
+      // gradient is the sum of its eight children, (d, h, w) order, this wave's 2 x 2 rows
+      // and lane pairs along w.
+      const int h = cur.h0 + 2 * wave;
+      const bool in = cur.d0 < v.D && h < v.H && w < v.W;  // extents are even: whole groups
+      const long long vi = vox_id(v, cur.b, cur.d0, h, w);
+      const Vol vc{v.B, v.D / 2, v.H / 2, v.W / 2};
+      const long long vcI = vox_id(vc, cur.b, cur.d0 >> 1, h >> 1, w >> 1);
+      const int cup = COUT - out.split;
 #pragma unroll
-  for (int f = 0; f < MF; ++f) {
-    const int row = wave * MF + f;
-    const int rd = row / TH, rh = row - rd * TH;
+      for (int n = 0; n < NTB; ++n) {
+        const int c = n0 + n * 16 + q * 4;
+        if (n0 + n * 16 < out.split) {
+          if (in)
 #pragma unroll
-    for (int nt = 0; nt < NTB; ++nt) {
-      const int n = n0 + nt * 16 + r;
+            for (int f = 0; f < MF; ++f)
+              *(f32x4*)((float*)out.y + (vi + ((long long)(f >> 1) * v.H + (f & 1)) * v.W) * out.ys + out.yo + c) = acc[f][n];
+          continue;
+        }
+        float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const long long o = vox_id(v, b, d0 + rd, h0 + rh, w0 + q * 4 + i);
-        float val = acc[f][nt][i];
-        if (bias) val += bias[n];
-        if (RELU) val = fmaxf(val, 0.f);
-        Y[o * ys + yo + n] = f2bf(val);
+        for (int f = 0; f < MF; ++f)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            s[j] += acc[f][n][j];
+            s[j] += __shfl_xor(acc[f][n][j], 1, 64);
+          }
+        if (in && !(r & 1)) {
+          const int cc = c - out.split;
+          const bf16x4 m = *(const bf16x4*)(out.m + vcI * out.ms + out.mo + cc);
+          bf16x4 y;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) y[j] = f2bf(bf2f(m[j]) > 0.f ? s[j] : 0.f);
+          *(bf16x4*)(out.up + vcI * cup + cc) = y;
+        }
       }
     }
   }
 }
 
-// Launches k_conv3_tile when the extents divide into its tiles (W % 16, H % 8 and,
-// for TD = 2, D % 2), with ReLU. Two depths TD and one or two channel tiles per
-// block, chosen so that the grid still has about 512 or more blocks.
-template <int CIN, int COUT, int CH>
-static bool conv3_tile_fwd(const Vol& v, const __bf16* X, int xs, int xo, const __bf16* Wk, const float* bias,
-                           __bf16* Y, int ys, int yo, hipStream_t s) {
-  if (v.W % 16 || v.H % 8) return false;
-  const long long tiles1 = (long long)v.B * v.D * (v.H / 8) * (v.W / 16);
-  const bool td2 = v.D % 2 == 0 && tiles1 / 2 * (COUT / 16) >= 512;
-  const long long tiles = td2 ? tiles1 / 2 : tiles1;
-  const bool ntb2 = COUT >= 32 && tiles * (COUT / 32) >= 512;
-  const dim3 grid((unsigned)tiles, ntb2 ? COUT / 32 : COUT / 16);
+// Output tiles per launch: enough blocks to fill the chip, each walking several tiles
+// when there are more (kConvBlocks: 4 blocks of 256 threads per CU).
+constexpr int kConvBlocks = 1024;
+template <int CIN, int COUT, int CH, int TD, int NTB, int EPI>
+static void conv3_tile_launch(const Vol& v, const __bf16* X, int xs, int xo, const __bf16* Wk, const ConvOut& out,
+                              hipStream_t s) {
+  const long long tiles = (long long)v.B * ((v.D + TD - 1) / TD) * ((v.H + 7) / 8) * ((v.W + 15) / 16);
+  const unsigned nb = (unsigned)std::min<long long>(tiles, std::max(8, kConvBlocks / (COUT / (16 * NTB)) / 8 * 8));
+  hipLaunchKernelGGL((k_conv3_tile<CIN, COUT, CH, TD, NTB, EPI>), dim3(nb, COUT / (16 * NTB)), dim3(256), 0, s, v,
+                     (int)tiles, X, xs, xo, Wk, out);
+}
+
+// Tile depth and channel tiles per block: two planes and two channel tiles where the
+// launch still has at least 512 blocks (two per CU), else one.
+template <int CIN, int COUT, int CH, int EPI>
+static void conv3_tile_pick(const Vol& v, const __bf16* X, int xs, int xo, const __bf16* Wk, const ConvOut& out,
+                            hipStream_t s) {
+  constexpr bool kDeep = 4 * 180 * (CH + 8) * 2 <= 80 * 1024;  // two blocks' two-plane tiles fit a CU's LDS
+  const long long tiles1 = (long long)v.B * v.D * ((v.H + 7) / 8) * ((v.W + 15) / 16);
+  const bool td2 = kDeep && v.D % 2 == 0 && tiles1 / 2 * (COUT / 16) >= 512;
+  const bool ntb2 = COUT >= 32 && (td2 ? tiles1 / 2 : tiles1) * (COUT / 32) >= 512;
+  constexpr int TD2 = kDeep ? 2 : 1, NT2 = COUT >= 32 ? 2 : 1;
   if (td2 && ntb2)
-    hipLaunchKernelGGL((k_conv3_tile<CIN, COUT, CH, 2, 2, true>), grid, dim3(256), 0, s, v, X, xs, xo, Wk, bias, Y, ys, yo);
+    conv3_tile_launch<CIN, COUT, CH, TD2, NT2, EPI>(v, X, xs, xo, Wk, out, s);
   else if (td2)
-    hipLaunchKernelGGL((k_conv3_tile<CIN, COUT, CH, 2, 1, true>), grid, dim3(256), 0, s, v, X, xs, xo, Wk, bias, Y, ys, yo);
+    conv3_tile_launch<CIN, COUT, CH, TD2, 1, EPI>(v, X, xs, xo, Wk, out, s);
   else if (ntb2)
-    hipLaunchKernelGGL((k_conv3_tile<CIN, COUT, CH, 1, 2, true>), grid, dim3(256), 0, s, v, X, xs, xo, Wk, bias, Y, ys, yo);
+    conv3_tile_launch<CIN, COUT, CH, 1, NT2, EPI>(v, X, xs, xo, Wk, out, s);
   else
-    hipLaunchKernelGGL((k_conv3_tile<CIN, COUT, CH, 1, 1, true>), grid, dim3(256), 0, s, v, X, xs, xo, Wk, bias, Y, ys, yo);
-  return true;
+    conv3_tile_launch<CIN, COUT, CH, 1, 1, EPI>(v, X, xs, xo, Wk, out, s);
 }
 
+// Layers with more than 32 input channels are staged in chunks where the extents divide
+// into tiles, and whole otherwise: the two orders of k that the forward pass has always
+// had there.
 template <int CIN, int COUT>
 static void conv3_fwd_t(const Vol& v, const __bf16* X, int xs, int xo, const __bf16* Wk,
-                        const float* bias, __bf16* Y, int ys, int yo, bool relu, hipStream_t s) {
-  constexpr int CH = CIN % 32 == 0 ? 32 : CIN % 16 == 0 ? 16 : 8;
-  if (relu && conv3_tile_enabled() && conv3_tile_fwd<CIN, COUT, CH>(v, X, xs, xo, Wk, bias, Y, ys, yo, s)) return;
-  const long long V = (long long)v.B * v.D * v.H * v.W;
-  if (V >= 1024 * (long long)kConvVox) {  // enough blocks: 4 fragments per wave, all tiles
-    const int nb = (int)((V + kConvVox - 1) / kConvVox);
-    if (relu)
-      hipLaunchKernelGGL((k_conv3<CIN, COUT, true, false, false>), dim3(nb), dim3(256), 0, s, v, X, xs, xo, Wk, bias, (void*)Y, ys, yo);
-    else
-      hipLaunchKernelGGL((k_conv3<CIN, COUT, false, false, false>), dim3(nb), dim3(256), 0, s, v, X, xs, xo, Wk, bias, (void*)Y, ys, yo);
-  } else {  // small grids: one fragment per wave, one 16-channel tile per block
-    const dim3 grid((unsigned)((V + 63) / 64), COUT / 16);
-    if (relu)
-      hipLaunchKernelGGL((k_conv3<CIN, COUT, true, false, false, 1, 1>), grid, dim3(256), 0, s, v, X, xs, xo, Wk, bias, (void*)Y, ys, yo);
-    else
-      hipLaunchKernelGGL((k_conv3<CIN, COUT, false, false, false, 1, 1>), grid, dim3(256), 0, s, v, X, xs, xo, Wk, bias, (void*)Y, ys, yo);
+                        const float* bias, __bf16* Y, int ys, int yo, hipStream_t s) {
+  constexpr int CH = CIN <= 32 ? CIN : CIN % 32 == 0 ? 32 : 16;
+  if (!conv3_tile_enabled()) {
+    const long long V = (long long)v.B * v.D * v.H * v.W;
+    hipLaunchKernelGGL((k_conv3<CIN, COUT>), dim3((unsigned)((V + 63) / 64), COUT / 16), dim3(256), 0, s, v, X, xs,
+                       xo, Wk, bias, Y, ys, yo);
+    return;
   }
-}
-template <int CIN, int COUT>
-static void conv3_dgrad_t(const Vol& v, const __bf16* dY, const __bf16* Wt, float* dX, int dxs, int dxo,
-                          hipStream_t s) {
-  // transposed problem: input dYpre has CIN (= the layer's COUT) channels, output COUT (= its CIN)
-  const long long V = (long long)v.B * v.D * v.H * v.W;
-  const int nb = (int)((V + kConvVox - 1) / kConvVox);
-  hipLaunchKernelGGL((k_conv3<CIN, COUT, false, true, false>), dim3(nb), dim3(256), 0, s, v, dY, CIN, 0, Wt, (const float*)nullptr, (void*)dX, dxs, dxo);
+  const ConvOut out{bias, Y, ys, yo, nullptr, 0, 0, 0, nullptr};
+  if (CH == CIN || (v.W % 16 == 0 && v.H % 8 == 0))
+    conv3_tile_pick<CIN, COUT, CH, kConvFwd>(v, X, xs, xo, Wk, out, s);
+  else
+    conv3_tile_pick<CIN, COUT, CIN, kConvFwd>(v, X, xs, xo, Wk, out, s);
 }
 
 void conv3_forward(int cin, int cout, const Vol& v, const __bf16* X, int xs, int xo, const __bf16* Wk,
-                   const float* bias, __bf16* Y, int ys, int yo, bool relu, hipStream_t s) {
+                   const float* bias, __bf16* Y, int ys, int yo, hipStream_t s) {
 #define AQU_FWD(CI, CO) \
-  if (cin == CI && cout == CO) return conv3_fwd_t<CI, CO>(v, X, xs, xo, Wk, bias, Y, ys, yo, relu, s);
+  if (cin == CI && cout == CO) return conv3_fwd_t<CI, CO>(v, X, xs, xo, Wk, bias, Y, ys, yo, s);
   AQU_FWD(8, 16) AQU_FWD(16, 16) AQU_FWD(16, 32) AQU_FWD(32, 32) AQU_FWD(32, 64) AQU_FWD(64, 64)
   AQU_FWD(96, 32) AQU_FWD(48, 16)
 #undef AQU_FWD
 }
 
 // Input gradient: dX[v, c] = sum_{tap, n} dYpre[v - off(tap), n] * W[n, tap, c], computed as a
-// forward convolution of dYpre (cout channels) with Wt[c, tap', n] = W[n, 26 - tap', c].
-void conv3_dgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* Wt, float* dX,
-                 int dxs, int dxo, hipStream_t s) {
-#define AQU_DG(CI, CO) \
-  if (cin == CI && cout == CO) return conv3_dgrad_t<CO, CI>(v, dY, Wt, dX, dxs, dxo, s);
-  AQU_DG(16, 16) AQU_DG(16, 32) AQU_DG(32, 32) AQU_DG(32, 64) AQU_DG(64, 64) AQU_DG(96, 32)
-  AQU_DG(48, 16)
-#undef AQU_DG
+// convolution of dYpre (cout channels) with Wt[c, tap', n] = W[n, 26 - tap', c].
+// dX in FP32 (the pooled layers, whose gradient is added to another).
+void conv3_dgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* Wt, float* dX, hipStream_t s) {
+  const ConvOut out{nullptr, dX, cin, 0, nullptr, 0, 0, 0, nullptr};
+  if (cin == 16 && cout == 32) return conv3_tile_pick<32, 16, 32, kConvF32>(v, dY, 32, 0, Wt, out, s);
+  if (cin == 32 && cout == 64) return conv3_tile_pick<64, 32, 64, kConvF32>(v, dY, 64, 0, Wt, out, s);
+}
+// The same through the ReLU whose outputs are M: dYpre of the layer below, bf16, dense.
+void conv3_dgrad_relu(int c, const Vol& v, const __bf16* dY, const __bf16* Wt, const __bf16* M, int ms, int mo,
+                      __bf16* dYpre, hipStream_t s) {
+  const ConvOut out{nullptr, dYpre, c, 0, M, ms, mo, 0, nullptr};
+  if (c == 16) return conv3_tile_pick<16, 16, 16, kConvMask>(v, dY, 16, 0, Wt, out, s);
+  if (c == 32) return conv3_tile_pick<32, 32, 32, kConvMask>(v, dY, 32, 0, Wt, out, s);
+  if (c == 64) return conv3_tile_pick<64, 64, 64, kConvMask>(v, dY, 64, 0, Wt, out, s);
+}
+// The same for a concatenated input of `cin` channels: the skip part's gradient (the first
+// cin/3 channels) in FP32, the upsampled part's through its upsampling and ReLU (outputs
+// M, dense, half extents) to dYpre of that layer.
+void conv3_dgrad_concat(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16* Wt, float* skip,
+                        const __bf16* M, __bf16* up, hipStream_t s) {
+  const int split = cin / 3;
+  const ConvOut out{nullptr, skip, split, 0, M, cin - split, 0, split, up};
+  if (cin == 48 && cout == 16) return conv3_tile_launch<16, 48, 16, 2, 3, kConvUp>(v, dY, 16, 0, Wt, out, s);
+  if (cin == 96 && cout == 32) return conv3_tile_launch<32, 96, 32, 2, 2, kConvUp>(v, dY, 32, 0, Wt, out, s);
 }
 
 // ------------------------------------------------------------------ weight gradient
@@ -561,23 +655,34 @@ void conv3_wgrad(int cin, int cout, const Vol& v, const __bf16* dY, const __bf16
 #undef AQU_WG
 }
 
-// ------------------------------------------------------------------ ReLU backward
-// dYpre = dY * (Y > 0) as bf16 (dense, C channels), 8 channels per thread.
-__global__ void k_relu_bwd(long long n8, int C8, const __bf16* __restrict__ Y, int ysd, int yo,
-                           const float* __restrict__ dY, int dys, int dyo, __bf16* __restrict__ dYpre) {
+// ------------------------------------------------------------------ skip connections backward
+// dYpre of a layer whose output goes to a skip connection (gradient dS, FP32, dense) and
+// to an average pooling (gradient dP of the pooled tensor, vo): (dS + dP / 8) * (Y > 0) as
+// bf16, 8 channels per thread.
+__global__ void k_skip_bwd(Vol v, int C8, const __bf16* __restrict__ Y, int ys, const float* __restrict__ dS,
+                           const float* __restrict__ dP, __bf16* __restrict__ dYpre) {
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n8) return;
   const long long vv = e / C8;
+  if (vv >= (long long)v.B * v.D * v.H * v.W) return;
   const int c = (int)(e - vv * C8) * 8;
-  const bf16x8 y = *(const bf16x8*)(Y + vv * ysd + yo + c);
-  const f32x4 g0 = *(const f32x4*)(dY + vv * dys + dyo + c), g1 = *(const f32x4*)(dY + vv * dys + dyo + c + 4);
+  const VoxelPos p = vox_of(v, vv);
+  const Vol vo{v.B, v.D / 2, v.H / 2, v.W / 2};
+  const float* pp = dP + vox_id(vo, p.b, p.d >> 1, p.h >> 1, p.w >> 1) * (C8 * 8) + c;
+  const bf16x8 y = *(const bf16x8*)(Y + vv * ys + c);
+  const f32x4 s0 = *(const f32x4*)(dS + e * 8), s1 = *(const f32x4*)(dS + e * 8 + 4);
+  const f32x4 p0 = *(const f32x4*)pp, p1 = *(const f32x4*)(pp + 4);
   bf16x8 o;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    const float g = k < 4 ? g0[k & 3] : g1[k & 3];
+    const float g = (k < 4 ? s0[k & 3] : s1[k & 3]) + (k < 4 ? p0[k & 3] : p1[k & 3]) * 0.125f;
     o[k] = f2bf(bf2f(y[k]) > 0.f ? g : 0.f);
   }
   *(bf16x8*)(dYpre + e * 8) = o;
+}
+void skip_bwd(const Vol& v, int C, const __bf16* Y, int ys, const float* dS, const float* dP, __bf16* dYpre,
+              hipStream_t s) {
+  const long long n8 = (long long)v.B * v.D * v.H * v.W * (C / 8);
+  hipLaunchKernelGGL(k_skip_bwd, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, s, v, C / 8, Y, ys, dS, dP, dYpre);
 }
 
 // out[c] = sum over rows (in order) of part[row][c], C <= 64: the rows are staged in LDS
@@ -599,15 +704,8 @@ __global__ __launch_bounds__(256) void k_fold_rows(const float* __restrict__ par
   if ((int)threadIdx.x < C) out[threadIdx.x] = s;
 }
 
-void relu_bwd(long long V, int C, const __bf16* Y, int ys, int yo, const float* dY, int dys, int dyo,
-              __bf16* dYpre, hipStream_t s) {
-  const long long n8 = V * (C / 8);
-  hipLaunchKernelGGL(k_relu_bwd, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, s, n8, C / 8, Y, ys, yo, dY, dys,
-                     dyo, dYpre);
-}
-
 // ------------------------------------------------------------------ pooling / upsampling
-// 2x2x2 average pooling (forward, bf16) and its adjoint (accumulating FP32).
+// 2x2x2 average pooling (bf16).
 // One thread per output voxel and 8 consecutive channels; the eight children are
 // summed in the same (d, h, w) order for every channel.
 __global__ void k_avgpool(Vol vo, int C, const __bf16* __restrict__ X, int xs, int xo,
@@ -634,23 +732,7 @@ __global__ void k_avgpool(Vol vo, int C, const __bf16* __restrict__ X, int xs, i
   for (int c = 0; c < 8; ++c) o8[c] = f2bf(acc[c] * 0.125f);
   *(bf16x8*)(Y + vox_id(vo, b, d, h, w) * C + 8 * j) = o8;
 }
-__global__ void k_avgpool_bwd(Vol vo, int C, const float* __restrict__ dY, float* __restrict__ dX,
-                              int dxs, int dxo) {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long V = (long long)vo.B * vo.D * vo.H * vo.W;
-  if (e >= V * C) return;
-  const int c = (int)(e % C);
-  const VoxelPos p = vox_of(vo, e / C);
-  const Vol vi{vo.B, vo.D * 2, vo.H * 2, vo.W * 2};
-  const float g = dY[e] * 0.125f;
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    float* o = dX + vox_id(vi, p.b, 2 * p.d + (k >> 2), 2 * p.h + ((k >> 1) & 1), 2 * p.w + (k & 1)) * dxs + dxo + c;
-    *o += g;
-  }
-}
-// Nearest 2x upsampling into a channel slice (forward) and its adjoint (sum of the
-// eight children, FP32).
+// Nearest 2x upsampling into a channel slice.
 // One thread per output voxel and 8 consecutive channels (a 16-byte load and store).
 __global__ void k_upsample(Vol vi, int C, const __bf16* __restrict__ X, __bf16* __restrict__ Y, int ys,
                            int yo, int row0) {
@@ -668,21 +750,6 @@ __global__ void k_upsample(Vol vi, int C, const __bf16* __restrict__ X, __bf16* 
   const long long i = vox_id(vi, b, d >> 1, h >> 1, w >> 1);
   *(bf16x8*)(Y + o * ys + yo + 8 * j) = *(const bf16x8*)(X + i * C + 8 * j);
 }
-__global__ void k_upsample_bwd(Vol vi, int C, const float* __restrict__ dY, int dys, int dyo,
-                               float* __restrict__ dX) {
-  const Vol vo{vi.B, vi.D * 2, vi.H * 2, vi.W * 2};
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long V = (long long)vi.B * vi.D * vi.H * vi.W;
-  if (e >= V * C) return;
-  const int c = (int)(e % C);
-  const VoxelPos p = vox_of(vi, e / C);
-  float s = 0.f;
-#pragma unroll
-  for (int k = 0; k < 8; ++k)
-    s += dY[vox_id(vo, p.b, 2 * p.d + (k >> 2), 2 * p.h + ((k >> 1) & 1), 2 * p.w + (k & 1)) * dys + dyo + c];
-  dX[e] = s;
-}
-
 static inline int nb1(long long n) { return (int)((n + 255) / 256); }
 void avgpool(const Vol& vo, int C, const __bf16* X, int xs, int xo, __bf16* Y, hipStream_t s) {
   const int rows = vo.B * vo.D * vo.H;
@@ -691,20 +758,12 @@ void avgpool(const Vol& vo, int C, const __bf16* X, int xs, int xo, __bf16* Y, h
     hipLaunchKernelGGL(k_avgpool, grid, dim3(256), 0, s, vo, C, X, xs, xo, Y, r0);
   }
 }
-void avgpool_bwd(const Vol& vo, int C, const float* dY, float* dX, int dxs, int dxo, hipStream_t s) {
-  const long long n = (long long)vo.B * vo.D * vo.H * vo.W * C;
-  hipLaunchKernelGGL(k_avgpool_bwd, dim3(nb1(n)), dim3(256), 0, s, vo, C, dY, dX, dxs, dxo);
-}
 void upsample(const Vol& vi, int C, const __bf16* X, __bf16* Y, int ys, int yo, hipStream_t s) {
   const int rows = vi.B * vi.D * 2 * vi.H * 2;
   for (int r0 = 0; r0 < rows; r0 += 65535) {  // grid.y limit
     const dim3 grid((unsigned)((vi.W * 2 * (C / 8) + 255) / 256), (unsigned)std::min(65535, rows - r0));
     hipLaunchKernelGGL(k_upsample, grid, dim3(256), 0, s, vi, C, X, Y, ys, yo, r0);
   }
-}
-void upsample_bwd(const Vol& vi, int C, const float* dY, int dys, int dyo, float* dX, hipStream_t s) {
-  const long long n = (long long)vi.B * vi.D * vi.H * vi.W * C;
-  hipLaunchKernelGGL(k_upsample_bwd, dim3(nb1(n)), dim3(256), 0, s, vi, C, dY, dys, dyo, dX);
 }
 
 // ------------------------------------------------------------------ output head (1x1x1, C -> 1)
@@ -720,38 +779,56 @@ __global__ void k_head(long long V, int C, const __bf16* __restrict__ X, const f
   }
   y[i] = s;
 }
-__global__ void k_head_bwd(long long V, int C, const __bf16* __restrict__ X, const float* __restrict__ w,
-                           const float* __restrict__ dy, float* __restrict__ dX, float* __restrict__ part,
-                           int vpb) {
-  __shared__ float red[256 * 17];
-  float acc[17];
+// Head backward: dYpre of the layer below, dy * w through its ReLU (outputs X) as bf16,
+// and per-block partial sums of the head's own gradient: dy * X per channel and dy.
+template <int C>
+__global__ __launch_bounds__(256) void k_head_bwd(long long V, const __bf16* __restrict__ X,
+                                                  const float* __restrict__ w, const float* __restrict__ dy,
+                                                  __bf16* __restrict__ dYpre, float* __restrict__ part, int vpb) {
+  constexpr int RS = 257;  // rows of one channel's partials, one bank apart
+  __shared__ float red[(C + 1) * RS];
+  float acc[C + 1], wc[C];
+#pragma unroll
   for (int c = 0; c <= C; ++c) acc[c] = 0.f;
+#pragma unroll
+  for (int c = 0; c < C; ++c) wc[c] = w[c];
   const long long v0 = (long long)blockIdx.x * vpb;
   for (int i = threadIdx.x; i < vpb; i += 256) {
     const long long vv = v0 + i;
     if (vv >= V) break;
     const float g = dy[vv];
-    for (int c = 0; c < C; ++c) {
-      dX[vv * C + c] = g * w[c];
-      acc[c] += g * bf2f(X[vv * C + c]);
+#pragma unroll
+    for (int c0 = 0; c0 < C; c0 += 8) {
+      const bf16x8 x8 = *(const bf16x8*)(X + vv * C + c0);
+      bf16x8 o;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        const float x = bf2f(x8[c]);
+        o[c] = f2bf(x > 0.f ? g * wc[c0 + c] : 0.f);
+        acc[c0 + c] += g * x;
+      }
+      *(bf16x8*)(dYpre + vv * C + c0) = o;
     }
     acc[C] += g;
   }
-  for (int c = 0; c <= C; ++c) red[c * 256 + threadIdx.x] = acc[c];
+#pragma unroll
+  for (int c = 0; c <= C; ++c) red[c * RS + threadIdx.x] = acc[c];
   __syncthreads();
   if ((int)threadIdx.x <= C) {
     float s = 0.f;
-    for (int k = 0; k < 256; ++k) s += red[threadIdx.x * 256 + k];
+#pragma unroll 16
+    for (int k = 0; k < 256; ++k) s += red[threadIdx.x * RS + k];
     part[(long long)blockIdx.x * (C + 1) + threadIdx.x] = s;
   }
 }
 void head_fwd(long long V, int C, const __bf16* X, const float* w, const float* b, float* y, hipStream_t s) {
   hipLaunchKernelGGL(k_head, dim3(nb1(V)), dim3(256), 0, s, V, C, X, w, b, y);
 }
-void head_bwd(long long V, int C, const __bf16* X, const float* w, const float* dy, float* dX,
-              float* part, int nblk, float* dwb, hipStream_t s) {
+void head_bwd(long long V, const __bf16* X, const float* w, const float* dy, __bf16* dYpre, float* part,
+              int nblk, float* dwb, hipStream_t s) {
+  constexpr int C = 16;
   const int vpb = (int)((V + nblk - 1) / nblk);
-  hipLaunchKernelGGL(k_head_bwd, dim3(nblk), dim3(256), 0, s, V, C, X, w, dy, dX, part, vpb);
+  hipLaunchKernelGGL(k_head_bwd<C>, dim3(nblk), dim3(256), 0, s, V, X, w, dy, dYpre, part, vpb);
   hipLaunchKernelGGL(k_fold_rows, dim3(1), dim3(256), 0, s, part, nblk, C + 1, dwb);
 }
 
@@ -786,15 +863,26 @@ __global__ void k_loss_partial(long long V, const float* __restrict__ y, const f
     part[2 * blockIdx.x + 1] = s2[0];
   }
 }
-__global__ void k_loss_fold(const double* __restrict__ part, int n, double* __restrict__ out) {
-  if (threadIdx.x != 0) return;
-  double a = 0, c = 0;
-  for (int i = 0; i < n; ++i) {
-    a += part[2 * i];
-    c += part[2 * i + 1];
+// The partials are staged in LDS by the whole block; one thread per column adds them in
+// order (from memory, one dependent load per term took 36 us).
+__global__ __launch_bounds__(256) void k_loss_fold(const double* __restrict__ part, int n, double* __restrict__ out) {
+  __shared__ double sp[2048], tot[2];
+  double s = 0;
+  for (int i0 = 0; i0 < n; i0 += 1024) {
+    const int m = min(1024, n - i0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2 * m; i += 256) sp[i] = part[2 * i0 + i];
+    __syncthreads();
+    if (threadIdx.x < 2)
+#pragma unroll 8
+      for (int i = 0; i < m; ++i) s += sp[2 * i + threadIdx.x];
   }
-  out[0] = c > 0 ? a / c : 0.0;
-  out[1] = c;
+  if (threadIdx.x < 2) tot[threadIdx.x] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    out[0] = tot[1] > 0 ? tot[0] / tot[1] : 0.0;
+    out[1] = tot[1];
+  }
 }
 __global__ void k_loss_grad(long long V, const float* __restrict__ y, const float* __restrict__ t,
                             const float* __restrict__ m, const double* __restrict__ tot,
@@ -808,7 +896,7 @@ void masked_mse(long long V, const float* y, const float* t, const float* m, dou
                 double* out, float* dy, hipStream_t s) {
   const int vpb = (int)((V + nblk - 1) / nblk);
   hipLaunchKernelGGL(k_loss_partial, dim3(nblk), dim3(256), 0, s, V, y, t, m, part, vpb);
-  hipLaunchKernelGGL(k_loss_fold, dim3(1), dim3(64), 0, s, part, nblk, out);
+  hipLaunchKernelGGL(k_loss_fold, dim3(1), dim3(256), 0, s, part, nblk, out);
   if (dy) hipLaunchKernelGGL(k_loss_grad, dim3(nb1(V)), dim3(256), 0, s, V, y, t, m, out, dy);
 }
 

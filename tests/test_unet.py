@@ -232,6 +232,26 @@ def test_gradients_at_row_lengths(shape):
 
 
 @pytest.mark.gpu
+def test_gradients_of_a_repeated_sample():
+    """A batch of eight copies of a sample has the sample's gradients: 8 x 64^3 runs the
+    two-plane, two-channel-tile variants, 64^3 alone the single ones. Every product is exact
+    (exact_problem; the mask count grows by 2^3), so the two differ by the order of FP32
+    sums of up to 2^21 terms in 256 runs: 1e-5 of a layer's norm holds a few hundred
+    roundings of 2^-24."""
+    from aquarius_amd.unet import UNet
+    p, x, t, m = exact_problem((1, 64, 64, 64), seed=9)
+    net = UNet()
+    net.set_params(p)
+    l1, g1 = net.gradients(x, t, m)
+    l8, g8 = net.gradients(*(np.repeat(a, 8, 0) for a in (x, t, m)))
+    assert l8 == pytest.approx(l1, rel=1e-12)
+    blocks, hw, hb, total = U.layout()
+    for l, ((w, b), (ci, co)) in enumerate(zip(blocks, U.CONVS)):
+        assert np.any(g1[w:b]), l
+        assert rel_l2(g8[w:b], g1[w:b]) <= 1e-5 and rel_l2(g8[b:b + co], g1[b:b + co]) <= 1e-5, l
+
+
+@pytest.mark.gpu
 def test_gradient_descent_on_gpu_gradients_reduces_loss():
     """Plain gradient descent driven by the GPU gradients (host-tensor path) lowers
     the loss on a fixed batch: the gradients point downhill."""
