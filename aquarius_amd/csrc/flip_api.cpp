@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -133,12 +134,22 @@ struct aq_flip {
   };
   std::vector<SweepGraph> sweep_graphs;
   static constexpr size_t kMaxSweepGraphs = 16;
-  // Multigrid-preconditioned CG (allocated on first use).
+  // Multigrid-preconditioned CG (allocated on first use). The iteration's launches are
+  // captured once per parity from the handle's second solve on.
   struct MgState {
-    MgHierarchy H;
-    double *b = nullptr, *x = nullptr, *r = nullptr, *z = nullptr, *d = nullptr, *q = nullptr;
-    double *part = nullptr, *S = nullptr;
-    int nparts = 256;
+    MgLevels H{};
+    MgVectors V{};
+    MgReport* report = nullptr;  // pinned
+    long long solves = 0;
+    hipGraph_t graph[2] = {};
+    hipGraphExec_t exec[2] = {};
+    ~MgState() {
+      for (int k = 0; k < 2; ++k) {
+        if (exec[k]) hipGraphExecDestroy(exec[k]);
+        if (graph[k]) hipGraphDestroy(graph[k]);
+      }
+      if (report) hipHostFree(report);
+    }
   };
   MgState* mg = nullptr;
   std::vector<hipEvent_t> event_pool;
@@ -530,74 +541,91 @@ aq_status run_stage(aq_flip* h, int st) {
 // ---- multigrid-preconditioned CG ---------------------------------------------
 aq_status mg_setup(aq_flip* h) {
   if (h->mg) return AQ_OK;
-  auto* M = new aq_flip::MgState;
-  h->mg = M;
+  std::unique_ptr<aq_flip::MgState> M(new aq_flip::MgState);
   const Geom& G = h->G;
+  MgLevels& H = M->H;
   int X = G.X, Y = G.Y, Z = G.Z;
+  auto guarded = [&](auto** p, const MgLevel& L) -> aq_status {
+    AQ_TRY(h->allocT(p, (size_t)L.n + 2 * (size_t)mg_guard(L)));
+    *p += mg_guard(L);
+    return AQ_OK;
+  };
   for (;;) {  // halve every axis down to a few cells
-    MgLevel L{X, Y, Z, (long long)X * Y * Z, nullptr};
-    AQ_TRY(h->allocT(&L.fluid, (size_t)L.n));
-    float *f, *u, *t;
-    AQ_TRY(h->allocT(&f, (size_t)L.n));
-    AQ_TRY(h->allocT(&u, (size_t)L.n));
-    AQ_TRY(h->allocT(&t, (size_t)L.n));
-    M->H.levels.push_back(L);
-    M->H.f.push_back(f);
-    M->H.u.push_back(u);
-    M->H.t.push_back(t);
-    if (std::max(X, std::max(Y, Z)) <= 4 || M->H.levels.size() >= 12) break;
+    MgLevel& L = H.L[H.count++];
+    L = mg_level(X, Y, Z);
+    AQ_TRY(guarded(&L.code, L));
+    for (float** p : {&L.f, &L.u, &L.t}) AQ_TRY(guarded(p, L));
+    if (std::max(X, std::max(Y, Z)) <= 4) break;
     X = (X + 1) / 2, Y = (Y + 1) / 2, Z = (Z + 1) / 2;
   }
-  const size_t n0 = (size_t)M->H.levels[0].n;
-  for (double** v : {&M->b, &M->x, &M->r, &M->z, &M->d, &M->q}) AQ_TRY(h->allocT(v, n0));
-  AQ_TRY(h->allocT(&M->part, (size_t)M->nparts * 2));
-  AQ_TRY(h->allocT(&M->S, 8));
+  H.tail = mg_tail_level(H);
+  MgVectors& V = M->V;
+  for (double** p : {&V.x, &V.r, &V.q, &V.d[0], &V.d[1]}) AQ_TRY(guarded(p, H.L[0]));
+  AQ_TRY(h->allocT(&V.part, mg_part_size(H)));
+  AQ_TRY(h->allocT(&V.S, 1));
+  HIP_TRY(hipHostMalloc((void**)&M->report, sizeof(MgReport), hipHostMallocMapped));
+  HIP_TRY(hipHostGetDevicePointer((void**)&V.report, M->report, 0));
+  h->mg = M.release();
+  return AQ_OK;
+}
+
+// Waits until the solve has reported `seq`. Every report is written by a kernel already
+// queued on the stream; if the stream runs empty without it, a launch failed.
+aq_status mg_wait(aq_flip* h, int seq) {
+  const MgReport* r = h->mg->report;
+  auto there = [&] { return __atomic_load_n(&r->seq, __ATOMIC_ACQUIRE) >= seq; };
+  for (unsigned spin = 1; !there(); ++spin) {
+    if (spin % 4096) continue;
+    const hipError_t e = hipStreamQuery(h->stream);
+    if (e == hipErrorNotReady) continue;
+    if (e != hipSuccess) return fail(AQ_EHIP, std::string("MG-PCG: ") + hipGetErrorString(e));
+    if (!there()) return fail(AQ_EHIP, "MG-PCG: the residual was not reported");
+  }
+  return AQ_OK;
+}
+
+aq_status mg_enqueue(aq_flip* h, int odd) {
+  aq_flip::MgState& M = *h->mg;
+  if (h->timing || !h->use_graphs || M.solves == 0) {
+    mg_iterate(M.H, M.V, odd, h->stream);
+    return AQ_OK;
+  }
+  if (!M.exec[odd]) {
+    HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
+    mg_iterate(M.H, M.V, odd, h->stream);
+    const hipError_t e = hipStreamEndCapture(h->stream, &M.graph[odd]);
+    if (e != hipSuccess) return fail(AQ_EHIP, std::string("MG-PCG capture: ") + hipGetErrorString(e));
+    HIP_TRY(hipGraphInstantiate(&M.exec[odd], M.graph[odd], nullptr, nullptr, 0));
+  }
+  HIP_TRY(hipGraphLaunch(M.exec[odd], h->stream));
   return AQ_OK;
 }
 
 // Solve A p = b to an FP64 relative residual <= tol with MG-preconditioned CG in FP64,
-// starting from the current pressure (or zero), and store the result as FP32.
+// starting from the current pressure (or zero), and store the result as FP32. The
+// residual of an iteration is reported before its V-cycle, so the next iteration is
+// queued while the V-cycle runs.
 aq_status mgpcg_solve(aq_flip* h, double tol, int max_iters, int check_every, bool from_current,
                       int* iters, double* rel) {
   AQ_TRY(mg_setup(h));
   aq_flip::MgState& M = *h->mg;
-  const MgLevel& L0 = M.H.levels[0];
-  const long long n = L0.n;
-  hipStream_t s = h->stream;
-  mg_gather(h->G, h->gr.content, h->gr.rhs, h->gr.p[h->pb], from_current, L0, M.b, M.x, s);
-  for (size_t l = 1; l < M.H.levels.size(); ++l) mg_coarsen_flags(M.H.levels[l - 1], M.H.levels[l], s);
-  cg_residual(L0, M.b, M.x, M.r, s);
-  cg_dot2(n, M.b, M.b, nullptr, nullptr, M.part, M.nparts, M.S, 6, s);   // S[6] = b.b
-  mg_vcycle(M.H, M.r, M.z, s);
-  cg_copy(n, M.z, M.d, s);
-  cg_dot2(n, M.r, M.z, M.r, M.r, M.part, M.nparts, M.S, 0, s);           // S[0] = r.z, S[1] = r.r
-  double hs[8] = {0};
-  HIP_TRY(hipMemcpyAsync(hs, M.S, sizeof(hs), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  const double bb = hs[6];
-  auto relres = [&](double rr) { return bb > 0 ? std::sqrt(rr / bb) : std::sqrt(rr); };
-  double res = relres(hs[1]);
+  M.report->seq = 0;  // the previous solve's kernels have completed
+  float* p = h->gr.p[h->pb];
+  mg_start(h->G, M.H, M.V, h->gr.content, h->gr.rhs, from_current ? p : nullptr, tol, max_iters, check_every,
+           h->stream);
+  AQ_TRY(mg_wait(h, 1));
   int it = 0;
-  while (!(res <= tol) && it < max_iters && std::isfinite(res)) {
-    cg_apply(L0, M.d, M.q, s);
-    cg_dot2(n, M.d, M.q, nullptr, nullptr, M.part, M.nparts, M.S, 2, s);  // S[2] = d.q
-    cg_update_xr(n, M.S, M.d, M.q, M.x, M.r, s);
-    mg_vcycle(M.H, M.r, M.z, s);
-    cg_dot2(n, M.r, M.z, M.r, M.r, M.part, M.nparts, M.S, 4, s);          // S[4] = r.z, S[5] = r.r
-    cg_update_d(n, M.S, M.z, M.d, s);
-    cg_shift(M.S, s);
-    ++it;
-    if (it % check_every == 0 || it == max_iters) {
-      HIP_TRY(hipMemcpyAsync(hs, M.S, sizeof(hs), hipMemcpyDeviceToHost, s));
-      HIP_TRY(hipStreamSynchronize(s));
-      res = relres(hs[1]);
-    }
+  while (!M.report->stop && it < max_iters) {
+    const int next = (int)std::min<long long>(max_iters, ((long long)it / check_every + 1) * check_every);
+    for (; it < next; ++it) AQ_TRY(mg_enqueue(h, it & 1));
+    AQ_TRY(mg_wait(h, it + 1));
   }
-  mg_scatter(h->G, L0, M.x, h->gr.p[h->pb], s);
+  mg_finish(h->G, M.H, M.V, p, h->stream);
   HIP_TRY(hipGetLastError());
+  ++M.solves;
   h->air_clean[h->pb] = true;  // AIR cells written 0
   *iters = it;
-  *rel = res;
+  *rel = M.report->res;
   return AQ_OK;
 }
 
