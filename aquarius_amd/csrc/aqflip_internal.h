@@ -144,14 +144,34 @@ void launch_seed_write(const SeedVolume& v, const SeedParams& sp, long long nc, 
                        long long out0, Particles P, hipStream_t s);
 int seed_block_size();
 void launch_hash_count(const Geom& G, Particles P, long long Np, Bins B, hipStream_t s);
-void launch_scan(const Geom& G, Bins B, hipStream_t s);
+// start / end (either may be null): the cell ranges, see k_scan_final.
+void launch_scan(const Geom& G, Bins B, hipStream_t s, int* start = nullptr, int* end = nullptr);
 void launch_scatter_sort_gather(const Geom& G, Particles cur, Particles alt, long long Np, int K,
                                 Bins B, hipStream_t s);
 // Standalone spatial hashing (records of `stride` floats, position first).
 void launch_hash_records(const Geom& G, const float* pos, long long n, int stride, Bins B, hipStream_t s);
 void launch_scatter_segsort(const Geom& G, long long n, Bins B, hipStream_t s);
-void launch_hash_outputs(const Geom& G, long long n, int stride, Bins B, const float* rec, int* start, int* end,
-                         int* sorted_hash, float* sorted_rec, hipStream_t s);
+// The same permutation by a stable radix sort of the hashes (crowded grids).
+struct RadixBufs {
+  uint32_t* keys[2];        // n each
+  int* vals[2];             // n each; vals[1] only with two passes or more
+  int *counts, *offsets, *partials;  // radix_counts(n), one more, and a scan's partials of it
+};
+int radix_passes(const Geom& G);
+size_t radix_counts(long long n);
+// Sorted slot -> record index in R.vals[0]; returns the sorted hashes.
+uint32_t* launch_radix_sort(const Geom& G, const float* rec, long long n, int stride, const RadixBufs& R,
+                            hipStream_t s);
+// What the outputs are written from: the permutation, and the hashes per record or (sorted)
+// per slot; then start / end (either may be null) receive the ranges of the non-empty cells.
+struct HashSorted {
+  const int* perm;
+  const int* hash;
+  bool sorted;
+  int *start, *end;
+};
+void launch_hash_outputs(long long n, int stride, const HashSorted& in, const float* rec, int* perm, int* sorted_hash,
+                         float* sorted_rec, hipStream_t s);
 void launch_p2g(const Geom& G, Particles P, long long Np, int K, Bins B, Grid gr, int nv,
                 int hv, int nf, StepParams sp, hipStream_t s);
 void launch_gravity_boundary(const Geom& G, Grid gr, int nv, StepParams sp, int doGravity,

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <climits>
+#include <type_traits>
 
 #include "aqflip_internal.h"
 
@@ -147,6 +148,29 @@ __device__ __forceinline__ void bin_particle(int hh, bool valid, int* __restrict
   rank = base + __popcll(group & lt);
 }
 
+// The same for records in any order. Where neighbouring lanes share their hashes the groups
+// are few and bin_particle's loop is short; in a wave of mostly different hashes it would
+// take up to 64 rounds to save no atomic, so every lane takes its own slot. (Which lane of a
+// cell gets which slot is then arbitrary; every slot but a cell's first marks the cell, so
+// the segment sort orders it.) Sorted records at 8 per cell make 8 to 16 runs per wave;
+// 1 M unordered ones of 16 bytes in 100^3 cells took 169 us in all with the loop, 122 now.
+constexpr int kMaxRuns = 24;
+__device__ __forceinline__ void bin_record(int hh, bool valid, int* __restrict__ count, uint8_t* __restrict__ multi,
+                                           int& rank) {
+  const int lane = (int)(threadIdx.x & 63);
+  const int prev = __shfl_up(hh, 1, 64);
+  const unsigned long long starts = __ballot(valid && (lane == 0 || hh != prev));
+  if (__popcll(starts) <= kMaxRuns) {
+    bin_particle(hh, valid, count, multi, rank);
+    return;
+  }
+  rank = 0;
+  if (valid) {
+    rank = atomicAdd(&count[hh], 1);
+    if (rank > 0) multi[hh] = 1;
+  }
+}
+
 __global__ void k_hash_bin(Geom G, Particles P, long long Np, int* __restrict__ hash,
                            int* __restrict__ rank, int* __restrict__ count, uint8_t* __restrict__ multi) {
   const int i = gtid();
@@ -245,9 +269,14 @@ __global__ void k_scan_parts(int* __restrict__ partials, int nparts) {
 // Block b adds the totals of blocks 0..b-1 (read here, with its counts, in the same
 // round trip; or, when `prefixed`, their sum already formed by k_scan_parts) to its own
 // exclusive scan; the last block also writes offsets[n]. Integer sums, so any
-// association gives the same offsets.
+// association gives the same offsets. RANGES: also the cell ranges in the reference's
+// convention (findCellStartEndImpl, Fluid/Fluid_kernels.cuh:3-22), first and last
+// (inclusive) sorted slot of every cell, -1 for empty ones, into either array that is not
+// null (any 4-byte alignment).
+template <bool RANGES>
 __global__ void k_scan_final(int* __restrict__ count, int n, const int* __restrict__ partials,
-                             int nparts, int* __restrict__ offsets, int prefixed) {
+                             int nparts, int* __restrict__ offsets, int prefixed, int* __restrict__ start,
+                             int* __restrict__ end) {
   __shared__ int wsum[kBlock / 64], wpre[kBlock / 64];
   const int b = blockIdx.x;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -297,6 +326,26 @@ __global__ void k_scan_final(int* __restrict__ count, int n, const int* __restri
       if (base + k < n) offsets[base + k] = o[k];
   }
   if (b == nparts - 1 && threadIdx.x == 0) offsets[n] = prefix + tot;
+  if (RANGES) {
+    typedef int i32x4u __attribute__((ext_vector_type(4), aligned(4)));
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+      int* __restrict__ out = which ? end : start;
+      if (!out) continue;
+      int r[kScanPerThread];
+#pragma unroll
+      for (int k = 0; k < kScanPerThread; ++k) r[k] = v[k] > 0 ? o[k] + (which ? v[k] - 1 : 0) : -1;
+      if (base + kScanPerThread <= n) {
+#pragma unroll
+        for (int k = 0; k < kScanPerThread; k += 4)
+          *(i32x4u*)(out + base + k) = i32x4u{r[k], r[k + 1], r[k + 2], r[k + 3]};
+      } else {
+#pragma unroll
+        for (int k = 0; k < kScanPerThread; ++k)
+          if (base + k < n) out[base + k] = r[k];
+      }
+    }
+  }
   // The counts' last reader: the nonzero ones (the cells holding particles, a quarter of
   // the grid in the 128^3 scenes) are set back to zero, so the next binning needs no
   // clearing pass. (Zeroing all of them here cost as much as the clearing pass.)
@@ -312,14 +361,19 @@ __global__ void k_scan_final(int* __restrict__ count, int n, const int* __restri
   }
 }
 
-void launch_scan(const Geom& G, Bins B, hipStream_t s) {
+void launch_scan(const Geom& G, Bins B, hipStream_t s, int* start, int* end) {
   const int n = G.ncells_hash;
   const int nparts = (n + kScanChunk - 1) / kScanChunk;
-  hipLaunchKernelGGL(k_scan_reduce, dim3(nparts), dim3(kBlock), 0, s, B.count, n, B.partials);
+  if (nparts > 1)  // a single block has no totals before it
+    hipLaunchKernelGGL(k_scan_reduce, dim3(nparts), dim3(kBlock), 0, s, B.count, n, B.partials);
   const int prefixed = nparts > kScanDirectParts ? 1 : 0;
   if (prefixed) hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kBlock), 0, s, B.partials, nparts);
-  hipLaunchKernelGGL(k_scan_final, dim3(nparts), dim3(kBlock), 0, s, B.count, n, B.partials, nparts,
-                     B.offsets, prefixed);
+  if (start || end)
+    hipLaunchKernelGGL(k_scan_final<true>, dim3(nparts), dim3(kBlock), 0, s, B.count, n, B.partials, nparts,
+                       B.offsets, prefixed, start, end);
+  else
+    hipLaunchKernelGGL(k_scan_final<false>, dim3(nparts), dim3(kBlock), 0, s, B.count, n, B.partials, nparts,
+                       B.offsets, prefixed, nullptr, nullptr);
 }
 
 // ------------------------------------------------------------------ stable counting sort
@@ -342,12 +396,14 @@ __global__ void k_scatter(const int* __restrict__ hash, const int* __restrict__ 
 // are loaded into registers in one round trip (predicated loads, INT_MAX past the end),
 // sorted there by a bitonic network (every index a compile-time constant, so the array
 // stays in registers) and written back once; the entries are distinct particle indices,
-// so any correct sort gives the same order. Longer segments are checked by a loop and,
-// when unsorted, insertion-sorted in place. (After the ball of the 128^3 multiphase
-// scene meets the pool, 100-180 cells hold 17-30 particles: by the insertion sort, one
-// dependent load and store per step, they took the kernel from 12.5 to 81 us.)
+// so any correct sort gives the same order. (After the ball of the 128^3 multiphase
+// scene meets the pool, 100-180 cells hold 17-30 particles: by an insertion sort in memory
+// they took the kernel from 12.5 to 81 us.) Longer segments are sorted by their whole wave,
+// one after another (wave_sort): a settled pool's clumps of 33-100 particles, and grids of
+// few cells, whose segments of thousands took a lone lane's insertion sort seconds.
 constexpr int kSegFast = 16;
 constexpr int kSegMid = 32;
+constexpr int kSegLds = 1024;  // entries a wave sorts in LDS
 template <int N>
 __device__ __forceinline__ void bitonic_sort(int (&v)[N]) {
 #pragma unroll
@@ -380,31 +436,96 @@ __device__ __forceinline__ void sort_segment(int* __restrict__ perm, int s, int 
   for (int k = 0; k < N; ++k)
     if (s + k < e) perm[s + k] = v[k];
 }
-__global__ void k_segsort(const int* __restrict__ offsets, int ncells, int* __restrict__ perm,
-                          uint8_t* __restrict__ multi) {
-  const int c = gtid();
-  if (c >= ncells || !multi[c]) return;
-  multi[c] = 0;
-  const int s = offsets[c], e = offsets[c + 1];
-  if (e - s <= kSegFast) {
-    sort_segment<kSegFast>(perm, s, e);
-    return;
+// Ascending bitonic network on a[0, n) by one wave, from blocks of `k0` that are in order
+// (k0 = 1: from scratch) to blocks of `k1`; every comparator keeps the smaller value at the
+// lower index (a merge starts with mirrored pairs), so entries past n, which would sort
+// last, can simply be left out. `lo`: merge steps of a smaller distance are left to the
+// caller. a is in LDS or in memory; the wave's
+// own accesses are ordered by the fences.
+__device__ __forceinline__ void bitonic_pair(int* a, uint32_t n, uint32_t i, uint32_t l) {
+  if (l >= n) return;
+  const int x = a[i], y = a[l];
+  if (x > y) {
+    a[i] = y;
+    a[l] = x;
   }
-  if (e - s <= kSegMid) {
-    sort_segment<kSegMid>(perm, s, e);
+}
+// One merge step: pairs (i, i + j), i's bit j clear, the first `pairs` of them.
+__device__ __forceinline__ void bitonic_step(int* a, uint32_t n, uint32_t j, uint32_t pairs) {
+  for (uint32_t t = threadIdx.x & 63; t < pairs; t += 64) {
+    const uint32_t o = t & (j - 1), i = 2 * (t - o) + o;
+    bitonic_pair(a, n, i, i + j);
+  }
+  __threadfence_block();
+}
+__device__ void bitonic_wave(int* a, uint32_t n, uint32_t k0, uint32_t k1, uint32_t lo) {
+  for (uint32_t k = 2 * k0; k && k <= k1; k <<= 1) {
+    const uint32_t half = k / 2, pairs = ((n - 1) / k + 1) * half;
+    for (uint32_t t = threadIdx.x & 63; t < pairs; t += 64) {
+      const uint32_t o = t & (half - 1), b = 2 * (t - o);
+      bitonic_pair(a, n, b + o, b + (k - 1) - o);
+    }
+    __threadfence_block();
+    for (uint32_t j = half / 2; j >= lo && j; j >>= 1) bitonic_step(a, n, j, pairs);
+  }
+}
+// Sort p[0, n) by one wave: in LDS (kSegLds entries) when it fits, else chunks in LDS and
+// the merges' wide steps in memory.
+__device__ void wave_sort(int* __restrict__ p, int n, int* lds) {
+  const int lane = (int)(threadIdx.x & 63);
+  if (n <= 64) {  // one entry per lane, exchanged by lane permutation
+    int v = lane < n ? p[lane] : INT_MAX;
+    for (int k = 2; k <= 64; k <<= 1)
+      for (int m = k - 1, j = k / 2; j > 0; j >>= 1, m = j) {
+        const int w = __shfl_xor(v, m, 64);
+        v = (lane & j) == 0 ? min(v, w) : max(v, w);
+      }
+    if (lane < n) p[lane] = v;
     return;
   }
   bool sorted = true;
-  for (int i = s + 1; i < e; ++i) sorted &= perm[i - 1] < perm[i];
-  if (sorted) return;
-  for (int i = s + 1; i < e; ++i) {
-    const int v = perm[i];
-    int j = i - 1;
-    while (j >= s && perm[j] > v) {
-      perm[j + 1] = perm[j];
-      --j;
+  for (int i = lane; i + 1 < n; i += 64) sorted &= p[i] < p[i + 1];
+  if (__ballot(!sorted) == 0) return;
+  auto chunk = [&](int c, bool first) {
+    const int m = min(kSegLds, n - c);
+    for (int i = lane; i < m; i += 64) lds[i] = p[c + i];
+    __threadfence_block();
+    if (first) {
+      int k1 = 64;
+      while (k1 < m) k1 <<= 1;
+      bitonic_wave(lds, m, 1, k1, 1);
+    } else {
+      for (int j = kSegLds / 2; j > 0; j >>= 1) bitonic_step(lds, m, j, kSegLds / 2);
     }
-    perm[j + 1] = v;
+    for (int i = lane; i < m; i += 64) p[c + i] = lds[i];
+    __threadfence_block();
+  };
+  for (int c = 0; c < n; c += kSegLds) chunk(c, true);
+  for (uint32_t k = 2 * kSegLds; k && k / 2 < (uint32_t)n; k <<= 1) {
+    bitonic_wave(p, n, k / 2, k, kSegLds);
+    for (int c = 0; c < n; c += kSegLds) chunk(c, false);
+  }
+}
+__global__ __launch_bounds__(kBlock) void k_segsort(const int* __restrict__ offsets, int ncells,
+                                                    int* __restrict__ perm, uint8_t* __restrict__ multi) {
+  __shared__ int lds[kBlock / 64][kSegLds];
+  const int c = gtid();
+  const bool flagged = c < ncells && multi[c];
+  if (__ballot(flagged) == 0) return;
+  int s = 0, e = 0;
+  if (flagged) {
+    multi[c] = 0;
+    s = offsets[c];
+    e = offsets[c + 1];
+    if (e - s <= kSegFast)
+      sort_segment<kSegFast>(perm, s, e);
+    else if (e - s <= kSegMid)
+      sort_segment<kSegMid>(perm, s, e);
+  }
+  for (unsigned long long rest = __ballot(e - s > kSegMid); rest; rest &= rest - 1) {
+    const int l = __ffsll((long long)rest) - 1;
+    const int ls = __shfl(s, l, 64), le = __shfl(e, l, 64);
+    wave_sort(perm + ls, le - ls, lds[threadIdx.x >> 6]);
   }
 }
 
@@ -444,7 +565,7 @@ __global__ void k_hash_records(Geom G, const float* __restrict__ pos, long long 
     hh = cell_hash(G, p[0], p[1], p[2]);
   }
   int r;
-  bin_particle(hh, valid, count, multi, r);
+  bin_record(hh, valid, count, multi, r);
   if (valid) {
     hash[i] = hh;
     rank[i] = r;
@@ -460,36 +581,205 @@ void launch_scatter_segsort(const Geom& G, long long n, Bins B, hipStream_t s) {
   hipLaunchKernelGGL(k_segsort, dim3(nblocks(G.ncells_hash)), dim3(kBlock), 0, s, B.offsets,
                      G.ncells_hash, B.perm, B.multi);
 }
-// findCellStartEndImpl (Fluid/Fluid_kernels.cuh:3-22) from the offsets: first and
-// last (inclusive) sorted slot of every cell, -1 for empty cells.
-__global__ void k_cell_ranges(int ncells, const int* __restrict__ offsets, int* __restrict__ start,
-                              int* __restrict__ end) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= ncells) return;
-  const int s = offsets[c], e = offsets[c + 1];
-  if (start) start[c] = e > s ? s : -1;
-  if (end) end[c] = e > s ? e - 1 : -1;
+// ---- stable radix sort of the hashes, least digit first
+// The counting sort above leaves each cell's segment in the order its waves reserved slots,
+// and sorts segments one by one: with many records per cell that is nearly all of its
+// time (1.07 M records in 210 cells: seconds by insertion, 39 ms by waves, 72 us here). A
+// radix pass needs neither atomics on cells nor segments: a block counts its tile's digits in LDS, the counts (digit-major) are
+// scanned as the cell counts are, and each wave then places its keys in order, 64 at a
+// time, finding the lanes that share a digit with one ballot per bit. Digits of up to 9
+// bits, so that grids of up to 64^3 cells take two passes.
+constexpr int kRadixBits = 9;
+constexpr int kRadixBins = 1 << kRadixBits;
+// Keys of a tile: kBlock / 64 waves, ROUNDS rounds of 64 keys each.
+template <int ROUNDS>
+constexpr int kRadixTile = kBlock * ROUNDS;
+template <int ROUNDS, bool FIRST>
+__global__ __launch_bounds__(kBlock) void k_radix_count(Geom G, const float* __restrict__ rec, int stride, long long n,
+                                                        uint32_t* __restrict__ keys, int shift, int bins,
+                                                        int* __restrict__ counts) {
+  __shared__ int hist[kRadixBins];
+  for (int b = threadIdx.x; b < kRadixBins; b += kBlock) hist[b] = 0;
+  __syncthreads();
+  const long long k0 = (long long)blockIdx.x * kRadixTile<ROUNDS> + threadIdx.x;
+  uint32_t key[ROUNDS];
+#pragma unroll
+  for (int i = 0; i < ROUNDS; ++i) {
+    const long long k = k0 + i * kBlock;
+    key[i] = 0;
+    if (k < n) {
+      if (FIRST) {
+        const float* p = rec + k * stride;
+        key[i] = (uint32_t)cell_hash(G, p[0], p[1], p[2]);
+        keys[k] = key[i];
+      } else {
+        key[i] = keys[k];
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < ROUNDS; ++i)
+    if (k0 + i * kBlock < n) atomicAdd(&hist[(key[i] >> shift) & (bins - 1)], 1);
+  __syncthreads();
+  for (int b = threadIdx.x; b < bins; b += kBlock) counts[b * gridDim.x + blockIdx.x] = hist[b];
 }
-// Sorted hashes and, optionally, the records in sorted order (applySortImpl,
-// Fluid/Fluid_3D_kernels.cuh:95-102).
+template <int ROUNDS, bool FIRST>
+__global__ __launch_bounds__(kBlock) void k_radix_scatter(long long n, const uint32_t* __restrict__ keys,
+                                                          const int* __restrict__ vals, int shift, int bins,
+                                                          const int* __restrict__ offsets,
+                                                          uint32_t* __restrict__ keys_out, int* __restrict__ vals_out) {
+  constexpr int W = kBlock / 64;
+  __shared__ int at[W][kRadixBins];  // counts, then the next slot, of each wave and digit
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int b = threadIdx.x; b < W * kRadixBins; b += kBlock) at[0][b] = 0;
+  __syncthreads();
+  const long long k0 = (long long)blockIdx.x * kRadixTile<ROUNDS> + wave * (64 * ROUNDS) + lane;
+  uint32_t key[ROUNDS];
+  int val[ROUNDS];
+#pragma unroll
+  for (int i = 0; i < ROUNDS; ++i) {
+    const long long k = k0 + i * 64;
+    key[i] = k < n ? keys[k] : 0;
+    val[i] = FIRST ? (int)k : (k < n ? vals[k] : 0);
+  }
+#pragma unroll
+  for (int i = 0; i < ROUNDS; ++i)
+    if (k0 + i * 64 < n) atomicAdd(&at[wave][(key[i] >> shift) & (bins - 1)], 1);
+  __syncthreads();
+  for (int b = threadIdx.x; b < bins; b += kBlock) {
+    int base = offsets[b * gridDim.x + blockIdx.x];
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const int c = at[w][b];
+      at[w][b] = base;
+      base += c;
+    }
+  }
+  __syncthreads();
+  const unsigned long long lt = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int i = 0; i < ROUNDS; ++i) {
+    const bool valid = k0 + i * 64 < n;
+    const uint32_t d = (key[i] >> shift) & (bins - 1);
+    unsigned long long same = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < kRadixBits; ++b) {
+      const unsigned long long one = __ballot((d >> b) & 1);
+      same &= (d >> b) & 1 ? one : ~one;
+    }
+    int slot = 0;
+    if (valid) slot = at[wave][d] + __popcll(same & lt);
+    __threadfence_block();  // every lane has read its slot
+    if (valid && (same & lt) == 0) at[wave][d] += __popcll(same);
+    __threadfence_block();
+    if (valid) {
+      keys_out[slot] = key[i];
+      vals_out[slot] = val[i];
+    }
+  }
+}
+static int radix_rounds(long long n) { return n >= (1 << 19) ? 16 : 4; }
+size_t radix_counts(long long n) {
+  const long long tile = (long long)kBlock * radix_rounds(n);
+  return (size_t)((n + tile - 1) / tile * kRadixBins);
+}
+int radix_passes(const Geom& G) {
+  int bits = 1;
+  while ((1ll << bits) < G.ncells_hash) ++bits;
+  return (bits + kRadixBits - 1) / kRadixBits;
+}
+uint32_t* launch_radix_sort(const Geom& G, const float* rec, long long n, int stride, const RadixBufs& R,
+                            hipStream_t s) {
+  int bits = 1;
+  while ((1ll << bits) < G.ncells_hash) ++bits;
+  const int passes = radix_passes(G), width = (bits + passes - 1) / passes, bins = 1 << width;
+  const int rounds = radix_rounds(n);
+  const int tiles = (int)((n + (long long)kBlock * rounds - 1) / ((long long)kBlock * rounds));
+  Geom S{};
+  S.ncells_hash = bins * tiles;
+  Bins B{};
+  B.count = R.counts, B.offsets = R.offsets, B.partials = R.partials;
+  // the last pass leaves the indices in vals[0]
+  int k = 0, v = passes & 1 ? 1 : 0;
+  for (int p = 0; p < passes; ++p, k ^= 1, v ^= 1) {
+    const int shift = p * width;
+    auto pass = [&](auto r, auto first) {
+      constexpr int ROUNDS = decltype(r)::value;
+      constexpr bool FIRST = decltype(first)::value;
+      hipLaunchKernelGGL((k_radix_count<ROUNDS, FIRST>), dim3(tiles), dim3(kBlock), 0, s, G, rec, stride, n, R.keys[k],
+                         shift, bins, R.counts);
+      launch_scan(S, B, s);
+      hipLaunchKernelGGL((k_radix_scatter<ROUNDS, FIRST>), dim3(tiles), dim3(kBlock), 0, s, n, R.keys[k], R.vals[v],
+                         shift, bins, R.offsets, R.keys[k ^ 1], R.vals[v ^ 1]);
+    };
+    auto both = [&](auto r) {
+      if (p == 0)
+        pass(r, std::true_type{});
+      else
+        pass(r, std::false_type{});
+    };
+    if (rounds == 16)
+      both(std::integral_constant<int, 16>{});
+    else
+      both(std::integral_constant<int, 4>{});
+  }
+  return R.keys[k];
+}
+
+// The permutation, the sorted hashes and the records in sorted order (applySortImpl,
+// Fluid/Fluid_3D_kernels.cuh:95-102), each where its output is not null. A thread moves one
+// piece (T: 16, 8 or 4 bytes) of a record, S pieces per record, so that neighbouring lanes
+// write neighbouring bytes whatever the stride. 1 M records of 48 bytes: 278 -> 44 us
+// (a thread per record wrote 4 bytes every 48). SORTED: `hash` is already in sorted order,
+// and the cell ranges (see k_scan_final; their empty cells are set beforehand) are read off it.
+template <typename T, bool SORTED>
 __global__ void k_sorted_outputs(long long n, const int* __restrict__ perm, const int* __restrict__ hash,
-                                 int* __restrict__ sorted_hash, const float* __restrict__ rec,
-                                 float* __restrict__ sorted_rec, int stride) {
-  const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+                                 int* __restrict__ perm_out, int* __restrict__ sorted_hash,
+                                 const T* __restrict__ rec, T* __restrict__ sorted_rec, int S, FastDiv divS,
+                                 int* __restrict__ start, int* __restrict__ end) {
+  const long long e0 = (long long)blockIdx.x * kBlock, k0 = e0 / S;
+  const uint32_t r = (uint32_t)(e0 - k0 * S) + threadIdx.x;
+  const uint32_t dk = fast_div(r, divS);
+  const long long k = k0 + dk;
+  const int f = (int)(r - dk * (uint32_t)S);
   if (k >= n) return;
   const int j = perm[k];
-  if (sorted_hash) sorted_hash[k] = hash[j];
-  if (sorted_rec)
-    for (int f = 0; f < stride; ++f) sorted_rec[k * stride + f] = rec[(long long)j * stride + f];
+  if (sorted_rec) sorted_rec[k * S + f] = rec[(long long)j * S + f];
+  if (f == 0) {
+    if (perm_out && perm_out != perm) perm_out[k] = j;
+    if (SORTED) {
+      const int h = hash[k];
+      if (sorted_hash) sorted_hash[k] = h;
+      if (start && (k == 0 || hash[k - 1] != h)) start[h] = (int)k;
+      if (end && (k == n - 1 || hash[k + 1] != h)) end[h] = (int)k;
+    } else if (sorted_hash) {
+      sorted_hash[k] = hash[j];
+    }
+  }
 }
-void launch_hash_outputs(const Geom& G, long long n, int stride, Bins B, const float* rec, int* start, int* end,
-                         int* sorted_hash, float* sorted_rec, hipStream_t s) {
-  if (start || end)
-    hipLaunchKernelGGL(k_cell_ranges, dim3(nblocks(G.ncells_hash)), dim3(kBlock), 0, s, G.ncells_hash,
-                       B.offsets, start, end);
-  if ((sorted_hash || sorted_rec) && n > 0)
-    hipLaunchKernelGGL(k_sorted_outputs, dim3(nblocks(n)), dim3(kBlock), 0, s, n, B.perm, B.hash,
-                       sorted_hash, rec, sorted_rec, stride);
+template <typename T>
+static void sorted_outputs(long long n, int stride, const HashSorted& in, const float* rec, int* perm,
+                           int* sorted_hash, float* sorted_rec, hipStream_t s) {
+  const int S = sorted_rec ? stride / (int)(sizeof(T) / 4) : 1;
+  const dim3 grid((unsigned)((n * S + kBlock - 1) / kBlock));
+  if (in.sorted)
+    hipLaunchKernelGGL((k_sorted_outputs<T, true>), grid, dim3(kBlock), 0, s, n, in.perm, in.hash, perm, sorted_hash,
+                       (const T*)rec, (T*)sorted_rec, S, make_fastdiv((uint32_t)S), in.start, in.end);
+  else
+    hipLaunchKernelGGL((k_sorted_outputs<T, false>), grid, dim3(kBlock), 0, s, n, in.perm, in.hash, perm, sorted_hash,
+                       (const T*)rec, (T*)sorted_rec, S, make_fastdiv((uint32_t)S), nullptr, nullptr);
+}
+void launch_hash_outputs(long long n, int stride, const HashSorted& in, const float* rec, int* perm, int* sorted_hash,
+                         float* sorted_rec, hipStream_t s) {
+  if (n <= 0 || !(perm || sorted_hash || sorted_rec || (in.sorted && (in.start || in.end)))) return;
+  // The widest piece that divides the stride and that both arrays are aligned to.
+  const uintptr_t at = sorted_rec ? (uintptr_t)rec | (uintptr_t)sorted_rec | (uintptr_t)(stride * 4) : 4;
+  if (at % 16 == 0)
+    sorted_outputs<float4>(n, stride, in, rec, perm, sorted_hash, sorted_rec, s);
+  else if (at % 8 == 0)
+    sorted_outputs<float2>(n, stride, in, rec, perm, sorted_hash, sorted_rec, s);
+  else
+    sorted_outputs<float>(n, stride, in, rec, perm, sorted_hash, sorted_rec, s);
 }
 
 // ------------------------------------------------------------------ P2G

@@ -42,11 +42,13 @@ struct aq_hash {
   hipStream_t stream = nullptr;
   Bins B{};
   long long cap = 0;  // particles the per-particle buffers hold
+  int *vals2 = nullptr, *rcounts = nullptr, *roffsets = nullptr, *rpartials = nullptr;  // radix sort, on first use
   // staging for the host entry point
   float *d_rec = nullptr, *d_sorted = nullptr;
   int *d_start = nullptr, *d_end = nullptr, *d_shash = nullptr;
   size_t rec_cap = 0;
   std::vector<void*> fixed, per_particle, staging;
+  bool counts_zero = false;  // B.count holds zeros
 
   ~aq_hash() {
     if (stream) hipStreamSynchronize(stream);
@@ -70,6 +72,30 @@ struct aq_hash {
     HTRY(alloc(&B.rank, (size_t)n, per_particle));
     HTRY(alloc(&B.perm, (size_t)n, per_particle));
     cap = n;
+    vals2 = nullptr;  // the radix sort's buffers went with the others
+    rcounts = roffsets = rpartials = nullptr;
+    return AQ_OK;
+  }
+  // Which of the two sorts. The radix sort's time depends on neither the records' order nor
+  // their spread; the counting sort's grows with the records per cell and with disorder,
+  // but takes one pass where the records come nearly sorted. us, counting / radix, for
+  // records in random order, moved a little since the last sort, and sorted:
+  //   1 M in 50^3 cells     149 / 115   112 / 99    68 / 95
+  //   1 M in 40^3 cells     184 / 92    148 / 85    70 / 82
+  //   3 M in 100^3 cells    359 / 257   225 / 224  134 / 207
+  //   100,000 in 30^3        44 / 52     39 / 56    35 / 50
+  //   100,000 in 16^3       126 / 53    119 / 52    80 / 52
+  // so the line lies at 4 records per cell for large sorts, and at 16 below them, where the
+  // extra launches weigh more.
+  bool crowded(long long n) const {
+    return n >= (1 << 18) ? n >= 4LL * G.ncells_hash : n >= 2048 && n > 16LL * G.ncells_hash;
+  }
+  aq_status ensure_radix(long long n) {
+    if (!vals2) HTRY(alloc(&vals2, (size_t)cap, per_particle));
+    const size_t c = std::max(radix_counts(cap), radix_counts(std::min<long long>(cap, (1 << 19) - 1)));
+    if (!rcounts) HTRY(alloc(&rcounts, c, per_particle));
+    if (!roffsets) HTRY(alloc(&roffsets, c + 1, per_particle));
+    if (!rpartials) HTRY(alloc(&rpartials, c / 4096 + 2, per_particle));
     return AQ_OK;
   }
   aq_status ensure_staging(long long n, int stride) {
@@ -90,13 +116,24 @@ struct aq_hash {
   aq_status run(const float* rec, long long n, int stride, int* perm, int* shash, int* start, int* end,
                 float* sorted, hipStream_t s) {
     HTRY(ensure(n));
-    const int ncells = G.ncells_hash;
-    launch_fill_u32(B.count, 0u, ncells, s);
+    if (crowded(n)) {
+      HTRY(ensure_radix(n));
+      const RadixBufs R{{(uint32_t*)B.hash, (uint32_t*)B.rank}, {B.perm, vals2}, rcounts, roffsets, rpartials};
+      if (start) launch_fill_u32(start, 0xffffffffu, G.ncells_hash, s);
+      if (end) launch_fill_u32(end, 0xffffffffu, G.ncells_hash, s);
+      const uint32_t* keys = launch_radix_sort(G, rec, n, stride, R, s);
+      launch_hash_outputs(n, stride, HashSorted{B.perm, (const int*)keys, true, start, end}, rec, perm, shash, sorted, s);
+      HHIP(hipGetLastError());
+      return AQ_OK;
+    }
+    // The scan, the counts' last reader, leaves them at zero; only after a call that failed
+    // part-way are they cleared first.
+    if (!counts_zero) launch_fill_u32(B.count, 0u, G.ncells_hash, s);
+    counts_zero = false;
     if (n > 0) launch_hash_records(G, rec, n, stride, B, s);
-    launch_scan(G, B, s);
+    launch_scan(G, B, s, start, end);
     if (n > 0) launch_scatter_segsort(G, n, B, s);
-    launch_hash_outputs(G, n, stride, B, rec, start, end, shash, sorted, s);
-    if (perm && n > 0) HHIP(hipMemcpyAsync(perm, B.perm, n * sizeof(int), hipMemcpyDeviceToDevice, s));
+    launch_hash_outputs(n, stride, HashSorted{B.perm, B.hash, false, nullptr, nullptr}, rec, perm, shash, sorted, s);
     HHIP(hipGetLastError());
     return AQ_OK;
   }
@@ -210,9 +247,11 @@ aq_status aq_hash_create(int32_t sx, int32_t sy, int32_t sz, float cell_size, in
   if (st == AQ_OK) st = h->alloc(&h->B.offsets, (size_t)nch + 1, h->fixed);
   if (st == AQ_OK) st = h->alloc(&h->B.partials, (size_t)(nch + 4095) / 4096 + 1, h->fixed);
   if (st == AQ_OK) st = h->alloc(&h->B.multi, (size_t)nch, h->fixed);
-  // the multi-run flags start at zero; k_segsort clears each flag it reads
-  if (st == AQ_OK && hipMemsetAsync(h->B.multi, 0, (size_t)nch, h->stream) != hipSuccess)
+  // the counts and the multi-run flags start at zero; k_scan_final and k_segsort leave them so
+  if (st == AQ_OK && (hipMemsetAsync(h->B.multi, 0, (size_t)nch, h->stream) != hipSuccess ||
+                      hipMemsetAsync(h->B.count, 0, (size_t)nch * sizeof(int), h->stream) != hipSuccess))
     st = hfail(AQ_EHIP, "clearing the bins failed");
+  h->counts_zero = true;
   if (st == AQ_OK) st = h->alloc(&h->d_start, (size_t)nch, h->fixed);
   if (st == AQ_OK) st = h->alloc(&h->d_end, (size_t)nch, h->fixed);
   if (st == AQ_OK) st = h->ensure(std::max<int64_t>(capacity, 1));
@@ -245,6 +284,7 @@ aq_status aq_hash_sort_host(aq_hash* h, const float* rec, int64_t n, int32_t str
   if (end) HHIP(hipMemcpyAsync(end, h->d_end, cb, hipMemcpyDeviceToHost, h->stream));
   if (sorted && n > 0) HHIP(hipMemcpyAsync(sorted, h->d_sorted, bytes, hipMemcpyDeviceToHost, h->stream));
   HHIP(hipStreamSynchronize(h->stream));
+  h->counts_zero = true;
   if (cell_count > ncells) {
     if (start) std::fill(start + ncells, start + cell_count, -1);
     if (end) std::fill(end + ncells, end + cell_count, -1);
@@ -270,6 +310,7 @@ aq_status aq_hash_sort_device(aq_hash* h, const float* d_rec, int64_t n, int32_t
     HHIP(hipGetLastError());
   }
   HHIP(hipStreamSynchronize(s));
+  h->counts_zero = true;
   return AQ_OK;
 }
 
@@ -304,10 +345,9 @@ aq_status aq_hash_sort_device_noalloc(int32_t sx, int32_t sy, int32_t sz, float 
   launch_fill_u32(B.count, 0u, G.ncells_hash, s);
   launch_fill_u32(B.multi, 0u, (G.ncells_hash + 3) / 4, s);
   if (n > 0) launch_hash_records(G, d_rec, n, stride, B, s);
-  launch_scan(G, B, s);
+  launch_scan(G, B, s, d_start, d_end);
   if (n > 0) launch_scatter_segsort(G, n, B, s);
-  launch_hash_outputs(G, n, stride, B, d_rec, d_start, d_end, d_shash, d_sorted, s);
-  if (d_perm && n > 0) HHIP(hipMemcpyAsync(d_perm, B.perm, n * sizeof(int), hipMemcpyDeviceToDevice, s));
+  launch_hash_outputs(n, stride, HashSorted{B.perm, B.hash, false, nullptr, nullptr}, d_rec, d_perm, d_shash, d_sorted, s);
   if (cell_count > G.ncells_hash) {
     if (d_start) launch_fill_u32(d_start + G.ncells_hash, 0xffffffffu, cell_count - G.ncells_hash, s);
     if (d_end) launch_fill_u32(d_end + G.ncells_hash, 0xffffffffu, cell_count - G.ncells_hash, s);

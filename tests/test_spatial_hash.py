@@ -89,6 +89,58 @@ def test_gpu_segments_of_17_to_32_records():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("counts", [(33, 64, 65, 1, 0, 32), (1023, 1024, 1025, 2), (2048, 2049, 3073), (20001, 5, 70)])
+def test_gpu_long_segments(counts):
+    """Cells with more records than the register networks take, in random order: around the
+    wave sort's own limits (64 lanes, 1,024 entries in LDS, merges in memory)."""
+    rng = np.random.default_rng(counts[0])
+    x = np.repeat(np.arange(len(counts)), counts).astype(np.float32) + 0.5
+    rec = np.stack([x, np.full_like(x, 0.5), np.full_like(x, 0.5), np.arange(x.size, dtype=np.float32)], 1)
+    gpu_case((len(counts), 1, 1), 1.0, rec[rng.permutation(x.size)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,n", [((1, 1, 1), 2048), ((3, 1, 2), 4097), ((16, 16, 1), 70_000), ((17, 16, 1), 70_001),
+                                     ((40, 41, 40), 1_100_000), ((5, 4, 3), 524_289), ((5, 4, 3), 524_287)])
+def test_gpu_crowded_grids(sizes, n):
+    """Grids sorted by radix: one, two and three digits, both tile sizes with remainders, and
+    records crowded into part of the grid, some outside it."""
+    rng = np.random.default_rng(n)
+    rec = rng.uniform(-0.3, 0.7, (n, 5)).astype(np.float32)
+    rec[:, :3] *= np.array(sizes, np.float32)
+    gpu_case(sizes, 1.0, rec)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stride,skew", [(3, 0), (4, 0), (4, 1), (5, 0), (6, 0), (6, 2), (8, 2), (12, 1), (12, 0), (700, 0)])
+def test_gpu_record_pieces(stride, skew):
+    """Sorted records of every piece width: strides and array starts (`skew` floats past an
+    aligned address) that allow 16, 8 or 4 bytes, outputs in runs that no block divides."""
+    import torch
+    from aquarius_amd.spatial_hash import SpatialHash
+    n, sizes = 20_011, (9, 11, 13)
+    rng = np.random.default_rng(stride)
+    rec = rng.uniform(0, 9, (n, stride)).astype(np.float32)
+    src = torch.zeros(n * stride + 8, device="cuda")
+    src[skew:skew + n * stride] = torch.from_numpy(rec.ravel()).cuda()
+    dst = torch.full_like(src, -7.0)
+    ranges = torch.full((2, 9 * 11 * 13 + 2), -7, dtype=torch.int32, device="cuda")  # rows start unaligned
+    perm = torch.empty(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    sh = SpatialHash(sizes, 1.0, n)
+    sh.sort_device(src.data_ptr() + 4 * skew, n, stride, d_perm=perm.data_ptr(), d_cell_start=ranges[0].data_ptr() + 4,
+                   d_cell_end=ranges[1].data_ptr() + 4, d_sorted_records=dst.data_ptr() + 4 * skew)
+    sh.close()
+    want = R.spatial_hash(rec, sizes, 1.0)
+    assert np.array_equal(perm.cpu().numpy(), want["perm"])
+    out = dst.cpu().numpy()
+    assert np.array_equal(out[skew:skew + n * stride].reshape(n, stride), want["sorted_records"])
+    assert np.all(out[:skew] == -7) and np.all(out[skew + n * stride:] == -7)
+    for got, key in zip(ranges.cpu().numpy(), ("cell_start", "cell_end")):
+        assert np.array_equal(got[1:-1], want[key]) and got[0] == got[-1] == -7
+
+
+@pytest.mark.gpu
 def test_gpu_edge_cases():
     gpu_case((3, 4, 5), 1.0, np.zeros((0, 3), np.float32))                      # empty
     gpu_case((3, 4, 5), 1.0, np.array([[2.5, 0.5, 4.9]], np.float32))            # one particle
