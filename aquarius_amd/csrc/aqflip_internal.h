@@ -148,6 +148,14 @@ void launch_hash_count(const Geom& G, Particles P, long long Np, Bins B, hipStre
 void launch_scan(const Geom& G, Bins B, hipStream_t s, int* start = nullptr, int* end = nullptr);
 void launch_scatter_sort_gather(const Geom& G, Particles cur, Particles alt, long long Np, int K,
                                 Bins B, hipStream_t s);
+// Exports in the layouts of the C ABI.
+void launch_export_particles(Particles P, long long Np, int K, float* pos, float* vel, float4* frac, hipStream_t s);
+struct ExportField {
+  enum Kind { kScalar, kByte, kBits, kVector, kCount } kind;
+  bool face;           // the face extent instead of the interior
+  const void* src[4];  // kVector: the components, null = 0
+};
+void launch_export_field(const Geom& G, const ExportField& f, long long n, void* out, hipStream_t s);
 // Standalone spatial hashing (records of `stride` floats, position first).
 void launch_hash_records(const Geom& G, const float* pos, long long n, int stride, Bins B, hipStream_t s);
 void launch_scatter_segsort(const Geom& G, long long n, Bins B, hipStream_t s);

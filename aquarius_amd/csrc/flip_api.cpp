@@ -101,6 +101,8 @@ struct aq_flip {
   aq_flip_solver solver{AQ_SOLVE_FIXED, 1e-4, 100000, 50, 20, 0};
   aq_unet* net = nullptr;
   aq_flip_solver_stats sstats{};
+  void* export_buf = nullptr;  // scratch of field exports larger than a particle array
+  size_t export_cap = 0;
   float* p_keep = nullptr;  // the iterate before a U-Net correction (allocated on first use)
 
   bool timing = false;
@@ -1300,32 +1302,19 @@ aq_status aq_flip_run_stage(aq_flip* h, int32_t stage) {
 
 int64_t aq_flip_particle_count(const aq_flip* h) { return h ? h->Np : 0; }
 
+// The arrays of the particle buffer a step would overwrite next serve as scratch between
+// steps: 48 bytes per particle, an export takes 40.
 aq_status aq_flip_get_particles(aq_flip* h, float* pos, float* vel, float* frac4) {
   if (!h) return fail(AQ_EINVAL, "null handle");
-  const long long n = h->Np;
-  std::vector<float4> a, b, c;
-  const Particles& P = h->P[h->cur];
-  AQ_TRY(d2h(h, a, P.a, (size_t)n));
-  AQ_TRY(d2h(h, b, P.b, (size_t)n));
-  if (h->K > 2) AQ_TRY(d2h(h, c, P.c, (size_t)n));
-  for (long long i = 0; i < n; ++i) {
-    if (pos) {
-      pos[3 * i] = a[i].x;
-      pos[3 * i + 1] = a[i].y;
-      pos[3 * i + 2] = a[i].z;
-    }
-    if (vel) {
-      vel[3 * i] = a[i].w;
-      vel[3 * i + 1] = b[i].x;
-      vel[3 * i + 2] = b[i].y;
-    }
-    if (frac4) {
-      frac4[4 * i] = b[i].z;
-      frac4[4 * i + 1] = h->K > 1 ? b[i].w : 0.f;
-      frac4[4 * i + 2] = h->K > 2 ? c[i].x : 0.f;
-      frac4[4 * i + 3] = h->K > 3 ? c[i].y : 0.f;
-    }
-  }
+  const size_t n = (size_t)h->Np;
+  const Particles& S = h->P[h->cur ^ 1];
+  launch_export_particles(h->P[h->cur], h->Np, h->K, pos ? (float*)S.a : nullptr, vel ? (float*)S.b : nullptr,
+                          frac4 ? S.c : nullptr, h->stream);
+  HIP_TRY(hipGetLastError());
+  if (pos) HIP_TRY(hipMemcpyAsync(pos, S.a, n * 3 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+  if (vel) HIP_TRY(hipMemcpyAsync(vel, S.b, n * 3 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+  if (frac4) HIP_TRY(hipMemcpyAsync(frac4, S.c, n * 4 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipStreamSynchronize(h->stream));
   return AQ_OK;
 }
 
@@ -1355,77 +1344,37 @@ aq_status aq_flip_get_field(aq_flip* h, int32_t field, void* dst, size_t bytes) 
   const size_t n = field_elems(h, field, &w, &isInt);
   if (n == 0) return fail(AQ_EINVAL, "unknown field");
   if (bytes != n * w * 4) return fail(AQ_EINVAL, "byte count does not match the field");
-  const Geom& G = h->G;
-  const size_t nc = (size_t)G.ncell;
-  float* F = (float*)dst;
-  int32_t* I = (int32_t*)dst;
-  const bool face = (field == AQ_FIELD_CONTENT || field == AQ_FIELD_VELOCITY ||
-                     field == AQ_FIELD_NEW_VELOCITY);
-  const int EX = face ? G.X + 1 : G.X, EYe = face ? G.Y + 1 : G.Y, EZe = face ? G.Z + 1 : G.Z;
-  auto each = [&](auto&& fn) {
-    size_t o = 0;
-    for (int x = 0; x < EX; ++x)
-      for (int y = 0; y < EYe; ++y)
-        for (int z = 0; z < EZe; ++z, ++o) fn(o, (size_t)G.g(x, y, z));
-  };
+  const Grid& gr = h->gr;
+  ExportField f{ExportField::kScalar, false, {}};
   switch (field) {
-    case AQ_FIELD_CONTENT: {
-      std::vector<uint8_t> c;
-      AQ_TRY(d2h(h, c, h->gr.content, nc));
-      each([&](size_t o, size_t g) { I[o] = c[g]; });
+    case AQ_FIELD_CONTENT: f = {ExportField::kByte, true, {gr.content}}; break;
+    case AQ_FIELD_VELOCITY: f = {ExportField::kVector, true, {gr.vel[0], gr.vel[1], gr.vel[2]}}; break;
+    case AQ_FIELD_NEW_VELOCITY:
+      f = {ExportField::kVector, true, {gr.nvel[h->nv][0], gr.nvel[h->nv][1], gr.nvel[h->nv][2]}};
       break;
-    }
-    case AQ_FIELD_VELOCITY:
-    case AQ_FIELD_NEW_VELOCITY: {
-      std::vector<float> comp[3];
-      for (int a = 0; a < 3; ++a)
-        AQ_TRY(d2h(h, comp[a], field == AQ_FIELD_VELOCITY ? h->gr.vel[a] : h->gr.nvel[h->nv][a], nc));
-      each([&](size_t o, size_t g) {
-        for (int a = 0; a < 3; ++a) F[4 * o + a] = comp[a][g];
-        F[4 * o + 3] = 0.f;
-      });
-      break;
-    }
-    case AQ_FIELD_PRESSURE:
-    case AQ_FIELD_DIVERGENCE:
-    case AQ_FIELD_DENSITY: {
-      const float* src = field == AQ_FIELD_PRESSURE ? h->gr.p[h->pb]
-                         : field == AQ_FIELD_DIVERGENCE ? h->gr.div
-                                                        : h->gr.density;
-      std::vector<float> v;
-      AQ_TRY(d2h(h, v, src, nc));
-      each([&](size_t o, size_t g) { F[o] = v[g]; });
-      break;
-    }
-    case AQ_FIELD_PARTICLE_COUNT: {
-      std::vector<int> off;
-      AQ_TRY(d2h(h, off, h->B.offsets, (size_t)G.ncells_hash + 1));
-      for (int c = 0; c < G.ncells_hash; ++c) {
-        const int cnt = off[c + 1] - off[c];
-        I[c] = cnt > 0 ? cnt - 1 : 0;  // cellEnd - cellStart (Fluid_3D_FLIP.cu:180)
-      }
-      break;
-    }
-    case AQ_FIELD_HAS_VELOCITY: {
-      std::vector<uint8_t> v;
-      AQ_TRY(d2h(h, v, h->gr.hasvel[h->hv], nc));
-      each([&](size_t o, size_t g) {
-        for (int a = 0; a < 3; ++a) I[4 * o + a] = (v[g] >> a) & 1;
-        I[4 * o + 3] = 0;
-      });
-      break;
-    }
-    case AQ_FIELD_VOLUME_FRACTIONS:
-    case AQ_FIELD_NEW_VOLUME_FRACTIONS: {
-      std::vector<float> comp[4];
-      for (int a = 0; a < h->K; ++a)
-        AQ_TRY(d2h(h, comp[a], field == AQ_FIELD_VOLUME_FRACTIONS ? h->gr.vf[a] : h->gr.nvf[h->nf][a], nc));
-      each([&](size_t o, size_t g) {
-        for (int a = 0; a < 4; ++a) F[4 * o + a] = a < h->K ? comp[a][g] : 0.f;
-      });
-      break;
-    }
+    case AQ_FIELD_PRESSURE: f.src[0] = gr.p[h->pb]; break;
+    case AQ_FIELD_DIVERGENCE: f.src[0] = gr.div; break;
+    case AQ_FIELD_DENSITY: f.src[0] = gr.density; break;
+    case AQ_FIELD_PARTICLE_COUNT: f = {ExportField::kCount, false, {h->B.offsets}}; break;
+    case AQ_FIELD_HAS_VELOCITY: f = {ExportField::kBits, false, {gr.hasvel[h->hv]}}; break;
+    default:  // the volume fractions
+      f.kind = ExportField::kVector;
+      for (int a = 0; a < h->K; ++a) f.src[a] = field == AQ_FIELD_VOLUME_FRACTIONS ? gr.vf[a] : gr.nvf[h->nf][a];
   }
+  // scratch: an array of the idle particle buffer (see aq_flip_get_particles) if it is large
+  // enough, else one of its own, kept
+  void* scratch = h->P[h->cur ^ 1].a;
+  if (bytes > (size_t)h->Np * sizeof(float4)) {
+    if (bytes > h->export_cap) {
+      AQ_TRY(h->alloc(&h->export_buf, bytes));
+      h->export_cap = bytes;
+    }
+    scratch = h->export_buf;
+  }
+  launch_export_field(h->G, f, (long long)n, scratch, h->stream);
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(dst, scratch, bytes, hipMemcpyDeviceToHost, h->stream));
+  HIP_TRY(hipStreamSynchronize(h->stream));
   return AQ_OK;
 }
 

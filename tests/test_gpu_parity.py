@@ -131,6 +131,29 @@ def test_stagewise_multiphase_24():
     run_stagewise(cfg, steps=2, label="multiphase_24")
 
 
+@pytest.mark.parametrize("n,phases", [(1, 1), (3, 3), (40, 2), (3000, 4)])
+def test_exports_with_few_particles(n, phases):
+    """Every export of a handle whose particle arrays are smaller than its fields (the
+    exports' scratch) and, with 3,000 particles, larger than some: against the oracle, on
+    odd extents, before and after a step."""
+    cfg = configs.make_config(12, dt=0.01, pressure_iters=8, diffusion_iters=4, phase_count=phases, extent=(9, 12, 7))
+    rng = np.random.default_rng(n)
+    h = 10 / 12
+    pos = (rng.uniform(0.3, 0.7, (n, 3)) * np.array([9, 12, 7]) * h).astype(np.float32)
+    vel = rng.standard_normal((n, 3)).astype(np.float32)
+    frac = np.zeros((n, 4), np.float32)
+    frac[np.arange(n), rng.integers(0, phases, n)] = 1
+    gpu, orc = FlipHandle(cfg, pos, vel, frac), ob.Oracle(cfg, pos=pos, vel=vel, frac4=frac)
+    for step in range(2):
+        for name in aq.FIELDS:
+            if step or name != "particle_count":  # the oracle counts inside a step
+                check_field(name, gpu, orc, f"step {step} ")
+        check_particles(gpu, orc)
+        gpu.step()
+        orc.step()
+    gpu.close()
+
+
 def test_stagewise_edge_configs():
     # non-cubic grid, full boundary coverage, warm-started pressure, 4 phases
     cfg = configs.make_config(0, dt=0.01, pressure_iters=25, diffusion_iters=5, extent=(12, 16, 20),
