@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -51,6 +52,84 @@ aq_status fail(aq_status s, const std::string& msg) {
     if (s_ != AQ_OK) return s_;   \
   } while (0)
 
+// Device memory of handles, kept for the next handle. Mapping and unmapping a handle's
+// memory cost more than a short scene's steps (64^3: 1 + 7 ms against 0.37 ms a step;
+// 256^3: 7 + 11 ms, and 150 ms once a process had cycled through the card's memory), so a
+// destroyed handle's blocks are kept and handed to the next request that they fit. Blocks
+// enter after their handle's streams have been synchronised and are cleared by whoever
+// takes them, so neither threads nor streams matter beyond the lock. Bounded: at most
+// kKeepBytes per device, a block that kKeepPuts later ones passed over is freed, and all
+// are when an allocation fails. Blocks below kKeepMin are not kept: the runtime serves
+// those from its own chunks.
+class BlockCache {
+ public:
+  hipError_t get(size_t bytes, void** p, size_t* size) {
+    *size = (bytes + kGranule - 1) / kGranule * kGranule;
+    if (bytes < kKeepMin) {
+      *size = bytes;
+      return hipMalloc(p, bytes);
+    }
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+    std::lock_guard<std::mutex> lock(mutex_);
+    auto best = blocks_.end();
+    for (auto b = blocks_.begin(); b != blocks_.end(); ++b)
+      if (b->dev == dev && b->size >= bytes && b->size <= *size + *size / 4 &&
+          (best == blocks_.end() || b->size < best->size))
+        best = b;
+    if (best != blocks_.end()) {
+      *p = best->p;
+      *size = best->size;
+      blocks_.erase(best);
+      return hipSuccess;
+    }
+    hipError_t e = hipMalloc(p, *size);
+    if (e != hipErrorOutOfMemory || blocks_.empty()) return e;
+    (void)hipGetLastError();
+    for (const Block& b : blocks_) (void)hipFree(b.p);
+    blocks_.clear();
+    return hipMalloc(p, *size);
+  }
+  // p: no work on it is pending.
+  void put(void* p, size_t size, int dev) {
+    if (size < kKeepMin) {
+      (void)hipFree(p);
+      return;
+    }
+    std::lock_guard<std::mutex> lock(mutex_);
+    blocks_.push_back(Block{p, size, dev, ++puts_});
+    size_t held = 0;  // newest first, what fits the bound stays
+    for (size_t i = blocks_.size(); i-- > 0;) {
+      const Block& b = blocks_[i];
+      if (b.dev != dev) continue;
+      held += b.size;
+      if (held <= kKeepBytes && puts_ - b.at < kKeepPuts) continue;
+      held -= b.size;
+      (void)hipFree(b.p);
+      blocks_.erase(blocks_.begin() + (long)i);
+    }
+  }
+
+ private:
+  static constexpr size_t kGranule = 1 << 21, kKeepMin = 1 << 20, kKeepBytes = 12ull << 30;
+  static constexpr uint64_t kKeepPuts = 64;
+  struct Block {
+    void* p;
+    size_t size;
+    int dev;
+    uint64_t at;
+  };
+  std::mutex mutex_;
+  std::vector<Block> blocks_;
+  uint64_t puts_ = 0;
+};
+// Never destroyed: at process exit the runtime may be gone before it, and the memory goes
+// with the process.
+BlockCache& block_cache() {
+  static BlockCache* c = new BlockCache;
+  return *c;
+}
+
 int boundary_coverage(int A, int B, bool ref) {
   const int pairs = (A + 1) * (B + 1);
   if (!ref) return pairs;
@@ -82,7 +161,12 @@ struct aq_flip {
   // Paired diffusion sweeps after one that changed no bit skip their identical work.
   bool skip_fixed = true;
   int listed_grid = 0;  // 0: the default listed sweep grids; n: at most n workgroups
-  std::vector<void*> allocs;
+  struct Alloc {
+    void* p;
+    size_t size;
+  };
+  std::vector<Alloc> allocs;
+  int dev = 0;
 
   Particles P[2]{};
   int cur = 0;
@@ -170,18 +254,20 @@ struct aq_flip {
       hipGraphExecDestroy(g.exec);
       hipGraphDestroy(g.graph);
     }
-    for (void* p : allocs) hipFree(p);
-    for (hipEvent_t e : event_pool) hipEventDestroy(e);
     if (side) hipStreamSynchronize(side);
+    for (const Alloc& a : allocs) block_cache().put(a.p, a.size, dev);
+    for (hipEvent_t e : event_pool) hipEventDestroy(e);
     if (ev_fork) hipEventDestroy(ev_fork);
     if (ev_join) hipEventDestroy(ev_join);
     if (side) hipStreamDestroy(side);
     if (stream) hipStreamDestroy(stream);
   }
 
+  // Zeroed.
   aq_status alloc(void** p, size_t bytes) {
-    HIP_TRY(hipMalloc(p, bytes));
-    allocs.push_back(*p);
+    size_t size = 0;
+    HIP_TRY(block_cache().get(bytes, p, &size));
+    allocs.push_back({*p, size});
     HIP_TRY(hipMemsetAsync(*p, 0, bytes, stream));
     return AQ_OK;
   }
@@ -278,6 +364,66 @@ aq_status check_positions(const aq_flip* h, const float* pos, long long n) {
   return AQ_OK;
 }
 
+// Hands out the arrays of one block, 256 bytes apart at least; without a base it only
+// measures.
+struct Carver {
+  char* base = nullptr;
+  size_t at = 0;
+  template <typename T>
+  void take(T** p, size_t n) {
+    *p = base ? (T*)(base + at) : nullptr;
+    at += (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
+  }
+};
+void carve_arrays(aq_flip* h, Carver& c) {
+  const Geom& G = h->G;
+  const size_t Np = (size_t)h->Np, nc = (size_t)G.ncell, nch = (size_t)G.ncells_hash;
+  for (int b = 0; b < 2; ++b) {
+    c.take(&h->P[b].a, Np);
+    c.take(&h->P[b].b, Np);
+    c.take(&h->P[b].c, Np);
+  }
+  Grid& gr = h->gr;
+  c.take(&gr.content, nc);
+  for (int a = 0; a < 3; ++a) {
+    c.take(&gr.vel[a], nc);
+    c.take(&gr.nvel[0][a], nc);
+    c.take(&gr.nvel[1][a], nc);
+    c.take(&gr.nvo[a], nc);
+  }
+  for (int b = 0; b < 2; ++b) {
+    c.take(&gr.hasvel[b], nc);
+    c.take(&gr.p[b], nc);
+  }
+  c.take(&gr.div, nc);
+  c.take(&gr.rhs, nc);
+  c.take(&gr.density, nc);
+  // One flag per 256-cell block plus one slot that stays 0, so the sweep kernels'
+  // pairs of blocks never read past the array.
+  c.take(&gr.active, (nch + 255) / 256 + 1);
+  c.take(&gr.alist, (size_t)sweep_chunks(G) + 1);
+  c.take(&gr.btab, (size_t)sweep_table_entries(G));
+  c.take(&gr.dchange, 4);
+  c.take(&gr.stepstamp, 1);
+  c.take(&gr.rowstamp, (size_t)(G.X + 1) * (G.Y + 1));
+  for (int a = 0; a < 4; ++a) {
+    c.take(&gr.vf[a], nc);
+    c.take(&gr.nvf[0][a], nc);
+    c.take(&gr.nvf[1][a], nc);
+  }
+  c.take(&h->B.count, nch);
+  c.take(&h->B.offsets, nch + 1);
+  c.take(&h->B.partials, (nch + 4095) / 4096 + 1);
+  c.take(&h->B.hash, Np);
+  c.take(&h->B.rank, Np);
+  c.take(&h->B.perm, Np);
+  c.take(&h->B.multi, nch);  // zeroed here; k_segsort clears what it reads
+  h->nparts_red = 512;  // volume statistics: 512 partial rows of 16 columns
+  // (the residual uses two columns per sweep chunk)
+  c.take(&h->red_partial, std::max<size_t>((size_t)h->nparts_red * 16, 2 * (size_t)sweep_chunks(G)));
+  c.take(&h->red_out, 16);
+}
+
 aq_status setup(aq_flip* h, const aq_flip_config* cfg, long long Np) {
   h->cfg = *cfg;
   Geom& G = h->G;
@@ -314,53 +460,14 @@ aq_status setup(aq_flip* h, const aq_flip_config* cfg, long long Np) {
   HIP_TRY(hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking));
   HIP_TRY(hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming));
   HIP_TRY(hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming));
-  for (int b = 0; b < 2; ++b) {
-    AQ_TRY(h->allocT(&h->P[b].a, (size_t)Np));
-    AQ_TRY(h->allocT(&h->P[b].b, (size_t)Np));
-    AQ_TRY(h->allocT(&h->P[b].c, (size_t)Np));
-  }
-  const size_t nc = (size_t)G.ncell;
-  Grid& gr = h->gr;
-  AQ_TRY(h->allocT(&gr.content, nc));
-  for (int a = 0; a < 3; ++a) {
-    AQ_TRY(h->allocT(&gr.vel[a], nc));
-    AQ_TRY(h->allocT(&gr.nvel[0][a], nc));
-    AQ_TRY(h->allocT(&gr.nvel[1][a], nc));
-  }
-  for (int a = 0; a < 3; ++a) AQ_TRY(h->allocT(&gr.nvo[a], nc));
-  AQ_TRY(h->allocT(&gr.hasvel[0], nc));
-  AQ_TRY(h->allocT(&gr.hasvel[1], nc));
-  AQ_TRY(h->allocT(&gr.p[0], nc));
-  AQ_TRY(h->allocT(&gr.p[1], nc));
-  AQ_TRY(h->allocT(&gr.div, nc));
-  AQ_TRY(h->allocT(&gr.rhs, nc));
-  AQ_TRY(h->allocT(&gr.density, nc));
-  // One flag per 256-cell block plus one slot that stays 0, so the sweep kernels'
-  // pairs of blocks never read past the array.
-  AQ_TRY(h->allocT(&gr.active, (size_t)(G.ncells_hash + 255) / 256 + 1));
-  AQ_TRY(h->allocT(&gr.alist, (size_t)sweep_chunks(G) + 1));
-  AQ_TRY(h->allocT(&gr.btab, (size_t)sweep_table_entries(G)));
-  set_listed_grids(G, gr, h->listed_grid);
-  AQ_TRY(h->allocT(&gr.dchange, 4));
-  AQ_TRY(h->allocT(&gr.stepstamp, 1));
-  AQ_TRY(h->allocT(&gr.rowstamp, (size_t)(G.X + 1) * (G.Y + 1)));
-  for (int a = 0; a < 4; ++a) {
-    AQ_TRY(h->allocT(&gr.vf[a], nc));
-    AQ_TRY(h->allocT(&gr.nvf[0][a], nc));
-    AQ_TRY(h->allocT(&gr.nvf[1][a], nc));
-  }
-  const int nch = G.ncells_hash;
-  AQ_TRY(h->allocT(&h->B.count, (size_t)nch));
-  AQ_TRY(h->allocT(&h->B.offsets, (size_t)nch + 1));
-  AQ_TRY(h->allocT(&h->B.partials, (size_t)(nch + 4095) / 4096 + 1));
-  AQ_TRY(h->allocT(&h->B.hash, (size_t)Np));
-  AQ_TRY(h->allocT(&h->B.rank, (size_t)Np));
-  AQ_TRY(h->allocT(&h->B.perm, (size_t)Np));
-  AQ_TRY(h->allocT(&h->B.multi, (size_t)nch));  // zeroed here; k_segsort clears what it reads
-  h->nparts_red = 512;  // volume statistics: 512 partial rows of 16 columns
-  // (the residual uses two columns per sweep chunk)
-  AQ_TRY(h->allocT(&h->red_partial, std::max<size_t>((size_t)h->nparts_red * 16, 2 * (size_t)sweep_chunks(G))));
-  AQ_TRY(h->allocT(&h->red_out, 16));
+  HIP_TRY(hipGetDevice(&h->dev));
+  // One block for every array: measured first, then carved.
+  Carver c;
+  carve_arrays(h, c);
+  AQ_TRY(h->alloc((void**)&c.base, c.at));
+  c.at = 0;
+  carve_arrays(h, c);
+  set_listed_grids(G, h->gr, h->listed_grid);
   return AQ_OK;
 }
 

@@ -154,6 +154,27 @@ def test_exports_with_few_particles(n, phases):
     gpu.close()
 
 
+def test_handles_take_over_each_others_memory():
+    """A handle's memory goes to later handles of a similar size: a scene gives the same bits
+    in memory that other scenes (other sizes, phases, solver state) have left, and with
+    several threads creating and destroying handles at once."""
+    from concurrent.futures import ThreadPoolExecutor
+    scenes = [configs.make_config(n, dt=0.01, pressure_iters=20, diffusion_iters=6, phase_count=k, sphere_phase=k - 1,
+                                  extent=(n, n + 2, n - 3)) for n, k in ((24, 1), (24, 2), (23, 4), (40, 2))]
+
+    def run(i):
+        with FlipHandle(scenes[i]) as h:
+            h.steps(3)
+            h.solve_pressure_mgpcg(1e-6)
+            h.steps(1)
+            return [h.get_field(f) for f in aq.FIELDS] + list(h.get_particles())
+    first = [run(i) for i in range(4)]
+    with ThreadPoolExecutor(4) as pool:
+        for i, got in zip([0, 1, 2, 3] * 4, pool.map(run, [0, 1, 2, 3] * 4)):
+            for a, b in zip(got, first[i]):
+                assert np.array_equal(a.view(np.int32), b.view(np.int32))
+
+
 def test_stagewise_edge_configs():
     # non-cubic grid, full boundary coverage, warm-started pressure, 4 phases
     cfg = configs.make_config(0, dt=0.01, pressure_iters=25, diffusion_iters=5, extent=(12, 16, 20),
