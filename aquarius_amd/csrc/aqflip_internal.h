@@ -200,6 +200,10 @@ void launch_fill_pressure_zero(const Geom& G, Grid gr, int pb, hipStream_t s);
 // cells and AIR cells are skipped -- valid once both buffers hold 0 on AIR.
 // pzero = 1: the input is the zero guess (not read); needs full = 1.
 void launch_jacobi(const Geom& G, Grid gr, int pin, int full, int pzero, hipStream_t s);
+// All sweeps of a step in one launch, on grids that fit in a workgroup's LDS (K channel sets).
+bool small_grid(const Geom& G, int K);
+void launch_sweeps_small(const Geom& G, Grid gr, int K, int pb, int pzero, int nj, int nf, float lambda, double inv_cc,
+                         int nd, int npaired, int skip_ok, hipStream_t s);
 void launch_air_pressure_zero(const Geom& G, Grid gr, int pb, hipStream_t s);
 void launch_project(const Geom& G, Grid gr, int nv, int hv, int pb, hipStream_t s);
 // near_rows: only the face rows stamped by this step's P2G (passes 2 and 3 of a step, see

@@ -174,6 +174,7 @@ struct aq_flip {
   int nv = 0, hv = 0, pb = 0, nf = 0;  // current buffer of each ping-pong pair
   // air_clean[i]: pressure buffer i holds 0 on every AIR cell of the current content.
   bool air_clean[2] = {false, false};
+  bool p2g_content = false;  // every interior cell is AIR or FLUID (see content_changed)
   Bins B{};
   StepParams sp{};
   int nparts_red = 0;
@@ -498,7 +499,11 @@ aq_status upload_particles(aq_flip* h, const float* pos, const float* vel, const
 // ---- stages --------------------------------------------------------------
 
 // New FLUID/AIR marking: AIR cells of either pressure buffer may hold old values.
-void content_changed(aq_flip* h) { h->air_clean[0] = h->air_clean[1] = false; }
+// p2g: the marking is P2G's, AIR or FLUID on every interior cell (an upload may hold others).
+void content_changed(aq_flip* h, bool p2g) {
+  h->air_clean[0] = h->air_clean[1] = false;
+  h->p2g_content = p2g;
+}
 
 // hash is already binned (count filled): scan, scatter, segment sort, gather, P2G.
 // Inside a step the P2G kernel is timed in its own bucket (split = true).
@@ -512,7 +517,7 @@ void transfer_after_count(aq_flip* h, bool split = false) {
   }
   launch_p2g(h->G, h->P[h->cur], h->Np, h->K, h->B, h->gr, h->nv, h->hv, h->nf, h->sp, h->stream);
   if (split) h->end(AQ_STAGE_P2G);
-  content_changed(h);
+  content_changed(h, true);
 }
 
 void clear_bins(aq_flip* h) { launch_fill_u32(h->B.count, 0u, h->G.ncells_hash, h->stream); }
@@ -529,7 +534,27 @@ void stage_transfer(aq_flip* h) {
 // from_zero: the sweeps start from the zero guess; the first one does not read the
 // input buffer (its neighbours are 0) and writes every cell, so neither buffer needs
 // clearing first.
+//
+// Small grids run all n sweeps in one launch, in place. One workgroup per chain does the
+// work, so the rule weighs the FLUID cells (times K with the diffusion chain beside it),
+// taken from the seeding density of 8 particles per cell, against launches that cost about
+// 2 us each. Microseconds per step, one launch / a launch per sweep, sweep counts in brackets:
+// 16^3 with 1,160 FLUID cells 110/270 (100), 80/87 (8); 20^3 with 7,600 205/287 (100), 100/98
+// (8); 24^3 with 13,100 453/356 (100); both chains, 100 sweeps each: K = 2 with 3,900 cells
+// 287/428 (all 16^3) and 163/366 (24^3), 7,600 cells 732/441; K = 4 with 3,900 cells 586/478.
+constexpr int kSmallSweeps = 16;
+constexpr long long kSmallPressure = 7000, kSmallPaired = 8192;
+bool small_sweeps(const aq_flip* h, int n, int K) {
+  const long long fluid = std::min((long long)h->G.ncells_hash, (h->Np + 7) / 8);
+  return n >= kSmallSweeps && h->p2g_content && small_grid(h->G, K) &&
+         (K > 1 ? fluid * K <= kSmallPaired : fluid <= kSmallPressure);
+}
 void jacobi_sweeps(aq_flip* h, int n, bool from_zero = false) {
+  if (small_sweeps(h, n, 1)) {
+    launch_sweeps_small(h->G, h->gr, 1, h->pb, from_zero ? 1 : 0, n, h->nf, 0.f, 1.0, 0, 0, 0, h->stream);
+    h->air_clean[h->pb] = true;
+    return;
+  }
   for (int i = 0; i < n; ++i) {
     const int out = h->pb ^ 1;
     const bool z = from_zero && i == 0;
@@ -582,7 +607,13 @@ void fused_pressure_diffusion(aq_flip* h) {
   const bool zero = h->cfg.pressure_init == AQ_PRESSURE_ZERO;  // first sweep from the zero guess
   const int n = std::min(h->cfg.pressure_iters, h->cfg.diffusion_iters);
   h->begin(AQ_STAGE_PRESSURE_DIFFUSION);
-  for (int i = 0; i < n; ++i) {
+  const bool small = small_sweeps(h, n, h->K);
+  if (small) {  // both chains whole, side by side
+    launch_sweeps_small(h->G, h->gr, h->K, h->pb, zero ? 1 : 0, h->cfg.pressure_iters, h->nf, h->sp.lambda,
+                        h->sp.inv_cc, h->cfg.diffusion_iters, n, h->skip_fixed ? 1 : 0, h->stream);
+    h->air_clean[h->pb] = true;
+  }
+  for (int i = 0; i < n && !small; ++i) {
     const int out = h->pb ^ 1;
     const bool z = zero && i == 0;
     launch_jacobi_diffusion(h->G, h->gr, h->K, h->pb, (z || !h->air_clean[out]) ? 1 : 0, h->nf,
@@ -594,10 +625,10 @@ void fused_pressure_diffusion(aq_flip* h) {
   }
   h->end(AQ_STAGE_PRESSURE_DIFFUSION, n);
   h->begin(AQ_STAGE_PRESSURE);
-  jacobi_sweeps(h, h->cfg.pressure_iters - n);
+  if (!small) jacobi_sweeps(h, h->cfg.pressure_iters - n);
   h->end(AQ_STAGE_PRESSURE, h->cfg.pressure_iters - n);
   h->begin(AQ_STAGE_DIFFUSION);
-  diffusion_sweeps(h, h->stream, n);
+  if (!small) diffusion_sweeps(h, h->stream, n);
   h->end(AQ_STAGE_DIFFUSION, h->cfg.diffusion_iters - n);
 }
 
@@ -1514,7 +1545,7 @@ aq_status aq_flip_set_field(aq_flip* h, int32_t field, const void* src, size_t b
       AQ_TRY(d2h(h, c, h->gr.content, nc));
       each([&](size_t o, size_t g) { c[g] = (uint8_t)I[o]; });
       AQ_TRY(h2d(h, h->gr.content, c));
-      content_changed(h);
+      content_changed(h, false);
       refresh_rhs(h);
       HIP_TRY(hipStreamSynchronize(h->stream));
       break;

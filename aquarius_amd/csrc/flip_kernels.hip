@@ -2142,6 +2142,263 @@ void launch_jacobi_diffusion(const Geom& G, Grid gr, int K, int pin, int fullJ, 
   }
 }
 
+// ------------------------------------------------------------------ small grids
+// All of a step's sweeps in one launch, where the grid fits in a workgroup's LDS. A sweep
+// launch cannot take less than about 2 us; here a sweep is the FLUID cells' LDS reads, one
+// barrier (two for diffusion) and the writes. Block 0 runs the pressure sweeps and block 1
+// the diffusion sweeps (independent chains, see k_jacobi_diffusion). The FLUID cells are
+// listed first, NP per thread, and stay with their thread: index and the sides that have a
+// neighbour in one register, the right-hand side in another. Same arithmetic and order as
+// jacobi_value and diffusion_cell, so the same bits. Interior cells must be AIR or FLUID.
+// Bound by instruction issue on its one CU per chain: at 16^3 with 1,500 FLUID cells 60
+// sweeps take 27 us, against about 125 us as launches of their own. With both buffers in LDS
+// a pressure sweep has one barrier; border copies written by their owners instead of the
+// clamped neighbour indices cost 61 us.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallCells = 20000;
+constexpr int kSmallLds = 2 * kSmallCells;  // pressure: two buffers; diffusion: one per fraction
+constexpr int kSmallMost = (kSmallCells + kSmallThreads - 1) / kSmallThreads;
+struct SmallArgs {
+  const uint8_t* content;
+  const float* rhs;
+  float* p;          // in and out
+  int pzero, nj;     // from zero (p not read); pressure sweeps
+  float* f[4];       // fractions, in and out
+  int nd, npaired;   // diffusion sweeps; how many of them are paired ones (counted in dchange[3])
+  int skip_ok;
+  float lambda;
+  double inv_cc;
+  uint32_t* dchange;
+};
+struct SmallShared {
+  float v[kSmallLds];
+  int cells;
+};
+constexpr int kSmallBatch = 4;  // cells per thread whose loads are in flight together
+// A field into LDS in the order of the linear cell index.
+__device__ __forceinline__ void small_load(const Geom& G, const float* __restrict__ src, float* v) {
+  for (int n0 = (int)threadIdx.x; n0 < G.ncells_hash; n0 += kSmallBatch * kSmallThreads) {
+    float t[kSmallBatch];
+#pragma unroll
+    for (int k = 0; k < kSmallBatch; ++k) {
+      const int n = min(n0 + k * kSmallThreads, G.ncells_hash - 1);
+      int x, y, z;
+      cell_of(G, n, x, y, z);
+      t[k] = src[G.g(x, y, z)];
+    }
+#pragma unroll
+    for (int k = 0; k < kSmallBatch; ++k)
+      if (n0 + k * kSmallThreads < G.ncells_hash) v[n0 + k * kSmallThreads] = t[k];
+  }
+}
+__device__ __forceinline__ void small_store(const Geom& G, float* __restrict__ dst, const float* v) {
+  for (int n = threadIdx.x; n < G.ncells_hash; n += kSmallThreads) {
+    int x, y, z;
+    cell_of(G, n, x, y, z);
+    dst[G.g(x, y, z)] = v[n];
+  }
+}
+__device__ __forceinline__ void small_zero(const Geom& G, float* v) {
+  for (int n = threadIdx.x; n < G.ncells_hash; n += kSmallThreads) v[n] = 0.f;
+}
+// The FLUID cells' linear indices, in m.v as 16-bit values; their number.
+__device__ __forceinline__ int small_list(const Geom& G, const uint8_t* __restrict__ content, SmallShared& m) {
+  uint16_t* list = (uint16_t*)m.v;
+  if (threadIdx.x == 0) m.cells = 0;
+  __syncthreads();
+  const int lane = (int)(threadIdx.x & 63);
+  for (int n0 = 0; n0 < G.ncells_hash; n0 += kSmallBatch * kSmallThreads) {
+    uint8_t c[kSmallBatch];
+#pragma unroll
+    for (int k = 0; k < kSmallBatch; ++k) {
+      const int n = n0 + k * kSmallThreads + (int)threadIdx.x;
+      int x, y, z;
+      cell_of(G, min(n, G.ncells_hash - 1), x, y, z);
+      c[k] = content[G.g(x, y, z)];
+    }
+#pragma unroll
+    for (int k = 0; k < kSmallBatch; ++k) {
+      const int n = n0 + k * kSmallThreads + (int)threadIdx.x;
+      const bool fl = n < G.ncells_hash && c[k] == FLUID;
+      const unsigned long long mask = __ballot(fl);
+      int base = 0;
+      if (lane == 0 && mask) base = atomicAdd(&m.cells, __popcll(mask));
+      base = __shfl(base, 0, 64);
+      if (fl) list[base + __popcll(mask & ((1ull << lane) - 1ull))] = (uint16_t)n;
+    }
+  }
+  __syncthreads();
+  return m.cells;
+}
+// This thread's cells in one register each: linear index (16 bits), bits 16-21 for the sides
+// with a neighbour inside (+x, -x, +y, -y, +z, -z; the others read the cell itself, clamp to
+// edge), and whether the entry is one of the list's; entries past it repeat its first cell
+// and are not written.
+constexpr uint32_t kSmallOwn = 1u << 24;
+template <int NP>
+__device__ __forceinline__ void small_cells(const Geom& G, const SmallShared& m, int cells, uint32_t c[NP]) {
+  const uint16_t* list = (const uint16_t*)m.v;
+#pragma unroll
+  for (int k = 0; k < NP; ++k) {
+    const int e = k * kSmallThreads + (int)threadIdx.x;
+    const bool own = e < cells;
+    const int n = cells > 0 ? list[own ? e : 0] : 0;
+    int x, y, z;
+    cell_of(G, n, x, y, z);
+    const uint32_t sides = (x < G.X - 1 ? 1u : 0u) | (x > 0 ? 2u : 0u) | (y < G.Y - 1 ? 4u : 0u) |
+                           (y > 0 ? 8u : 0u) | (z < G.Z - 1 ? 16u : 0u) | (z > 0 ? 32u : 0u);
+    c[k] = (uint32_t)n | sides << 16 | (own ? kSmallOwn : 0u);
+  }
+  __syncthreads();  // the list's place is free
+}
+// A cell and its six neighbours. With many cells per thread c is made opaque, so that the
+// indices are formed at each use: kept over the sweeps, they spill.
+template <int NP>
+struct SmallAt {
+  int i, n[6];
+  __device__ __forceinline__ SmallAt(const Geom& G, uint32_t& c) {
+    if constexpr (NP > 8) asm volatile("" : "+v"(c));
+    i = (int)(c & 0xffffu);
+    const int sx = G.Y * G.Z, sy = G.Z;
+    n[0] = i + (side(c, 0) & sx);
+    n[1] = i - (side(c, 1) & sx);
+    n[2] = i + (side(c, 2) & sy);
+    n[3] = i - (side(c, 3) & sy);
+    n[4] = i + (side(c, 4) & 1);
+    n[5] = i - (side(c, 5) & 1);
+  }
+  static __device__ __forceinline__ int side(uint32_t c, int b) { return (int)(c << (15 - b)) >> 31; }  // all bits or none
+};
+template <int NP>
+__device__ __forceinline__ void small_pressure(const Geom& G, const SmallArgs& A, SmallShared& m, int cells) {
+  uint32_t c[NP];
+  float b[NP];
+  small_cells<NP>(G, m, cells, c);
+  float* v = m.v;
+  float* w = m.v + kSmallCells;
+  small_load(G, A.rhs, v);
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NP; ++k) b[k] = v[c[k] & 0xffffu];
+  __syncthreads();
+  if (A.pzero)
+    small_zero(G, v);
+  else
+    small_load(G, A.p, v);
+  small_zero(G, w);
+  __syncthreads();
+  for (int it = 0; it < A.nj; ++it) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      if (k * kSmallThreads >= cells) continue;
+      const SmallAt<NP> at(G, c[k]);
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 6; ++j) s += v[at.n[j]];
+      s += b[k];
+      if (c[k] & kSmallOwn) w[at.i] = div_exact(s, 1.0 / 6.0);
+    }
+    __syncthreads();
+    if (it == 0 && !A.pzero) {  // the first sweep read what AIR cells held; it leaves 0 there
+      small_zero(G, v);
+      __syncthreads();
+    }
+    float* t = v;
+    v = w;
+    w = t;
+  }
+  small_store(G, A.p, v);
+}
+template <int K, int NP>
+__device__ __forceinline__ void small_diffusion(const Geom& G, const SmallArgs& A, SmallShared& m, int cells) {
+  uint32_t c[NP];
+  small_cells<NP>(G, m, cells, c);
+  const int size = G.ncells_hash;
+#pragma unroll
+  for (int a = 0; a < K; ++a) small_load(G, A.f[a], m.v + a * size);
+  __syncthreads();
+  int done = 0;
+  for (bool go = true; go && done < A.nd; ++done) {
+    float r[NP][K];
+    bool changed = false;
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      if (k * kSmallThreads >= cells) continue;
+      const SmallAt<NP> at(G, c[k]);
+#pragma unroll
+      for (int a = 0; a < K; ++a) {
+        const float* v = m.v + a * size;
+        float t = 0.f;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) t += v[at.n[j]] * A.lambda;
+        t += v[at.i];
+        r[k][a] = div_exact(t, A.inv_cc);
+      }
+      float sum = r[k][0];
+#pragma unroll
+      for (int a = 1; a < K; ++a) sum += r[k][a];
+#pragma unroll
+      for (int a = 0; a < K; ++a) {
+        const float f = r[k][a] / sum;
+        changed |= (c[k] & kSmallOwn) && __float_as_uint(f) != __float_as_uint(m.v[a * size + at.i]);
+        r[k][a] = f;
+      }
+    }
+    // a sweep that changed nothing: all later ones would write the same values
+    go = __syncthreads_or(changed) || (!A.skip_ok && done + 1 < A.npaired);
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      if constexpr (NP > 8) asm volatile("" : "+v"(c[k]));
+      if (k * kSmallThreads < cells && (c[k] & kSmallOwn))
+#pragma unroll
+        for (int a = 0; a < K; ++a) m.v[a * size + (int)(c[k] & 0xffffu)] = r[k][a];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) A.dchange[3] += (uint32_t)min(done, A.npaired);  // paired sweeps computed
+#pragma unroll
+  for (int a = 0; a < K; ++a) small_store(G, A.f[a], m.v + a * size);
+}
+template <int K>
+__global__ __launch_bounds__(kSmallThreads) void k_sweeps_small(SmallArgs A, Geom G) {
+  __shared__ SmallShared m;
+  const int cells = small_list(G, A.content, m);
+  const int np = (cells + kSmallThreads - 1) / kSmallThreads;
+  if (blockIdx.x == 0) {
+    if (np <= 4)
+      small_pressure<4>(G, A, m, cells);
+    else if (np <= 8)
+      small_pressure<8>(G, A, m, cells);
+    else
+      small_pressure<kSmallMost>(G, A, m, cells);
+  } else if constexpr (K > 1) {
+    constexpr int kMost = std::min(kSmallMost, (kSmallLds / K + kSmallThreads - 1) / kSmallThreads);
+    if (np <= 4)
+      small_diffusion<K, 4>(G, A, m, cells);
+    else
+      small_diffusion<K, kMost>(G, A, m, cells);
+  }
+}
+bool small_grid(const Geom& G, int K) {
+  return G.ncells_hash <= kSmallCells && G.ncells_hash * std::max(K, 1) <= kSmallLds;
+}
+// nj pressure sweeps on p[pb], in place; with nd > 0 (K > 1) also nd diffusion sweeps on
+// nvf[nf], in place, of which the first npaired are the paired ones.
+void launch_sweeps_small(const Geom& G, Grid gr, int K, int pb, int pzero, int nj, int nf, float lambda, double inv_cc,
+                         int nd, int npaired, int skip_ok, hipStream_t s) {
+  SmallArgs A{gr.content, gr.rhs, gr.p[pb], pzero, nj, {}, nd, npaired, skip_ok, lambda, inv_cc, gr.dchange};
+  for (int a = 0; a < 4; ++a) A.f[a] = gr.nvf[nf][a];
+  const dim3 block(kSmallThreads);
+  if (nd == 0 || K == 1)
+    hipLaunchKernelGGL(k_sweeps_small<1>, dim3(1), block, 0, s, A, G);
+  else if (K == 2)
+    hipLaunchKernelGGL(k_sweeps_small<2>, dim3(2), block, 0, s, A, G);
+  else if (K == 3)
+    hipLaunchKernelGGL(k_sweeps_small<3>, dim3(2), block, 0, s, A, G);
+  else
+    hipLaunchKernelGGL(k_sweeps_small<4>, dim3(2), block, 0, s, A, G);
+}
+
 // ------------------------------------------------------------------ G2P and advection
 // getInterpolatedValueAtPoint (Fluid/MAC_Grid_3D.cuh:66-97) on one face component:
 // clamp to [0, N-1], trilinear lerps in the order z, y, x.

@@ -375,6 +375,40 @@ def test_full_steps_match_oracle_mixing_24(pressure_iters, diffusion_iters):
     gpu.close()
 
 
+@pytest.mark.parametrize("extent,phases,pressure_iters,diffusion_iters,keep,depth,sparse", [
+    ((5, 3, 4), 1, 16, 0, False, 0.5, False),     # fewer cells than a wave
+    ((16, 16, 16), 4, 16, 40, False, 0.25, False),  # diffusion goes on alone
+    ((20, 18, 27), 3, 41, 16, True, 0.1, False),  # pressure goes on alone, from the last step's
+    ((24, 24, 24), 1, 30, 0, False, 0.45, False),  # five to eight cells per thread
+    ((26, 26, 26), 2, 20, 17, True, 1.0, True),   # more, in both chains
+    ((27, 27, 27), 1, 17, 0, True, 1.0, True),    # nearly the most cells
+    ((27, 27, 28), 1, 17, 0, True, 0.1, False),   # one launch per sweep: too many cells
+])
+def test_sweeps_of_small_grids(extent, phases, pressure_iters, diffusion_iters, keep, depth, sparse):
+    """All sweeps of a step in one launch (grids that fit in LDS), over the numbers of
+    cells per thread, phases and chain lengths. sparse: one particle in every cell, so
+    that all are FLUID."""
+    cfg = configs.make_config(0, dt=0.01, extent=extent, pressure_iters=pressure_iters,
+                              diffusion_iters=diffusion_iters, pool_depth=depth, radius=0.2,
+                              center=(0.5, 0.5, 0.5), sphere_phase=phases - 1, phase_count=phases,
+                              diffusion_coeff=0.05, seed=31,
+                              pressure_init=configs.AQ_PRESSURE_PREVIOUS if keep else configs.AQ_PRESSURE_ZERO)
+    pos, frac = ob.seed(cfg)
+    if sparse:
+        cell = (pos / np.float32(cfg.grid_physical_size / extent[0])).astype(np.int64)
+        _, one = np.unique((cell[:, 0] * extent[1] + cell[:, 1]) * extent[2] + cell[:, 2], return_index=True)
+        pos, frac = pos[one], frac[one]
+    gpu = FlipHandle(cfg, pos=pos, frac4=frac)
+    orc = ob.Oracle(cfg, pos=pos, frac4=frac)
+    log(f"[small {extent} K{phases} J{pressure_iters} D{diffusion_iters}] {len(pos)} particles")
+    gpu.steps(3)
+    orc.step(3)
+    check_particles(gpu, orc)
+    for f in ("content", "pressure", "new_velocity", "new_volume_fractions", "volume_fractions", "density"):
+        check_field(f, gpu, orc)
+    gpu.close()
+
+
 @pytest.mark.parametrize("scene", ["separated", "mixing"])
 def test_fixed_point_skip_equals_full_compute_64(monkeypatch, scene):
     """Paired diffusion sweeps after a sweep that changed nothing skip their work; the
