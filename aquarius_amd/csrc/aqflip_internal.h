@@ -89,6 +89,9 @@ struct Grid {
   uint4* btab;          // per workgroup of a listed sweep grid: {chunks, first list
                         // position, first two chunk ids}; the pressure grid's entries,
                         // then the paired grid's (launch_active_list writes both)
+  uint32_t* tactive;    // per tile: any FLUID (set with `active`, cleared when listed)
+  uint32_t* tlist;      // [0] = count, then the ids of the tiles holding FLUID
+  uint4* ttab;          // as btab, per workgroup of a listed tile sweep
   int listed[2];        // workgroups of a listed pressure sweep and of a listed paired sweep
   uint32_t* dchange;    // words 0-2: paired diffusion sweep i changed a bit -> word i % 3 != 0;
                         // word 3: paired diffusion sweeps computed (not skipped)
@@ -200,6 +203,12 @@ void launch_fill_pressure_zero(const Geom& G, Grid gr, int pb, hipStream_t s);
 // cells and AIR cells are skipped -- valid once both buffers hold 0 on AIR.
 // pzero = 1: the input is the zero guess (not read); needs full = 1.
 void launch_jacobi(const Geom& G, Grid gr, int pin, int full, int pzero, hipStream_t s);
+// tile_sweeps() sweeps from gr.p[pin] to gr.p[pin ^ 1]; same flags. AIR or FLUID cells only.
+void launch_jacobi_tile(const Geom& G, Grid gr, int pin, int full, int pzero, hipStream_t s);
+int tile_sweeps();
+bool tile_full(const Geom& G);  // full = 1 is taken
+int sweep_tiles(const Geom& G);
+int tile_grid(const Geom& G);
 // All sweeps of a step in one launch, on grids that fit in a workgroup's LDS (K channel sets).
 bool small_grid(const Geom& G, int K);
 void launch_sweeps_small(const Geom& G, Grid gr, int K, int pb, int pzero, int nj, int nf, float lambda, double inv_cc,
@@ -213,8 +222,9 @@ void launch_extrapolate(const Geom& G, Grid gr, int nvin, int hvin, bool near_ro
 // gr.nvo from newVelocity buffer nv and velocity, every face.
 void launch_build_nvo(const Geom& G, Grid gr, int nv, hipStream_t s);
 // full = 1: AIR cells copied to the output buffer; full = 0: AIR cells and blocks
-// without FLUID skipped -- valid once both buffers agree on AIR cells.
-void launch_diffusion(const Geom& G, Grid gr, int K, int fin, float lambda, double inv_cc, int full,
+// without FLUID skipped -- valid once both buffers agree on AIR cells. sweep > 0: the
+// sweep of that number after paired ones, skipped once one has changed nothing.
+void launch_diffusion(const Geom& G, Grid gr, int K, int fin, float lambda, double inv_cc, int full, int sweep,
                       hipStream_t s);
 // One Jacobi sweep (p[pin] -> p[pin^1]) and one diffusion sweep (nvf[fin] ->
 // nvf[fin^1]) in one launch; fullJ / fullD as `full` above.

@@ -404,6 +404,9 @@ void carve_arrays(aq_flip* h, Carver& c) {
   c.take(&gr.active, (nch + 255) / 256 + 1);
   c.take(&gr.alist, (size_t)sweep_chunks(G) + 1);
   c.take(&gr.btab, (size_t)sweep_table_entries(G));
+  c.take(&gr.tactive, (size_t)sweep_tiles(G));
+  c.take(&gr.tlist, (size_t)sweep_tiles(G) + 1);
+  c.take(&gr.ttab, (size_t)tile_grid(G));
   c.take(&gr.dchange, 4);
   c.take(&gr.stepstamp, 1);
   c.take(&gr.rowstamp, (size_t)(G.X + 1) * (G.Y + 1));
@@ -555,15 +558,20 @@ void jacobi_sweeps(aq_flip* h, int n, bool from_zero = false) {
     h->air_clean[h->pb] = true;
     return;
   }
-  for (int i = 0; i < n; ++i) {
+  for (int i = 0; i < n;) {
     const int out = h->pb ^ 1;
-    const bool z = from_zero && i == 0;
-    launch_jacobi(h->G, h->gr, h->pb, (z || !h->air_clean[out]) ? 1 : 0, z ? 1 : 0, h->stream);
+    const bool z = from_zero && i == 0, full = z || !h->air_clean[out];
+    if (h->p2g_content && n - i >= tile_sweeps() && (!full || tile_full(h->G))) {
+      launch_jacobi_tile(h->G, h->gr, h->pb, full ? 1 : 0, z ? 1 : 0, h->stream);
+      i += tile_sweeps();
+    } else {
+      launch_jacobi(h->G, h->gr, h->pb, full ? 1 : 0, z ? 1 : 0, h->stream);
+      ++i;
+    }
     h->air_clean[out] = true;
     h->pb = out;
   }
 }
-
 
 // Zero pressure start: both buffers cleared.
 void zero_pressure(aq_flip* h) {
@@ -592,10 +600,11 @@ void stage_extrapolate(aq_flip* h, bool in_step = false) {
   }
 }
 
-// Diffusion sweeps first..diffusion_iters-1 of the step.
+// Diffusion sweeps first..diffusion_iters-1 of the step (first > 0: after paired ones).
 void diffusion_sweeps(aq_flip* h, hipStream_t s, int first = 0) {
   for (int i = first; i < h->cfg.diffusion_iters; ++i) {  // the first sweep also copies AIR cells across
-    launch_diffusion(h->G, h->gr, h->K, h->nf, h->sp.lambda, h->sp.inv_cc, i == 0 ? 1 : 0, s);
+    launch_diffusion(h->G, h->gr, h->K, h->nf, h->sp.lambda, h->sp.inv_cc, i == 0 ? 1 : 0,
+                     first > 0 && h->skip_fixed ? i : 0, s);
     h->nf ^= 1;
   }
 }

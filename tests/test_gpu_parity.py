@@ -409,6 +409,48 @@ def test_sweeps_of_small_grids(extent, phases, pressure_iters, diffusion_iters, 
     gpu.close()
 
 
+@pytest.mark.parametrize("extent,sweeps,keep,depth", [
+    ((5, 3, 4), 9, True, 0.5),          # less than a tile; two tile launches and a single
+    ((8, 16, 24), 4, False, 0.5),       # whole tiles, one launch
+    ((33, 17, 26), 11, True, 0.25),     # ragged in every axis
+    ((25, 40, 39), 8, False, 0.9),
+    ((16, 16, 16), 21, True, 0.25),     # all sweeps in one launch
+    ((104, 100, 101), 11, True, 0.25),  # long tiles, rows that end inside a thread's cells
+    ((104, 101, 100), 14, False, 0.9),  # and that do not
+])
+def test_sweeps_per_launch_keep_the_bits(extent, sweeps, keep, depth):
+    """Several pressure sweeps to a launch against one (the path of a field whose content
+    was uploaded), from arbitrary values: zeros of both signs, subnormal and very large
+    ones, and AIR cells that hold something."""
+    cfg = configs.make_config(0, dt=0.01, extent=extent, pressure_iters=sweeps, pool_depth=depth, radius=0.2,
+                              center=(0.5, 0.6, 0.5), seed=37,
+                              pressure_init=configs.AQ_PRESSURE_PREVIOUS if keep else configs.AQ_PRESSURE_ZERO)
+    rng = np.random.default_rng(5)
+    out = []
+    fields = None
+    for uploaded in (False, True):
+        h = FlipHandle(cfg)
+        if fields is None:
+            shape = h.get_field("pressure").shape
+
+            def values():
+                v = rng.standard_normal(shape) * 10.0 ** rng.integers(-3, 4, shape)
+                v = np.where(rng.random(shape) < 0.1, rng.choice([0.0, -0.0, 1e-44, -3e-42, 1e-38, 1e30], shape), v)
+                return v.astype(np.float32)
+
+            fields = {"divergence": values(), "pressure": values(), "content": h.get_field("content")}
+        if uploaded:
+            h.set_field("content", fields["content"])
+        for f in ("divergence", "pressure"):
+            h.set_field(f, fields[f])
+        for _ in range(2):  # the second solve starts in the other buffer and with clean AIR cells
+            h.run_stage("pressure")
+            out.append(h.get_field("pressure").view(np.uint32))
+        h.close()
+    assert np.isfinite(out[1].view(np.float32)).all()
+    assert np.array_equal(out[0], out[2]) and np.array_equal(out[1], out[3])
+
+
 @pytest.mark.parametrize("scene", ["separated", "mixing"])
 def test_fixed_point_skip_equals_full_compute_64(monkeypatch, scene):
     """Paired diffusion sweeps after a sweep that changed nothing skip their work; the
