@@ -1652,9 +1652,9 @@ void launch_jacobi(const Geom& G, Grid gr, int pin, int full, int pzero, hipStre
 // tiles, 5.5 with short ones), about 15 instructions each, on top of some 2.5 us of launch,
 // loads and stores. Microseconds per sweep, single launches before and this: 64^3 with 25 % /
 // 90 % FLUID 2.26 -> 1.20 / 2.49 -> 1.49, 128^3 3.33 -> 2.19 / 5.86 -> 5.31, 256^3 with 33 %
-// 18.5 -> 14.5. Dividing through double as in div_exact took the same time as before AIR
-// cells' marker (a NaN) was kept out of the sums, and sent most waves down the slow branch.
-// 512 workgroups, two per CU, measured the same as 1024.
+// 18.5 -> 14.1. A sixth in single precision (product and correction, with a test for
+// subnormal results) took as long as div_exact's three instructions. 512 workgroups, two
+// per CU, measured the same as 1024.
 constexpr int kTileSweeps = 4;
 constexpr int kTileSpan = kTile + 2 * kTileSweeps;  // 16
 constexpr int kTileThreads = kTileSpan * kTileSpan * 4;
@@ -1668,15 +1668,6 @@ __device__ __forceinline__ float lane_below(float x) {  // lane - 1's, within 16
 }
 __device__ __forceinline__ float lane_above(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x101, 0xf, 0xf, true));
-}
-// A sixth by a product and one correction step: the same bits as div_exact(s, 1.0 / 6.0)
-// for every float (all 2^32 compared) unless the result is subnormal, infinite or NaN, which
-// `odd` collects, or s is -0, which no sum here is (see tile_sweep).
-__device__ __forceinline__ float sixth(float s, bool& odd) {
-  const float q = s * (1.f / 6.f);
-  const float f = __builtin_fmaf(__builtin_fmaf(-6.f, q, s), 1.f / 6.f, q);
-  odd |= __builtin_isfpclass(f, 0x0001 | 0x0002 | 0x0004 | 0x0200 | 0x0010 | 0x0080);  // NaN, infinite, subnormal
-  return f;
 }
 // Four values of a row, `in` of them inside the grid, written through (see st_wt).
 __device__ __forceinline__ void tile_store(float* __restrict__ p, const float* v, int in) {
@@ -1737,7 +1728,7 @@ __device__ __forceinline__ void tile_sweep(const Geom& G, const TileCells<RUNS>&
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     air[i] = __float_as_uint(c.b[i]) == kAirRhsBits;
-    b[i] = air[i] ? 0.f : c.b[i];  // the marker is a NaN, which would make its sum odd
+    b[i] = air[i] ? 0.f : c.b[i];  // keeps the comparison out of the sweeps: 9.98 -> 9.18 us at 128^3
     v[i] = c.v[i] + 0.f;           // no -0 from here on: the sums can start from their first term
   }
   auto edge = [&] {  // cells outside repeat the grid's first or last
@@ -1776,15 +1767,8 @@ __device__ __forceinline__ void tile_sweep(const Geom& G, const TileCells<RUNS>&
         s[i] += b[i];
       }
     }
-    bool odd = false;
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = sixth(s[i], odd);
-    if (odd) {
-#pragma unroll
-      for (int i = 0; i < N; ++i) v[i] = div_exact(s[i], 1.0 / 6.0);
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = air[i] ? 0.f : v[i];
+    for (int i = 0; i < N; ++i) v[i] = air[i] ? 0.f : div_exact(s[i], 1.0 / 6.0);
     edge();
   }
 #pragma unroll
