@@ -207,6 +207,11 @@ void launch_jacobi(const Geom& G, Grid gr, int pin, int full, int pzero, hipStre
 void launch_jacobi_tile(const Geom& G, Grid gr, int pin, int full, int pzero, hipStream_t s);
 int tile_sweeps();
 bool tile_full(const Geom& G);  // full = 1 is taken
+// tile_sweeps() pressure and diffusion sweeps in one launch (K >= 2, AIR cells as `full` = 0
+// asks); `launch` as `sweep` of launch_jacobi_diffusion.
+bool tile_pairs(const Geom& G, int K);
+void launch_tile_pair(const Geom& G, Grid gr, int K, int pin, int fin, float lambda, double inv_cc, int launch,
+                      int skip_ok, hipStream_t s);
 int sweep_tiles(const Geom& G);
 int tile_grid(const Geom& G);
 // All sweeps of a step in one launch, on grids that fit in a workgroup's LDS (K channel sets).

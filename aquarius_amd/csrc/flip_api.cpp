@@ -600,18 +600,19 @@ void stage_extrapolate(aq_flip* h, bool in_step = false) {
   }
 }
 
-// Diffusion sweeps first..diffusion_iters-1 of the step (first > 0: after paired ones).
-void diffusion_sweeps(aq_flip* h, hipStream_t s, int first = 0) {
-  for (int i = first; i < h->cfg.diffusion_iters; ++i) {  // the first sweep also copies AIR cells across
+// Diffusion sweeps first..diffusion_iters-1 of the step (first > 0: after `launch` paired
+// launches).
+void diffusion_sweeps(aq_flip* h, hipStream_t s, int first = 0, int launch = 0) {
+  for (int i = first; i < h->cfg.diffusion_iters; ++i, ++launch) {  // the first sweep also copies AIR cells across
     launch_diffusion(h->G, h->gr, h->K, h->nf, h->sp.lambda, h->sp.inv_cc, i == 0 ? 1 : 0,
-                     first > 0 && h->skip_fixed ? i : 0, s);
+                     first > 0 && h->skip_fixed ? launch : 0, s);
     h->nf ^= 1;
   }
 }
 
 // Fixed-sweep pressure solve and the diffusion sweeps together: the first
-// min(pressure_iters, diffusion_iters) sweeps of each run pairwise in one launch,
-// the rest of the longer chain on its own. Same iterates as the two loops.
+// min(pressure_iters, diffusion_iters) sweeps of each share launches, one or several of
+// each at a time, the rest of the longer chain has its own. Same iterates as the two loops.
 void fused_pressure_diffusion(aq_flip* h) {
   const bool zero = h->cfg.pressure_init == AQ_PRESSURE_ZERO;  // first sweep from the zero guess
   const int n = std::min(h->cfg.pressure_iters, h->cfg.diffusion_iters);
@@ -622,12 +623,19 @@ void fused_pressure_diffusion(aq_flip* h) {
                         h->sp.inv_cc, h->cfg.diffusion_iters, n, h->skip_fixed ? 1 : 0, h->stream);
     h->air_clean[h->pb] = true;
   }
-  for (int i = 0; i < n && !small; ++i) {
+  int launch = 0;  // the step's paired launches, numbered for the diffusion's skipping
+  for (int i = 0; i < n && !small; ++launch) {
     const int out = h->pb ^ 1;
-    const bool z = zero && i == 0;
-    launch_jacobi_diffusion(h->G, h->gr, h->K, h->pb, (z || !h->air_clean[out]) ? 1 : 0, h->nf,
-                            h->sp.lambda, h->sp.inv_cc, i == 0 ? 1 : 0, z ? 1 : 0, i,
-                            h->skip_fixed ? 1 : 0, h->stream);
+    const bool z = zero && i == 0, full = z || !h->air_clean[out];
+    if (i > 0 && !full && n - i >= tile_sweeps() && tile_pairs(h->G, h->K)) {
+      launch_tile_pair(h->G, h->gr, h->K, h->pb, h->nf, h->sp.lambda, h->sp.inv_cc, launch, h->skip_fixed ? 1 : 0,
+                       h->stream);
+      i += tile_sweeps();
+    } else {
+      launch_jacobi_diffusion(h->G, h->gr, h->K, h->pb, full ? 1 : 0, h->nf, h->sp.lambda, h->sp.inv_cc,
+                              i == 0 ? 1 : 0, z ? 1 : 0, launch, h->skip_fixed ? 1 : 0, h->stream);
+      ++i;
+    }
     h->air_clean[out] = true;
     h->pb = out;
     h->nf ^= 1;
@@ -637,7 +645,7 @@ void fused_pressure_diffusion(aq_flip* h) {
   if (!small) jacobi_sweeps(h, h->cfg.pressure_iters - n);
   h->end(AQ_STAGE_PRESSURE, h->cfg.pressure_iters - n);
   h->begin(AQ_STAGE_DIFFUSION);
-  if (!small) diffusion_sweeps(h, h->stream, n);
+  if (!small) diffusion_sweeps(h, h->stream, n, launch);
   h->end(AQ_STAGE_DIFFUSION, h->cfg.diffusion_iters - n);
 }
 

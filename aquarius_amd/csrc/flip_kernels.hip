@@ -2423,6 +2423,159 @@ void launch_jacobi_diffusion(const Geom& G, Grid gr, int K, int pin, int fullJ, 
     default: launch_paired<4>(G, gr, pin, fullJ, fin, lambda, inv_cc, fullD, pzero, sweep, skip_ok, s); break;
   }
 }
+// kTileSweeps pressure sweeps and as many diffusion sweeps in one launch: the first half of
+// the workgroups are k_jacobi_tile's, the second half sweep the fractions of the same tiles
+// in the same way (one LDS buffer per fraction, two barriers a sweep; diffusion_cell's sums).
+// `launch` numbers the step's paired launches: one that changes no bit lets the diffusion
+// part of the next ones skip, as in k_jacobi_diffusion. Steps of 100 + 100 sweeps with two
+// phases, a launch per sweep pair before and this, in us: apart (one diffusion launch
+// computes) 33^3 330 -> 207, 50^3 354 -> 232, 64^3 396 -> 266; mixing (all compute) 483 -> 341,
+// 518 -> 387, 546 -> 513.
+struct PairFields {
+  const float* fin[4];
+  float* fout[4];
+};
+template <int K>
+union PairShared {
+  TileShared<1> p;
+  float4 f[K][kTileThreads];
+};
+template <int K>
+__device__ __forceinline__ bool diffusion_tile(const Geom& G, const TileGeom& T, const float* __restrict__ rhs,
+                                               const PairFields& F, float lambda, double inv_cc, int tile,
+                                               PairShared<K>& m) {
+  TileCells<1> c;
+  tile_load<true, 1>(G, T, rhs, nullptr, tile, c);
+  const int tid = (int)threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), ly = (tid >> 2) & 15;
+  const int in = G.Z - c.z;
+  const bool ragged = G.Z % 4 != 0, own = tile_own<1>(G, c, 0);
+  const int ixp = w == kTileSpan - 1 || c.x == G.X - 1 ? tid : tid + 64, ixm = w == 0 || c.x == 0 ? tid : tid - 64;
+  const int iyp = ly == kTileSpan - 1 || c.y == G.Y - 1 ? tid : tid + 4, iym = ly == 0 || c.y == 0 ? tid : tid - 4;
+  const long long gi = c.row + clampi(c.z, 0, (G.Z - 1) & ~3);
+  float v[K][4];
+  bool air[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) air[i] = __float_as_uint(c.b[i]) == kAirRhsBits;
+#pragma unroll
+  for (int a = 0; a < K; ++a) *reinterpret_cast<float4*>(v[a]) = *reinterpret_cast<const float4*>(F.fin[a] + gi);
+  auto edge = [&] {
+    if (ragged)
+#pragma unroll
+      for (int a = 0; a < K; ++a)
+#pragma unroll
+        for (int i = 1; i < 4; ++i) v[a][i] = in <= i ? v[a][i - 1] : v[a][i];
+  };
+  edge();
+  bool changed = false;
+#pragma unroll 1
+  for (int t = 1; t <= kTileSweeps; ++t) {
+    __syncthreads();  // the previous sweep's (or tile's) reads are done
+#pragma unroll
+    for (int a = 0; a < K; ++a) m.f[a][tid] = make_float4(v[a][0], v[a][1], v[a][2], v[a][3]);
+    __syncthreads();
+    if (w < t || w >= kTileSpan - t) continue;
+    float r[K][4];
+#pragma unroll
+    for (int a = 0; a < K; ++a) {
+      const float below = lane_below(v[a][3]), above = lane_above(v[a][0]);  // all lanes take part
+      const float before = c.z == 0 ? v[a][0] : below, after = in == 4 ? v[a][3] : above;
+      float n[4][4];
+      *reinterpret_cast<float4*>(n[0]) = m.f[a][ixp];
+      *reinterpret_cast<float4*>(n[1]) = m.f[a][ixm];
+      *reinterpret_cast<float4*>(n[2]) = m.f[a][iyp];
+      *reinterpret_cast<float4*>(n[3]) = m.f[a][iym];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float s = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) s += n[k][i] * lambda;
+        s += (i < 3 ? v[a][i < 3 ? i + 1 : i] : after) * lambda;
+        s += (i > 0 ? v[a][i > 0 ? i - 1 : i] : before) * lambda;
+        s += v[a][i];
+        r[a][i] = div_exact(s, inv_cc);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float sum = r[0][i];
+#pragma unroll
+      for (int a = 1; a < K; ++a) sum += r[a][i];
+#pragma unroll
+      for (int a = 0; a < K; ++a) {
+        const float f = air[i] ? v[a][i] : r[a][i] / sum;
+        changed |= own && i < in && __float_as_uint(f) != __float_as_uint(v[a][i]);
+        v[a][i] = f;
+      }
+    }
+    edge();
+  }
+  if (own)
+#pragma unroll
+    for (int a = 0; a < K; ++a) tile_store(F.fout[a] + gi, v[a], in);
+  return changed;
+}
+template <int K>
+__global__ __launch_bounds__(kTileThreads, K <= 2 ? 8 : 4) void k_tile_pair(
+    const uint4* __restrict__ tab, const uint32_t* __restrict__ list, uint32_t* __restrict__ dchange,
+    const float* __restrict__ rhs, const float* __restrict__ pin, float* __restrict__ pout, int launch, int skip_ok,
+    int nb, PairFields F, float lambda, double inv_cc, Geom G, TileGeom T) {
+  __shared__ PairShared<K> m;
+  const bool diff = (int)blockIdx.x >= nb;
+  const uint4 e = tab[diff ? blockIdx.x - nb : blockIdx.x];
+  const uint32_t prev = dchange[(launch + 2) % 3];
+  const int nj = nb >= kXCD ? nb / kXCD : nb;
+  AQF_SGPR_READY(G, e, "s"(nj), "s"(nb), "s"(prev), "s"(T.ny), "s"(T.nz), "s"(T.dny.m), "s"(T.dny.s), "s"(T.dnz.m),
+                 "s"(T.dnz.s));
+  const int n = (int)e.x;
+  if (!diff) {
+    for (int k = 0; k < n; ++k) {
+      TileCells<1> c;
+      tile_load<false, 1>(G, T, rhs, pin, (int)(k == 0 ? e.z : k == 1 ? e.w : list[1 + e.y + k * nj]), c);
+      tile_sweep<1>(G, c, pout, m.p);
+    }
+    return;
+  }
+  const bool skip = skip_ok && prev == 0u;
+  if ((int)blockIdx.x == nb && threadIdx.x == 0) {
+    st_wt(&dchange[(launch + 1) % 3], 0u);
+    if (!skip) atomicAdd(&dchange[3], (uint32_t)kTileSweeps);  // paired diffusion sweeps computed
+  }
+  if (skip) return;
+  bool changed = false;
+  for (int k = 0; k < n; ++k)
+    changed |= diffusion_tile<K>(G, T, rhs, F, lambda, inv_cc,
+                                 (int)(k == 0 ? e.z : k == 1 ? e.w : list[1 + e.y + k * nj]), m);
+  if (__ballot(changed) && (threadIdx.x & 63) == 0) dchange[launch % 3] = 1u;
+}
+// Computing diffusion in tiles costs its border too, which outweighs the launches on larger
+// grids and with more phases: mixing 96^3, K = 2 817 -> 799 us, but K = 4 984 -> 1,256;
+// 64^3, K = 4 608 -> 624 (apart: 392 -> 269).
+bool tile_pairs(const Geom& G, int K) { return tile_geom(G).runs == 1 && (long long)K * G.ncells_hash < 7 << 18; }
+void launch_tile_pair(const Geom& G, Grid gr, int K, int pin, int fin, float lambda, double inv_cc, int launch,
+                      int skip_ok, hipStream_t s) {
+  const TileGeom T = tile_geom(G);
+  PairFields F;
+  for (int a = 0; a < 4; ++a) {
+    F.fin[a] = gr.nvf[fin][a];
+    F.fout[a] = gr.nvf[fin ^ 1][a];
+  }
+  const int nb = tile_grid(G);
+  const dim3 grid(2 * nb), block(kTileThreads);
+  switch (K) {
+    case 2:
+      hipLaunchKernelGGL(k_tile_pair<2>, grid, block, 0, s, gr.ttab, gr.tlist, gr.dchange, gr.rhs, gr.p[pin],
+                         gr.p[pin ^ 1], launch, skip_ok, nb, F, lambda, inv_cc, G, T);
+      break;
+    case 3:
+      hipLaunchKernelGGL(k_tile_pair<3>, grid, block, 0, s, gr.ttab, gr.tlist, gr.dchange, gr.rhs, gr.p[pin],
+                         gr.p[pin ^ 1], launch, skip_ok, nb, F, lambda, inv_cc, G, T);
+      break;
+    default:
+      hipLaunchKernelGGL(k_tile_pair<4>, grid, block, 0, s, gr.ttab, gr.tlist, gr.dchange, gr.rhs, gr.p[pin],
+                         gr.p[pin ^ 1], launch, skip_ok, nb, F, lambda, inv_cc, G, T);
+  }
+}
+
 // ------------------------------------------------------------------ small grids
 // All of a step's sweeps in one launch, where the grid fits in a workgroup's LDS. A sweep
 // launch cannot take less than about 2 us; here a sweep is the FLUID cells' LDS reads, one

@@ -451,6 +451,37 @@ def test_sweeps_per_launch_keep_the_bits(extent, sweeps, keep, depth):
     assert np.array_equal(out[0], out[2]) and np.array_equal(out[1], out[3])
 
 
+@pytest.mark.parametrize("extent,phases,pressure_iters,diffusion_iters", [
+    ((9, 10, 13), 3, 10, 11),   # two launches of four pairs, a diffusion sweep after them
+    ((33, 17, 26), 2, 15, 12),
+    ((16, 24, 20), 4, 14, 40),
+    ((97, 66, 65), 4, 11, 10),  # a pair per launch: too many cells for four phases
+])
+def test_paired_launches_of_several_sweeps(monkeypatch, extent, phases, pressure_iters, diffusion_iters):
+    """Several pressure and diffusion sweeps to a launch give the bits of the sequential
+    order, and count every pair when none is skipped. The ball rests in the pool, so that
+    the phases mix."""
+    cfg = configs.make_config(0, dt=0.01, extent=extent, pressure_iters=pressure_iters,
+                              diffusion_iters=diffusion_iters, radius=0.2, center=(0.5, 0.2, 0.5),
+                              sphere_phase=phases - 1, phase_count=phases, diffusion_coeff=0.05, seed=41)
+    pos, frac = ob.seed(cfg)
+    out, computed = [], []
+    for env in ({"AQFLIP_NO_FUSE": "1", "AQFLIP_NO_OVERLAP": "1"}, {}, {"AQFLIP_NO_FIXED_POINT_SKIP": "1"}):
+        with monkeypatch.context() as m:
+            for k, v in env.items():
+                m.setenv(k, v)
+            h = FlipHandle(cfg, pos=pos, frac4=frac)
+        h.steps(3)
+        out.append([h.get_field(f).view(np.uint32) for f in ("pressure", "new_volume_fractions")])
+        computed.append(h.paired_diffusion_computed())
+        h.close()
+    for k in (1, 2):
+        for a, b in zip(out[0], out[k]):
+            assert np.array_equal(a, b)
+    paired = 3 * min(pressure_iters, diffusion_iters)
+    assert computed[2] == paired and computed[1] <= paired
+
+
 @pytest.mark.parametrize("scene", ["separated", "mixing"])
 def test_fixed_point_skip_equals_full_compute_64(monkeypatch, scene):
     """Paired diffusion sweeps after a sweep that changed nothing skip their work; the
