@@ -244,7 +244,15 @@ void launch_advect(const Geom& G, Particles P, long long Np, Grid gr, int nv, St
 void launch_g2p_advect_hash(const Geom& G, Particles P, long long Np, int K, Grid gr, int nv,
                             int nf, StepParams sp, Bins B, hipStream_t s);
 // FP64 reductions: residual terms (sum r^2, sum b^2) and volume statistics.
-void launch_residual(const Geom& G, Grid gr, int pb, double* partial, double* out, hipStream_t s);
+// Sums of the FP64 residual, pinned: written before seq.
+struct SweepReport {
+  double rr, bb;
+  int seq;
+};
+// reports: device count of the reports so far.
+void launch_residual(const Geom& G, Grid gr, int pb, double* partial, double* out, hipStream_t s,
+                     SweepReport* report = nullptr, int* reports = nullptr);
+void launch_copy_cells(const Geom& G, const float* src, float* dst, hipStream_t s);
 void launch_stats(const Geom& G, Particles P, long long Np, int K, Grid gr, double* partial,
                   int nparts, double* out, hipStream_t s);
 

@@ -214,13 +214,18 @@ struct aq_flip {
   // Tolerance solves: k Jacobi sweeps plus the FP64 residual kernels between two
   // host checks, captured once per (pressure buffer, AIR-clean state, k).
   struct SweepGraph {
-    int key[4];   // pb, air_clean[0], air_clean[1], k
+    int key[5];   // pb, air_clean[0], air_clean[1], k, whether the iterate is kept first
     int next[3];  // pb, air_clean[0], air_clean[1] afterwards
     hipGraph_t graph;
     hipGraphExec_t exec;
   };
   std::vector<SweepGraph> sweep_graphs;
   static constexpr size_t kMaxSweepGraphs = 16;
+  SweepReport* report = nullptr;  // pinned, two; the device's view of it
+  SweepReport* report_dev = nullptr;
+  int* reports = nullptr;         // device count of the reports written
+  int reports_due = 0;            // and of those enqueued
+  float* p_ahead = nullptr;       // the iterate before the chunk that runs ahead
   // Multigrid-preconditioned CG (allocated on first use). The iteration's launches are
   // captured once per parity from the handle's second solve on.
   struct MgState {
@@ -247,6 +252,7 @@ struct aq_flip {
   ~aq_flip() {
     if (stream) hipStreamSynchronize(stream);
     delete mg;
+    if (report) hipHostFree(report);
     for (StepGraph& g : graphs) {
       hipGraphExecDestroy(g.exec);
       hipGraphDestroy(g.graph);
@@ -726,20 +732,20 @@ aq_status mg_setup(aq_flip* h) {
   return AQ_OK;
 }
 
-// Waits until the solve has reported `seq`. Every report is written by a kernel already
+// Waits until *seq has reached want. Every report is written by a kernel already
 // queued on the stream; if the stream runs empty without it, a launch failed.
-aq_status mg_wait(aq_flip* h, int seq) {
-  const MgReport* r = h->mg->report;
-  auto there = [&] { return __atomic_load_n(&r->seq, __ATOMIC_ACQUIRE) >= seq; };
+aq_status wait_report(aq_flip* h, const int* seq, int want) {
+  auto there = [&] { return __atomic_load_n(seq, __ATOMIC_ACQUIRE) >= want; };
   for (unsigned spin = 1; !there(); ++spin) {
     if (spin % 4096) continue;
     const hipError_t e = hipStreamQuery(h->stream);
     if (e == hipErrorNotReady) continue;
-    if (e != hipSuccess) return fail(AQ_EHIP, std::string("MG-PCG: ") + hipGetErrorString(e));
-    if (!there()) return fail(AQ_EHIP, "MG-PCG: the residual was not reported");
+    if (e != hipSuccess) return fail(AQ_EHIP, std::string("solver: ") + hipGetErrorString(e));
+    if (!there()) return fail(AQ_EHIP, "solver: the residual was not reported");
   }
   return AQ_OK;
 }
+aq_status mg_wait(aq_flip* h, int seq) { return wait_report(h, &h->mg->report->seq, seq); }
 
 aq_status mg_enqueue(aq_flip* h, int odd) {
   aq_flip::MgState& M = *h->mg;
@@ -801,31 +807,46 @@ aq_status residual_now(aq_flip* h, double* rel) {
   return residual_read(h, rel);
 }
 
-// k Jacobi sweeps, then the FP64 residual of the result. Replayed from a captured
+// k Jacobi sweeps, then the FP64 residual of the result; with `keep` the iterate before
+// them is copied to p_ahead first. Replayed from a captured
 // graph (host-launched sweeps cannot keep up with the GPU: about 5.6 against 3.6 us
 // per sweep at 128^3); eager while stage timing is on or graphs are switched off.
-aq_status sweeps_then_residual(aq_flip* h, int k, double* rel) {
-  if (h->timing || !h->use_graphs) {
-    jacobi_sweeps(h, k);
-    return residual_now(h, rel);
+aq_status enqueue_sweeps(aq_flip* h, int k, bool keep) {
+  if (!h->report) {
+    AQ_TRY(h->allocT(&h->reports, 1));
+    HIP_TRY(hipHostMalloc((void**)&h->report, 2 * sizeof(SweepReport), hipHostMallocMapped));
+    h->report[0].seq = h->report[1].seq = 0;
+    HIP_TRY(hipHostGetDevicePointer((void**)&h->report_dev, h->report, 0));
   }
-  const int key[4] = {h->pb, h->air_clean[0], h->air_clean[1], k};
-  for (auto& g : h->sweep_graphs) {
-    if (std::memcmp(g.key, key, sizeof(key)) == 0) {
-      HIP_TRY(hipGraphLaunch(g.exec, h->stream));
-      h->pb = g.next[0], h->air_clean[0] = g.next[1] != 0, h->air_clean[1] = g.next[2] != 0;
-      return residual_read(h, rel);
+  if (keep && !h->p_ahead) AQ_TRY(h->allocT(&h->p_ahead, (size_t)h->G.ncell));
+  auto enqueue = [&] {
+    if (keep) launch_copy_cells(h->G, h->gr.p[h->pb], h->p_ahead, h->stream);
+    jacobi_sweeps(h, k);
+    launch_residual(h->G, h->gr, h->pb, h->red_partial, h->red_out, h->stream, h->report_dev, h->reports);
+  };
+  const int due = h->reports_due + 1;
+  const int key[5] = {h->pb, h->air_clean[0], h->air_clean[1], k, keep};
+  const bool graphs = !h->timing && h->use_graphs;
+  if (graphs) {
+    for (auto& g : h->sweep_graphs) {
+      if (std::memcmp(g.key, key, sizeof(key)) == 0) {
+        HIP_TRY(hipGraphLaunch(g.exec, h->stream));
+        h->pb = g.next[0], h->air_clean[0] = g.next[1] != 0, h->air_clean[1] = g.next[2] != 0;
+        h->reports_due = due;
+        return AQ_OK;
+      }
     }
   }
-  if (h->sweep_graphs.size() >= aq_flip::kMaxSweepGraphs) {  // unusual chunk lengths: eager
-    jacobi_sweeps(h, k);
-    return residual_now(h, rel);
+  if (!graphs || h->sweep_graphs.size() >= aq_flip::kMaxSweepGraphs) {  // (unusual chunk lengths)
+    enqueue();
+    HIP_TRY(hipGetLastError());
+    h->reports_due = due;
+    return AQ_OK;
   }
   aq_flip::SweepGraph g{};
   std::memcpy(g.key, key, sizeof(key));
   HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-  jacobi_sweeps(h, k);
-  launch_residual(h->G, h->gr, h->pb, h->red_partial, h->red_out, h->stream);
+  enqueue();
   hipGraph_t graph = nullptr;
   const hipError_t e = hipStreamEndCapture(h->stream, &graph);
   if (e != hipSuccess) {
@@ -837,8 +858,53 @@ aq_status sweeps_then_residual(aq_flip* h, int k, double* rel) {
   g.next[0] = h->pb, g.next[1] = h->air_clean[0], g.next[2] = h->air_clean[1];
   h->sweep_graphs.push_back(g);
   HIP_TRY(hipGraphLaunch(g.exec, h->stream));
-  return residual_read(h, rel);
+  h->reports_due = due;
+  return AQ_OK;
 }
+
+// Sweeps in chunks of `every` up to `budget`, each chunk's residual read while the next
+// one already runs: a chunk is queued before its predecessor's residual is known when the
+// fall of the last two lets expect that this will not end the solve, and undone by finish()
+// where it did. 64^3, a check every 50 sweeps: 24.0 -> 20.4 ms for 10,700 sweeps.
+struct ChunkedSweeps {
+  aq_flip* h;
+  int every, budget;
+  double tol, res;             // res: the last known residual
+  double before = 0;           // and the one before it (0: none)
+  int done = 0, flying = 0;    // sweeps reported; of the chunk queued ahead
+  int pb = 0;                  // state before that chunk
+  bool clean[2] = {false, false};
+  // Up to here: the copy then takes 7 us (8 bytes a cell), and a wait is little next to a chunk.
+  static constexpr long long kMaxCells = 1 << 22;
+
+  aq_status next() {
+    const int k = flying ? flying : std::min(every, budget - done);
+    if (!flying) AQ_TRY(enqueue_sweeps(h, k, false));
+    const int due = h->reports_due;
+    flying = std::min(every, budget - done - k);
+    if (flying > 0 && before > 0 && res * (res / before) > tol && res < before && !h->timing && h->use_graphs &&
+        h->G.ncell <= kMaxCells) {
+      pb = h->pb;
+      std::copy(h->air_clean, h->air_clean + 2, clean);
+      AQ_TRY(enqueue_sweeps(h, flying, true));
+    } else {
+      flying = 0;
+    }
+    AQ_TRY(wait_report(h, &h->report[due & 1].seq, due));
+    const SweepReport& r = h->report[due & 1];
+    before = res;
+    res = r.bb > 0 ? std::sqrt(r.rr) / std::sqrt(r.bb) : std::sqrt(r.rr);
+    done += k;
+    return AQ_OK;
+  }
+  void finish() {
+    if (!flying) return;
+    launch_copy_cells(h->G, h->p_ahead, h->gr.p[pb], h->stream);
+    h->pb = pb;
+    std::copy(clean, clean + 2, h->air_clean);
+    flying = 0;
+  }
+};
 
 // Jacobi sweeps from the current pressure until the FP64 relative residual is
 // <= tol (checked every check_every sweeps) or `budget` sweeps are spent. With
@@ -850,26 +916,28 @@ aq_status sweep_to_tol(aq_flip* h, int budget, bool detect_stall, int* sweeps, d
   *sweeps = 0;
   *stalled = false;
   AQ_TRY(residual_now(h, res));
+  ChunkedSweeps C{h, S.check_every, budget, S.tol, *res};
   double best = *res;
   int flat = 0;
-  while (!(*res <= S.tol) && *sweeps < budget) {
-    if (!std::isfinite(*res)) {
+  while (!(C.res <= S.tol) && C.done < budget) {
+    if (!std::isfinite(C.res)) {
       *stalled = true;
       break;
     }
-    const int k = std::min(S.check_every, budget - *sweeps);
-    AQ_TRY(sweeps_then_residual(h, k, res));
-    *sweeps += k;
+    AQ_TRY(C.next());
     if (detect_stall) {
-      if (std::isfinite(*res) && *res < 0.99 * best) {
-        best = *res;
+      if (std::isfinite(C.res) && C.res < 0.99 * best) {
+        best = C.res;
         flat = 0;
-      } else if (++flat >= S.stall_checks || !std::isfinite(*res)) {
+      } else if (++flat >= S.stall_checks || !std::isfinite(C.res)) {
         *stalled = true;
         break;
       }
     }
   }
+  C.finish();
+  *sweeps = C.done;
+  *res = C.res;
   return AQ_OK;
 }
 
@@ -1697,11 +1765,11 @@ aq_status aq_flip_solve_pressure(aq_flip* h, double tol, int32_t max_iters, int3
   int it = 0;
   double rel = 0;
   AQ_TRY(aq_flip_residual_fp64(h, &rel));
-  while (!(rel <= tol) && it < max_iters) {
-    const int k = std::min(check_every, max_iters - it);
-    AQ_TRY(sweeps_then_residual(h, k, &rel));
-    it += k;
-  }
+  ChunkedSweeps C{h, check_every, max_iters, tol, rel};
+  while (!(C.res <= tol) && C.done < max_iters) AQ_TRY(C.next());
+  C.finish();
+  it = C.done;
+  rel = C.res;
   if (iters_out) *iters_out = it;
   if (rel_out) *rel_out = rel;
   if (!(rel <= tol)) return fail(AQ_ESTALL, "pressure solve reached its iteration cap");

@@ -3180,8 +3180,11 @@ __global__ void k_fold_partials(const double* __restrict__ partial, int nparts, 
 
 // Fold of the residual's per-chunk pairs: 1024 threads, thread t adds pairs t,
 // t + 1024, ... in order, then a fixed-shape tree (deterministic).
+// With a report the sums also go to pinned host memory, to slot c & 1 for the c-th report, so
+// that the host can read them while later work runs.
 __global__ __launch_bounds__(1024) void k_fold_pairs_1024(const double* __restrict__ partial, int n,
-                                                          double* __restrict__ out) {
+                                                          double* __restrict__ out, SweepReport* report,
+                                                          int* reports) {
   __shared__ double s1[1024], s2[1024];
   double a = 0.0, b = 0.0;
   for (int i = (int)threadIdx.x; i < n; i += 1024) {
@@ -3201,13 +3204,31 @@ __global__ __launch_bounds__(1024) void k_fold_pairs_1024(const double* __restri
   if (threadIdx.x == 0) {
     out[0] = s1[0];
     out[1] = s2[0];
+    if (report) {
+      const int c = ++*reports;
+      SweepReport* r = report + (c & 1);
+      r->rr = s1[0];
+      r->bb = s2[0];
+      __hip_atomic_store(&r->seq, c, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
-void launch_residual(const Geom& G, Grid gr, int pb, double* partial, double* out, hipStream_t s) {
+void launch_residual(const Geom& G, Grid gr, int pb, double* partial, double* out, hipStream_t s, SweepReport* report,
+                     int* reports) {
   const int nch = sweep_chunks(G);
   hipLaunchKernelGGL(k_residual_partial, dim3(nch), dim3(kBlock), 0, s, G, gr.content, gr.rhs,
                      gr.p[pb], gr.active, partial);
-  hipLaunchKernelGGL(k_fold_pairs_1024, dim3(1), dim3(1024), 0, s, partial, nch, out);
+  hipLaunchKernelGGL(k_fold_pairs_1024, dim3(1), dim3(1024), 0, s, partial, nch, out, report,
+                     reports);
+}
+
+__global__ void k_copy(const float4* __restrict__ src, float4* __restrict__ dst, long long n) {
+  const long long i = (long long)blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+void launch_copy_cells(const Geom& G, const float* src, float* dst, hipStream_t s) {
+  const long long n = G.ncell / 4;  // rows are a multiple of 8 floats
+  hipLaunchKernelGGL(k_copy, dim3(nblocks(n)), dim3(kBlock), 0, s, (const float4*)src, (float4*)dst, n);
 }
 
 // Volume and mass checks: per phase the sum of particle fractions, the number of

@@ -314,6 +314,30 @@ def test_solve_pressure_to_tolerance_16():
     gpu2.close()
 
 
+@pytest.mark.parametrize("n,every,tol,limit", [(16, 7, 1e-3, 4000), (33, 20, 1e-3, 4000), (33, 1, 3e-2, 4000),
+                                               (40, 50, 1e-5, 333)])
+def test_solves_that_run_ahead(monkeypatch, n, every, tol, limit):
+    """Chunks of sweeps queued before the last residual is known, and undone where it ends
+    the solve: the same sweeps, residual and bits as waiting for each one (no graphs),
+    in a second solve and the step after it as well."""
+    cfg = configs.make_config(n, dt=0.01, pressure_iters=20, pool_depth=0.4, seed=43)
+    out = []
+    for no_graph in ("1", "0"):
+        monkeypatch.setenv("AQFLIP_NO_GRAPH", no_graph)
+        h = FlipHandle(cfg)
+        h.steps(2)
+        got = []
+        for t in (tol, tol / 3):
+            sweeps, res, _ = h.solve_pressure(t, limit, every)
+            got += [sweeps, res, h.get_field("pressure")]
+        h.steps(1)
+        out.append(got + [h.get_field("pressure"), h.residual()])
+        h.close()
+    assert out[0][0] > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 def test_cpp_driver_runs():
     from aquarius_amd.build import DRIVER
     out = subprocess.run([str(DRIVER), "--n", "16", "--steps", "5"], capture_output=True, text=True,
