@@ -596,32 +596,44 @@ __global__ __launch_bounds__(128) void k_bias_part(long long V, int C, const __b
   }
 }
 
-// dW[n][tap*CIN + c] = sum over splits (in order) of part[split][tap][n][c], and the bias
-// gradient db[n] likewise of bpart[block][n]. The loads of kFoldAhead rows are in
-// flight together; the sums stay in row order.
-constexpr int kFoldAhead = 32;
-__global__ __launch_bounds__(64) void k_fold_wgrad(const float* __restrict__ part, const float* __restrict__ bpart,
-                                                   int nsplit, int cin, int cout, float* __restrict__ dW,
-                                                   float* __restrict__ db) {
-  const int total = 27 * cout * cin;
-  const int e = blockIdx.x * 64 + threadIdx.x;
-  if (e >= total + cout) return;
-  const bool isw = e < total;
-  const float* p = isw ? part + e : bpart + (e - total);
-  const long long stride = isw ? total : cout;
-  const int rows = isw ? nsplit : kBiasBlocks;
+// Sum of base[e], base[stride + e], ... over `rows` values, in order, kFoldAhead loads in
+// flight together: a chain of round trips and of additions, so as few of the former as
+// registers allow. base and stride are the block's, so that the rows' addresses are scalar.
+// Per layer of a 2 x 24 x 20 x 28 batch (256 splits, 512 bias rows): 32 loads 10.2 us, 128
+// 7.7. (Four groups of lanes taking 128 bias rows each at once: 8.2.)
+constexpr int kFoldAhead = 128;
+__device__ __forceinline__ float fold_column(const float* __restrict__ base, uint32_t e, long long stride, int rows) {
   float s = 0.f;
-  int sp = 0;
-  for (; sp + kFoldAhead <= rows; sp += kFoldAhead) {
+  int r = 0;
+  for (; r + kFoldAhead <= rows; r += kFoldAhead) {
     float t[kFoldAhead];
 #pragma unroll
-    for (int k = 0; k < kFoldAhead; ++k) t[k] = p[(sp + k) * stride];
+    for (int k = 0; k < kFoldAhead; ++k) t[k] = (base + (r + k) * stride)[e];
 #pragma unroll
     for (int k = 0; k < kFoldAhead; ++k) s += t[k];
   }
-  for (; sp < rows; ++sp) s += p[sp * stride];
+  for (; r + 8 <= rows; r += 8) {
+    float t[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t[k] = (base + (r + k) * stride)[e];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += t[k];
+  }
+  for (; r < rows; ++r) s += (base + r * stride)[e];
+  return s;
+}
+// dW[n][tap*CIN + c] = sum over splits (in order) of part[split][tap][n][c], and the bias
+// gradient db[n] likewise of bpart[block][n].
+__global__ __launch_bounds__(64) void k_fold_wgrad(const float* __restrict__ part, const float* __restrict__ bpart,
+                                                   int nsplit, int cin, int cout, float* __restrict__ dW,
+                                                   float* __restrict__ db) {
+  const int total = 27 * cout * cin;  // a multiple of 64: a block folds weights or biases
+  const bool isw = (int)blockIdx.x * 64 < total;
+  const int e = (int)(blockIdx.x * 64 + threadIdx.x) - (isw ? 0 : total);
+  if (!isw && e >= cout) return;
+  const float s = fold_column(isw ? part : bpart, (uint32_t)e, isw ? total : cout, isw ? nsplit : kBiasBlocks);
   if (!isw) {
-    db[e - total] = s;
+    db[e] = s;
     return;
   }
   const int c = e % cin, t2 = e / cin;
@@ -685,23 +697,11 @@ void skip_bwd(const Vol& v, int C, const __bf16* Y, int ys, const float* dS, con
   hipLaunchKernelGGL(k_skip_bwd, dim3((unsigned)((n8 + 255) / 256)), dim3(256), 0, s, v, C / 8, Y, ys, dS, dP, dYpre);
 }
 
-// out[c] = sum over rows (in order) of part[row][c], C <= 64: the rows are staged in LDS
-// kFoldRows at a time by the whole block, then thread c adds its column.
-constexpr int kFoldRows = 256;
-__global__ __launch_bounds__(256) void k_fold_rows(const float* __restrict__ part, int rows, int C,
-                                                   float* __restrict__ out) {
-  __shared__ float sp[kFoldRows * 64];
-  float s = 0.f;
-  for (int r0 = 0; r0 < rows; r0 += kFoldRows) {
-    const int nr = min(kFoldRows, rows - r0);
-    __syncthreads();
-    for (int e = threadIdx.x; e < nr * C; e += 256) sp[e] = part[(long long)r0 * C + e];
-    __syncthreads();
-    if ((int)threadIdx.x < C)
-#pragma unroll 16
-      for (int r = 0; r < nr; ++r) s += sp[r * C + threadIdx.x];
-  }
-  if ((int)threadIdx.x < C) out[threadIdx.x] = s;
+// out[c] = sum over rows (in order) of part[row][c], C <= 64. 512 rows: 14.7 -> 6.1 us against
+// staging them in LDS.
+__global__ __launch_bounds__(64) void k_fold_rows(const float* __restrict__ part, int rows, int C,
+                                                  float* __restrict__ out) {
+  if ((int)threadIdx.x < C) out[threadIdx.x] = fold_column(part, threadIdx.x, C, rows);
 }
 
 // ------------------------------------------------------------------ pooling / upsampling
@@ -829,7 +829,7 @@ void head_bwd(long long V, const __bf16* X, const float* w, const float* dy, __b
   constexpr int C = 16;
   const int vpb = (int)((V + nblk - 1) / nblk);
   hipLaunchKernelGGL(k_head_bwd<C>, dim3(nblk), dim3(256), 0, s, V, X, w, dy, dYpre, part, vpb);
-  hipLaunchKernelGGL(k_fold_rows, dim3(1), dim3(256), 0, s, part, nblk, C + 1, dwb);
+  hipLaunchKernelGGL(k_fold_rows, dim3(1), dim3(64), 0, s, part, nblk, C + 1, dwb);
 }
 
 // ------------------------------------------------------------------ loss
