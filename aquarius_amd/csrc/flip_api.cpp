@@ -546,13 +546,14 @@ void stage_transfer(aq_flip* h) {
 //
 // Small grids run all n sweeps in one launch, in place. One workgroup per chain does the
 // work, so the rule weighs the FLUID cells (times K with the diffusion chain beside it),
-// taken from the seeding density of 8 particles per cell, against launches that cost about
-// 2 us each. Microseconds per step, one launch / a launch per sweep, sweep counts in brackets:
-// 16^3 with 1,160 FLUID cells 110/270 (100), 80/87 (8); 20^3 with 7,600 205/287 (100), 100/98
-// (8); 24^3 with 13,100 453/356 (100); both chains, 100 sweeps each: K = 2 with 3,900 cells
-// 287/428 (all 16^3) and 163/366 (24^3), 7,600 cells 732/441; K = 4 with 3,900 cells 586/478.
+// taken from the seeding density of 8 particles per cell, against tile launches of four
+// sweeps. Microseconds per step, one launch / tiles, sweep counts in brackets: 16^3 with 1,160
+// FLUID cells 109/164 (100), 81/86 (16), with 3,900 146/170 (100); 24^3 with 3,900 165/175
+// (100), 102/94 (16); 27^3 with 5,600 205/177 (100). Both chains, 100 sweeps each, K = 2: 16^3
+// with 1,160 107/175, with 3,900 and phases mixing 286/296, 18^3 with 5,500 608/464; K = 4,
+// mixing: 12^3 with 1,640 403/430, 16^3 with 3,900 587/440.
 constexpr int kSmallSweeps = 16;
-constexpr long long kSmallPressure = 7000, kSmallPaired = 8192;
+constexpr long long kSmallPressure = 4096, kSmallPaired = 8192;
 bool small_sweeps(const aq_flip* h, int n, int K) {
   const long long fluid = std::min((long long)h->G.ncells_hash, (h->Np + 7) / 8);
   return n >= kSmallSweeps && h->p2g_content && small_grid(h->G, K) &&

@@ -403,7 +403,7 @@ def test_full_steps_match_oracle_mixing_24(pressure_iters, diffusion_iters):
     ((5, 3, 4), 1, 16, 0, False, 0.5, False),     # fewer cells than a wave
     ((16, 16, 16), 4, 16, 40, False, 0.25, False),  # diffusion goes on alone
     ((20, 18, 27), 3, 41, 16, True, 0.1, False),  # pressure goes on alone, from the last step's
-    ((24, 24, 24), 1, 30, 0, False, 0.45, False),  # five to eight cells per thread
+    ((20, 20, 20), 1, 30, 0, False, 1.0, True),   # five to eight cells per thread
     ((26, 26, 26), 2, 20, 17, True, 1.0, True),   # more, in both chains
     ((27, 27, 27), 1, 17, 0, True, 1.0, True),    # nearly the most cells
     ((27, 27, 28), 1, 17, 0, True, 0.1, False),   # one launch per sweep: too many cells
