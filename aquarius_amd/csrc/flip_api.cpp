@@ -155,8 +155,8 @@ struct aq_flip {
   hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   bool overlap = true;
-  // With the fixed-sweep solver, diffusion sweep i runs in the same launch as
-  // pressure sweep i (k_jacobi_diffusion) instead of on the second stream.
+  // With the fixed-sweep solver, diffusion sweeps share launches with pressure sweeps
+  // (fused_pressure_diffusion) instead of running on the second stream.
   bool fuse = true;
   // Paired diffusion sweeps after one that changed no bit skip their identical work.
   bool skip_fixed = true;
