@@ -212,9 +212,9 @@ struct aq_flip {
   bool use_graphs = true;
   bool nvo_valid = false;  // gr.nvo matches newVelocity and velocity (see graph_step)
   // Tolerance solves: k Jacobi sweeps plus the FP64 residual kernels between two
-  // host checks, captured once per (pressure buffer, AIR-clean state, k).
+  // host checks, captured once per (pressure buffer, AIR-clean state, kind of content, k).
   struct SweepGraph {
-    int key[5];   // pb, air_clean[0], air_clean[1], k, whether the iterate is kept first
+    int key[6];   // pb, air_clean[0], air_clean[1], p2g_content, k, whether the iterate is kept first
     int next[3];  // pb, air_clean[0], air_clean[1] afterwards
     hipGraph_t graph;
     hipGraphExec_t exec;
@@ -826,7 +826,7 @@ aq_status enqueue_sweeps(aq_flip* h, int k, bool keep) {
     launch_residual(h->G, h->gr, h->pb, h->red_partial, h->red_out, h->stream, h->report_dev, h->reports);
   };
   const int due = h->reports_due + 1;
-  const int key[5] = {h->pb, h->air_clean[0], h->air_clean[1], k, keep};
+  const int key[6] = {h->pb, h->air_clean[0], h->air_clean[1], h->p2g_content, k, keep};
   const bool graphs = !h->timing && h->use_graphs;
   if (graphs) {
     for (auto& g : h->sweep_graphs) {

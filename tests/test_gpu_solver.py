@@ -98,3 +98,29 @@ def test_coarse_inference_path():
     it, rel, ok = h.solve_pressure(1e-4, 50000, check_every=20)
     assert ok and rel <= 1e-4
     h.close()
+
+
+@pytest.mark.parametrize("n", [16, 33])
+def test_replayed_sweeps_follow_uploaded_content(n):
+    """A solve after a content upload that puts SOLID cells inside the grid, on a handle
+    whose earlier solve captured the same chunk of sweeps for P2G's content (AIR and FLUID
+    only), against the same upload and solve on a fresh handle."""
+    cfg = configs.make_config(n, dt=0.01, pressure_iters=20, pool_depth=0.5, seed=43)
+    out = []
+    for solved_before in (False, True):
+        h = FlipHandle(cfg)
+        rng = np.random.default_rng(7)
+        divergence = rng.standard_normal((n, n, n)).astype(np.float32)
+        h.set_field("divergence", divergence)
+        if solved_before:
+            h.solve_pressure(1e-12, 40, 40)
+        content = h.get_field("content")
+        inner = content[:n, :n, :n]
+        inner[rng.random(inner.shape) < 0.1] = 2  # SOLID
+        h.set_field("content", content)
+        h.set_field("pressure", np.zeros((n, n, n), np.float32))
+        rel = [h.solve_pressure(1e-12, 40, 40)[1] for _ in range(2)]
+        out.append((rel, h.get_field("pressure")))
+        h.close()
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1].view(np.uint32), out[1][1].view(np.uint32))
