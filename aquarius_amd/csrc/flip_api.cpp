@@ -1526,18 +1526,26 @@ aq_status aq_flip_run_stage(aq_flip* h, int32_t stage) {
 
 int64_t aq_flip_particle_count(const aq_flip* h) { return h ? h->Np : 0; }
 
-// The arrays of the particle buffer a step would overwrite next serve as scratch between
-// steps: 48 bytes per particle, an export takes 40.
+// Arrays a and b of the particle buffer that a step overwrites next serve as scratch between
+// steps, 16 bytes per particle each. (c does not: with up to two phases no step writes it, and
+// the fractions in it have to stay 0.) Fractions follow in a launch of their own, in order
+// behind the copies that read the scratch.
 aq_status aq_flip_get_particles(aq_flip* h, float* pos, float* vel, float* frac4) {
   if (!h) return fail(AQ_EINVAL, "null handle");
   const size_t n = (size_t)h->Np;
-  const Particles& S = h->P[h->cur ^ 1];
-  launch_export_particles(h->P[h->cur], h->Np, h->K, pos ? (float*)S.a : nullptr, vel ? (float*)S.b : nullptr,
-                          frac4 ? S.c : nullptr, h->stream);
-  HIP_TRY(hipGetLastError());
-  if (pos) HIP_TRY(hipMemcpyAsync(pos, S.a, n * 3 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-  if (vel) HIP_TRY(hipMemcpyAsync(vel, S.b, n * 3 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-  if (frac4) HIP_TRY(hipMemcpyAsync(frac4, S.c, n * 4 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+  const Particles &P = h->P[h->cur], &S = h->P[h->cur ^ 1];
+  if (pos || vel) {
+    launch_export_particles(P, h->Np, h->K, pos ? (float*)S.a : nullptr, vel ? (float*)S.b : nullptr, nullptr,
+                            h->stream);
+    HIP_TRY(hipGetLastError());
+    if (pos) HIP_TRY(hipMemcpyAsync(pos, S.a, n * 3 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+    if (vel) HIP_TRY(hipMemcpyAsync(vel, S.b, n * 3 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+  }
+  if (frac4) {
+    launch_export_particles(P, h->Np, h->K, nullptr, nullptr, S.a, h->stream);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(frac4, S.a, n * 4 * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+  }
   HIP_TRY(hipStreamSynchronize(h->stream));
   return AQ_OK;
 }

@@ -648,3 +648,20 @@ def test_steps_after_a_field_upload_match_an_uninterrupted_run():
         np.testing.assert_array_equal(x, y)
     a.close()
     b.close()
+
+
+def test_an_export_leaves_fractions_the_handle_does_not_carry_at_zero():
+    """Two phases: an export, a step, and a field upload that raises the phases to four.
+    The particles have never held fractions 2 and 3, so both are 0 (also in the sums)."""
+    cfg = configs.make_config(16, dt=0.01, pressure_iters=20, diffusion_iters=5, sphere_phase=1, phase_count=2, seed=47)
+    h = FlipHandle(cfg)
+    h.get_particles()
+    h.steps(1)
+    f = h.get_field("volume_fractions")
+    f[0, 0, 0, 3] = 0.5
+    h.set_field("volume_fractions", f)
+    frac = h.get_particles()[2]
+    assert frac[:, :2].sum() > 0 and not frac[:, 2:].any()
+    sums = h.stats()["phase_sum"]
+    assert sums[0] > 0 and sums[2:] == [0.0, 0.0]
+    h.close()
