@@ -1911,6 +1911,10 @@ aq_status aq_flip_load(const char* path, aq_flip** out) {
   aq_flip* h = new aq_flip;
   read_env(h);
   aq_status st = setup(h, &cfg, np);
+  // The sections arrive by copies that do not wait for the handle's stream: the clear of its
+  // memory has to be over before the first.
+  if (st == AQ_OK && hipStreamSynchronize(h->stream) != hipSuccess)
+    st = fail(AQ_EHIP, "snapshot: clearing the handle's memory failed");
   if (st != AQ_OK) {
     delete h;
     return bail(st, aq_last_error());

@@ -1,0 +1,73 @@
+// host_cases.cpp -- the library's host code over fake_hip.hpp, one case per run:
+//   host_cases NAME DIR      exit status 0: passed
+#include "fake_hip.hpp"
+
+#include <fstream>
+#include <iterator>
+
+#define REQUIRE(cond)                                                         \
+  do {                                                                        \
+    if (!(cond)) {                                                            \
+      std::fprintf(stderr, "line %d: %s (%s)\n", __LINE__, #cond, aq_last_error()); \
+      std::exit(1);                                                           \
+    }                                                                         \
+  } while (0)
+
+namespace {
+
+std::string dir;
+
+aq_flip_config config(int n, int phases = 1) {
+  aq_flip_config c;
+  REQUIRE(aq_flip_config_default(&c) == AQ_OK);
+  c.size[0] = c.size[1] = c.size[2] = n;
+  c.phase_count = phases;
+  return c;
+}
+// A handle with `np` particles spread over the grid.
+aq_flip* create(const aq_flip_config& c, int np = 64) {
+  std::vector<float> pos(3 * np), frac(4 * np, 0.f);
+  const float h = c.grid_physical_size / (float)c.size[1];
+  for (int i = 0; i < np; ++i) {
+    for (int a = 0; a < 3; ++a) pos[3 * i + a] = h * (0.5f + (float)((i + a) % c.size[a]));
+    frac[4 * i] = 1.f;
+  }
+  aq_flip* f = nullptr;
+  REQUIRE(aq_flip_create_with_particles(&c, pos.data(), nullptr, frac.data(), np, &f) == AQ_OK);
+  return f;
+}
+std::string saved(aq_flip* f, const std::string& name) {
+  const std::string path = dir + "/" + name;
+  REQUIRE(aq_flip_save(f, path.c_str()) == AQ_OK);
+  std::ifstream in(path, std::ios::binary);
+  return std::string(std::istreambuf_iterator<char>(in), {});
+}
+
+// The clear of a new handle's memory must not run over the sections of its snapshot.
+void load_after_clear() {
+  aq_flip* f = create(config(32));
+  const std::vector<float> p(32 * 32 * 32, 1.5f);
+  REQUIRE(aq_flip_set_field(f, AQ_FIELD_PRESSURE, p.data(), p.size() * 4) == AQ_OK);
+  const std::string first = saved(f, "first");
+  aq_flip_destroy(f);
+  aq_flip* g = nullptr;
+  REQUIRE(aq_flip_load((dir + "/first").c_str(), &g) == AQ_OK);
+  REQUIRE(saved(g, "second") == first);
+  aq_flip_destroy(g);
+}
+
+const std::map<std::string, void (*)()> cases = {
+    {"load_after_clear", load_after_clear},
+};
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  if (argc == 1) {
+    for (const auto& c : cases) std::puts(c.first.c_str());
+    return 0;
+  }
+  dir = argc > 2 ? argv[2] : ".";
+  cases.at(argv[1])();
+  return 0;
+}
