@@ -192,7 +192,9 @@ __device__ __forceinline__ double block_sum(double v) {
 
 // ---- start of a solve
 // Level 0 from the FLIP grid: code, x (the start p, or 0) and r = b; u, t and both search
-// directions cleared; partial sums of b.b.
+// directions cleared; partial sums of b.b. The FP64 vectors are also cleared in the guard
+// cells that the last thread of a pass updates with its own (0 times a scalar, but a solve
+// that overflowed multiplied by an infinity there).
 __global__ void k_mg_gather(Geom G, const uint8_t* __restrict__ content, const float* __restrict__ rhs,
                             const float* __restrict__ p, MgLevel L, MgVectors V) {
   const int n = mg_block() * kMgBlock + (int)threadIdx.x;
@@ -211,6 +213,11 @@ __global__ void k_mg_gather(Geom G, const uint8_t* __restrict__ content, const f
     L.u[n] = 0.f;
     L.t[n] = 0.f;
     bb = b * b;
+  } else if (n < (L.n + 3) / 4 * 4) {
+    V.x[n] = 0.0;
+    V.r[n] = 0.0;
+    V.d[0][n] = 0.0;
+    V.d[1][n] = 0.0;
   }
   bb = block_sum<kMgBlock>(bb);
   if (threadIdx.x == 0) V.part[blockIdx.x] = bb;

@@ -130,3 +130,31 @@ def test_mgpcg_solver_mode_steps():
     assert st["solves"] == 3 and st["capped"] == 0
     assert st["last_residual"] < 1e-5
     h.close()
+
+
+def test_solves_after_one_that_overflowed():
+    """81^3 cells, four to a thread, so that the last thread owns cells past the grid's end.
+    A right-hand side that overflows the FP32 preconditioner ends a solve without a result;
+    the next solve on the handle equals that of a fresh handle bit for bit."""
+    n = 81
+    rng = np.random.default_rng(53)
+    divergence = rng.standard_normal((n, n, n)).astype(np.float32)
+    cfg = configs.make_config(n, dt=0.01, pressure_iters=20, pool_depth=0.5, center=(0.95, 0.95, 0.95), radius=0.15,
+                              seed=53)
+    out = []
+    for overflow in (False, True):
+        h = FlipHandle(cfg)
+        zero = np.zeros((n, n, n), np.float32)
+        assert h.get_field("content")[n - 1, n - 1, n - 1] == FLUID  # the last thread has work
+        if overflow:
+            h.set_field("divergence", np.abs(divergence) * np.float32(1e37))
+            it, rel, ok = h.solve_pressure_mgpcg(1e-6, max_iters=20)
+            assert not ok and it > 0
+        h.set_field("divergence", divergence)
+        h.set_field("pressure", zero)
+        it, rel, ok = h.solve_pressure_mgpcg(1e-6, max_iters=60)
+        out.append((it, rel, ok, h.get_field("pressure")))
+        h.close()
+    assert out[0][2]
+    assert out[0][:3] == out[1][:3]
+    assert np.array_equal(out[0][3].view(np.uint32), out[1][3].view(np.uint32))
