@@ -49,6 +49,7 @@ struct aq_hash {
   size_t rec_cap = 0;
   std::vector<void*> fixed, per_particle, staging;
   bool counts_zero = false;  // B.count holds zeros
+  bool counting = false;     // the sort last queued without an error was a counting sort
 
   ~aq_hash() {
     if (stream) hipStreamSynchronize(stream);
@@ -115,6 +116,7 @@ struct aq_hash {
   // pointers (may be null).
   aq_status run(const float* rec, long long n, int stride, int* perm, int* shash, int* start, int* end,
                 float* sorted, hipStream_t s) {
+    counting = false;
     HTRY(ensure(n));
     if (crowded(n)) {
       HTRY(ensure_radix(n));
@@ -126,8 +128,8 @@ struct aq_hash {
       HHIP(hipGetLastError());
       return AQ_OK;
     }
-    // The scan, the counts' last reader, leaves them at zero; only after a call that failed
-    // part-way are they cleared first.
+    // The scan, the counts' last reader, leaves them at zero; only after a counting sort that
+    // failed part-way are they cleared first.
     if (!counts_zero) launch_fill_u32(B.count, 0u, G.ncells_hash, s);
     counts_zero = false;
     if (n > 0) launch_hash_records(G, rec, n, stride, B, s);
@@ -135,8 +137,11 @@ struct aq_hash {
     if (n > 0) launch_scatter_segsort(G, n, B, s);
     launch_hash_outputs(n, stride, HashSorted{B.perm, B.hash, false, nullptr, nullptr}, rec, perm, shash, sorted, s);
     HHIP(hipGetLastError());
+    counting = true;
     return AQ_OK;
   }
+  // After the stream of the last run() has been synchronised.
+  void done() { counts_zero |= counting; }
 };
 
 namespace {
@@ -284,7 +289,7 @@ aq_status aq_hash_sort_host(aq_hash* h, const float* rec, int64_t n, int32_t str
   if (end) HHIP(hipMemcpyAsync(end, h->d_end, cb, hipMemcpyDeviceToHost, h->stream));
   if (sorted && n > 0) HHIP(hipMemcpyAsync(sorted, h->d_sorted, bytes, hipMemcpyDeviceToHost, h->stream));
   HHIP(hipStreamSynchronize(h->stream));
-  h->counts_zero = true;
+  h->done();
   if (cell_count > ncells) {
     if (start) std::fill(start + ncells, start + cell_count, -1);
     if (end) std::fill(end + ncells, end + cell_count, -1);
@@ -310,7 +315,7 @@ aq_status aq_hash_sort_device(aq_hash* h, const float* d_rec, int64_t n, int32_t
     HHIP(hipGetLastError());
   }
   HHIP(hipStreamSynchronize(s));
-  h->counts_zero = true;
+  h->done();
   return AQ_OK;
 }
 

@@ -50,7 +50,8 @@ inline size_t capacity = (size_t)-1;  // of a device
 inline int device = 0;
 inline std::string fail_launch;       // the next launch of this name fails
 inline hipError_t last_error = hipSuccess;
-inline long long launches = 0, graph_launches = 0, captures = 0, kernels_failed = 0;
+inline bool check_bins = true;        // a scatter's offsets have to end at its record count
+inline long long launches = 0, graph_launches = 0, captures = 0;
 inline std::map<std::string, long long> count;  // launches by name, replayed ones too
 inline double rate = 0.99;                      // the residual's factor per sweep
 
@@ -91,7 +92,6 @@ inline void launch(const char* name, hipStream_t s, Work w = [] {}) {
   if (fail_launch == name) {
     fail_launch.clear();
     last_error = hipErrorLaunchFailure;
-    ++kernels_failed;
     return;
   }
   ++launches;
@@ -254,7 +254,7 @@ void launch_scan(const Geom& G, Bins B, hipStream_t s, int*, int*) {
 void launch_scatter_segsort(const Geom& G, long long n, Bins B, hipStream_t s) {
   launch("scatter", s, [B, n, nc = G.ncells_hash] {
     fake::check(B.perm, (size_t)n * 4);
-    if (B.offsets[nc] != n) std::fprintf(stderr, "offsets hold %d records of %lld\n", B.offsets[nc], n), std::exit(4);
+    if (fake::check_bins && B.offsets[nc] != n) std::fprintf(stderr, "offsets hold %d records of %lld\n", B.offsets[nc], n), std::exit(4);
   });
 }
 size_t radix_counts(long long n) { return (size_t)((n + 1023) / 1024 * 512); }

@@ -56,7 +56,25 @@ void load_after_clear() {
   aq_flip_destroy(g);
 }
 
+// A counting sort that fails after its counts leaves them dirty, whatever succeeds next.
+void hash_after_a_failed_sort() {
+  aq_hash* h = nullptr;
+  REQUIRE(aq_hash_create(4, 4, 4, 1.f, 4096, &h) == AQ_OK);
+  const std::vector<float> rec(3 * 4096, 0.5f);
+  REQUIRE(aq_hash_sort_host(h, rec.data(), 100, 3, nullptr, nullptr, nullptr, nullptr, 0, nullptr) == AQ_OK);
+  fake::check_bins = false;
+  fake::fail_launch = "scan";
+  REQUIRE(aq_hash_sort_host(h, rec.data(), 100, 3, nullptr, nullptr, nullptr, nullptr, 0, nullptr) != AQ_OK);
+  REQUIRE(aq_hash_sort_host(h, rec.data(), 4096, 3, nullptr, nullptr, nullptr, nullptr, 0, nullptr) == AQ_OK);
+  REQUIRE(fake::count["radix"] == 1);  // the crowded sort, which does not touch the counts
+  fake::check_bins = true;
+  for (int i = 0; i < 2; ++i)
+    REQUIRE(aq_hash_sort_host(h, rec.data(), 100, 3, nullptr, nullptr, nullptr, nullptr, 0, nullptr) == AQ_OK);
+  aq_hash_destroy(h);
+}
+
 const std::map<std::string, void (*)()> cases = {
+    {"hash_after_a_failed_sort", hash_after_a_failed_sort},
     {"load_after_clear", load_after_clear},
 };
 
