@@ -69,12 +69,13 @@ struct aq_hash {
     HHIP(hipStreamSynchronize(stream));
     for (void* p : per_particle) hipFree(p);
     per_particle.clear();
+    cap = 0;  // until all of the new ones are there
+    vals2 = nullptr;  // the radix sort's buffers went with the others
+    rcounts = roffsets = rpartials = nullptr;
     HTRY(alloc(&B.hash, (size_t)n, per_particle));
     HTRY(alloc(&B.rank, (size_t)n, per_particle));
     HTRY(alloc(&B.perm, (size_t)n, per_particle));
     cap = n;
-    vals2 = nullptr;  // the radix sort's buffers went with the others
-    rcounts = roffsets = rpartials = nullptr;
     return AQ_OK;
   }
   // Which of the two sorts. The radix sort's time depends on neither the records' order nor
@@ -105,6 +106,7 @@ struct aq_hash {
     HHIP(hipStreamSynchronize(stream));
     for (void* p : staging) hipFree(p);
     staging.clear();
+    rec_cap = 0;
     HTRY(alloc(&d_rec, need, staging));
     HTRY(alloc(&d_sorted, need, staging));
     HTRY(alloc(&d_shash, (size_t)std::max<long long>(n, 1), staging));

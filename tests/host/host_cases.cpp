@@ -73,7 +73,32 @@ void hash_after_a_failed_sort() {
   aq_hash_destroy(h);
 }
 
+// A sort that runs out of memory while its buffers grow leaves none of the old ones in use.
+void hash_after_failed_growth() {
+  const auto sort = [](aq_hash* h, const float* rec, long long n) {
+    return aq_hash_sort_host(h, rec, n, 3, nullptr, nullptr, nullptr, nullptr, 0, nullptr);
+  };
+  const std::vector<float> rec(3 * 8192, 0.5f);
+  for (int cells : {4, 2}) {  // 4^3: 1,000 records are no crowded sort there; 2^3: 2,100 are one
+    const long long n = cells == 4 ? 1000 : 2100;
+    for (int room = 1; room <= 40; ++room) {  // each allocation of the growth in turn
+      aq_hash* h = nullptr;
+      fake::capacity = (size_t)-1;
+      REQUIRE(aq_hash_create(cells, cells, cells, 1.f, n, &h) == AQ_OK);
+      REQUIRE(sort(h, rec.data(), n) == AQ_OK);
+      fake::capacity = fake::used(0) + (size_t)room * 8192;
+      (void)sort(h, rec.data(), 8192);
+      (void)sort(h, rec.data(), n);  // may fail for the larger buffers that are there by now
+      fake::capacity = (size_t)-1;
+      REQUIRE(sort(h, rec.data(), n) == AQ_OK);
+      aq_hash_destroy(h);
+      REQUIRE(fake::used(0) == 0);
+    }
+  }
+}
+
 const std::map<std::string, void (*)()> cases = {
+    {"hash_after_failed_growth", hash_after_failed_growth},
     {"hash_after_a_failed_sort", hash_after_a_failed_sort},
     {"load_after_clear", load_after_clear},
 };
