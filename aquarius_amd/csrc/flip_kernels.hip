@@ -810,8 +810,8 @@ template <typename T, bool SORTED>
 __global__ void k_sorted_outputs(long long n, const int* __restrict__ perm, const int* __restrict__ hash,
                                  int* __restrict__ perm_out, int* __restrict__ sorted_hash,
                                  const T* __restrict__ rec, T* __restrict__ sorted_rec, int S, FastDiv divS,
-                                 int* __restrict__ start, int* __restrict__ end) {
-  const long long e0 = (long long)blockIdx.x * kBlock, k0 = e0 / S;
+                                 int* __restrict__ start, int* __restrict__ end, long long block0) {
+  const long long e0 = (block0 + blockIdx.x) * kBlock, k0 = e0 / S;
   const uint32_t r = (uint32_t)(e0 - k0 * S) + threadIdx.x;
   const uint32_t dk = fast_div(r, divS);
   const long long k = k0 + dk;
@@ -835,13 +835,17 @@ template <typename T>
 static void sorted_outputs(long long n, int stride, const HashSorted& in, const float* rec, int* perm,
                            int* sorted_hash, float* sorted_rec, hipStream_t s) {
   const int S = sorted_rec ? stride / (int)(sizeof(T) / 4) : 1;
-  const dim3 grid((unsigned)((n * S + kBlock - 1) / kBlock));
-  if (in.sorted)
-    hipLaunchKernelGGL((k_sorted_outputs<T, true>), grid, dim3(kBlock), 0, s, n, in.perm, in.hash, perm, sorted_hash,
-                       (const T*)rec, (T*)sorted_rec, S, make_fastdiv((uint32_t)S), in.start, in.end);
-  else
-    hipLaunchKernelGGL((k_sorted_outputs<T, false>), grid, dim3(kBlock), 0, s, n, in.perm, in.hash, perm, sorted_hash,
-                       (const T*)rec, (T*)sorted_rec, S, make_fastdiv((uint32_t)S), nullptr, nullptr);
+  const long long blocks = (n * S + kBlock - 1) / kBlock;
+  constexpr long long kMost = 1 << 23;  // blocks of a launch, which takes fewer than 2^32 work-items
+  for (long long b = 0; b < blocks; b += kMost) {
+    const dim3 grid((unsigned)(blocks - b < kMost ? blocks - b : kMost));
+    if (in.sorted)
+      hipLaunchKernelGGL((k_sorted_outputs<T, true>), grid, dim3(kBlock), 0, s, n, in.perm, in.hash, perm, sorted_hash,
+                         (const T*)rec, (T*)sorted_rec, S, make_fastdiv((uint32_t)S), in.start, in.end, b);
+    else
+      hipLaunchKernelGGL((k_sorted_outputs<T, false>), grid, dim3(kBlock), 0, s, n, in.perm, in.hash, perm, sorted_hash,
+                         (const T*)rec, (T*)sorted_rec, S, make_fastdiv((uint32_t)S), nullptr, nullptr, b);
+  }
 }
 void launch_hash_outputs(long long n, int stride, const HashSorted& in, const float* rec, int* perm, int* sorted_hash,
                          float* sorted_rec, hipStream_t s) {

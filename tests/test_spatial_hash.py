@@ -237,3 +237,26 @@ def test_gpu_grid_with_more_than_1024_scan_blocks():
     rng = np.random.default_rng(11)
     pos = rng.uniform(0, 1, (1_500_000, 3)).astype(np.float32) * np.array([256, 256, 80], np.float32) * 0.5
     gpu_case((256, 256, 80), 0.5, pos)
+
+
+@pytest.mark.gpu
+def test_gpu_more_output_words_than_one_launch_has_work_items():
+    """1,048,705 records of 4,097 floats, not aligned to more than a float: 2^32 + 2.6 M
+    words of sorted records, past the 2^32 work-items that a launch can have."""
+    import torch
+    from aquarius_amd.spatial_hash import SpatialHash
+    n, stride, side = 1_048_705, 4097, 64
+    assert n * stride > 1 << 32
+    rec = torch.empty((n, stride), device="cuda")
+    rec.uniform_(0, side)
+    out = torch.empty_like(rec)
+    perm = torch.empty(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    sh = SpatialHash((side, side, side), 1.0, capacity=n)
+    sh.sort_device(rec.data_ptr(), n, stride, d_perm=perm.data_ptr(), d_sorted_records=out.data_ptr())
+    sh.close()
+    for k in range(0, n, 100_000):  # the gather in pieces: a copy of all would be 17 GB more
+        assert torch.equal(out[k:k + 100_000], rec[perm[k:k + 100_000].long()])
+    cell = rec[:, :3].floor().long()
+    h = ((cell[:, 0] * side + cell[:, 1]) * side + cell[:, 2])[perm.long()]
+    assert bool((h[1:] >= h[:-1]).all())
