@@ -866,7 +866,9 @@ aq_status enqueue_sweeps(aq_flip* h, int k, bool keep) {
 // Sweeps in chunks of `every` up to `budget`, each chunk's residual read while the next
 // one already runs: a chunk is queued before its predecessor's residual is known when the
 // fall of the last two lets expect that this will not end the solve, and undone by finish()
-// where it did. 64^3, a check every 50 sweeps: 24.0 -> 20.4 ms for 10,700 sweeps.
+// where it did. 64^3, a check every 50 sweeps: 24.0 -> 20.4 ms for 10,700 sweeps. A solve that
+// ends sooner than expected has queued up to kMaxAhead sweeps for nothing, which the entry
+// points wait for; longer chunks gain less than they risk and are not queued ahead.
 struct ChunkedSweeps {
   aq_flip* h;
   int every, budget;
@@ -877,13 +879,14 @@ struct ChunkedSweeps {
   bool clean[2] = {false, false};
   // Up to here: the copy then takes 7 us (8 bytes a cell), and a wait is little next to a chunk.
   static constexpr long long kMaxCells = 1 << 22;
+  static constexpr int kMaxAhead = 128;
 
   aq_status next() {
     const int k = flying ? flying : std::min(every, budget - done);
     if (!flying) AQ_TRY(enqueue_sweeps(h, k, false));
     const int due = h->reports_due;
     flying = std::min(every, budget - done - k);
-    if (flying > 0 && before > 0 && res * (res / before) > tol && res < before && !h->timing && h->use_graphs &&
+    if (flying > 0 && flying <= kMaxAhead && before > 0 && res * (res / before) > tol && res < before && !h->timing && h->use_graphs &&
         h->G.ncell <= kMaxCells) {
       pb = h->pb;
       std::copy(h->air_clean, h->air_clean + 2, clean);
@@ -898,12 +901,14 @@ struct ChunkedSweeps {
     done += k;
     return AQ_OK;
   }
-  void finish() {
-    if (!flying) return;
+  aq_status finish() {
+    if (!flying) return AQ_OK;
     launch_copy_cells(h->G, h->p_ahead, h->gr.p[pb], h->stream);
+    HIP_TRY(hipGetLastError());
     h->pb = pb;
     std::copy(clean, clean + 2, h->air_clean);
     flying = 0;
+    return AQ_OK;
   }
 };
 
@@ -936,7 +941,7 @@ aq_status sweep_to_tol(aq_flip* h, int budget, bool detect_stall, int* sweeps, d
       }
     }
   }
-  C.finish();
+  AQ_TRY(C.finish());
   *sweeps = C.done;
   *res = C.res;
   return AQ_OK;
@@ -1411,6 +1416,7 @@ aq_status aq_flip_solve_pressure_nn(aq_flip* h, aq_unet* net, double tol, int32_
   }
   h->solver = keep;
   if (st != AQ_OK) return st;
+  HIP_TRY(hipStreamSynchronize(h->stream));  // a chunk queued ahead may still be running
   if (iters_out) *iters_out = total;
   if (rel_out) *rel_out = res;
   if (corrections_out) *corrections_out = (int32_t)corr;
@@ -1776,7 +1782,8 @@ aq_status aq_flip_solve_pressure(aq_flip* h, double tol, int32_t max_iters, int3
   AQ_TRY(aq_flip_residual_fp64(h, &rel));
   ChunkedSweeps C{h, check_every, max_iters, tol, rel};
   while (!(C.res <= tol) && C.done < max_iters) AQ_TRY(C.next());
-  C.finish();
+  AQ_TRY(C.finish());
+  HIP_TRY(hipStreamSynchronize(h->stream));  // a chunk queued ahead may still be running
   it = C.done;
   rel = C.res;
   if (iters_out) *iters_out = it;

@@ -53,7 +53,7 @@ inline hipError_t last_error = hipSuccess;
 inline bool check_bins = true;        // a scatter's offsets have to end at its record count
 inline long long launches = 0, graph_launches = 0, captures = 0;
 inline std::map<std::string, long long> count;  // launches by name, replayed ones too
-inline double rate = 0.99;                      // the residual's factor per sweep
+inline double rate = 0.99, drop_at = 1e30;      // the residual's factor per sweep; 1e-3 of it from drop_at on
 
 inline size_t used(int dev) {
   size_t n = 0;
@@ -202,7 +202,7 @@ void launch_fill_u32(void* p, uint32_t v, long long n, hipStream_t s) {
 void launch_residual(const Geom&, Grid gr, int pb, double*, double* out, hipStream_t s, SweepReport* report,
                      int* reports) {
   launch("residual", s, [=] {
-    const double r = std::pow(fake::rate, gr.p[pb][0]);
+    const double r = std::pow(fake::rate, gr.p[pb][0]) * (gr.p[pb][0] >= fake::drop_at ? 1e-3 : 1.0);
     out[0] = r * r, out[1] = 1.0;
     if (!report) return;
     const int c = ++*reports;

@@ -97,7 +97,28 @@ void hash_after_failed_growth() {
   }
 }
 
+// A solve that ends while its next chunk is queued ahead returns with nothing left on the
+// stream, and with the iterate, sweep count and residual of the chunk that reached tol.
+void solve_returns_idle() {
+  aq_flip* f = create(config(16));
+  const std::vector<float> zero(16 * 16 * 16, 0.f);
+  fake::drop_at = 195;  // sooner than the last two residuals let expect
+  for (int every : {10, 20}) {
+    REQUIRE(aq_flip_set_field(f, AQ_FIELD_PRESSURE, zero.data(), zero.size() * 4) == AQ_OK);
+    int32_t it = 0;
+    double rel = 0, now = 0;
+    const long long undone = fake::count["copy_cells"];
+    REQUIRE(aq_flip_solve_pressure(f, 0.01, 5000, every, &it, &rel) == AQ_OK);
+    REQUIRE(fake::pending() == 0);
+    REQUIRE(fake::count["copy_cells"] > undone);  // a chunk was queued ahead
+    REQUIRE(it == 200 && std::abs(rel - 1e-3 * std::pow(0.99, 200)) < 1e-12);
+    REQUIRE(aq_flip_residual_fp64(f, &now) == AQ_OK && now == rel);
+  }
+  aq_flip_destroy(f);
+}
+
 const std::map<std::string, void (*)()> cases = {
+    {"solve_returns_idle", solve_returns_idle},
     {"hash_after_failed_growth", hash_after_failed_growth},
     {"hash_after_a_failed_sort", hash_after_a_failed_sort},
     {"load_after_clear", load_after_clear},
