@@ -225,6 +225,7 @@ struct aq_flip {
   SweepReport* report_dev = nullptr;
   int* reports = nullptr;         // device count of the reports written
   int reports_due = 0;            // and of those enqueued
+  bool reports_lost = false;      // an error came between: the two may differ
   float* p_ahead = nullptr;       // the iterate before the chunk that runs ahead
   // Multigrid-preconditioned CG (allocated on first use). The iteration's launches are
   // captured once per parity from the handle's second solve on.
@@ -820,12 +821,21 @@ aq_status enqueue_sweeps(aq_flip* h, int k, bool keep) {
     HIP_TRY(hipHostGetDevicePointer((void**)&h->report_dev, h->report, 0));
   }
   if (keep && !h->p_ahead) AQ_TRY(h->allocT(&h->p_ahead, (size_t)h->G.ncell));
+  if (h->reports_lost) {
+    HIP_TRY(hipMemcpyAsync(&h->reports_due, h->reports, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    HIP_TRY(hipStreamSynchronize(h->stream));
+  }
+  h->reports_lost = true;  // until this report is queued
+  auto queued = [h] {
+    ++h->reports_due;
+    h->reports_lost = false;
+    return AQ_OK;
+  };
   auto enqueue = [&] {
     if (keep) launch_copy_cells(h->G, h->gr.p[h->pb], h->p_ahead, h->stream);
     jacobi_sweeps(h, k);
     launch_residual(h->G, h->gr, h->pb, h->red_partial, h->red_out, h->stream, h->report_dev, h->reports);
   };
-  const int due = h->reports_due + 1;
   const int key[6] = {h->pb, h->air_clean[0], h->air_clean[1], h->p2g_content, k, keep};
   const bool graphs = !h->timing && h->use_graphs;
   if (graphs) {
@@ -833,16 +843,14 @@ aq_status enqueue_sweeps(aq_flip* h, int k, bool keep) {
       if (std::memcmp(g.key, key, sizeof(key)) == 0) {
         HIP_TRY(hipGraphLaunch(g.exec, h->stream));
         h->pb = g.next[0], h->air_clean[0] = g.next[1] != 0, h->air_clean[1] = g.next[2] != 0;
-        h->reports_due = due;
-        return AQ_OK;
+        return queued();
       }
     }
   }
   if (!graphs || h->sweep_graphs.size() >= aq_flip::kMaxSweepGraphs) {  // (unusual chunk lengths)
     enqueue();
     HIP_TRY(hipGetLastError());
-    h->reports_due = due;
-    return AQ_OK;
+    return queued();
   }
   aq_flip::SweepGraph g{};
   std::memcpy(g.key, key, sizeof(key));
@@ -859,8 +867,7 @@ aq_status enqueue_sweeps(aq_flip* h, int k, bool keep) {
   g.next[0] = h->pb, g.next[1] = h->air_clean[0], g.next[2] = h->air_clean[1];
   h->sweep_graphs.push_back(g);
   HIP_TRY(hipGraphLaunch(g.exec, h->stream));
-  h->reports_due = due;
-  return AQ_OK;
+  return queued();
 }
 
 // Sweeps in chunks of `every` up to `budget`, each chunk's residual read while the next
@@ -894,7 +901,10 @@ struct ChunkedSweeps {
     } else {
       flying = 0;
     }
-    AQ_TRY(wait_report(h, &h->report[due & 1].seq, due));
+    if (const aq_status st = wait_report(h, &h->report[due & 1].seq, due); st != AQ_OK) {
+      h->reports_lost = true;
+      return st;
+    }
     const SweepReport& r = h->report[due & 1];
     before = res;
     res = r.bb > 0 ? std::sqrt(r.rr) / std::sqrt(r.bb) : std::sqrt(r.rr);

@@ -32,6 +32,7 @@ using Work = std::function<void()>;
 struct Stream {
   std::deque<Work> queue;
   std::vector<Work>* capture = nullptr;
+  bool invalid = false;  // a launch failed during the capture
 };
 struct Graph {
   std::vector<Work> work;
@@ -92,6 +93,7 @@ inline void launch(const char* name, hipStream_t s, Work w = [] {}) {
   if (fail_launch == name) {
     fail_launch.clear();
     last_error = hipErrorLaunchFailure;
+    if (s && ((Stream*)s)->capture) ((Stream*)s)->invalid = true;
     return;
   }
   ++launches;
@@ -149,9 +151,12 @@ hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
   return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
-  *g = (hipGraph_t) new fake::Graph{*((fake::Stream*)s)->capture};
-  ((fake::Stream*)s)->capture = nullptr;
-  return hipSuccess;
+  fake::Stream* f = (fake::Stream*)s;
+  *g = f->invalid ? nullptr : (hipGraph_t) new fake::Graph{*f->capture};
+  f->capture = nullptr;
+  const hipError_t e = f->invalid ? hipErrorStreamCaptureInvalidated : hipSuccess;
+  f->invalid = false;
+  return e;
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t g, hipGraphNode_t*, char*, size_t) {
   *e = (hipGraphExec_t) new fake::Graph(*(fake::Graph*)g);

@@ -117,7 +117,30 @@ void solve_returns_idle() {
   aq_flip_destroy(f);
 }
 
+// One failed launch in a tolerance solve fails that solve only.
+void solves_after_a_failed_launch() {
+  for (const char* eager : {"1", "0"}) {
+    setenv("AQFLIP_NO_GRAPH", eager, 1);
+    aq_flip* f = create(config(16));
+    const std::vector<float> zero(16 * 16 * 16, 0.f);
+    for (const char* name : {"", "residual", "small", "copy_cells", ""}) {
+      REQUIRE(aq_flip_set_field(f, AQ_FIELD_PRESSURE, zero.data(), zero.size() * 4) == AQ_OK);
+      REQUIRE(aq_flip_solve_pressure(f, 0.9, 20, 20, nullptr, nullptr) == AQ_OK);
+      fake::fail_launch = name;
+      const aq_status st = aq_flip_solve_pressure(f, 0.2, 1000, 20, nullptr, nullptr);
+      REQUIRE(st != AQ_OK || !fake::fail_launch.empty() || !*name);
+      fake::fail_launch.clear();
+      REQUIRE(aq_flip_set_field(f, AQ_FIELD_PRESSURE, zero.data(), zero.size() * 4) == AQ_OK);
+      int32_t it = 0;
+      REQUIRE(aq_flip_solve_pressure(f, 0.5, 1000, 20, &it, nullptr) == AQ_OK);
+      REQUIRE(it == 80);
+    }
+    aq_flip_destroy(f);
+  }
+}
+
 const std::map<std::string, void (*)()> cases = {
+    {"solves_after_a_failed_launch", solves_after_a_failed_launch},
     {"solve_returns_idle", solve_returns_idle},
     {"hash_after_failed_growth", hash_after_failed_growth},
     {"hash_after_a_failed_sort", hash_after_a_failed_sort},

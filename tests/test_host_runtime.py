@@ -22,6 +22,7 @@ def host_cases(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", [
+    "solves_after_a_failed_launch",
     "solve_returns_idle",
     "hash_after_failed_growth",
     "hash_after_a_failed_sort",
