@@ -234,6 +234,7 @@ struct aq_flip {
     MgVectors V{};
     MgReport* report = nullptr;  // pinned
     long long solves = 0;
+    bool running = false;  // a solve has begun and has not come to its end
     hipGraph_t graph[2] = {};
     hipGraphExec_t exec[2] = {};
     ~MgState() {
@@ -774,7 +775,10 @@ aq_status mgpcg_solve(aq_flip* h, double tol, int max_iters, int check_every, bo
                       int* iters, double* rel) {
   AQ_TRY(mg_setup(h));
   aq_flip::MgState& M = *h->mg;
-  M.report->seq = 0;  // the previous solve's kernels have completed
+  // A completed solve has no report left to write; one that failed may have some queued.
+  if (M.running) HIP_TRY(hipStreamSynchronize(h->stream));
+  M.running = true;
+  M.report->seq = 0;
   float* p = h->gr.p[h->pb];
   mg_start(h->G, M.H, M.V, h->gr.content, h->gr.rhs, from_current ? p : nullptr, tol, max_iters, check_every,
            h->stream);
@@ -788,6 +792,7 @@ aq_status mgpcg_solve(aq_flip* h, double tol, int max_iters, int check_every, bo
   mg_finish(h->G, M.H, M.V, p, h->stream);
   HIP_TRY(hipGetLastError());
   ++M.solves;
+  M.running = false;
   h->air_clean[h->pb] = true;  // AIR cells written 0
   *iters = it;
   *rel = M.report->res;

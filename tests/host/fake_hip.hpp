@@ -49,12 +49,15 @@ inline std::map<char*, Block> live;
 inline std::vector<Stream*> streams;
 inline size_t capacity = (size_t)-1;  // of a device
 inline int device = 0;
-inline std::string fail_launch;       // the next launch of this name fails
+inline std::string fail_launch;       // a launch of this name fails,
+inline int fail_skip = 0;             // after so many of them
 inline hipError_t last_error = hipSuccess;
 inline bool check_bins = true;        // a scatter's offsets have to end at its record count
 inline long long launches = 0, graph_launches = 0, captures = 0;
 inline std::map<std::string, long long> count;  // launches by name, replayed ones too
 inline double rate = 0.99, drop_at = 1e30;      // the residual's factor per sweep; 1e-3 of it from drop_at on
+
+inline int mg_iters = 0;
 
 inline size_t used(int dev) {
   size_t n = 0;
@@ -90,7 +93,8 @@ inline void put(hipStream_t s, Work w) {
     f->queue.push_back(std::move(w));
 }
 inline void launch(const char* name, hipStream_t s, Work w = [] {}) {
-  if (fail_launch == name) {
+  if (fail_launch == name && fail_skip-- == 0) {
+    fail_skip = 0;
     fail_launch.clear();
     last_error = hipErrorLaunchFailure;
     if (s && ((Stream*)s)->capture) ((Stream*)s)->invalid = true;
@@ -142,7 +146,14 @@ hipError_t hipStreamSynchronize(hipStream_t s) {
   if (s) fake::run((fake::Stream*)s);
   return hipSuccess;
 }
-hipError_t hipStreamQuery(hipStream_t s) { return hipStreamSynchronize(s); }
+hipError_t hipStreamQuery(hipStream_t s) {  // polling lets the stream go on by one piece of work
+  fake::Stream* f = (fake::Stream*)s;
+  if (f->queue.empty()) return hipSuccess;
+  fake::Work w = std::move(f->queue.front());
+  f->queue.pop_front();
+  w();
+  return hipErrorNotReady;
+}
 hipError_t hipStreamDestroy(hipStream_t s) { return hipStreamSynchronize(s); }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) {
@@ -304,10 +315,22 @@ MgLevel mg_level(int X, int Y, int Z) {
 }
 int mg_tail_level(const MgLevels& H) { return H.count - 1; }
 size_t mg_part_size(const MgLevels&) { return 64; }
-void mg_start(const Geom&, const MgLevels&, const MgVectors& V, const uint8_t*, const float*, const float*, double, int,
-              int, hipStream_t s) {
-  launch("mg_start", s, [V] { V.report->res = 0, V.report->stop = 1, V.report->seq = 1; });
+// Solved after fake::mg_iters iterations.
+void mg_start(const Geom&, const MgLevels&, const MgVectors& V, const uint8_t*, const float*, const float*, double,
+              int max_iters, int check_every, hipStream_t s) {
+  launch("mg_start", s, [=] {
+    *V.S = MgScalars{};
+    V.S->max_iters = max_iters, V.S->check_every = check_every;
+    *V.report = MgReport{1.0, fake::mg_iters == 0, 1};
+  });
 }
-void mg_iterate(const MgLevels&, const MgVectors&, int, hipStream_t s) { launch("mg_iterate", s); }
+void mg_iterate(const MgLevels&, const MgVectors& V, int, hipStream_t s) {
+  launch("mg_iterate", s, [V] {
+    MgScalars& S = *V.S;
+    if (++S.it % S.check_every && S.it != S.max_iters) return;
+    const bool stop = S.it >= fake::mg_iters;
+    *V.report = MgReport{stop ? 0.0 : 1.0, stop, S.it + 1};
+  });
+}
 void mg_finish(const Geom&, const MgLevels&, const MgVectors&, float*, hipStream_t s) { launch("mg_finish", s); }
 }  // namespace aqf

@@ -139,7 +139,22 @@ void solves_after_a_failed_launch() {
   }
 }
 
+// What a failed MG-PCG solve has left on the stream does not answer for the next one.
+void mgpcg_after_a_failed_solve() {
+  aq_flip* f = create(config(16));
+  const auto solve = [&](int* it) { return aq_flip_solve_pressure_mgpcg(f, 1e-6, 100, 2, 0, it, nullptr); };
+  int32_t it = 0;
+  fake::mg_iters = 8;
+  REQUIRE(solve(&it) == AQ_OK && it == 8);
+  fake::fail_launch = "mg_iterate";  // the capture of the odd iterations, behind a queued even one
+  fake::fail_skip = 1;
+  REQUIRE(solve(&it) != AQ_OK && fake::pending() > 0);
+  for (int i = 0; i < 2; ++i) REQUIRE(solve(&it) == AQ_OK && it == 8);
+  aq_flip_destroy(f);
+}
+
 const std::map<std::string, void (*)()> cases = {
+    {"mgpcg_after_a_failed_solve", mgpcg_after_a_failed_solve},
     {"solves_after_a_failed_launch", solves_after_a_failed_launch},
     {"solve_returns_idle", solve_returns_idle},
     {"hash_after_failed_growth", hash_after_failed_growth},
