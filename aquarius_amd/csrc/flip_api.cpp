@@ -760,7 +760,10 @@ aq_status mg_enqueue(aq_flip* h, int odd) {
     HIP_TRY(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     mg_iterate(M.H, M.V, odd, h->stream);
     const hipError_t e = hipStreamEndCapture(h->stream, &M.graph[odd]);
-    if (e != hipSuccess) return fail(AQ_EHIP, std::string("MG-PCG capture: ") + hipGetErrorString(e));
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // reported here, not by the next call
+      return fail(AQ_EHIP, std::string("MG-PCG capture: ") + hipGetErrorString(e));
+    }
     HIP_TRY(hipGraphInstantiate(&M.exec[odd], M.graph[odd], nullptr, nullptr, 0));
   }
   HIP_TRY(hipGraphLaunch(M.exec[odd], h->stream));
@@ -865,6 +868,8 @@ aq_status enqueue_sweeps(aq_flip* h, int k, bool keep) {
   const hipError_t e = hipStreamEndCapture(h->stream, &graph);
   if (e != hipSuccess) {
     if (graph) hipGraphDestroy(graph);
+    (void)hipGetLastError();  // reported here, not by the next call
+    h->pb = key[0], h->air_clean[0] = key[1] != 0, h->air_clean[1] = key[2] != 0;  // no sweep has run
     return fail(AQ_EHIP, std::string("sweep capture: ") + hipGetErrorString(e));
   }
   g.graph = graph;

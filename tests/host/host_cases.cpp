@@ -139,6 +139,19 @@ void solves_after_a_failed_launch() {
   }
 }
 
+// Sweeps whose capture fails have not run: the pressure is still the iterate before them.
+void iterate_after_a_failed_capture() {
+  aq_flip* f = create(config(33));
+  const std::vector<float> zero(33 * 33 * 33, 0.f);
+  REQUIRE(aq_flip_set_field(f, AQ_FIELD_PRESSURE, zero.data(), zero.size() * 4) == AQ_OK);
+  REQUIRE(aq_flip_solve_pressure(f, 1e-9, 20, 20, nullptr, nullptr) == AQ_ESTALL);
+  fake::fail_launch = "tile";
+  REQUIRE(aq_flip_solve_pressure(f, 1e-9, 12, 12, nullptr, nullptr) == AQ_EHIP);
+  double rel = 0;
+  REQUIRE(aq_flip_residual_fp64(f, &rel) == AQ_OK && std::abs(rel - std::pow(0.99, 20)) < 1e-12);
+  aq_flip_destroy(f);
+}
+
 // What a failed MG-PCG solve has left on the stream does not answer for the next one.
 void mgpcg_after_a_failed_solve() {
   aq_flip* f = create(config(16));
@@ -154,6 +167,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"iterate_after_a_failed_capture", iterate_after_a_failed_capture},
     {"mgpcg_after_a_failed_solve", mgpcg_after_a_failed_solve},
     {"solves_after_a_failed_launch", solves_after_a_failed_launch},
     {"solve_returns_idle", solve_returns_idle},
