@@ -1176,6 +1176,7 @@ aq_status graph_step(aq_flip* h) {
     if (std::memcmp(g.key, key, sizeof(key)) == 0) {
       HIP_TRY(hipGraphLaunch(g.exec, h->stream));
       set_state(h, g.next);
+      h->p2g_content = true;
       h->physicalTime += h->cfg.dt;
       return AQ_OK;
     }

@@ -152,6 +152,23 @@ void iterate_after_a_failed_capture() {
   aq_flip_destroy(f);
 }
 
+// A step marks every interior cell AIR or FLUID, replayed or not: solves after it take
+// several sweeps to a launch again.
+void replayed_step_marks_content() {
+  aq_flip* f = create(config(33));
+  std::vector<int32_t> content(34 * 34 * 34, 0);
+  const long long captured = fake::captures;
+  for (int i = 0; i < 8; ++i) {
+    REQUIRE(aq_flip_set_field(f, AQ_FIELD_CONTENT, content.data(), content.size() * 4) == AQ_OK);
+    REQUIRE(aq_flip_step(f) == AQ_OK);
+  }
+  REQUIRE(fake::captures - captured < 8);  // some of the steps were replayed
+  const long long single = fake::count["jacobi"];
+  REQUIRE(aq_flip_solve_pressure(f, 1e-9, 40, 40, nullptr, nullptr) == AQ_ESTALL);
+  REQUIRE(fake::count["jacobi"] == single && fake::count["tile"] >= 10);
+  aq_flip_destroy(f);
+}
+
 // What a failed MG-PCG solve has left on the stream does not answer for the next one.
 void mgpcg_after_a_failed_solve() {
   aq_flip* f = create(config(16));
@@ -167,6 +184,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"replayed_step_marks_content", replayed_step_marks_content},
     {"iterate_after_a_failed_capture", iterate_after_a_failed_capture},
     {"mgpcg_after_a_failed_solve", mgpcg_after_a_failed_solve},
     {"solves_after_a_failed_launch", solves_after_a_failed_launch},
