@@ -627,9 +627,10 @@ void fused_pressure_diffusion(aq_flip* h) {
   const int n = std::min(h->cfg.pressure_iters, h->cfg.diffusion_iters);
   h->begin(AQ_STAGE_PRESSURE_DIFFUSION);
   const bool small = small_sweeps(h, n, h->K);
-  if (small) {  // both chains whole, side by side
-    launch_sweeps_small(h->G, h->gr, h->K, h->pb, zero ? 1 : 0, h->cfg.pressure_iters, h->nf, h->sp.lambda,
-                        h->sp.inv_cc, h->cfg.diffusion_iters, n, h->skip_fixed ? 1 : 0, h->stream);
+  const bool whole = small && !h->timing;  // both chains to their ends, side by side
+  if (small) {  // (timed, the longer chain's rest has launches and a bucket of its own)
+    launch_sweeps_small(h->G, h->gr, h->K, h->pb, zero ? 1 : 0, whole ? h->cfg.pressure_iters : n, h->nf, h->sp.lambda,
+                        h->sp.inv_cc, whole ? h->cfg.diffusion_iters : n, n, h->skip_fixed ? 1 : 0, h->stream);
     h->air_clean[h->pb] = true;
   }
   int launch = 0;  // the step's paired launches, numbered for the diffusion's skipping
@@ -651,10 +652,14 @@ void fused_pressure_diffusion(aq_flip* h) {
   }
   h->end(AQ_STAGE_PRESSURE_DIFFUSION, n);
   h->begin(AQ_STAGE_PRESSURE);
-  if (!small) jacobi_sweeps(h, h->cfg.pressure_iters - n);
+  if (!whole) jacobi_sweeps(h, h->cfg.pressure_iters - n);
   h->end(AQ_STAGE_PRESSURE, h->cfg.pressure_iters - n);
   h->begin(AQ_STAGE_DIFFUSION);
-  if (!small) diffusion_sweeps(h, h->stream, n, launch);
+  if (!small)
+    diffusion_sweeps(h, h->stream, n, launch);
+  else if (!whole && h->cfg.diffusion_iters > n)
+    launch_sweeps_small(h->G, h->gr, h->K, h->pb, 0, 0, h->nf, h->sp.lambda, h->sp.inv_cc, h->cfg.diffusion_iters - n, 0,
+                        1, h->stream);
   h->end(AQ_STAGE_DIFFUSION, h->cfg.diffusion_iters - n);
 }
 

@@ -169,6 +169,25 @@ void replayed_step_marks_content() {
   aq_flip_destroy(f);
 }
 
+// Timed steps of small grids: a stage that counts sweeps has the launches that ran them.
+void timed_small_steps() {
+  for (const auto& iters : {std::pair<int, int>{100, 30}, {30, 100}, {40, 40}, {20, 25}, {25, 20}}) {
+    aq_flip_config c = config(16, 2);
+    c.pressure_iters = iters.first, c.diffusion_iters = iters.second;
+    aq_flip* f = create(c);
+    REQUIRE(aq_flip_set_timing(f, 1) == AQ_OK && aq_flip_steps(f, 2) == AQ_OK);
+    double ms[AQ_STAGE_COUNT];
+    int64_t passes[AQ_STAGE_COUNT];
+    REQUIRE(aq_flip_get_timing(f, ms, passes) == AQ_OK);
+    const int n = std::min(iters.first, iters.second);
+    REQUIRE(fake::count["small"] > 0 && passes[AQ_STAGE_PRESSURE_DIFFUSION] == 2 * n);
+    REQUIRE(passes[AQ_STAGE_PRESSURE] == 2 * (iters.first - n) && passes[AQ_STAGE_DIFFUSION] == 2 * (iters.second - n));
+    for (int st : {AQ_STAGE_PRESSURE_DIFFUSION, AQ_STAGE_PRESSURE, AQ_STAGE_DIFFUSION})
+      REQUIRE((passes[st] > 0) == (ms[st] > 0));  // (the stand-in's milliseconds are launches)
+    aq_flip_destroy(f);
+  }
+}
+
 // What a failed MG-PCG solve has left on the stream does not answer for the next one.
 void mgpcg_after_a_failed_solve() {
   aq_flip* f = create(config(16));
@@ -184,6 +203,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"timed_small_steps", timed_small_steps},
     {"replayed_step_marks_content", replayed_step_marks_content},
     {"iterate_after_a_failed_capture", iterate_after_a_failed_capture},
     {"mgpcg_after_a_failed_solve", mgpcg_after_a_failed_solve},

@@ -665,3 +665,21 @@ def test_an_export_leaves_fractions_the_handle_does_not_carry_at_zero():
     sums = h.stats()["phase_sum"]
     assert sums[0] > 0 and sums[2:] == [0.0, 0.0]
     h.close()
+
+
+@pytest.mark.parametrize("pressure_iters,diffusion_iters", [(40, 20), (20, 40), (18, 21), (24, 24)])
+def test_timed_small_steps_keep_the_bits(pressure_iters, diffusion_iters):
+    """Both chains of sweeps in one launch, and with stage timing on, where the longer
+    chain's rest has launches of its own. The ball rests in the pool, so the phases mix."""
+    cfg = configs.make_config(14, dt=0.01, pressure_iters=pressure_iters, diffusion_iters=diffusion_iters, radius=0.2,
+                              center=(0.5, 0.2, 0.5), sphere_phase=1, phase_count=2, diffusion_coeff=0.05, seed=59)
+    out = []
+    for timed in (False, True):
+        h = FlipHandle(cfg)
+        h.set_timing(timed)
+        h.steps(3)
+        out.append([h.get_field(f).view(np.uint32) for f in ("pressure", "new_velocity", "new_volume_fractions")])
+        out[-1].append(h.paired_diffusion_computed())
+        h.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
