@@ -220,7 +220,9 @@ struct aq_flip {
     hipGraphExec_t exec;
   };
   std::vector<SweepGraph> sweep_graphs;
-  static constexpr size_t kMaxSweepGraphs = 16;
+  // 16 chunk lengths and buffer states, each on either kind of content and with the iterate
+  // kept or not.
+  static constexpr size_t kMaxSweepGraphs = 16 * 4;
   SweepReport* report = nullptr;  // pinned, two; the device's view of it
   SweepReport* report_dev = nullptr;
   int* reports = nullptr;         // device count of the reports written

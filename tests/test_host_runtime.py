@@ -22,6 +22,7 @@ def host_cases(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", [
+    "eight_chunk_lengths_replay",
     "timed_small_steps",
     "replayed_step_marks_content",
     "iterate_after_a_failed_capture",
