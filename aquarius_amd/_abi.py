@@ -144,6 +144,7 @@ PROTOTYPES = {
     "aq_flip_create": (C.c_int, [C.POINTER(Config), C.POINTER(_P)]),
     "aq_flip_create_with_particles": (C.c_int, [C.POINTER(Config), _FP, _FP, _FP, C.c_int64, C.POINTER(_P)]),
     "aq_flip_destroy": (None, [_P]),
+    "aq_flip_release_memory": (None, []),
     "aq_flip_step": (C.c_int, [_P]),
     "aq_flip_steps": (C.c_int, [_P, C.c_int32]),
     "aq_flip_run_stage": (C.c_int, [_P, C.c_int32]),

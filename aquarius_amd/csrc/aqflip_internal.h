@@ -140,6 +140,10 @@ struct SeedParams {
   int S[3];
 };
 
+// hipMalloc, tried again without the memory kept from destroyed handles when there is too
+// little (flip_api.cpp). The library's allocations all go through it.
+hipError_t device_malloc(void** p, size_t bytes);
+
 // ---- launchers (flip_kernels.hip, seed_kernels.hip) ----
 void launch_fill_u32(void* p, uint32_t v, long long n, hipStream_t s);
 void launch_seed_count(const SeedVolume& v, const SeedParams& sp, long long nc, int* counts, hipStream_t s);

@@ -58,37 +58,33 @@ aq_status fail(aq_status s, const std::string& msg) {
 // destroyed handle's blocks are kept and handed to the next request that they fit. Blocks
 // enter after their handle's streams have been synchronised and are cleared by whoever
 // takes them, so neither threads nor streams matter beyond the lock. Bounded: at most
-// kKeepBytes per device, a block that kKeepPuts later ones passed over is freed, and all
-// are when an allocation fails. Blocks below kKeepMin are not kept: the runtime serves
-// those from its own chunks.
+// kKeepBytes per device, and a block that kKeepPuts later ones passed over is freed. All are
+// when an allocation of this library fails (device_malloc) and when the caller asks for it
+// (aq_flip_release_memory); nothing else in the process or outside it can. Blocks below
+// kKeepMin are not kept: the runtime serves those from its own chunks.
 class BlockCache {
  public:
   hipError_t get(size_t bytes, void** p, size_t* size) {
+    *size = bytes;
+    if (bytes < kKeepMin) return device_malloc(p, bytes);
     *size = (bytes + kGranule - 1) / kGranule * kGranule;
-    if (bytes < kKeepMin) {
-      *size = bytes;
-      return hipMalloc(p, bytes);
-    }
     int dev = 0;
     if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lock(mutex_);
-    auto best = blocks_.end();
-    for (auto b = blocks_.begin(); b != blocks_.end(); ++b)
-      if (b->dev == dev && b->size >= bytes && b->size <= *size + *size / 4 &&
-          (best == blocks_.end() || b->size < best->size))
-        best = b;
-    if (best != blocks_.end()) {
-      *p = best->p;
-      *size = best->size;
-      blocks_.erase(best);
-      return hipSuccess;
+    {
+      std::lock_guard<std::mutex> lock(mutex_);
+      auto best = blocks_.end();
+      for (auto b = blocks_.begin(); b != blocks_.end(); ++b)
+        if (b->dev == dev && b->size >= bytes && b->size <= *size + *size / 4 &&
+            (best == blocks_.end() || b->size < best->size))
+          best = b;
+      if (best != blocks_.end()) {
+        *p = best->p;
+        *size = best->size;
+        blocks_.erase(best);
+        return hipSuccess;
+      }
     }
-    hipError_t e = hipMalloc(p, *size);
-    if (e != hipErrorOutOfMemory || blocks_.empty()) return e;
-    (void)hipGetLastError();
-    for (const Block& b : blocks_) (void)hipFree(b.p);
-    blocks_.clear();
-    return hipMalloc(p, *size);
+    return device_malloc(p, *size);
   }
   // p: no work on it is pending.
   void put(void* p, size_t size, int dev) {
@@ -97,7 +93,12 @@ class BlockCache {
       return;
     }
     std::lock_guard<std::mutex> lock(mutex_);
-    blocks_.push_back(Block{p, size, dev, ++puts_});
+    try {
+      blocks_.push_back(Block{p, size, dev, ++puts_});
+    } catch (const std::bad_alloc&) {
+      (void)hipFree(p);
+      return;
+    }
     size_t held = 0;  // newest first, what fits the bound stays
     for (size_t i = blocks_.size(); i-- > 0;) {
       const Block& b = blocks_[i];
@@ -108,6 +109,14 @@ class BlockCache {
       (void)hipFree(b.p);
       blocks_.erase(blocks_.begin() + (long)i);
     }
+  }
+  // Frees every block; whether there was one.
+  bool release() {
+    std::lock_guard<std::mutex> lock(mutex_);
+    const bool any = !blocks_.empty();
+    for (const Block& b : blocks_) (void)hipFree(b.p);
+    blocks_.clear();
+    return any;
   }
 
  private:
@@ -1280,7 +1289,7 @@ aq_status plan_seeding(const aq_flip_config& cfg, SeedPlan* plan) {
   long long maxb = 1;
   for (long long nc : plan->nc) maxb = std::max(maxb, (nc + B - 1) / B);
   int* d_counts = nullptr;
-  hipError_t e = hipMalloc((void**)&d_counts, (size_t)maxb * sizeof(int));
+  hipError_t e = device_malloc((void**)&d_counts, (size_t)maxb * sizeof(int));
   for (size_t i = 0; i < plan->vols.size() && e == hipSuccess; ++i) {
     const long long nb = (plan->nc[i] + B - 1) / B;
     launch_seed_count(plan->vols[i], plan->sp, plan->nc[i], d_counts, s);
@@ -1309,7 +1318,7 @@ aq_status write_seeded(aq_flip* h, const SeedPlan& plan) {
   long long maxb = 1;
   for (const auto& o : plan.offsets) maxb = std::max<long long>(maxb, (long long)o.size());
   int* d_off = nullptr;
-  HIP_TRY(hipMalloc((void**)&d_off, (size_t)maxb * sizeof(int)));
+  HIP_TRY(device_malloc((void**)&d_off, (size_t)maxb * sizeof(int)));
   hipError_t e = hipSuccess;
   for (size_t i = 0; i < plan.vols.size() && e == hipSuccess; ++i) {
     e = hipMemcpyAsync(d_off, plan.offsets[i].data(), plan.offsets[i].size() * sizeof(int),
@@ -1405,6 +1414,12 @@ aq_status h2d(aq_flip* h, void* dst, const std::vector<T>& src) {
 }  // namespace
 
 namespace aqf {
+hipError_t device_malloc(void** p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory || !block_cache().release()) return e;
+  (void)hipGetLastError();
+  return hipMalloc(p, bytes);
+}
 FlipView flip_view(aq_flip* h) { return FlipView{h->G, &h->gr, &h->pb, h->stream}; }
 void set_last_error(const std::string& msg) { g_err = msg; }
 }  // namespace aqf
@@ -1535,6 +1550,8 @@ aq_status aq_flip_create_with_particles(const aq_flip_config* cfg, const float* 
 }
 
 void aq_flip_destroy(aq_flip* h) { delete h; }
+
+void aq_flip_release_memory(void) { block_cache().release(); }
 
 aq_status aq_flip_step(aq_flip* h) {
   if (!h) return fail(AQ_EINVAL, "null handle");

@@ -60,7 +60,7 @@ struct aq_hash {
   }
   template <typename T>
   aq_status alloc(T** p, size_t n, std::vector<void*>& list) {
-    HHIP(hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T)));
+    HHIP(device_malloc((void**)p, std::max<size_t>(n, 1) * sizeof(T)));
     list.push_back(*p);
     return AQ_OK;
   }

@@ -105,7 +105,7 @@ struct aq_unet {
   }
   template <typename T>
   aq_status alloc(T** p, size_t n, std::vector<void*>& list) {
-    UHIP(hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T)));
+    UHIP(aqf::device_malloc((void**)p, std::max<size_t>(n, 1) * sizeof(T)));
     list.push_back(*p);
     UHIP(hipMemsetAsync(*p, 0, std::max<size_t>(n, 1) * sizeof(T), stream));
     return AQ_OK;
@@ -620,9 +620,9 @@ aq_status aq_flip_nn_correct(aq_flip* flip, aq_unet* net) {
 aq_status aq_unet_mfma_probe(const float* A, const float* B, float* D) {
   if (!A || !B || !D) return ufail(AQ_EINVAL, "null argument");
   float *dA, *dB, *dD;
-  UHIP(hipMalloc((void**)&dA, 16 * 32 * sizeof(float)));
-  UHIP(hipMalloc((void**)&dB, 32 * 16 * sizeof(float)));
-  UHIP(hipMalloc((void**)&dD, 16 * 16 * sizeof(float)));
+  UHIP(aqf::device_malloc((void**)&dA, 16 * 32 * sizeof(float)));
+  UHIP(aqf::device_malloc((void**)&dB, 32 * 16 * sizeof(float)));
+  UHIP(aqf::device_malloc((void**)&dD, 16 * 16 * sizeof(float)));
   UHIP(hipMemcpy(dA, A, 16 * 32 * sizeof(float), hipMemcpyHostToDevice));
   UHIP(hipMemcpy(dB, B, 32 * 16 * sizeof(float), hipMemcpyHostToDevice));
   mfma_probe(dA, dB, dD, nullptr);

@@ -38,6 +38,11 @@ def seed_particles(cfg: Config) -> tuple[np.ndarray, np.ndarray]:
     return pos, frac
 
 
+def release_memory() -> None:
+    """Give the device memory kept from closed handles back to the device."""
+    load().aq_flip_release_memory()
+
+
 class FlipHandle:
     """One simulation on one GPU (an aq_flip handle)."""
 

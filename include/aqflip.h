@@ -143,7 +143,11 @@ aq_status aq_flip_create_with_particles(const aq_flip_config* cfg, const float* 
                                         const float* vel, const float* frac4, int64_t n,
                                         aq_flip** out);
 
+/* The device memory of a destroyed handle is kept for the next one, up to 12 GiB per
+ * device, until another allocation of this library needs it or aq_flip_release_memory
+ * gives it back to the device (for another library's allocations, say). */
 void aq_flip_destroy(aq_flip* h);
+void aq_flip_release_memory(void);
 
 /* = Fluid::simulationStep (Fluid/Fluid_3D_FLIP.cu:316-352). */
 aq_status aq_flip_step(aq_flip* h);

@@ -1,5 +1,5 @@
 // fake_hip.hpp -- a stand-in for the HIP runtime and the library's kernels, so that the
-// host code (flip_api.cpp, hash_api.cpp) runs on a machine without a GPU.
+// host code (flip_api.cpp, hash_api.cpp, unet_api.cpp) runs on a machine without a GPU.
 //
 // Device memory is host memory in a table of live allocations. Work on a stream is queued
 // and runs only when something waits for that stream; a copy on the null stream does not
@@ -25,6 +25,7 @@
 #include "aqflip_internal.h"
 #include "aqflip_unet.h"
 #include "mgpcg.h"
+#include "unet_internal.h"
 
 namespace fake {
 
@@ -205,8 +206,6 @@ hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t s) {
   return hipSuccess;
 }
 hipError_t hipGetSymbolAddress(void** p, const void* s) { return *p = (void*)s, hipSuccess; }
-aq_status aq_flip_nn_guess(aq_flip*, aq_unet*) { return AQ_OK; }
-aq_status aq_flip_nn_correct(aq_flip*, aq_unet*) { return AQ_OK; }
 }
 
 // ---- the library's kernels
@@ -288,7 +287,9 @@ void launch_hash_outputs(long long, int, const HashSorted&, const float*, int*, 
 }
 #define AQ_FAKE(name, ...) \
   void launch_##name(__VA_ARGS__, hipStream_t s) { launch(#name, s); }
-AQ_FAKE(seed_count, const SeedVolume&, const SeedParams&, long long, int*)
+void launch_seed_count(const SeedVolume&, const SeedParams&, long long nc, int* counts, hipStream_t s) {
+  launch("seed_count", s, [=] { std::fill_n(counts, (nc + 255) / 256, 0); });
+}
 AQ_FAKE(seed_write, const SeedVolume&, const SeedParams&, long long, const int*, long long, Particles)
 AQ_FAKE(hash_count, const Geom&, Particles, long long, Bins)
 AQ_FAKE(scatter_sort_gather, const Geom&, Particles, Particles, long long, int, Bins)
@@ -334,3 +335,45 @@ void mg_iterate(const MgLevels&, const MgVectors& V, int, hipStream_t s) {
 }
 void mg_finish(const Geom&, const MgLevels&, const MgVectors&, float*, hipStream_t s) { launch("mg_finish", s); }
 }  // namespace aqf
+
+// ---- the network's kernels
+namespace aqu {
+using aqf::Geom;
+#define AQ_FAKE(name, ...) \
+  void name(__VA_ARGS__, hipStream_t s) { fake::launch(#name, s); }
+AQ_FAKE(conv3_dgrad, int, int, const Vol&, const __bf16*, const __bf16*, float*)
+AQ_FAKE(conv3_dgrad_relu, int, const Vol&, const __bf16*, const __bf16*, const __bf16*, int, int, __bf16*)
+AQ_FAKE(conv3_dgrad_concat, int, int, const Vol&, const __bf16*, const __bf16*, float*, const __bf16*, __bf16*)
+AQ_FAKE(conv3_wgrad, int, int, const Vol&, const __bf16*, const __bf16*, int, int, float*, float*, int, float*, float*)
+AQ_FAKE(skip_bwd, const Vol&, int, const __bf16*, int, const float*, const float*, __bf16*)
+AQ_FAKE(avgpool, const Vol&, int, const __bf16*, int, int, __bf16*)
+AQ_FAKE(upsample, const Vol&, int, const __bf16*, __bf16*, int, int)
+AQ_FAKE(head_bwd, long long, const __bf16*, const float*, const float*, __bf16*, float*, int, float*)
+AQ_FAKE(masked_mse, long long, const float*, const float*, const float*, double*, int, double*, float*)
+AQ_FAKE(adam, long long, float*, const float*, float*, float*, float, float, float, float)
+AQ_FAKE(pack_weights, int, int, const float*, __bf16*, __bf16*)
+AQ_FAKE(mfma_probe, const float*, const float*, float*)
+AQ_FAKE(nn_sigma, const Geom&, const uint8_t*, const float*, double*, int, double*)
+AQ_FAKE(nn_input, const Geom&, const uint8_t*, const float*, const double*, __bf16*, float*)
+AQ_FAKE(nn_target, const Geom&, const uint8_t*, const float*, const double*, float, float*)
+AQ_FAKE(nn_guess_gather, const Geom&, const uint8_t*, const float*, float*, float*)
+AQ_FAKE(nn_restrict, int, int, int, const float*, const float*, float*, float*)
+AQ_FAKE(nn_input_dense, long long, const float*, const float*, double*, int, double*, __bf16*)
+AQ_FAKE(nn_output_dense, long long, const float*, const float*, const double*, float, float*)
+AQ_FAKE(nn_prolong, int, int, int, const float*, float*)
+AQ_FAKE(nn_scatter_scaled, const Geom&, const uint8_t*, const float*, const float*, float*, double*, int, double*)
+AQ_FAKE(nn_residual, const Geom&, const uint8_t*, const float*, const float*, float*)
+AQ_FAKE(nn_axpy, const Geom&, const uint8_t*, const float*, float*)
+#undef AQ_FAKE
+void host_input(long long V, const float* x2, __bf16* x0, hipStream_t s) {
+  fake::launch("host_input", s, [=] { fake::check(x2, V * 8), fake::check(x0, V * 16); });
+}
+void conv3_forward(int cin, int cout, const Vol& v, const __bf16* X, int xs, int, const __bf16*, const float*, __bf16* Y,
+                   int ys, int, hipStream_t s) {
+  const size_t V = (size_t)v.B * v.D * v.H * v.W;
+  fake::launch("conv3_forward", s, [=] { fake::check(X, V * xs * 2), fake::check(Y, V * ys * 2); });
+}
+void head_fwd(long long V, int C, const __bf16* X, const float*, const float*, float* y, hipStream_t s) {
+  fake::launch("head_fwd", s, [=] { fake::check(X, (size_t)V * C * 2), fake::check(y, (size_t)V * 4); });
+}
+}  // namespace aqu

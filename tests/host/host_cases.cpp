@@ -213,6 +213,33 @@ void eight_chunk_lengths_replay() {
   aq_flip_destroy(f);
 }
 
+// The memory kept from destroyed handles serves the library's other allocations when there
+// is no more, and goes back to the device when asked.
+void kept_memory_is_given_back() {
+  const auto keep = [] {
+    fake::capacity = (size_t)-1;
+    aq_flip_destroy(create(config(112)));
+    REQUIRE(fake::used(0) > 1 << 20);
+    fake::capacity = fake::used(0);
+  };
+  keep();
+  aq_hash* h = nullptr;
+  REQUIRE(aq_hash_create(8, 8, 8, 1.f, 1000, &h) == AQ_OK);
+  aq_hash_destroy(h);
+  keep();
+  aq_unet_config uc;
+  aq_unet* net = nullptr;
+  REQUIRE(aq_unet_config_default(&uc) == AQ_OK && aq_unet_create(&uc, &net) == AQ_OK);
+  aq_unet_destroy(net);
+  keep();
+  aq_flip* f = nullptr;  // (the stand-in's seeder counts no particles)
+  const aq_flip_config c = config(64);
+  REQUIRE(aq_flip_create(&c, &f) == AQ_EINVAL);
+  keep();
+  aq_flip_release_memory();
+  REQUIRE(fake::used(0) == 0);
+}
+
 // What a failed MG-PCG solve has left on the stream does not answer for the next one.
 void mgpcg_after_a_failed_solve() {
   aq_flip* f = create(config(16));
@@ -228,6 +255,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"kept_memory_is_given_back", kept_memory_is_given_back},
     {"eight_chunk_lengths_replay", eight_chunk_lengths_replay},
     {"timed_small_steps", timed_small_steps},
     {"replayed_step_marks_content", replayed_step_marks_content},

@@ -1,4 +1,4 @@
-"""The library's host code (flip_api.cpp, hash_api.cpp) over a stand-in for the HIP runtime
+"""The library's host code (flip_api.cpp, hash_api.cpp, unet_api.cpp) over a stand-in for the HIP runtime
 that queues work until something waits for it and can run out of memory or fail a launch
 (host/fake_hip.hpp): what happens between calls, without a GPU."""
 import subprocess
@@ -17,11 +17,12 @@ def host_cases(tmp_path_factory):
     subprocess.run(["/opt/rocm/bin/amdclang++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__",
                     "-D__align__(n)=__attribute__((aligned(n)))", "-DHIP_SYMBOL(x)=(const void*)(x)", "-I/opt/rocm/include", f"-I{ROOT / 'include'}",
                     f"-I{CSRC}", str(HOST / "host_cases.cpp"), str(CSRC / "flip_api.cpp"), str(CSRC / "flip_seed.cpp"),
-                    str(CSRC / "hash_api.cpp"), "-o", str(exe), "-lpthread"], check=True)
+                    str(CSRC / "hash_api.cpp"), str(CSRC / "unet_api.cpp"), "-o", str(exe), "-lpthread"], check=True)
     return exe
 
 
 @pytest.mark.parametrize("name", [
+    "kept_memory_is_given_back",
     "eight_chunk_lengths_replay",
     "timed_small_steps",
     "replayed_step_marks_content",
