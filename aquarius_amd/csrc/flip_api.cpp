@@ -64,12 +64,14 @@ aq_status fail(aq_status s, const std::string& msg) {
 // kKeepMin are not kept: the runtime serves those from its own chunks.
 class BlockCache {
  public:
-  hipError_t get(size_t bytes, void** p, size_t* size) {
+  // size, device: the block's, for put().
+  hipError_t get(size_t bytes, void** p, size_t* size, int* device) {
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+    *device = dev;
     *size = bytes;
     if (bytes < kKeepMin) return device_malloc(p, bytes);
     *size = (bytes + kGranule - 1) / kGranule * kGranule;
-    int dev = 0;
-    if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
     {
       std::lock_guard<std::mutex> lock(mutex_);
       auto best = blocks_.end();
@@ -173,9 +175,9 @@ struct aq_flip {
   struct Alloc {
     void* p;
     size_t size;
+    int dev;
   };
   std::vector<Alloc> allocs;
-  int dev = 0;
 
   Particles P[2]{};
   int cur = 0;
@@ -275,7 +277,7 @@ struct aq_flip {
       hipGraphDestroy(g.graph);
     }
     if (side) hipStreamSynchronize(side);
-    for (const Alloc& a : allocs) block_cache().put(a.p, a.size, dev);
+    for (const Alloc& a : allocs) block_cache().put(a.p, a.size, a.dev);
     for (hipEvent_t e : event_pool) hipEventDestroy(e);
     if (ev_fork) hipEventDestroy(ev_fork);
     if (ev_join) hipEventDestroy(ev_join);
@@ -286,8 +288,9 @@ struct aq_flip {
   // Zeroed.
   aq_status alloc(void** p, size_t bytes) {
     size_t size = 0;
-    HIP_TRY(block_cache().get(bytes, p, &size));
-    allocs.push_back({*p, size});
+    int dev = 0;
+    HIP_TRY(block_cache().get(bytes, p, &size, &dev));
+    allocs.push_back({*p, size, dev});
     HIP_TRY(hipMemsetAsync(*p, 0, bytes, stream));
     return AQ_OK;
   }
@@ -483,7 +486,6 @@ aq_status setup(aq_flip* h, const aq_flip_config* cfg, long long Np) {
   HIP_TRY(hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking));
   HIP_TRY(hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming));
   HIP_TRY(hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming));
-  HIP_TRY(hipGetDevice(&h->dev));
   // One block for every array: measured first, then carved.
   Carver c;
   carve_arrays(h, c);

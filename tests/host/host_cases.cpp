@@ -240,6 +240,24 @@ void kept_memory_is_given_back() {
   REQUIRE(fake::used(0) == 0);
 }
 
+// A block that was allocated with another device current is kept for that device.
+void kept_blocks_stay_on_their_device() {
+  const aq_flip_config c = config(64);
+  const auto solve = [&](int device) {
+    aq_flip* f = create(c);
+    fake::device = device, fake::mg_iters = 2;
+    const size_t before = fake::used(device);
+    REQUIRE(aq_flip_solve_pressure_mgpcg(f, 1e-6, 10, 1, 0, nullptr, nullptr) == AQ_OK);
+    const size_t added = fake::used(device) - before;
+    fake::device = 0;
+    aq_flip_destroy(f);
+    return added;
+  };
+  const size_t size = solve(1);
+  REQUIRE(size > 0 && solve(0) == size);
+  aq_flip_release_memory();
+}
+
 // What a failed MG-PCG solve has left on the stream does not answer for the next one.
 void mgpcg_after_a_failed_solve() {
   aq_flip* f = create(config(16));
@@ -255,6 +273,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"kept_blocks_stay_on_their_device", kept_blocks_stay_on_their_device},
     {"kept_memory_is_given_back", kept_memory_is_given_back},
     {"eight_chunk_lengths_replay", eight_chunk_lengths_replay},
     {"timed_small_steps", timed_small_steps},
