@@ -117,6 +117,7 @@ struct aq_unet {
     UHIP(hipStreamSynchronize(stream));
     for (void* p : guess_allocs) hipFree(p);
     guess_allocs.clear();
+    guess_cap = 0;  // until all of the new ones are there
     gb.assign(levels + 1, nullptr);
     gm.assign(levels + 1, nullptr);
     gp.assign(levels + 1, nullptr);
@@ -136,6 +137,7 @@ struct aq_unet {
     UHIP(hipStreamSynchronize(stream));
     for (void* p : res_allocs) hipFree(p);
     res_allocs.clear();
+    res_cap = 0;
     UTRY(alloc(&res, ncell, res_allocs));
     UTRY(alloc(&corr, ncell, res_allocs));
     res_cap = ncell;
@@ -147,6 +149,7 @@ struct aq_unet {
     UHIP(hipStreamSynchronize(stream));
     for (void* p : act_allocs) hipFree(p);
     act_allocs.clear();
+    capV = 0;
     const long long V2 = V / 8 + 1, V3 = V / 64 + 1;
     auto& L = act_allocs;
     UTRY(alloc(&x0, V * 8, L));
@@ -502,6 +505,8 @@ aq_status aq_unet_dataset_reserve(aq_unet* net, int32_t cap, int32_t D, int32_t 
       hipFree(p);
       net->allocs.erase(std::remove(net->allocs.begin(), net->allocs.end(), p), net->allocs.end());
     }
+    net->ds_x = nullptr, net->ds_t = net->ds_m = nullptr;
+    net->ds_cap = net->ds_n = 0;
   }
   const long long V = (long long)D * H * W;
   UTRY(net->alloc(&net->ds_x, (size_t)cap * V * 8, net->allocs));

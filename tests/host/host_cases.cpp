@@ -258,6 +258,29 @@ void kept_blocks_stay_on_their_device() {
   aq_flip_release_memory();
 }
 
+// A network that runs out of memory while its activations grow leaves none of the old ones
+// in use.
+void network_after_failed_growth() {
+  aq_unet_config uc;
+  aq_unet* net = nullptr;
+  REQUIRE(aq_unet_config_default(&uc) == AQ_OK && aq_unet_create(&uc, &net) == AQ_OK);
+  std::vector<float> x(2 * 16 * 16 * 16, 0.f), y(16 * 16 * 16);
+  const auto forward = [&](int n) { return aq_unet_forward_host(net, x.data(), 1, n, n, n, y.data()); };
+  aq_flip* f = create(config(16));
+  const auto reserve = [&](int samples) { return aq_unet_dataset_reserve(net, samples, 16, 16, 16); };
+  REQUIRE(forward(8) == AQ_OK && reserve(2) == AQ_OK && aq_unet_dataset_add_flip(net, f) == AQ_OK);
+  fake::capacity = fake::used(0) + 200000;
+  REQUIRE(forward(16) != AQ_OK);
+  (void)forward(8);
+  REQUIRE(reserve(64) != AQ_OK && aq_unet_dataset_size(net) == 0);
+  fake::capacity = (size_t)-1;
+  REQUIRE(forward(8) == AQ_OK && forward(16) == AQ_OK);
+  REQUIRE(aq_unet_dataset_add_flip(net, f) != AQ_OK);  // nothing is reserved
+  REQUIRE(reserve(2) == AQ_OK && aq_unet_dataset_add_flip(net, f) == AQ_OK && aq_unet_dataset_size(net) == 1);
+  aq_flip_destroy(f);
+  aq_unet_destroy(net);
+}
+
 // What a failed MG-PCG solve has left on the stream does not answer for the next one.
 void mgpcg_after_a_failed_solve() {
   aq_flip* f = create(config(16));
@@ -273,6 +296,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"network_after_failed_growth", network_after_failed_growth},
     {"kept_blocks_stay_on_their_device", kept_blocks_stay_on_their_device},
     {"kept_memory_is_given_back", kept_memory_is_given_back},
     {"eight_chunk_lengths_replay", eight_chunk_lengths_replay},
