@@ -79,19 +79,22 @@ struct aq_hash {
     return AQ_OK;
   }
   // Which of the two sorts. The radix sort's time depends on neither the records' order nor
-  // their spread; the counting sort's grows with the records per cell and with disorder,
-  // but takes one pass where the records come nearly sorted. us, counting / radix, for
-  // records in random order, moved a little since the last sort, and sorted:
-  //   1 M in 50^3 cells     149 / 115   112 / 99    68 / 95
-  //   1 M in 40^3 cells     184 / 92    148 / 85    70 / 82
-  //   3 M in 100^3 cells    359 / 257   225 / 224  134 / 207
-  //   100,000 in 30^3        44 / 52     39 / 56    35 / 50
-  //   100,000 in 16^3       126 / 53    119 / 52    80 / 52
-  // so the line lies at 4 records per cell for large sorts, and at 16 below them, where the
-  // extra launches weigh more.
-  bool crowded(long long n) const {
-    return n >= (1 << 18) ? n >= 4LL * G.ncells_hash : n >= 2048 && n > 16LL * G.ncells_hash;
-  }
+  // their spread; the counting sort takes one pass, quickest where the records come nearly
+  // sorted, as they do from a step that sorted them before, but its segments' sorts grow with
+  // the records per cell. us per call, counting / radix, for 16-byte records in random order,
+  // moved a little since the last sort, and sorted:
+  //   1 M in 50^3 cells (8 a cell)   113 / 104    48 / 83     46 / 84
+  //   3 M in 80^3       (6)          312 / 210    86 / 158    79 / 156
+  //   300,000 in 30^3   (11)          56 / 74     36 / 71     37 / 73
+  //   100,000 in 16^3   (24)          47 / 76     36 / 74     36 / 74
+  //   1 M in 30^3       (37)         174 / 97    104 / 88     81 / 89
+  //   3 M in 44^3       (35)         353 / 209   129 / 138   107 / 138
+  //   20,000 in 8^3     (39)          94 / 33     90 / 33     68 / 33
+  //   1 M in 20^3       (125)        625 / 94    560 / 90    508 / 89
+  // so the line lies at 32 records per cell, where segments outgrow the sort in registers. (A
+  // million unordered records and more would gain below it too, but ordered ones would lose
+  // as much or more, and the order is not known here.)
+  bool crowded(long long n) const { return n >= 2048 && n > 32LL * G.ncells_hash; }
   aq_status ensure_radix(long long n) {
     if (!vals2) HTRY(alloc(&vals2, (size_t)cap, per_particle));
     const size_t c = std::max(radix_counts(cap), radix_counts(std::min<long long>(cap, (1 << 19) - 1)));

@@ -73,6 +73,22 @@ void hash_after_a_failed_sort() {
   aq_hash_destroy(h);
 }
 
+// Records are sorted by radix only where the cells are crowded: below that the counting sort
+// is the faster one for records that come nearly sorted.
+void sort_by_density() {
+  const std::vector<float> rec(3 * 70000, 0.5f);
+  for (const auto& c : {std::pair<int, int>{4, 64 * 32}, {4, 64 * 32 + 1}, {10, 4000}, {10, 20000}, {12, 60000}, {3, 800},
+                        {3, 2000}, {3, 2048}}) {
+    aq_hash* h = nullptr;
+    REQUIRE(aq_hash_create(c.first, c.first, c.first, 1.f, c.second, &h) == AQ_OK);
+    const long long before = fake::count["radix"];
+    REQUIRE(aq_hash_sort_host(h, rec.data(), c.second, 3, nullptr, nullptr, nullptr, nullptr, 0, nullptr) == AQ_OK);
+    const int cells = c.first * c.first * c.first;
+    REQUIRE(fake::count["radix"] - before == (c.second >= 2048 && c.second > 32 * cells));
+    aq_hash_destroy(h);
+  }
+}
+
 // A sort that runs out of memory while its buffers grow leaves none of the old ones in use.
 void hash_after_failed_growth() {
   const auto sort = [](aq_hash* h, const float* rec, long long n) {
@@ -296,6 +312,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"sort_by_density", sort_by_density},
     {"network_after_failed_growth", network_after_failed_growth},
     {"kept_blocks_stay_on_their_device", kept_blocks_stay_on_their_device},
     {"kept_memory_is_given_back", kept_memory_is_given_back},

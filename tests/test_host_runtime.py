@@ -22,6 +22,7 @@ def host_cases(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", [
+    "sort_by_density",
     "network_after_failed_growth",
     "kept_blocks_stay_on_their_device",
     "kept_memory_is_given_back",

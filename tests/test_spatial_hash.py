@@ -260,3 +260,13 @@ def test_gpu_more_output_words_than_one_launch_has_work_items():
     cell = rec[:, :3].floor().long()
     h = ((cell[:, 0] * side + cell[:, 1]) * side + cell[:, 2])[perm.long()]
     assert bool((h[1:] >= h[:-1]).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,n", [((10, 10, 11), 40_001), ((24, 25, 26), 530_001), ((64, 64, 65), 8_600_003)])
+def test_gpu_crowded_grids_of_two_and_three_digits(sizes, n):
+    """More than 32 records per cell on grids whose hashes take two radix digits (both tile
+    sizes) and three."""
+    rng = np.random.default_rng(n)
+    rec = rng.uniform(0, 1, (n, 3)).astype(np.float32) * np.array(sizes, np.float32)
+    gpu_case(sizes, 1.0, rec)
