@@ -41,9 +41,11 @@ aq_status fail(aq_status s, const std::string& msg) {
 #define HIP_TRY(expr)                                                                         \
   do {                                                                                        \
     hipError_t e_ = (expr);                                                                   \
-    if (e_ != hipSuccess)                                                                     \
+    if (e_ != hipSuccess) {                                                                   \
+      (void)hipGetLastError(); /* reported here, not by the next call */                      \
       return fail(e_ == hipErrorOutOfMemory ? AQ_ENOMEM : AQ_EHIP,                            \
                   std::string(#expr) + ": " + hipGetErrorString(e_));                         \
+    }                                                                                         \
   } while (0)
 
 #define AQ_TRY(expr)              \
@@ -1310,7 +1312,10 @@ aq_status plan_seeding(const aq_flip_config& cfg, SeedPlan* plan) {
   }
   if (d_counts) hipFree(d_counts);
   hipStreamDestroy(s);
-  if (e != hipSuccess) return fail(AQ_EHIP, std::string("seeding: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(AQ_EHIP, std::string("seeding: ") + hipGetErrorString(e));
+  }
   if (plan->total > (1ll << 31) - 1) return fail(AQ_EINVAL, "too many particles");
   return AQ_OK;
 }
@@ -1331,7 +1336,10 @@ aq_status write_seeded(aq_flip* h, const SeedPlan& plan) {
     }
   }
   hipFree(d_off);
-  if (e != hipSuccess) return fail(AQ_EHIP, std::string("seeding: ") + hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(AQ_EHIP, std::string("seeding: ") + hipGetErrorString(e));
+  }
   return AQ_OK;
 }
 

@@ -24,9 +24,11 @@ aq_status hfail(aq_status s, const std::string& m) {
 #define HHIP(expr)                                                                            \
   do {                                                                                        \
     hipError_t e_ = (expr);                                                                   \
-    if (e_ != hipSuccess)                                                                     \
+    if (e_ != hipSuccess) {                                                                   \
+      (void)hipGetLastError(); /* reported here, not by the next call */                      \
       return hfail(e_ == hipErrorOutOfMemory ? AQ_ENOMEM : AQ_EHIP,                           \
                    std::string(#expr) + ": " + hipGetErrorString(e_));                        \
+    }                                                                                         \
   } while (0)
 
 #define HTRY(expr)               \

@@ -32,12 +32,14 @@ aq_status ufail(aq_status s, const std::string& m) {
   return s;
 }
 
-#define UHIP(expr)                                                                              \
-  do {                                                                                          \
-    hipError_t e_ = (expr);                                                                     \
-    if (e_ != hipSuccess)                                                                       \
-      return ufail(e_ == hipErrorOutOfMemory ? AQ_ENOMEM : AQ_EHIP,                            \
-                   std::string(#expr) + ": " + hipGetErrorString(e_));                          \
+#define UHIP(expr)                                                                            \
+  do {                                                                                        \
+    hipError_t e_ = (expr);                                                                   \
+    if (e_ != hipSuccess) {                                                                   \
+      (void)hipGetLastError(); /* reported here, not by the next call */                      \
+      return ufail(e_ == hipErrorOutOfMemory ? AQ_ENOMEM : AQ_EHIP,                           \
+                   std::string(#expr) + ": " + hipGetErrorString(e_));                        \
+    }                                                                                         \
   } while (0)
 #define UTRY(expr)               \
   do {                           \

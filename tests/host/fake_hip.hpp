@@ -113,7 +113,7 @@ inline void launch(const char* name, hipStream_t s, Work w = [] {}) {
 // ---- the runtime
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
-  if (fake::used(fake::device) + n > fake::capacity) return hipErrorOutOfMemory;
+  if (fake::used(fake::device) + n > fake::capacity) return fake::last_error = hipErrorOutOfMemory;
   *p = std::malloc(n);
   std::memset(*p, 0xcd, n);
   fake::live[(char*)*p] = {n, fake::device};
