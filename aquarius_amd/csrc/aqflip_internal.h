@@ -162,7 +162,8 @@ struct ExportField {
   bool face;           // the face extent instead of the interior
   const void* src[4];  // kVector: the components, null = 0
 };
-void launch_export_field(const Geom& G, const ExportField& f, long long n, void* out, hipStream_t s);
+// Elements first .. first + n - 1.
+void launch_export_field(const Geom& G, const ExportField& f, long long first, long long n, void* out, hipStream_t s);
 // Standalone spatial hashing (records of `stride` floats, position first).
 void launch_hash_records(const Geom& G, const float* pos, long long n, int stride, Bins B, hipStream_t s);
 void launch_scatter_segsort(const Geom& G, long long n, Bins B, hipStream_t s);

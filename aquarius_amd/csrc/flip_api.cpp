@@ -199,8 +199,10 @@ struct aq_flip {
   aq_flip_solver solver{AQ_SOLVE_FIXED, 1e-4, 100000, 50, 20, 0};
   aq_unet* net = nullptr;
   aq_flip_solver_stats sstats{};
-  void* export_buf = nullptr;  // scratch of field exports larger than a particle array
+  // Scratch of field exports beyond a particle array, at most kExportBytes.
+  void* export_buf = nullptr;
   size_t export_cap = 0;
+  static constexpr size_t kExportBytes = 32 << 20;
   float* p_keep = nullptr;  // the iterate before a U-Net correction (allocated on first use)
 
   bool timing = false;
@@ -1654,19 +1656,23 @@ aq_status aq_flip_get_field(aq_flip* h, int32_t field, void* dst, size_t bytes) 
       f.kind = ExportField::kVector;
       for (int a = 0; a < h->K; ++a) f.src[a] = field == AQ_FIELD_VOLUME_FRACTIONS ? gr.vf[a] : gr.nvf[h->nf][a];
   }
-  // scratch: an array of the idle particle buffer (see aq_flip_get_particles) if it is large
-  // enough, else one of its own, kept
-  void* scratch = h->P[h->cur ^ 1].a;
-  if (bytes > (size_t)h->Np * sizeof(float4)) {
-    if (bytes > h->export_cap) {
-      AQ_TRY(h->alloc(&h->export_buf, bytes));
-      h->export_cap = bytes;
-    }
-    scratch = h->export_buf;
+  // Scratch: an array of the idle particle buffer (see aq_flip_get_particles), or one of its
+  // own, kept, where that is small; a field larger than it is exported in pieces.
+  const size_t elem = w * 4, particles = (size_t)h->Np * sizeof(float4);
+  char* scratch = (char*)h->P[h->cur ^ 1].a;
+  size_t cap = particles;
+  if (const size_t want = std::min(bytes, aq_flip::kExportBytes); particles < want) {
+    void* p = nullptr;
+    if (h->export_cap < want && h->alloc(&p, want) == AQ_OK) h->export_buf = p, h->export_cap = want;
+    if (h->export_cap > cap) scratch = (char*)h->export_buf, cap = h->export_cap;  // (else out of memory: make do)
   }
-  launch_export_field(h->G, f, (long long)n, scratch, h->stream);
-  HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpyAsync(dst, scratch, bytes, hipMemcpyDeviceToHost, h->stream));
+  for (size_t done = 0; done < n;) {
+    const size_t m = std::min(n - done, cap / elem);
+    launch_export_field(h->G, f, (long long)done, (long long)m, scratch, h->stream);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync((char*)dst + done * elem, scratch, m * elem, hipMemcpyDeviceToHost, h->stream));
+    done += m;
+  }
   HIP_TRY(hipStreamSynchronize(h->stream));
   return AQ_OK;
 }

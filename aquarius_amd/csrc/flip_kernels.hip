@@ -141,14 +141,16 @@ void launch_export_particles(Particles P, long long Np, int K, float* pos, float
     default: hipLaunchKernelGGL(k_export_particles<4>, grid, block, 0, s, P, Np, pos, vel, frac); break;
   }
 }
-// A grid field over the interior or (face) the face extent, z fastest.
-__global__ void k_export_field(Geom G, ExportField f, int n, uint32_t* __restrict__ out) {
-  const int o = (int)(blockIdx.x * kBlock + threadIdx.x);
-  if (o >= n) return;
+// n elements of a grid field from element `first` on, over the interior or (face) the face
+// extent, z fastest.
+__global__ void k_export_field(Geom G, ExportField f, int first, int n, uint32_t* __restrict__ out) {
+  const int i = (int)(blockIdx.x * kBlock + threadIdx.x);
+  if (i >= n) return;
+  const int o = first + i;
   if (f.kind == ExportField::kCount) {  // cellEnd - cellStart (Fluid/Fluid_3D_FLIP.cu:180)
     const int* off = (const int*)f.src[0];
     const int c = off[o + 1] - off[o];
-    out[o] = c > 0 ? c - 1 : 0;
+    out[i] = c > 0 ? c - 1 : 0;
     return;
   }
   int x, y, z;
@@ -158,21 +160,21 @@ __global__ void k_export_field(Geom G, ExportField f, int n, uint32_t* __restric
     cell_of(G, o, x, y, z);
   const long long g = G.g(x, y, z);
   if (f.kind == ExportField::kByte) {
-    out[o] = ((const uint8_t*)f.src[0])[g];
+    out[i] = ((const uint8_t*)f.src[0])[g];
   } else if (f.kind == ExportField::kBits) {  // bits 0-2 as int4
     const uint32_t v = ((const uint8_t*)f.src[0])[g];
-    ((uint4*)out)[o] = make_uint4(v & 1, (v >> 1) & 1, (v >> 2) & 1, 0);
+    ((uint4*)out)[i] = make_uint4(v & 1, (v >> 1) & 1, (v >> 2) & 1, 0);
   } else if (f.kind == ExportField::kScalar) {
-    out[o] = ((const uint32_t*)f.src[0])[g];
+    out[i] = ((const uint32_t*)f.src[0])[g];
   } else {  // up to four components, 0 where there is no array
     uint32_t v[4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) v[a] = f.src[a] ? ((const uint32_t*)f.src[a])[g] : 0u;
-    ((uint4*)out)[o] = make_uint4(v[0], v[1], v[2], v[3]);
+    ((uint4*)out)[i] = make_uint4(v[0], v[1], v[2], v[3]);
   }
 }
-void launch_export_field(const Geom& G, const ExportField& f, long long n, void* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_export_field, dim3(nblocks(n)), dim3(kBlock), 0, s, G, f, (int)n, (uint32_t*)out);
+void launch_export_field(const Geom& G, const ExportField& f, long long first, long long n, void* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_export_field, dim3(nblocks(n)), dim3(kBlock), 0, s, G, f, (int)first, (int)n, (uint32_t*)out);
 }
 
 // ------------------------------------------------------------------ hashing

@@ -285,6 +285,13 @@ uint32_t* launch_radix_sort(const Geom&, const float*, long long n, int, const R
 void launch_hash_outputs(long long, int, const HashSorted&, const float*, int*, int*, float*, hipStream_t s) {
   launch("outputs", s);
 }
+void launch_export_field(const Geom&, const ExportField& f, long long first, long long n, void* out, hipStream_t s) {
+  launch("export_field", s, [=] {
+    const size_t w = f.kind == ExportField::kVector || f.kind == ExportField::kBits ? 4 : 1;
+    fake::check(out, n * w * 4);
+    for (long long i = 0; i < n; ++i) std::fill_n((int*)out + i * w, w, (int)(first + i));
+  });
+}
 #define AQ_FAKE(name, ...) \
   void launch_##name(__VA_ARGS__, hipStream_t s) { launch(#name, s); }
 void launch_seed_count(const SeedVolume&, const SeedParams&, long long nc, int* counts, hipStream_t s) {
@@ -294,7 +301,6 @@ AQ_FAKE(seed_write, const SeedVolume&, const SeedParams&, long long, const int*,
 AQ_FAKE(hash_count, const Geom&, Particles, long long, Bins)
 AQ_FAKE(scatter_sort_gather, const Geom&, Particles, Particles, long long, int, Bins)
 AQ_FAKE(export_particles, Particles, long long, int, float*, float*, float4*)
-AQ_FAKE(export_field, const Geom&, const ExportField&, long long, void*)
 AQ_FAKE(p2g, const Geom&, Particles, long long, int, Bins, Grid, int, int, int, StepParams)
 AQ_FAKE(gravity_boundary, const Geom&, Grid, int, StepParams, int, int)
 AQ_FAKE(divergence, const Geom&, Grid, int, Bins)

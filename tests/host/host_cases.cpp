@@ -297,6 +297,23 @@ void network_after_failed_growth() {
   aq_unet_destroy(net);
 }
 
+// An export takes a bounded scratch buffer at most, and works without any memory left.
+void exports_need_little_memory() {
+  for (bool room : {true, false}) {
+    aq_flip* f = create(config(130), room ? 64 : 5000);
+    fake::capacity = fake::used(0) + (room ? 33 << 20 : 0);
+    for (int field : {AQ_FIELD_PRESSURE, AQ_FIELD_VELOCITY, AQ_FIELD_HAS_VELOCITY}) {
+      std::vector<int> out(aq_flip_field_bytes(f, field) / 4, -1);
+      REQUIRE(aq_flip_get_field(f, field, out.data(), out.size() * 4) == AQ_OK);
+      const size_t w = field == AQ_FIELD_PRESSURE ? 1 : 4;
+      for (size_t i = 0; i < out.size(); ++i) REQUIRE(out[i] == (int)(i / w));  // as the stand-in fills them
+    }
+    fake::capacity = (size_t)-1;
+    aq_flip_destroy(f);
+    aq_flip_release_memory();
+  }
+}
+
 // What a failed MG-PCG solve has left on the stream does not answer for the next one.
 void mgpcg_after_a_failed_solve() {
   aq_flip* f = create(config(16));
@@ -312,6 +329,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"exports_need_little_memory", exports_need_little_memory},
     {"sort_by_density", sort_by_density},
     {"network_after_failed_growth", network_after_failed_growth},
     {"kept_blocks_stay_on_their_device", kept_blocks_stay_on_their_device},

@@ -683,3 +683,21 @@ def test_timed_small_steps_keep_the_bits(pressure_iters, diffusion_iters):
         h.close()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+def test_fields_larger_than_the_export_scratch():
+    """130^3 cells and 64 particles: velocities (36 MB) and their flags (35 MB) leave in two
+    pieces of at most 32 MiB. What was uploaded comes back."""
+    n = 130
+    cfg = configs.make_config(n, dt=0.01, pressure_iters=4)
+    rng = np.random.default_rng(61)
+    h = FlipHandle(cfg, pos=(rng.uniform(0.3, 0.7, (64, 3)) * 10).astype(np.float32))
+    vel = rng.standard_normal((n + 1, n + 1, n + 1, 4)).astype(np.float32)
+    vel[..., 3] = 0
+    flags = rng.integers(0, 2, (n, n, n, 4)).astype(np.int32)
+    flags[..., 3] = 0
+    h.set_field("velocity", vel)
+    h.set_field("has_velocity", flags)
+    assert np.array_equal(h.get_field("velocity").view(np.uint32), vel.view(np.uint32))
+    assert np.array_equal(h.get_field("has_velocity"), flags)
+    h.close()

@@ -22,6 +22,7 @@ def host_cases(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", [
+    "exports_need_little_memory",
     "sort_by_density",
     "network_after_failed_growth",
     "kept_blocks_stay_on_their_device",
