@@ -208,6 +208,37 @@ void launch_fill_pressure_zero(const Geom& G, Grid gr, int pb, hipStream_t s);
 // cells and AIR cells are skipped -- valid once both buffers hold 0 on AIR.
 // pzero = 1: the input is the zero guess (not read); needs full = 1.
 void launch_jacobi(const Geom& G, Grid gr, int pin, int full, int pzero, hipStream_t s);
+// The tiles of launch_jacobi_tile: 8 x 8 cells in x and y, 8 or 24 in z.
+constexpr int kTile = 8;
+// Long tiles from here on. Microseconds per sweep with short / long tiles: 64^3 1.20 / 1.60,
+// 96^3 1.50 / 1.70 (25 % FLUID) and 3.58 / 3.11 (90 %), 112^3 2.49 / 2.10 and 5.14 / 3.87.
+constexpr int kTileLongCells = 1 << 20;
+struct TileGeom {
+  int ny, nz, n, runs;  // tiles in y, in z, all; 4-cell runs per thread (1: z 8, 2: z 24)
+  FastDiv dny, dnz;
+};
+inline TileGeom tile_geom(const Geom& G) {
+  TileGeom T;
+  T.runs = G.ncells_hash >= kTileLongCells ? 2 : 1;
+  const int tz = 16 * T.runs - 8;
+  T.ny = (G.Y + kTile - 1) / kTile;
+  T.nz = (G.Z + tz - 1) / tz;
+  T.n = (G.X + kTile - 1) / kTile * T.ny * T.nz;
+  T.dny = make_fastdiv((uint32_t)T.ny);
+  T.dnz = make_fastdiv((uint32_t)T.nz);
+  return T;
+}
+// Whether sweeps take less time on tiles than one per launch: a thin grid fills little of
+// its tiles, which costs nothing while they are few (a launch then takes what one tile takes)
+// but decides the time of many. Microseconds per 100 sweeps, single / tiles, FLUID nearly
+// everywhere: short tiles 256 x 256 x 1 444 / 228, 512 x 512 x 1 561 / 631, x 2 581 / 630, x 3
+// 690 / 634; long ones 512 x 512 x 4 541 / 932, x 8 801 / 1,000, x 12 907 / 978, x 16
+// 1,074 / 1,071; 1024 x 1024 x 1 1,987 / 3,575, x 8 2,549 / 3,702, x 16 5,997 / 4,526.
+inline bool tile_fits(const Geom& G) {
+  const TileGeom T = tile_geom(G);
+  const long long padded = (long long)T.n * kTile * kTile * (16 * T.runs - 8), cells = G.ncells_hash;
+  return T.runs == 1 ? padded <= 3 << 19 || padded <= 3 * cells : 5 * padded <= 8 * cells;
+}
 // tile_sweeps() sweeps from gr.p[pin] to gr.p[pin ^ 1]; same flags. AIR or FLUID cells only.
 void launch_jacobi_tile(const Geom& G, Grid gr, int pin, int full, int pzero, hipStream_t s);
 int tile_sweeps();

@@ -584,10 +584,11 @@ void jacobi_sweeps(aq_flip* h, int n, bool from_zero = false) {
     h->air_clean[h->pb] = true;
     return;
   }
+  const bool tiles = h->p2g_content && tile_fits(h->G);
   for (int i = 0; i < n;) {
     const int out = h->pb ^ 1;
     const bool z = from_zero && i == 0, full = z || !h->air_clean[out];
-    if (h->p2g_content && n - i >= tile_sweeps() && (!full || tile_full(h->G))) {
+    if (tiles && n - i >= tile_sweeps() && (!full || tile_full(h->G))) {
       launch_jacobi_tile(h->G, h->gr, h->pb, full ? 1 : 0, z ? 1 : 0, h->stream);
       i += tile_sweeps();
     } else {

@@ -1257,26 +1257,6 @@ __device__ __forceinline__ void mark_active(const Grid& gr, bool fluid) {
   if (threadIdx.x == 0) gr.active[xcd_block()] = any ? 1 : 0;
 }
 
-// The tiles of k_jacobi_tile: 8 x 8 cells in x and y, 8 or 24 in z.
-constexpr int kTile = 8;
-// Long tiles from here on. Microseconds per sweep with short / long tiles: 64^3 1.20 / 1.60,
-// 96^3 1.50 / 1.70 (25 % FLUID) and 3.58 / 3.11 (90 %), 112^3 2.49 / 2.10 and 5.14 / 3.87.
-constexpr int kTileLongCells = 1 << 20;
-struct TileGeom {
-  int ny, nz, n, runs;  // tiles in y, in z, all; 4-cell runs per thread (1: z 8, 2: z 24)
-  FastDiv dny, dnz;
-};
-TileGeom tile_geom(const Geom& G) {
-  TileGeom T;
-  T.runs = G.ncells_hash >= kTileLongCells ? 2 : 1;
-  const int tz = 16 * T.runs - 8;
-  T.ny = (G.Y + kTile - 1) / kTile;
-  T.nz = (G.Z + tz - 1) / tz;
-  T.n = (G.X + kTile - 1) / kTile * T.ny * T.nz;
-  T.dny = make_fastdiv((uint32_t)T.ny);
-  T.dnz = make_fastdiv((uint32_t)T.nz);
-  return T;
-}
 __device__ __forceinline__ int tile_of(const TileGeom& T, int x, int y, int z) {
   return ((x / kTile) * T.ny + y / kTile) * T.nz + (T.runs == 1 ? z / 8 : z / 24);
 }

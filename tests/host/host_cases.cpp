@@ -314,6 +314,29 @@ void exports_need_little_memory() {
   }
 }
 
+// Sweeps run on tiles where the grid fills them or needs few of them.
+void tiles_fit_the_grid() {
+  struct Case {
+    int x, y, z;
+    bool fits;
+  };
+  for (const Case& c : {Case{33, 33, 33, true}, {64, 64, 64, true}, {100, 100, 100, true}, {130, 130, 65, true},
+                        {256, 256, 256, true}, {256, 256, 1, true}, {1, 256, 256, true}, {1024, 8, 8, true},
+                        {512, 512, 3, true}, {512, 512, 1, false}, {512, 512, 2, false}, {512, 512, 4, false},
+                        {512, 512, 12, false}, {512, 512, 16, true}, {1024, 1024, 1, false}, {1024, 1, 1024, false},
+                        {1024, 1024, 8, false}, {1024, 1024, 16, true}, {1024, 1024, 1024, true}}) {
+    aqf::Geom G{};
+    G.X = c.x, G.Y = c.y, G.Z = c.z, G.ncells_hash = c.x * c.y * c.z;
+    REQUIRE(aqf::tile_fits(G) == c.fits);
+  }
+  aq_flip_config c = config(512);
+  c.size[2] = 2;
+  aq_flip* f = create(c);
+  REQUIRE(aq_flip_run_stage(f, AQ_STAGE_PRESSURE) == AQ_OK);
+  REQUIRE(fake::count["tile"] == 0 && fake::count["jacobi"] == c.pressure_iters);
+  aq_flip_destroy(f);
+}
+
 // What a failed MG-PCG solve has left on the stream does not answer for the next one.
 void mgpcg_after_a_failed_solve() {
   aq_flip* f = create(config(16));
@@ -329,6 +352,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"tiles_fit_the_grid", tiles_fit_the_grid},
     {"exports_need_little_memory", exports_need_little_memory},
     {"sort_by_density", sort_by_density},
     {"network_after_failed_growth", network_after_failed_growth},
