@@ -228,6 +228,17 @@ inline TileGeom tile_geom(const Geom& G) {
   T.dnz = make_fastdiv((uint32_t)T.nz);
   return T;
 }
+inline int sweep_tiles(const Geom& G) { return tile_geom(G).n; }
+// Workgroups of a launch over the listed tiles: kTileGrid, or where there are fewer tiles one
+// for each, in groups of the XCDs' number. (Rounded down, 27 or 125 full tiles left some
+// workgroups two: steps of 20^3 and 40^3 cells, two phases mixing, took 439 and 521 us, now
+// 292 and 365.)
+constexpr int kXCD = 8;
+constexpr int kTileGrid = 512;
+inline int tile_grid(const Geom& G) {
+  const int n = sweep_tiles(G), up = (n + kXCD - 1) / kXCD * kXCD;
+  return n < kXCD ? n : up < kTileGrid ? up : kTileGrid;
+}
 // Whether sweeps take less time on tiles than one per launch: a thin grid fills little of
 // its tiles, which costs nothing while they are few (a launch then takes what one tile takes)
 // but decides the time of many. Microseconds per 100 sweeps, single / tiles, FLUID nearly
@@ -248,8 +259,6 @@ bool tile_full(const Geom& G);  // full = 1 is taken
 bool tile_pairs(const Geom& G, int K);
 void launch_tile_pair(const Geom& G, Grid gr, int K, int pin, int fin, float lambda, double inv_cc, int launch,
                       int skip_ok, hipStream_t s);
-int sweep_tiles(const Geom& G);
-int tile_grid(const Geom& G);
 // All sweeps of a step in one launch, on grids that fit in a workgroup's LDS (K channel sets).
 bool small_grid(const Geom& G, int K);
 void launch_sweeps_small(const Geom& G, Grid gr, int K, int pb, int pzero, int nj, int nf, float lambda, double inv_cc,

@@ -17,7 +17,6 @@
 namespace aqf {
 
 constexpr int kBlock = 256;
-constexpr int kXCD = 8;
 
 // Workgroups of a launch are dispatched round-robin over the 8 XCDs. Map the
 // hardware block id so that each XCD walks one contiguous range of logical
@@ -1499,12 +1498,6 @@ __global__ __launch_bounds__(kListThreads) void k_active_list(int nchunks, const
   if (threadIdx.x == 0) dchange[0] = 0u;  // the first paired sweep of the next step records here
 }
 int sweep_grid(const Geom& G, bool full, int listed);
-int sweep_tiles(const Geom& G) { return tile_geom(G).n; }
-constexpr int kTileGrid = 512;
-int tile_grid(const Geom& G) {
-  const int n = sweep_tiles(G);
-  return n < kXCD ? n : std::min(n, kTileGrid) / kXCD * kXCD;
-}
 void launch_active_list(const Geom& G, Grid gr, hipStream_t s) {
   const TileLists T{gr.tactive, gr.tlist, gr.ttab, sweep_tiles(G), tile_grid(G)};
   hipLaunchKernelGGL(k_active_list, dim3(2), dim3(kListThreads), 0, s, sweep_chunks(G), gr.active, gr.alist,

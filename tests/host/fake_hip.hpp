@@ -250,8 +250,6 @@ void launch_fill_pressure_zero(const Geom& G, Grid gr, int pb, hipStream_t s) {
 }
 int sweep_chunks(const Geom& G) { return (G.ncells_hash + 511) / 512; }
 int sweep_table_entries(const Geom&) { return 64; }
-int sweep_tiles(const Geom& G) { return (G.ncells_hash + 511) / 512; }
-int tile_grid(const Geom& G) { return sweep_tiles(G); }
 void set_listed_grids(const Geom&, Grid&, int) {}
 int seed_block_size() { return 256; }
 void launch_hash_records(const Geom&, const float* rec, long long n, int stride, Bins B, hipStream_t s) {

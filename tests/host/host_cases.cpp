@@ -314,6 +314,16 @@ void exports_need_little_memory() {
   }
 }
 
+// Every tile has a workgroup of its own as long as there are enough, in whole groups.
+void one_workgroup_per_tile() {
+  for (int n : {1, 8, 9, 16, 17, 20, 28, 33, 40, 50, 56, 64, 72, 101}) {
+    aqf::Geom G{};
+    G.X = G.Y = G.Z = n, G.ncells_hash = n * n * n;
+    const int tiles = aqf::sweep_tiles(G), grid = aqf::tile_grid(G);
+    REQUIRE(grid <= 512 && (grid == 512 || grid >= tiles) && grid < tiles + 8 && (grid < 8 || grid % 8 == 0));
+  }
+}
+
 // Sweeps run on tiles where the grid fills them or needs few of them.
 void tiles_fit_the_grid() {
   struct Case {
@@ -352,6 +362,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"one_workgroup_per_tile", one_workgroup_per_tile},
     {"tiles_fit_the_grid", tiles_fit_the_grid},
     {"exports_need_little_memory", exports_need_little_memory},
     {"sort_by_density", sort_by_density},

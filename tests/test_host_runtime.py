@@ -22,6 +22,7 @@ def host_cases(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", [
+    "one_workgroup_per_tile",
     "tiles_fit_the_grid",
     "exports_need_little_memory",
     "sort_by_density",
