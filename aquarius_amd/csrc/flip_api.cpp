@@ -188,6 +188,7 @@ struct aq_flip {
   // air_clean[i]: pressure buffer i holds 0 on every AIR cell of the current content.
   bool air_clean[2] = {false, false};
   bool p2g_content = false;  // every interior cell is AIR or FLUID (see content_changed)
+  long long fluid = 0;       // FLUID cells to expect (see expect_fluid)
   Bins B{};
   StepParams sp{};
   int nparts_red = 0;
@@ -380,14 +381,24 @@ int channels_for(const aq_flip_config& c, const float* frac4, long long n) {
 }
 
 // Positions must hash into the grid (calcHashImpl would index out of range otherwise).
-aq_status check_positions(const aq_flip* h, const float* pos, long long n) {
+// cells: how many cells they lie in, where a choice of kernels depends on it (below 2^20 cells),
+// else 0.
+aq_status check_positions(const aq_flip* h, const float* pos, long long n, long long* cells) {
   const int S[3] = {h->G.X, h->G.Y, h->G.Z};
-  for (long long i = 0; i < n; ++i)
+  std::vector<bool> seen(h->G.ncells_hash < kTileLongCells ? (size_t)h->G.ncells_hash : 0);
+  *cells = 0;
+  for (long long i = 0; i < n; ++i) {
+    int c[3];
     for (int a = 0; a < 3; ++a) {
       const float v = pos[3 * i + a];
-      if (!(v >= 0.f) || (int)(v / h->G.h) >= S[a])
+      if (!(v >= 0.f) || (c[a] = (int)(v / h->G.h)) >= S[a])
         return fail(AQ_EINVAL, "particle " + std::to_string(i) + " lies outside the grid");
     }
+    if (seen.empty()) continue;
+    const size_t at = ((size_t)c[0] * S[1] + c[1]) * S[2] + c[2];
+    *cells += !seen[at];
+    seen[at] = true;
+  }
   return AQ_OK;
 }
 
@@ -564,19 +575,19 @@ void stage_transfer(aq_flip* h) {
 // clearing first.
 //
 // Small grids run all n sweeps in one launch, in place. One workgroup per chain does the
-// work, so the rule weighs the FLUID cells (times K with the diffusion chain beside it),
-// taken from the seeding density of 8 particles per cell, against tile launches of four
-// sweeps. Microseconds per step, one launch / tiles, sweep counts in brackets: 16^3 with 1,160
+// work, so the rule weighs the FLUID cells to expect (times K with the diffusion chain beside
+// it) against tile launches of four sweeps. Microseconds per step, one launch / tiles, sweep counts in brackets: 16^3 with 1,160
 // FLUID cells 109/164 (100), 81/86 (16), with 3,900 146/170 (100); 24^3 with 3,900 165/175
 // (100), 102/94 (16); 27^3 with 5,600 205/177 (100). Both chains, 100 sweeps each, K = 2: 16^3
 // with 1,160 107/175, with 3,900 and phases mixing 286/296, 18^3 with 5,500 608/464; K = 4,
 // mixing: 12^3 with 1,640 403/430, 16^3 with 3,900 587/440.
 constexpr int kSmallSweeps = 16;
 constexpr long long kSmallPressure = 4096, kSmallPaired = 8192;
+bool small_cells(const aq_flip* h, int K) {
+  return small_grid(h->G, K) && (K > 1 ? h->fluid * K <= kSmallPaired : h->fluid <= kSmallPressure);
+}
 bool small_sweeps(const aq_flip* h, int n, int K) {
-  const long long fluid = std::min((long long)h->G.ncells_hash, (h->Np + 7) / 8);
-  return n >= kSmallSweeps && h->p2g_content && small_grid(h->G, K) &&
-         (K > 1 ? fluid * K <= kSmallPaired : fluid <= kSmallPressure);
+  return n >= kSmallSweeps && h->p2g_content && small_cells(h, K);
 }
 void jacobi_sweeps(aq_flip* h, int n, bool from_zero = false) {
   if (small_sweeps(h, n, 1)) {
@@ -1171,6 +1182,23 @@ void drop_graphs(aq_flip* h) {
   h->graphs.clear();
 }
 
+// FLUID cells to expect: those that hold particles now, or what the particles fill at the
+// seeding density of 8 per cell if that is more. Captured launches that the choice of kernels
+// would no longer make are dropped. (27^3 cells with one particle in each, 100 sweeps a step:
+// 340 us with a sweep per launch, 550 in one launch as 8 per cell let expect, now 166.)
+void expect_fluid(aq_flip* h, long long cells) {
+  const auto routes = [h] { return (small_cells(h, 1) ? 1 : 0) | (small_cells(h, h->K) ? 2 : 0); };
+  const int before = routes();
+  h->fluid = std::min((long long)h->G.ncells_hash, std::max(cells, (h->Np + 7) / 8));
+  if (routes() == before) return;
+  drop_graphs(h);
+  for (auto& g : h->sweep_graphs) {
+    hipGraphExecDestroy(g.exec);
+    hipGraphDestroy(g.graph);
+  }
+  h->sweep_graphs.clear();
+}
+
 void state_of(const aq_flip* h, int k[7]) {
   k[0] = h->cur, k[1] = h->nv, k[2] = h->hv, k[3] = h->pb, k[4] = h->nf;
   k[5] = h->air_clean[0], k[6] = h->air_clean[1];
@@ -1365,11 +1393,14 @@ aq_status create_common(const aq_flip_config* cfg, const float* pos, const float
   aq_status st = setup(h, cfg, n);
   if (plan) {  // seeded on the device: positions are clamped into the domain by construction
     h->K = channels_for(*cfg, nullptr, 0);
+    if (st == AQ_OK) expect_fluid(h, 0);
     if (st == AQ_OK) st = write_seeded(h, *plan);
   } else {
-    if (st == AQ_OK) st = check_positions(h, pos, n);
+    long long cells = 0;
+    if (st == AQ_OK) st = check_positions(h, pos, n, &cells);
     if (st == AQ_OK) {
       h->K = channels_for(*cfg, frac4, n);
+      expect_fluid(h, cells);
       st = upload_particles(h, pos, vel, frac4);
     }
   }
@@ -1618,10 +1649,12 @@ aq_status aq_flip_set_particles(aq_flip* h, const float* pos, const float* vel, 
                                 int64_t n) {
   if (!h || !pos) return fail(AQ_EINVAL, "null argument");
   if (n != h->Np) return fail(AQ_EINVAL, "particle count differs from the handle's");
-  AQ_TRY(check_positions(h, pos, n));
+  long long cells = 0;
+  AQ_TRY(check_positions(h, pos, n, &cells));
   const int K = std::max(h->K, channels_for(h->cfg, frac4, n));
   if (K != h->K) drop_graphs(h);
   h->K = K;
+  expect_fluid(h, cells);
   return upload_particles(h, pos, vel, frac4);
 }
 
@@ -2009,6 +2042,12 @@ aq_status aq_flip_load(const char* path, aq_flip** out) {
     if (!ok || hipMemcpy(a.ptr, buf.data(), a.bytes, hipMemcpyHostToDevice) != hipSuccess) {
       delete h;
       return bail(AQ_EINVAL, "truncated snapshot section " + std::to_string(a.tag));
+    }
+    if (a.ptr == h->B.offsets) {  // as the particles were binned last
+      const int* off = (const int*)buf.data();
+      long long cells = 0;
+      for (int c = 0; c < h->G.ncells_hash; ++c) cells += off[c + 1] > off[c];
+      expect_fluid(h, cells);
     }
   }
   std::fclose(f);

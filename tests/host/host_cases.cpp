@@ -314,6 +314,41 @@ void exports_need_little_memory() {
   }
 }
 
+// Whether a small grid's sweeps run in one launch goes by the cells that hold particles, however
+// few there are in each, through uploads and snapshots.
+void sparse_particles_on_small_grids() {
+  const int n = 24;
+  aq_flip_config c = config(n);
+  c.diffusion_iters = 0;
+  const float h = c.grid_physical_size / n;
+  std::vector<float> everywhere, corner;
+  for (int i = 0; i < n * n * n; ++i)
+    for (int a : {i / (n * n), i / n % n, i % n}) {
+      everywhere.push_back(h * ((float)a + 0.5f));
+      corner.push_back(h * ((float)(a % 8) + 0.5f));
+    }
+  const auto one_launch = [](aq_flip* f) {
+    const long long small = fake::count["small"];
+    REQUIRE(aq_flip_steps(f, 3) == AQ_OK && fake::pending() == 0);
+    return fake::count["small"] > small;
+  };
+  aq_flip* f = nullptr;
+  REQUIRE(aq_flip_create_with_particles(&c, everywhere.data(), nullptr, nullptr, n * n * n, &f) == AQ_OK);
+  REQUIRE(!one_launch(f));  // 13,824 cells
+  REQUIRE(aq_flip_set_particles(f, corner.data(), nullptr, nullptr, n * n * n) == AQ_OK);
+  REQUIRE(one_launch(f));  // 512 cells; 1,728 at eight per cell
+  REQUIRE(aq_flip_set_particles(f, everywhere.data(), nullptr, nullptr, n * n * n) == AQ_OK);
+  REQUIRE(!one_launch(f));
+  aq_flip_destroy(f);
+  // a snapshot counts the cells of its bins (the stand-in bins nothing: none hold particles)
+  REQUIRE(aq_flip_create_with_particles(&c, everywhere.data(), nullptr, nullptr, n * n * n, &f) == AQ_OK);
+  (void)saved(f, "sparse");
+  aq_flip_destroy(f);
+  REQUIRE(aq_flip_load((dir + "/sparse").c_str(), &f) == AQ_OK);
+  REQUIRE(one_launch(f));
+  aq_flip_destroy(f);
+}
+
 // Every tile has a workgroup of its own as long as there are enough, in whole groups.
 void one_workgroup_per_tile() {
   for (int n : {1, 8, 9, 16, 17, 20, 28, 33, 40, 50, 56, 64, 72, 101}) {
@@ -362,6 +397,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"sparse_particles_on_small_grids", sparse_particles_on_small_grids},
     {"one_workgroup_per_tile", one_workgroup_per_tile},
     {"tiles_fit_the_grid", tiles_fit_the_grid},
     {"exports_need_little_memory", exports_need_little_memory},
