@@ -250,13 +250,25 @@ inline bool tile_fits(const Geom& G) {
   const long long padded = (long long)T.n * kTile * kTile * (16 * T.runs - 8), cells = G.ncells_hash;
   return T.runs == 1 ? padded <= 3 << 19 || padded <= 3 * cells : 5 * padded <= 8 * cells;
 }
+// Whether a step's paired sweeps take less time on tiles, with `fluid` FLUID cells. Where the
+// phases mix, all diffusion sweeps are computed, borders too, and the tiles' workgroups (two to
+// a CU with two phases, one with more, half of them for the pressure) should come to no more
+// than two rounds. Microseconds a step of 100 pairs, one pair a launch / tiles, mixing, tiles
+// with FLUID in brackets: K = 2 56^3 768 / 573 (326), 64^3 676 / 682 (486), 72^3 919 / 997
+// (692), 90^3 1,109 / 1,339 (920), 256 x 4 x 256 661 / 930 (1,024); K = 3 40^3 695 / 443
+// (125), 48^3 557 / 532 (205), 50^3 771 / 816 (326), 80^3 659 / 833 (300); K = 4 48^3
+// 586 / 605 (205), 50^3 830 / 964 (326). Apart, with one diffusion launch computed: 64^3
+// 368 / 254 (154), K = 4 375 / 269.
+inline bool tile_pairs(const Geom& G, int K, long long fluid) {
+  const TileGeom T = tile_geom(G);
+  return T.runs == 1 && T.n * fluid <= (K == 2 ? 512LL : 256LL) * G.ncells_hash;
+}
 // tile_sweeps() sweeps from gr.p[pin] to gr.p[pin ^ 1]; same flags. AIR or FLUID cells only.
 void launch_jacobi_tile(const Geom& G, Grid gr, int pin, int full, int pzero, hipStream_t s);
 int tile_sweeps();
 bool tile_full(const Geom& G);  // full = 1 is taken
 // tile_sweeps() pressure and diffusion sweeps in one launch (K >= 2, AIR cells as `full` = 0
 // asks); `launch` as `sweep` of launch_jacobi_diffusion.
-bool tile_pairs(const Geom& G, int K);
 void launch_tile_pair(const Geom& G, Grid gr, int K, int pin, int fin, float lambda, double inv_cc, int launch,
                       int skip_ok, hipStream_t s);
 // All sweeps of a step in one launch, on grids that fit in a workgroup's LDS (K channel sets).

@@ -666,7 +666,7 @@ void fused_pressure_diffusion(aq_flip* h) {
   for (int i = 0; i < n && !small; ++launch) {
     const int out = h->pb ^ 1;
     const bool z = zero && i == 0, full = z || !h->air_clean[out];
-    if (i > 0 && !full && n - i >= tile_sweeps() && tile_pairs(h->G, h->K)) {
+    if (i > 0 && !full && n - i >= tile_sweeps() && tile_pairs(h->G, h->K, h->fluid)) {
       launch_tile_pair(h->G, h->gr, h->K, h->pb, h->nf, h->sp.lambda, h->sp.inv_cc, launch, h->skip_fixed ? 1 : 0,
                        h->stream);
       i += tile_sweeps();
@@ -1187,7 +1187,9 @@ void drop_graphs(aq_flip* h) {
 // would no longer make are dropped. (27^3 cells with one particle in each, 100 sweeps a step:
 // 340 us with a sweep per launch, 550 in one launch as 8 per cell let expect, now 166.)
 void expect_fluid(aq_flip* h, long long cells) {
-  const auto routes = [h] { return (small_cells(h, 1) ? 1 : 0) | (small_cells(h, h->K) ? 2 : 0); };
+  const auto routes = [h] {
+    return (small_cells(h, 1) ? 1 : 0) | (small_cells(h, h->K) ? 2 : 0) | (tile_pairs(h->G, h->K, h->fluid) ? 4 : 0);
+  };
   const int before = routes();
   h->fluid = std::min((long long)h->G.ncells_hash, std::max(cells, (h->Np + 7) / 8));
   if (routes() == before) return;

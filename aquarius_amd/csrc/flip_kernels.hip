@@ -2526,10 +2526,6 @@ __global__ __launch_bounds__(kTileThreads, K <= 2 ? 8 : 4) void k_tile_pair(
                                  (int)(k == 0 ? e.z : k == 1 ? e.w : list[1 + e.y + k * nj]), m);
   if (__ballot(changed) && (threadIdx.x & 63) == 0) dchange[launch % 3] = 1u;
 }
-// Computing diffusion in tiles costs its border too, which outweighs the launches on larger
-// grids and with more phases: mixing 96^3, K = 2 817 -> 799 us, but K = 4 984 -> 1,256;
-// 64^3, K = 4 608 -> 624 (apart: 392 -> 269).
-bool tile_pairs(const Geom& G, int K) { return tile_geom(G).runs == 1 && (long long)K * G.ncells_hash < 7 << 18; }
 void launch_tile_pair(const Geom& G, Grid gr, int K, int pin, int fin, float lambda, double inv_cc, int launch,
                       int skip_ok, hipStream_t s) {
   const TileGeom T = tile_geom(G);

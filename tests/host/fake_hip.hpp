@@ -232,7 +232,6 @@ void launch_jacobi(const Geom&, Grid gr, int pin, int, int, hipStream_t s) {
 }
 int tile_sweeps() { return 4; }
 bool tile_full(const Geom&) { return true; }
-bool tile_pairs(const Geom&, int) { return true; }
 void launch_jacobi_tile(const Geom&, Grid gr, int pin, int, int, hipStream_t s) {
   launch("tile", s, [=] { gr.p[pin ^ 1][0] = gr.p[pin][0] + 4; });
 }

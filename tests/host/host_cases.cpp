@@ -349,6 +349,24 @@ void sparse_particles_on_small_grids() {
   aq_flip_destroy(f);
 }
 
+// Paired sweeps run on tiles where those that hold FLUID are few, by the number of phases.
+void paired_tiles_by_fluid() {
+  struct Case {
+    int x, y, z, phases;
+    double fluid;
+    bool tiles;
+  };
+  for (const Case& c : {Case{33, 33, 33, 4, 0.95, true}, {48, 48, 48, 4, 0.95, true}, {50, 50, 50, 4, 0.95, false},
+                        {48, 48, 48, 3, 0.95, true}, {50, 50, 50, 3, 0.95, false}, {50, 50, 50, 3, 0.3, true},
+                        {80, 80, 80, 3, 0.3, false}, {64, 64, 64, 2, 0.95, true}, {72, 72, 72, 2, 0.95, false},
+                        {72, 72, 72, 2, 0.3, true}, {90, 90, 90, 2, 0.53, false}, {256, 4, 256, 2, 1.0, false},
+                        {101, 101, 101, 2, 0.1, true}, {102, 102, 102, 2, 0.1, false}}) {
+    aqf::Geom G{};
+    G.X = c.x, G.Y = c.y, G.Z = c.z, G.ncells_hash = c.x * c.y * c.z;
+    REQUIRE(aqf::tile_pairs(G, c.phases, (long long)(c.fluid * G.ncells_hash)) == c.tiles);
+  }
+}
+
 // Every tile has a workgroup of its own as long as there are enough, in whole groups.
 void one_workgroup_per_tile() {
   for (int n : {1, 8, 9, 16, 17, 20, 28, 33, 40, 50, 56, 64, 72, 101}) {
@@ -397,6 +415,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"paired_tiles_by_fluid", paired_tiles_by_fluid},
     {"sparse_particles_on_small_grids", sparse_particles_on_small_grids},
     {"one_workgroup_per_tile", one_workgroup_per_tile},
     {"tiles_fit_the_grid", tiles_fit_the_grid},
