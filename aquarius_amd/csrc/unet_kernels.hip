@@ -58,8 +58,9 @@ __device__ __forceinline__ long long vox_id(const Vol& v, int b, int d, int h, i
 // the volume. M = voxels, N = COUT, K = 27*CIN in slices of 32.
 //
 // k_conv3 gathers its input per tap from memory, one fragment of 16 voxels and one
-// 16-channel output tile per wave: the reference for k_conv3_tile's forward pass, run
-// only under AQUNET_NO_TILE=1 (read at every launch).
+// 16-channel output tile per wave: for extents that would leave most of k_conv3_tile's tiles
+// empty (conv3_tile_fits), and the reference for its forward pass, run at every extent under
+// AQUNET_NO_TILE=1 (read at every launch).
 static bool conv3_tile_enabled() {
   const char* e = std::getenv("AQUNET_NO_TILE");
   return !(e && e[0] == '1');
@@ -369,6 +370,16 @@ static void conv3_tile_pick(const Vol& v, const __bf16* X, int xs, int xo, const
     conv3_tile_launch<CIN, COUT, CH, 1, 1, EPI>(v, X, xs, xo, Wk, out, s);
 }
 
+// Whether a layer's forward pass takes less time on tiles of 8 x 16 rows and columns: not where
+// over half of their voxels lie outside and these come to more than the launch itself costs.
+// Whole networks, us, gathered / tiled: 1 x 4096 x 4 x 4 271 / 585, 1 x 256 x 256 x 4 528 / 784,
+// 1 x 96 x 96 x 4 388 / 433, 1 x 64 x 64 x 4 272 / 249, 1 x 256 x 4 x 4 195 / 149, 1 x 128 x 128 x 8
+// 364 / 346, 1 x 256 x 256 x 12 1,156 / 1,037.
+static bool conv3_tile_fits(const Vol& v, int cin, int cout) {
+  const long long rows = (long long)v.B * v.D, padded = rows * ((v.H + 7) / 8 * 8) * ((v.W + 15) / 16 * 16);
+  return padded <= 2 * rows * v.H * v.W || padded * cin * cout <= 1 << 26;
+}
+
 // Layers with more than 32 input channels are staged in chunks where the extents divide
 // into tiles, and whole otherwise: the two orders of k that the forward pass has always
 // had there.
@@ -376,7 +387,7 @@ template <int CIN, int COUT>
 static void conv3_fwd_t(const Vol& v, const __bf16* X, int xs, int xo, const __bf16* Wk,
                         const float* bias, __bf16* Y, int ys, int yo, hipStream_t s) {
   constexpr int CH = CIN <= 32 ? CIN : CIN % 32 == 0 ? 32 : 16;
-  if (!conv3_tile_enabled()) {
+  if (!conv3_tile_enabled() || !conv3_tile_fits(v, CIN, COUT)) {
     const long long V = (long long)v.B * v.D * v.H * v.W;
     hipLaunchKernelGGL((k_conv3<CIN, COUT>), dim3((unsigned)((V + 63) / 64), COUT / 16), dim3(256), 0, s, v, X, xs,
                        xo, Wk, bias, Y, ys, yo);

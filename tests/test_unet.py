@@ -171,6 +171,19 @@ def test_tiled_forward_matches_untiled(monkeypatch, shape):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 2048, 4, 4), (1, 96, 96, 4), (2, 160, 8, 8), (1, 64, 4, 64)])
+def test_forward_of_thin_extents_matches_untiled(monkeypatch, shape):
+    """Extents that fill little of a tile, where a layer is tiled or gathered by its own
+    size: the same products in the same order, so the same bits as gathered throughout."""
+    from aquarius_amd.unet import UNet
+    net = UNet(seed=23)
+    x, _, _ = random_problem(*shape, seed=8)
+    y = net.forward(x)
+    monkeypatch.setenv("AQUNET_NO_TILE", "1")
+    assert np.array_equal(y.view(np.uint32), net.forward(x).view(np.uint32))
+
+
+@pytest.mark.gpu
 def test_gradients_match_oracle():
     from aquarius_amd.unet import UNet
     net = UNet(seed=11)
