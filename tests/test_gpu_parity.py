@@ -701,3 +701,23 @@ def test_fields_larger_than_the_export_scratch():
     assert np.array_equal(h.get_field("velocity").view(np.uint32), vel.view(np.uint32))
     assert np.array_equal(h.get_field("has_velocity"), flags)
     h.close()
+
+
+@pytest.mark.parametrize("extent,phases", [((33, 33, 33), 1), ((40, 40, 25), 3), ((40, 40, 26), 3), ((34, 33, 33), 1)])
+def test_exports_on_both_sides_of_the_small_sizes(extent, phases):
+    """Every export where a field or the particles are small enough to be rearranged on the
+    host (up to 40,000 elements and 4,096 particles), and just above: against the oracle."""
+    n = 4096 if extent[2] == 33 else 4097
+    cfg = configs.make_config(0, dt=0.01, pressure_iters=8, diffusion_iters=4, phase_count=phases, extent=extent)
+    rng = np.random.default_rng(n)
+    pos = (rng.uniform(0.2, 0.8, (n, 3)) * np.array(extent) * (10 / extent[1])).astype(np.float32)
+    vel = rng.standard_normal((n, 3)).astype(np.float32)
+    frac = np.zeros((n, 4), np.float32)
+    frac[np.arange(n), rng.integers(0, phases, n)] = 1
+    gpu, orc = FlipHandle(cfg, pos, vel, frac), ob.Oracle(cfg, pos=pos, vel=vel, frac4=frac)
+    gpu.step()
+    orc.step()
+    for name in aq.FIELDS:
+        check_field(name, gpu, orc)
+    check_particles(gpu, orc)
+    gpu.close()
