@@ -93,10 +93,16 @@ struct aq_hash {
   //   3 M in 44^3       (35)         353 / 209   129 / 138   107 / 138
   //   20,000 in 8^3     (39)          94 / 33     90 / 33     68 / 33
   //   1 M in 20^3       (125)        625 / 94    560 / 90    508 / 89
-  // so the line lies at 32 records per cell, where segments outgrow the sort in registers. (A
-  // million unordered records and more would gain below it too, but ordered ones would lose
-  // as much or more, and the order is not known here.)
-  bool crowded(long long n) const { return n >= 2048 && n > 32LL * G.ncells_hash; }
+  // so the line lies at 32 records per cell, where segments outgrow the sort in registers.
+  // Below it the order decides, which is not known here (a sample of it costs 20 us). Large
+  // sorts of wide records go by radix too: there it is the quicker one out of order and, in
+  // order, still quicker than a thread per record was (1 M records of 48 bytes in 50^3 cells,
+  // counting / radix / a thread per record: unordered and not in cache 155 / 126 / 423, in
+  // order 60 / 96 / 149; of 16 bytes in order 46 / 84 / 65).
+  bool crowded(long long n, int stride) const {
+    if (n < 2048) return false;
+    return n > 32LL * G.ncells_hash || (stride >= 12 && n >= 3 << 18 && n >= 4LL * G.ncells_hash);
+  }
   aq_status ensure_radix(long long n) {
     if (!vals2) HTRY(alloc(&vals2, (size_t)cap, per_particle));
     const size_t c = std::max(radix_counts(cap), radix_counts(std::min<long long>(cap, (1 << 19) - 1)));
@@ -125,7 +131,7 @@ struct aq_hash {
                 float* sorted, hipStream_t s) {
     counting = false;
     HTRY(ensure(n));
-    if (crowded(n)) {
+    if (crowded(n, stride)) {
       HTRY(ensure_radix(n));
       const RadixBufs R{{(uint32_t*)B.hash, (uint32_t*)B.rank}, {B.perm, vals2}, rcounts, roffsets, rpartials};
       if (start) launch_fill_u32(start, 0xffffffffu, G.ncells_hash, s);

@@ -73,18 +73,22 @@ void hash_after_a_failed_sort() {
   aq_hash_destroy(h);
 }
 
-// Records are sorted by radix only where the cells are crowded: below that the counting sort
-// is the faster one for records that come nearly sorted.
+// Records are sorted by radix only where the cells are crowded or the records many and wide:
+// elsewhere the counting sort is the faster one for records that come nearly sorted.
 void sort_by_density() {
-  const std::vector<float> rec(3 * 70000, 0.5f);
-  for (const auto& c : {std::pair<int, int>{4, 64 * 32}, {4, 64 * 32 + 1}, {10, 4000}, {10, 20000}, {12, 60000}, {3, 800},
-                        {3, 2000}, {3, 2048}}) {
+  struct Case {
+    int side, n, stride;
+    bool radix;
+  };
+  const std::vector<float> rec(12 * 786432, 0.5f);
+  for (const Case& c : {Case{4, 64 * 32, 3, false}, {4, 64 * 32 + 1, 3, true}, {10, 4000, 3, false}, {10, 20000, 12, false},
+                        {12, 60000, 3, true}, {3, 800, 3, false}, {3, 2000, 3, false}, {3, 2048, 3, true},
+                        {40, 786432, 8, false}, {40, 786432, 12, true}, {40, 786431, 12, false}, {59, 786432, 12, false}}) {
     aq_hash* h = nullptr;
-    REQUIRE(aq_hash_create(c.first, c.first, c.first, 1.f, c.second, &h) == AQ_OK);
+    REQUIRE(aq_hash_create(c.side, c.side, c.side, 1.f, c.n, &h) == AQ_OK);
     const long long before = fake::count["radix"];
-    REQUIRE(aq_hash_sort_host(h, rec.data(), c.second, 3, nullptr, nullptr, nullptr, nullptr, 0, nullptr) == AQ_OK);
-    const int cells = c.first * c.first * c.first;
-    REQUIRE(fake::count["radix"] - before == (c.second >= 2048 && c.second > 32 * cells));
+    REQUIRE(aq_hash_sort_host(h, rec.data(), c.n, c.stride, nullptr, nullptr, nullptr, nullptr, 0, nullptr) == AQ_OK);
+    REQUIRE(fake::count["radix"] - before == c.radix);
     aq_hash_destroy(h);
   }
 }

@@ -263,6 +263,14 @@ def test_gpu_more_output_words_than_one_launch_has_work_items():
 
 
 @pytest.mark.gpu
+def test_gpu_many_wide_records():
+    """800,003 records of 48 bytes, 13 per cell: by radix, in tiles of the larger size."""
+    rng = np.random.default_rng(71)
+    rec = rng.uniform(0, 39, (800_003, 12)).astype(np.float32)
+    gpu_case((39, 40, 39), 1.0, rec)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("sizes,n", [((10, 10, 11), 40_001), ((24, 25, 26), 530_001), ((64, 64, 65), 8_600_003)])
 def test_gpu_crowded_grids_of_two_and_three_digits(sizes, n):
     """More than 32 records per cell on grids whose hashes take two radix digits (both tile
