@@ -284,9 +284,10 @@ void launch_extrapolate(const Geom& G, Grid gr, int nvin, int hvin, bool near_ro
 // gr.nvo from newVelocity buffer nv and velocity, every face.
 void launch_build_nvo(const Geom& G, Grid gr, int nv, hipStream_t s);
 // full = 1: AIR cells copied to the output buffer; full = 0: AIR cells and blocks
-// without FLUID skipped -- valid once both buffers agree on AIR cells. sweep > 0: the
-// sweep of that number after paired ones, skipped once one has changed nothing.
-void launch_diffusion(const Geom& G, Grid gr, int K, int fin, float lambda, double inv_cc, int full, int sweep,
+// without FLUID skipped -- valid once both buffers agree on AIR cells. last >= 0: the sweep is
+// skipped if the one recorded under that number (paired launches record under theirs) has
+// changed nothing; mark >= 0: it is recorded under that one, the next after `last`.
+void launch_diffusion(const Geom& G, Grid gr, int K, int fin, float lambda, double inv_cc, int full, int last, int mark,
                       hipStream_t s);
 // One Jacobi sweep (p[pin] -> p[pin^1]) and one diffusion sweep (nvf[fin] ->
 // nvf[fin^1]) in one launch; fullJ / fullD as `full` above.

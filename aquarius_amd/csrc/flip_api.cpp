@@ -639,11 +639,16 @@ void stage_extrapolate(aq_flip* h, bool in_step = false) {
 }
 
 // Diffusion sweeps first..diffusion_iters-1 of the step (first > 0: after `launch` paired
-// launches).
+// launches). After paired sweeps every kRecordEvery-th, the first among them, records whether
+// it changed a bit, under the next launch's number.
+constexpr int kRecordEvery = 4;
 void diffusion_sweeps(aq_flip* h, hipStream_t s, int first = 0, int launch = 0) {
-  for (int i = first; i < h->cfg.diffusion_iters; ++i, ++launch) {  // the first sweep also copies AIR cells across
-    launch_diffusion(h->G, h->gr, h->K, h->nf, h->sp.lambda, h->sp.inv_cc, i == 0 ? 1 : 0,
-                     first > 0 && h->skip_fixed ? launch : 0, s);
+  const bool chained = first > 0 && h->skip_fixed;
+  for (int i = first; i < h->cfg.diffusion_iters; ++i) {  // the first sweep also copies AIR cells across
+    const bool record = chained && (i - first) % kRecordEvery == 0;
+    launch_diffusion(h->G, h->gr, h->K, h->nf, h->sp.lambda, h->sp.inv_cc, i == 0 ? 1 : 0, chained ? launch - 1 : -1,
+                     record ? launch : -1, s);
+    launch += record;
     h->nf ^= 1;
   }
 }

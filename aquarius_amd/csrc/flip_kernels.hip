@@ -2141,32 +2141,38 @@ __device__ __forceinline__ bool diffusion_cell(const Geom& G, const Grid& gr, in
   return changed;
 }
 
-// sweep > 0: the sweep continues a step's chain of paired ones (see k_jacobi_diffusion) and
-// is skipped like those, once a sweep has changed nothing. Steps of 30 pressure and 100
-// diffusion sweeps, two phases, before -> after: apart 64^3 478 -> 332 us, 128^3 1,283 -> 999;
-// mixing (no sweep skipped) 33^3 400 -> 425, 64^3 543 -> 554, 128^3 1,329 -> 1,302.
+// chained: *last says whether the step's last recorded diffusion sweep changed a bit (see
+// k_jacobi_diffusion); if it did not, neither would this one, and it is skipped. mark, unless
+// null: where this one records that; next, the word after it, is cleared. Recording costs
+// a store by every wave at its end, 0.2 - 0.4 us a sweep, so the host asks for it every fourth
+// sweep. Steps of 1 pressure and 41 diffusion sweeps, two phases, us, never skipped / recorded
+// by every sweep / by every fourth: mixing 16^3 171 / 186 / 172, 33^3 203 / 218 / 205, 64^3
+// 305 / 311 / 297, 128^3 856 / 881 / 850; apart 168 / 132 / 136, 187 / 146 / 150, 282 / 206 /
+// 209, 857 / 731 / 728.
 template <int K>
-__global__ void k_diffusion(Geom G, Grid gr, int fin, float lambda, double inv_cc, int full, int sweep) {
+__global__ void k_diffusion(const uint32_t* __restrict__ active, const uint32_t* __restrict__ last,
+                            uint32_t* __restrict__ mark, uint32_t* __restrict__ next, int chained, int full, Geom G,
+                            Grid gr, int fin, float lambda, double inv_cc) {
   // Both words, of the step's chain and of the block, in one round trip.
-  const uint32_t prev = gr.dchange[(sweep + 2) % 3], act = gr.active[xcd_block()];
+  const uint32_t prev = *last, act = active[xcd_block()];
   asm volatile("" ::"s"(prev), "s"(act));
-  if (sweep > 0) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) st_wt(&gr.dchange[(sweep + 1) % 3], 0u);
-    if (prev == 0u) return;
-  }
-  if (!full && !act) return;
+  if (mark && blockIdx.x == 0 && threadIdx.x == 0) st_wt(next, 0u);
+  if ((chained && prev == 0u) || (!full && !act)) return;
   const int n = gtid();
   const bool changed = n < G.ncells_hash && diffusion_cell<K>(G, gr, fin, lambda, inv_cc, n, full);
-  if (sweep > 0 && __ballot(changed) && (threadIdx.x & 63) == 0) gr.dchange[sweep % 3] = 1u;
+  if (mark && __ballot(changed) && (threadIdx.x & 63) == 0) *mark = 1u;
 }
-void launch_diffusion(const Geom& G, Grid gr, int K, int fin, float lambda, double inv_cc, int full, int sweep,
+void launch_diffusion(const Geom& G, Grid gr, int K, int fin, float lambda, double inv_cc, int full, int last, int mark,
                       hipStream_t s) {
   const dim3 grid(nblocks(G.ncells_hash)), block(kBlock);
+  const uint32_t* l = gr.dchange + (last >= 0 ? last % 3 : 0);
+  uint32_t *m = mark >= 0 ? gr.dchange + mark % 3 : nullptr, *x = gr.dchange + (mark + 1) % 3;
+  const int ch = last >= 0 ? 1 : 0;
   switch (K) {
-    case 1: hipLaunchKernelGGL(k_diffusion<1>, grid, block, 0, s, G, gr, fin, lambda, inv_cc, full, sweep); break;
-    case 2: hipLaunchKernelGGL(k_diffusion<2>, grid, block, 0, s, G, gr, fin, lambda, inv_cc, full, sweep); break;
-    case 3: hipLaunchKernelGGL(k_diffusion<3>, grid, block, 0, s, G, gr, fin, lambda, inv_cc, full, sweep); break;
-    default: hipLaunchKernelGGL(k_diffusion<4>, grid, block, 0, s, G, gr, fin, lambda, inv_cc, full, sweep); break;
+    case 1: hipLaunchKernelGGL(k_diffusion<1>, grid, block, 0, s, gr.active, l, m, x, ch, full, G, gr, fin, lambda, inv_cc); break;
+    case 2: hipLaunchKernelGGL(k_diffusion<2>, grid, block, 0, s, gr.active, l, m, x, ch, full, G, gr, fin, lambda, inv_cc); break;
+    case 3: hipLaunchKernelGGL(k_diffusion<3>, grid, block, 0, s, gr.active, l, m, x, ch, full, G, gr, fin, lambda, inv_cc); break;
+    default: hipLaunchKernelGGL(k_diffusion<4>, grid, block, 0, s, gr.active, l, m, x, ch, full, G, gr, fin, lambda, inv_cc); break;
   }
 }
 

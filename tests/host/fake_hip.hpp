@@ -243,7 +243,7 @@ bool small_grid(const Geom& G, int) { return G.ncells_hash <= 20000; }
 void launch_sweeps_small(const Geom&, Grid gr, int, int pb, int, int nj, int, float, double, int, int, int, hipStream_t s) {
   launch("small", s, [=] { gr.p[pb][0] += (float)nj; });
 }
-void launch_diffusion(const Geom&, Grid, int, int, float, double, int, int, hipStream_t s) { launch("diffusion", s); }
+void launch_diffusion(const Geom&, Grid, int, int, float, double, int, int, int, hipStream_t s) { launch("diffusion", s); }
 void launch_fill_pressure_zero(const Geom& G, Grid gr, int pb, hipStream_t s) {
   launch("pressure_zero", s, [=, n = G.ncell] { std::fill_n(gr.p[pb], n, 0.f); });
 }

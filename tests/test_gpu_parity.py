@@ -721,3 +721,25 @@ def test_exports_on_both_sides_of_the_small_sizes(extent, phases):
         check_field(name, gpu, orc)
     check_particles(gpu, orc)
     gpu.close()
+
+
+@pytest.mark.parametrize("coefficient", [0.05, 1e-5])
+@pytest.mark.parametrize("extent,rest", [((33, 17, 26), 1), ((33, 17, 26), 4), ((33, 17, 26), 9), ((64, 24, 40), 22)])
+def test_diffusion_sweeps_after_the_paired_ones(monkeypatch, extent, rest, coefficient):
+    """Diffusion sweeps beyond the pressure's, every fourth of which records whether it
+    changed anything so that later ones can be skipped, give the bits of the sequential
+    order: phases that mix, and ones that have settled after a few sweeps."""
+    cfg = configs.make_config(0, dt=0.01, extent=extent, pressure_iters=6, diffusion_iters=6 + rest, radius=0.2,
+                              center=(0.5, 0.2, 0.5), sphere_phase=1, phase_count=2, diffusion_coeff=coefficient,
+                              seed=67)
+    pos, frac = ob.seed(cfg)
+    out = []
+    for flag in ("1", "0"):
+        monkeypatch.setenv("AQFLIP_NO_FUSE", flag)
+        monkeypatch.setenv("AQFLIP_NO_OVERLAP", flag)
+        h = FlipHandle(cfg, pos=pos, frac4=frac)
+        h.steps(4)
+        out.append([h.get_field(f).view(np.uint32) for f in ("pressure", "new_volume_fractions")])
+        h.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
