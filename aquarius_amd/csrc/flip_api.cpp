@@ -582,9 +582,11 @@ void stage_transfer(aq_flip* h) {
 // with 1,160 107/175, with 3,900 and phases mixing 286/296, 18^3 with 5,500 608/464; K = 4,
 // mixing: 12^3 with 1,640 403/430, 16^3 with 3,900 587/440.
 constexpr int kSmallSweeps = 16;
-constexpr long long kSmallPressure = 4096, kSmallPaired = 8192;
+// With four phases the line lies lower for the sake of a longer diffusion chain, whose rest is
+// quicker in launches of its own (30 + 100 sweeps, 1,210 FLUID cells mixing: 394/364).
+constexpr long long kSmallPressure = 4096, kSmallPaired = 8192, kSmallPaired4 = 4500;
 bool small_cells(const aq_flip* h, int K) {
-  return small_grid(h->G, K) && (K > 1 ? h->fluid * K <= kSmallPaired : h->fluid <= kSmallPressure);
+  return small_grid(h->G, K) && (K > 1 ? h->fluid * K <= (K < 4 ? kSmallPaired : kSmallPaired4) : h->fluid <= kSmallPressure);
 }
 bool small_sweeps(const aq_flip* h, int n, int K) {
   return n >= kSmallSweeps && h->p2g_content && small_cells(h, K);

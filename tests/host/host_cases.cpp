@@ -371,6 +371,18 @@ void paired_tiles_by_fluid() {
   }
 }
 
+// With four phases fewer FLUID cells take the one launch.
+void four_phases_on_small_grids() {
+  for (int phases : {2, 3, 4}) {
+    aq_flip_config c = config(16, phases);
+    aq_flip* f = create(c, 8 * 1300);
+    const long long small = fake::count["small"];
+    REQUIRE(aq_flip_step(f) == AQ_OK);
+    REQUIRE((fake::count["small"] > small) == (phases < 4));
+    aq_flip_destroy(f);
+  }
+}
+
 // Every tile has a workgroup of its own as long as there are enough, in whole groups.
 void one_workgroup_per_tile() {
   for (int n : {1, 8, 9, 16, 17, 20, 28, 33, 40, 50, 56, 64, 72, 101}) {
@@ -419,6 +431,7 @@ void mgpcg_after_a_failed_solve() {
 }
 
 const std::map<std::string, void (*)()> cases = {
+    {"four_phases_on_small_grids", four_phases_on_small_grids},
     {"paired_tiles_by_fluid", paired_tiles_by_fluid},
     {"sparse_particles_on_small_grids", sparse_particles_on_small_grids},
     {"one_workgroup_per_tile", one_workgroup_per_tile},

@@ -22,6 +22,7 @@ def host_cases(tmp_path_factory):
 
 
 @pytest.mark.parametrize("name", [
+    "four_phases_on_small_grids",
     "paired_tiles_by_fluid",
     "sparse_particles_on_small_grids",
     "one_workgroup_per_tile",
