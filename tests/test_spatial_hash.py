@@ -263,6 +263,25 @@ def test_gpu_more_output_words_than_one_launch_has_work_items():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000, 70_001])
+@pytest.mark.parametrize("order", ["sorted", "pairs", "random", "one cell last"])
+def test_gpu_runs_of_equal_hashes(n, order):
+    """Runs of records in one cell of every length within a wave, across waves, and up to the
+    end of a last wave that is not full."""
+    rng = np.random.default_rng(n)
+    sizes = (23, 9, 11)
+    cell = rng.integers(0, 23 * 9 * 11, n)
+    if order in ("sorted", "one cell last"):
+        cell.sort()
+    if order == "pairs":
+        cell = np.repeat(cell[:(n + 1) // 2], 2)[:n]
+    if order == "one cell last":
+        cell[-(n // 3 + 1):] = 5
+    xyz = np.stack([cell // 99, cell // 11 % 9, cell % 11], 1) + rng.uniform(0.1, 0.9, (n, 3))
+    gpu_case(sizes, 1.0, xyz.astype(np.float32))
+
+
+@pytest.mark.gpu
 def test_gpu_many_wide_records():
     """800,003 records of 48 bytes, 13 per cell: by radix, in tiles of the larger size."""
     rng = np.random.default_rng(71)
