@@ -85,10 +85,10 @@ struct aq_hash {
   // sorted, as they do from a step that sorted them before, but its segments' sorts grow with
   // the records per cell. us per call, counting / radix, for 16-byte records in random order,
   // moved a little since the last sort, and sorted:
-  //   1 M in 50^3 cells (8 a cell)   113 / 104    48 / 83     46 / 84
-  //   3 M in 80^3       (6)          312 / 210    86 / 158    79 / 156
-  //   300,000 in 30^3   (11)          56 / 74     36 / 71     37 / 73
-  //   100,000 in 16^3   (24)          47 / 76     36 / 74     36 / 74
+  //   1 M in 50^3 cells (8 a cell)   113 / 104    47 / 83     45 / 84
+  //   3 M in 80^3       (6)          312 / 210    81 / 158    74 / 156
+  //   300,000 in 30^3   (11)          56 / 74     37 / 71     36 / 73
+  //   100,000 in 16^3   (24)          46 / 76     38 / 74     34 / 74
   //   1 M in 30^3       (37)         174 / 97    104 / 88     81 / 89
   //   3 M in 44^3       (35)         353 / 209   129 / 138   107 / 138
   //   20,000 in 8^3     (39)          94 / 33     90 / 33     68 / 33

@@ -73,7 +73,8 @@ aq_status aq_hash_sort_device(aq_hash* h, const float* d_records, int64_t n, int
  * in one static device array of 69 MB that every GPU the library runs on holds until
  * the process ends, so it takes at most 2,097,152 cells (size_x*size_y*size_z) and
  * 4,194,304 records; larger requests fail with AQ_EINVAL. Inputs, outputs, cell_count
- * and stream ordering are those of aq_hash_sort_device. Every call on one GPU shares
+ * and stream ordering are those of aq_hash_sort_device; it always takes the counting
+ * sort, which crowded cells slow down. Every call on one GPU shares
  * that GPU's array: calls that overlap on one GPU (other host threads, other streams)
  * race and must be serialised by the caller. */
 aq_status aq_hash_sort_device_noalloc(int32_t size_x, int32_t size_y, int32_t size_z, float cell_size,
